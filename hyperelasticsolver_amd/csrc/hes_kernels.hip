@@ -12,6 +12,7 @@
 // A 64-lane wave owns a tile of 62 cells plus one halo cell on each side, so
 // neighbour exchange is a lane shuffle and needs no LDS or barrier.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -23,6 +24,7 @@
 #include "hes_device.hpp"
 #include "hes_faces.hpp"
 #include "hes_host.hpp"
+#include "hes_resident.hpp"
 #include "hes_step.hpp"
 #include "../../include/hes.h"
 
@@ -145,6 +147,48 @@ __attribute__((amdgpu_waves_per_eu(NPH == 1 ? HES_STEP_WAVES_PER_EU : HES_STEP2_
   constexpr bool NOC = NPH == 1 && FLUX == FLUX_RUSANOV && PIN != 0;
   double lam = chunk_step<NPH, FLUX, FAST, PB, PIN != 0, SRC != 0, NOC>(ctx, i, q, cc, lmax);
   step_epilogue(a, lam, tcur, lmax);
+}
+
+// ---------------------------------------------------------------------------
+// Time loop of a small problem in one launch (hes_resident.hpp)
+// ---------------------------------------------------------------------------
+struct ResArgs {
+  ResTeam team;                // all but its rank
+  unsigned long long* slots;   // the handle's rings, left as k_step expects them
+  double* tring;
+  unsigned long long* jcnt;
+  ResOut* out;
+  long long step0;
+  MatDev mat[2];
+};
+
+// Shape of a team's workgroups: threads, and tiles of 64 cells that a wave holds.
+struct ResShape {
+  int block, tiles;
+};
+constexpr int RES_MAX_TEAM = 256;  // workgroups
+
+template <int FLUX, int FAST, int BLK, int T>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(BLK / 256)))
+void k_resident(ResArgs a) {
+  ResTeam tm = a.team;
+  tm.rank = (int)xcd_block();  // neighbours on one XCD
+  const ResOut o = resident_run1<FLUX, FAST, BLK, T, RES_MAX_TEAM>(tm, a.mat[0]);
+  if (tm.rank == 0 && threadIdx.x == 0) {
+    *a.out = o;
+    if (o.ok) {
+      const long long s = a.step0 + o.steps;
+      a.slots[s % 3] = (unsigned long long)__double_as_longlong(o.lmax);
+      a.slots[(s + 1) % 3] = 0ull;
+      a.slots[(s + 2) % 3] = 0ull;
+      a.tring[0] = o.t;
+      a.tring[1] = o.t;
+      if (a.jcnt) {
+        a.jcnt[0] = 0ull;
+        a.jcnt[1] = 0ull;
+      }
+    }
+  }
 }
 
 // Two phases: the faces with a volume-fraction jump of the step's input state,
@@ -499,6 +543,16 @@ struct hes_solver {
   hipStream_t stream;
   hipEvent_t ev0, ev1;
   bool has_state;
+  // the time loop in one launch (run_resident), for problems that fit the chip
+  int dev, cus;
+  ResShape shape;            // block 0: one launch per step
+  int res_g, res_own;        // workgroups and cells of each
+  unsigned long long* comm;  // their slots, then their halo words
+  unsigned res_tag;          // the last tag written there
+  struct ResMail {           // page-locked, written by the launch
+    ResOut out;
+    int status[4];
+  }* mail;
 };
 
 namespace {
@@ -627,6 +681,205 @@ int init_speeds(hes_solver* h) {
   return HES_OK;
 }
 
+// At most max_steps steps, one launch (for two phases one sequence) each.
+// Launches are issued in chunks of `chunk` steps (captured once into a
+// hipGraph when use_graph is set); with an end time the executed-step counter
+// is read back after each chunk.  Adds to *ms the time of the launches.
+int run_launches(hes_solver* h, long long max_steps, double t_end, int use_graph, double* hist,
+                 long long* steps_done, float* ms, int* bad) {
+  const long long chunk = 60;  // multiple of 6: ring phases repeat per chunk
+  HIP_TRY(hipMemsetAsync(h->status + 1, 0, sizeof(int), h->stream));
+  hipGraphExec_t gexec = nullptr;
+  hipGraph_t graph = nullptr;
+  long long graph_base = -1;  // step (mod 6) the captured graph starts from
+  long long launched = 0, done = 0;
+  const long long s0 = h->step;
+  HIP_TRY(hipEventRecord(h->ev0, h->stream));
+  int rc = HES_OK;
+  while (launched < max_steps) {
+    long long k = max_steps - launched < chunk ? max_steps - launched : chunk;
+    long long sb = s0 + launched;
+    bool graph_ok = use_graph && k == chunk && !hist;
+    if (graph_ok) {
+      if (!gexec || (graph_base % 6) != (sb % 6)) {
+        if (gexec) { (void)hipGraphExecDestroy(gexec); gexec = nullptr; }
+        if (graph) { (void)hipGraphDestroy(graph); graph = nullptr; }
+        hipError_t e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
+        if (e != hipSuccess) { rc = fail(HES_ERR_HIP, "stream capture failed"); break; }
+        for (long long j = 0; j < k; ++j) launch_step(h, make_args(h, sb + j, t_end, nullptr, 0));
+        e = hipStreamEndCapture(h->stream, &graph);
+        if (e == hipSuccess) e = hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0);
+        if (e != hipSuccess) { g_err = std::string("graph: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
+        graph_base = sb;
+      }
+      hipError_t e = hipGraphLaunch(gexec, h->stream);
+      if (e != hipSuccess) { g_err = std::string("graph launch: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
+    } else {
+      for (long long j = 0; j < k; ++j)
+        launch_step(h, make_args(h, sb + j, t_end, hist, (int)(launched + j)));
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) { g_err = std::string("launch: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
+    }
+    launched += k;
+    if (t_end < INFINITY || launched >= max_steps) {
+      int cnt = 0;
+      hipError_t e = hipMemcpyAsync(&cnt, h->status + 1, sizeof(int), hipMemcpyDeviceToHost, h->stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+      if (e != hipSuccess) { g_err = std::string("sync: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
+      done = cnt;
+      if (done < launched) break;  // t reached t_end inside this chunk
+    }
+  }
+  HIP_TRY(hipEventRecord(h->ev1, h->stream));
+  HIP_TRY(hipEventSynchronize(h->ev1));
+  if (gexec) (void)hipGraphExecDestroy(gexec);
+  if (graph) (void)hipGraphDestroy(graph);
+  if (rc != HES_OK) return rc;
+  float one = 0.f;
+  HIP_TRY(hipEventElapsedTime(&one, h->ev0, h->ev1));
+  *ms += one;
+  int st[2];
+  HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
+  done = st[1];
+  h->step = s0 + done;
+  double tr[2];
+  HIP_TRY(copy_on(h->stream, tr, h->tring, sizeof(tr), hipMemcpyDeviceToHost));
+  h->t = tr[h->step & 1];
+  *steps_done = done;
+  *bad = st[0];
+  return HES_OK;
+}
+
+// ---- the time loop in one launch ------------------------------------------------
+
+constexpr long long RES_STEPS = 1LL << 16;  // steps of one launch at most
+
+// How a problem is laid on the chip (block 0: it is not, and runs step by
+// step): the first of these shapes whose team has a compute unit for every
+// workgroup.  Fewer waves per SIMD come first, since a step's chain of
+// dependent FP64 operations is what a team of few waves waits for (us per
+// step, Rusanov / HLL, this shape against the next at the same cells, 59000:
+// 4.4 / 3.8 against 4.9 / 4.9; 123000: 5.3 / 5.1 against 7.1 / 8.2; 250000:
+// 7.6 / 8.2 against 9.3 / 11.8; the last against one launch per step, 300000:
+// 9.5 / 11.8 against 21.1 / 20.3).  Two tiles of 64 cells per wave and three
+// fill the registers of two waves per SIMD (200 to 256 VGPRs).
+constexpr ResShape RES_SHAPES[] = {{256, 1}, {512, 1}, {512, 2}, {512, 3}};
+
+void plan_resident(hes_solver* h) {
+  h->shape = {0, 0};
+  if (h->nph != 1) return;
+  for (const ResShape s : RES_SHAPES) {
+    const int cells = s.block / 64 * s.tiles * TILE + 2;  // of a team of one
+    const int per = cells - 2 * RES_HALO;
+    const long long g = h->n <= cells ? 1 : (h->n + per - 1) / per;
+    if (g > std::min(h->cus, RES_MAX_TEAM)) continue;
+    h->shape = s;
+    h->res_g = (int)g;
+    h->res_own = (int)((h->n + g - 1) / g);
+    return;
+  }
+}
+
+size_t comm_words(const hes_solver* h) {
+  return (size_t)2 * h->res_g * RES_SLOT + (size_t)2 * h->res_g * 2 * RES_HALO * 2 * h->nc;
+}
+
+// Two workgroups on one compute unit would share its SIMDs while other units
+// idle: a team's workgroups ask for more LDS than half a unit has.
+constexpr unsigned RES_ALONE_LDS = 84 * 1024;
+
+template <int FLUX, int FAST, int BLK, int T>
+hipError_t launch_resident_t(const ResArgs& a, hipStream_t st) {
+  auto* k = k_resident<FLUX, FAST, BLK, T>;
+  const unsigned lds = a.team.G > 1 ? RES_ALONE_LDS : 0;
+  if (lds) {
+    const hipError_t e = hipFuncSetAttribute((const void*)k,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)a.team.G), dim3(BLK), lds, st, a);
+  return hipGetLastError();
+}
+template <int FLUX, int FAST>
+hipError_t launch_resident_s(const hes_solver* h, const ResArgs& a) {
+  if (h->shape.block == 256) return launch_resident_t<FLUX, FAST, 256, 1>(a, h->stream);
+  if (h->shape.tiles == 1) return launch_resident_t<FLUX, FAST, 512, 1>(a, h->stream);
+  if (h->shape.tiles == 2) return launch_resident_t<FLUX, FAST, 512, 2>(a, h->stream);
+  return launch_resident_t<FLUX, FAST, 512, 3>(a, h->stream);
+}
+hipError_t launch_resident(const hes_solver* h, const ResArgs& a) {
+  const bool fast = all_fast(h);
+  if (h->flux == HES_FLUX_HLL)
+    return fast ? launch_resident_s<FLUX_HLL, 1>(h, a) : launch_resident_s<FLUX_HLL, 0>(h, a);
+  return fast ? launch_resident_s<FLUX_RUSANOV, 1>(h, a) : launch_resident_s<FLUX_RUSANOV, 0>(h, a);
+}
+
+// At most `steps` steps (<= RES_STEPS) in one launch.  *gave_up: no result
+// (the launch's workgroups were not on the chip together), the handle's state
+// is as before.  Adds to *ms the launch's time.
+int run_resident(hes_solver* h, long long steps, double t_end, double* dt_hist, long long* done,
+                 float* ms, bool* gave_up) {
+  ResArgs a;
+  std::memset((void*)&a, 0, sizeof(a));
+  const long long s0 = h->step;
+  ResTeam& tm = a.team;
+  tm.Qin = h->Q[s0 & 1];
+  tm.Qout = h->Q[(s0 + 1) & 1];
+  tm.Cout = h->C[(s0 + 1) & 1];
+  tm.pitch = h->pitch;
+  tm.lo = 0;
+  tm.hi = h->n;
+  tm.G = h->res_g;
+  tm.own = h->res_own;
+  tm.cfl = h->cfl;
+  tm.dx = h->dx;
+  tm.t = h->t;
+  tm.t_end = t_end;
+  tm.kmax = steps;
+  tm.dt_hist = dt_hist;
+  tm.status = h->status;
+  tm.lxf = h->flux == HES_FLUX_LXF;
+  tm.slots = h->comm;
+  tm.border = h->comm + (size_t)2 * h->res_g * RES_SLOT;
+  tm.tag0 = h->res_tag + 1;
+  tm.gave_up = h->status + 2;
+  a.slots = h->slots;
+  a.tring = h->tring;
+  a.jcnt = h->jcnt;
+  a.out = &h->mail->out;
+  a.step0 = s0;
+  a.mat[0] = h->mat[0];
+  a.mat[1] = h->mat[1];
+  h->res_tag += (unsigned)steps + 1;
+  {
+    ComputeUnits units(h->dev, h->cus, h->res_g > 1 ? h->res_g : 0);
+    HIP_TRY(hipEventRecord(h->ev0, h->stream));
+    HIP_TRY(hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * 2 * h->res_g * RES_SLOT, h->stream));
+    HIP_TRY(launch_resident(h, a));
+    HIP_TRY(hipEventRecord(h->ev1, h->stream));
+    HIP_TRY(hipMemcpyAsync(h->mail->status, h->status, sizeof(h->mail->status), hipMemcpyDeviceToHost,
+                           h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+  }
+  *gave_up = h->mail->status[2] != 0;
+  if (*gave_up) {
+    h->shape = {0, 0};  // step by step from here on
+    HIP_TRY(zero_on(h->stream, h->status + 2, sizeof(int)));
+    return init_speeds(h);
+  }
+  float one = 0.f;
+  HIP_TRY(hipEventElapsedTime(&one, h->ev0, h->ev1));
+  *ms += one;
+  *done = h->mail->out.steps;
+  h->step = s0 + *done;
+  h->t = h->mail->out.t;
+  if ((*done & 1) == 0) {  // the result is where an odd number of steps would have left it
+    std::swap(h->Q[0], h->Q[1]);
+    std::swap(h->C[0], h->C[1]);
+  }
+  return HES_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -660,8 +913,13 @@ int hes_solver_create(hes_solver** out, int nphase, int flux, long long ncells,
   for (int p = 0; p < nphase; ++p)
     if (!mat_ok(materials + 8 * p)) return fail(HES_ERR_ARG, "invalid material constants");
   if (!(cfl > 0) || !(dx > 0)) return fail(HES_ERR_ARG, "cfl and dx must be positive");
+  int dev = 0, cus = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   hes_solver* h = new hes_solver();
-  std::memset(h, 0, sizeof(*h));
+  std::memset((void*)h, 0, sizeof(*h));
+  h->dev = dev;
+  h->cus = cus;
   h->nph = nphase;
   h->flux = flux;
   h->nc = nphase == 1 ? 14 : 30;
@@ -675,6 +933,7 @@ int hes_solver_create(hes_solver** out, int nphase, int flux, long long ncells,
   h->mat[1] = make_mat(nphase == 2 ? materials + 8 : materials);
   h->cfl = cfl;
   h->dx = dx;
+  plan_resident(h);
   size_t qbytes = sizeof(double) * (size_t)h->nc * (size_t)h->pitch;
   size_t cbytes = sizeof(double) * (size_t)nphase * (size_t)h->pitch;
   hipError_t e = hipSuccess;
@@ -692,6 +951,12 @@ int hes_solver_create(hes_solver** out, int nphase, int flux, long long ncells,
   if (e == hipSuccess) e = hipEventCreate(&h->ev0);
   if (e == hipSuccess) e = hipEventCreate(&h->ev1);
   if (e == hipSuccess) e = zero_on(h->stream, h->status, 4 * sizeof(int));
+  if (h->shape.block) {
+    const size_t bytes = sizeof(unsigned long long) * comm_words(h);
+    if (e == hipSuccess) e = hipMalloc(&h->comm, bytes);
+    if (e == hipSuccess) e = hipMemsetAsync(h->comm, 0, bytes, h->stream);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&h->mail, sizeof(*h->mail));
+  }
   if (e != hipSuccess) {
     g_err = std::string("allocation failed: ") + hipGetErrorString(e);
     hes_solver_destroy(h);
@@ -731,6 +996,8 @@ int hes_solver_destroy(hes_solver* h) {
   if (h->tring) (void)hipFree(h->tring);
   if (h->status) (void)hipFree(h->status);
   if (h->dt_hist) (void)hipFree(h->dt_hist);
+  if (h->comm) (void)hipFree(h->comm);
+  if (h->mail) (void)hipHostFree(h->mail);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -860,15 +1127,14 @@ int hes_solver_next_dt(hes_solver* h, double* dt) {
   return HES_OK;
 }
 
-// Advance up to max_steps steps while t < t_end.  Launches are issued in
-// chunks of `chunk` steps (captured once into a hipGraph when use_graph is
-// set) and the executed-step counter is read back after each chunk.
+// Advance up to max_steps steps while t < t_end.  A problem that fits the chip
+// runs in one launch per RES_STEPS steps (run_resident), a larger one in one
+// launch per step (run_launches).
 int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_graph,
                    long long* steps_done, double* t_now, float* elapsed_ms, double* dt_out) {
   if (!h) return fail(HES_ERR_ARG, "null handle");
   if (!h->has_state) return fail(HES_ERR_ARG, "no state set");
   if (max_steps < 0) return fail(HES_ERR_ARG, "negative step count");
-  const long long chunk = 60;  // multiple of 6: ring phases repeat per chunk
   if (dt_out) {
     if (h->dt_cap < max_steps) {
       if (h->dt_hist) HIP_TRY(hipFree(h->dt_hist));
@@ -878,69 +1144,36 @@ int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_gra
       h->dt_cap = max_steps;
     }
   }
-  HIP_TRY(hipMemsetAsync(h->status + 1, 0, sizeof(int), h->stream));
-  hipGraphExec_t gexec = nullptr;
-  hipGraph_t graph = nullptr;
-  long long graph_base = -1;  // step (mod 6) the captured graph starts from
-  long long launched = 0, done = 0;
-  const long long s0 = h->step;
-  HIP_TRY(hipEventRecord(h->ev0, h->stream));
-  int rc = HES_OK;
-  while (launched < max_steps) {
-    long long k = max_steps - launched < chunk ? max_steps - launched : chunk;
-    long long sb = s0 + launched;
-    bool graph_ok = use_graph && k == chunk && !dt_out;
-    if (graph_ok) {
-      if (!gexec || (graph_base % 6) != (sb % 6)) {
-        if (gexec) { (void)hipGraphExecDestroy(gexec); gexec = nullptr; }
-        if (graph) { (void)hipGraphDestroy(graph); graph = nullptr; }
-        hipError_t e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess) { rc = fail(HES_ERR_HIP, "stream capture failed"); break; }
-        for (long long j = 0; j < k; ++j) launch_step(h, make_args(h, sb + j, t_end, nullptr, 0));
-        e = hipStreamEndCapture(h->stream, &graph);
-        if (e == hipSuccess) e = hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0);
-        if (e != hipSuccess) { g_err = std::string("graph: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
-        graph_base = sb;
-      }
-      hipError_t e = hipGraphLaunch(gexec, h->stream);
-      if (e != hipSuccess) { g_err = std::string("graph launch: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
-    } else {
-      for (long long j = 0; j < k; ++j)
-        launch_step(h, make_args(h, sb + j, t_end, dt_out ? h->dt_hist : nullptr, (int)(launched + j)));
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess) { g_err = std::string("launch: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
-    }
-    launched += k;
-    if (t_end < INFINITY || launched >= max_steps) {
-      int cnt = 0;
-      hipError_t e = hipMemcpyAsync(&cnt, h->status + 1, sizeof(int), hipMemcpyDeviceToHost, h->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-      if (e != hipSuccess) { g_err = std::string("sync: ") + hipGetErrorString(e); rc = HES_ERR_HIP; break; }
-      done = cnt;
-      if (done < launched) break;  // t reached t_end inside this chunk
-    }
-  }
-  HIP_TRY(hipEventRecord(h->ev1, h->stream));
-  HIP_TRY(hipEventSynchronize(h->ev1));
-  if (gexec) (void)hipGraphExecDestroy(gexec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (rc != HES_OK) return rc;
+  double* hist = dt_out ? h->dt_hist : nullptr;
+  long long done = 0;
   float ms = 0.f;
-  HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
-  int st[2];
-  HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
-  done = st[1];
-  h->step = s0 + done;
-  double tr[2];
-  HIP_TRY(copy_on(h->stream, tr, h->tring, sizeof(tr), hipMemcpyDeviceToHost));
-  h->t = tr[h->step & 1];
+  int bad = 0;
+  bool ended = max_steps == 0;
+  while (h->shape.block && !ended) {
+    const long long k = std::min(max_steps - done, RES_STEPS);
+    long long now = 0;
+    bool gave_up = false;
+    const int rc = run_resident(h, k, t_end, hist ? hist + done : nullptr, &now, &ms, &gave_up);
+    if (rc != HES_OK) return rc;
+    if (gave_up) break;
+    done += now;
+    bad = h->mail->status[0];
+    ended = now < k || done == max_steps;  // t reached t_end, or all steps done
+  }
+  if (!ended) {
+    long long now = 0;
+    const int rc = run_launches(h, max_steps - done, t_end, use_graph, hist ? hist + done : nullptr,
+                                &now, &ms, &bad);
+    if (rc != HES_OK) return rc;
+    done += now;
+  }
   if (steps_done) *steps_done = done;
   if (t_now) *t_now = h->t;
   if (elapsed_ms) *elapsed_ms = ms;
   if (dt_out && done > 0)
     HIP_TRY(copy_on(h->stream, dt_out, h->dt_hist, sizeof(double) * (size_t)done,
                     hipMemcpyDeviceToHost));
-  if (st[0]) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
+  if (bad) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
   return HES_OK;
 }
 
@@ -950,6 +1183,8 @@ int hes_solver_time_steps(hes_solver* h, long long reps, float* elapsed_ms) {
   if (!h || !elapsed_ms) return fail(HES_ERR_ARG, "null argument");
   if (!h->has_state) return fail(HES_ERR_ARG, "no state set");
   if (reps > 100000) return fail(HES_ERR_ARG, "at most 100000 timed steps");
+  if (h->shape.block)
+    return hes_solver_run(h, std::max(reps, 0LL), INFINITY, 0, nullptr, nullptr, elapsed_ms, nullptr);
   HIP_TRY(hipMemsetAsync(h->status + 1, 0, sizeof(int), h->stream));
   // capture the steps first (outside the timed region)
   hipGraph_t graph = nullptr;

@@ -1,0 +1,383 @@
+// hes_resident.hpp -- the time loop of one problem in one launch, its state on
+// the chip from the first step to the last.
+//
+// A step needs the maximum CFL speed of the whole state, so a launch per step
+// (k_step) streams every state through memory and pays a launch and its ramp
+// per step: 5.4 us per step at 1000 cells (Rusanov), 20.4 us at 2^18, of which
+// the arithmetic is 2 and 4.  Here a team of workgroups, all resident at once,
+// holds the problem: one cell per lane in registers for the whole run.
+//
+//   wave       64 consecutive cells; lanes 1..62 are updated by this wave,
+//              lanes 0 and 63 copy the neighbour waves' cells through LDS
+//   workgroup  `own` cells and `halo` cells on either side that a neighbour
+//              workgroup owns; the copies are stepped along with the own
+//              cells (the same arithmetic on the same values), lose one
+//              valid cell per step at their outer end, and are renewed from
+//              the neighbour every `halo` steps
+//   team       per step each workgroup publishes the maximum of its own
+//              cells' speeds in a slot of its own and reads all the others
+//
+// Two messages cross workgroups, both as single 64-bit words that carry their
+// own arrival mark, so no fence and no second round trip is needed: the
+// maximum's sign bit alternates with the use of its slot, and a halo word is
+// 32 bits of a value beside a 32-bit tag.  A slot (two by step parity) is
+// written again only after every workgroup has published the step between,
+// i.e. has read it.
+//
+// Every wait gives up after HES_RES_WAIT_TICKS, or at once when another workgroup
+// has: the launch then ends without a result and the caller's input is whole
+// (results go to another buffer, and only after the last wait).
+//
+// Measured, single phase, us per step, one launch per step against this:
+// 1000 cells 5.4 -> 3.4 (Rusanov) and 6.0 -> 3.7 (HLL), 30011 cells 7.2 -> 3.7
+// and 7.9 -> 3.5, 2^18 cells 20.4 -> 9.4 and 19.5 -> 11.8.  What is left: the
+// chain of dependent FP64 operations of one cell (2 us, a wave alone on its
+// SIMD), the team's maximum (1.3 us for 5 workgroups, 2.1 us for 256), and
+// from two waves per SIMD on the FP64 issue rate (0.95 us per tile and SIMD).
+#pragma once
+#include "hes_step.hpp"
+
+namespace hes {
+
+constexpr int RES_SLOT = 8;  // 64-bit words per slot: one per 64 B (stores of many
+                             // workgroups into one line serialise; 256 workgroups: 3.1 -> 2.1 us)
+#ifndef HES_RES_WAIT_TICKS
+#define HES_RES_WAIT_TICKS 400000000LL  // of the 100 MHz counter: 4 s
+#endif
+#ifndef HES_RES_POLLS
+#define HES_RES_POLLS 64  // polls between two looks at the time
+#endif
+constexpr int RES_HALO = 8;  // halo cells on either side of a workgroup (a team of one has none)
+
+// wave_max by DPP shifts instead of the LDS crossbar (a dependent chain of 6
+// moves and maxima, no ds_bpermute round trips): the maximum in every lane.
+template <int CTRL>
+__device__ __forceinline__ double dpp_max(double v) {
+  return fmax(v, dpp_shift<CTRL>(v));
+}
+__device__ __forceinline__ double wave_max_dpp(double v) {
+  v = dpp_max<0x111>(v);  // row_shr:1, 2, 4, 8: the rows of 16 lanes
+  v = dpp_max<0x112>(v);
+  v = dpp_max<0x114>(v);
+  v = dpp_max<0x118>(v);
+  v = dpp_max<0x142>(v);  // row_bcast:15, 31: across the rows, into lane 63
+  v = dpp_max<0x143>(v);
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// One workgroup's share of a problem, and the team's message buffers.
+struct ResTeam {
+  const double* __restrict__ Qin;
+  double* __restrict__ Qout;
+  double* __restrict__ Cout;
+  long long pitch, lo, hi;  // the problem's cells
+  int G, rank, own;         // workgroups, this one, its cells (at least RES_HALO for G > 1)
+  double cfl, dx, t, t_end;
+  long long kmax;           // steps at most
+  double* dt_hist;          // optional: dt of every step
+  int* status;
+  int lxf;
+  unsigned long long* slots;   // 2 G RES_SLOT words, zero at the start
+  unsigned long long* border;  // halo words: 2 G 2 RES_HALO 2 NC
+  unsigned tag0;               // larger than every tag in `border`
+  int* gave_up;                // nonzero: a wait ended without its message
+};
+
+struct ResOut {
+  long long steps;
+  double t, lmax;
+  bool ok;
+};
+
+__device__ __forceinline__ void res_store(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long res_load(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Barrier of the workgroup for LDS traffic alone: __syncthreads would also wait
+// for the messages on their way to memory.
+__device__ __forceinline__ void res_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// One check of a wait's end, every few polls: true when the wait is over
+// without its message (the time is up here, or another workgroup gave up).
+__device__ __forceinline__ bool res_expired(const ResTeam& a, int& polls, long long& since) {
+  if (++polls % HES_RES_POLLS) return false;
+  const long long now = wall_clock64();
+  if (since == 0) since = now;
+  if (__hip_atomic_load(a.gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return true;
+  if (now - since < HES_RES_WAIT_TICKS) return false;
+  __hip_atomic_store(a.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// The team's maximum of step s: publish this workgroup's, then wait for all
+// (one wave, every lane active).  A state without a positive speed (NaN) still
+// publishes a non-zero word.
+__device__ __forceinline__ void res_publish(const ResTeam& a, long long s, double m) {
+  const unsigned long long sign = (unsigned long long)((s >> 1) & 1) << 63;
+  const unsigned long long bits = m > 0.0 ? (unsigned long long)__double_as_longlong(m) : 1ull;
+  if ((threadIdx.x & 63) == 0)
+    res_store(a.slots + ((s & 1) * a.G + a.rank) * (long long)RES_SLOT, bits | sign);
+}
+template <int MAXG>
+__device__ __forceinline__ bool res_collect(const ResTeam& a, long long s, double& lmax) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long sign = (unsigned long long)((s >> 1) & 1) << 63;
+  const unsigned long long* sl = a.slots + (s & 1) * a.G * (long long)RES_SLOT;
+  int polls = 0;
+  long long since = 0;
+  for (;;) {
+    unsigned long long x[MAXG / 64];
+#pragma unroll
+    for (int k = 0; k < MAXG / 64; ++k) {
+      x[k] = sign | 1ull;
+      if (64 * k < a.G) {  // uniform; the loads of all slots are in flight together
+        const int b = 64 * k + lane;
+        x[k] = res_load(sl + (long long)(b < a.G ? b : a.rank) * RES_SLOT);
+      }
+    }
+    bool here = true;
+    double m = 0.0;
+#pragma unroll
+    for (int k = 0; k < MAXG / 64; ++k) {
+      here = here && x[k] != 0ull && ((x[k] ^ sign) >> 63) == 0ull;
+      m = fmax(m, __longlong_as_double((long long)(x[k] & 0x7fffffffffffffffull)));
+    }
+    if (__all(here)) {
+      lmax = wave_max_dpp(m);
+      return true;
+    }
+    if (res_expired(a, polls, since)) return false;
+  }
+}
+
+typedef unsigned __attribute__((may_alias)) u32_any;
+
+// Halo words of the cells a workgroup shares with its neighbours, renewed at
+// every RES_HALO-th step from and into LDS (word k of a side: 32-bit half k of
+// its RES_HALO cells' states): side 0 is read by the left neighbour (this
+// workgroup's first cells), side 1 by the right one (its last cells).  One
+// wave each, every lane active.
+template <int NC>
+__device__ __forceinline__ unsigned long long* res_words(const ResTeam& a, long long round,
+                                                         int rank, int side) {
+  return a.border + (((round & 1) * a.G + rank) * 2 + side) * (long long)(RES_HALO * 2 * NC);
+}
+template <int NC>
+__device__ __forceinline__ void res_send(const ResTeam& a, long long round, unsigned tag, int side,
+                                         const double* cells) {
+  unsigned long long* w = res_words<NC>(a, round, a.rank, side);
+  const u32_any* src = (const u32_any*)cells;
+#pragma unroll 1
+  for (int k = threadIdx.x & 63; k < RES_HALO * 2 * NC; k += 64)
+    res_store(w + k, (unsigned long long)src[k] | ((unsigned long long)tag << 32));
+}
+template <int NC>
+__device__ __forceinline__ bool res_receive(const ResTeam& a, long long round, unsigned tag,
+                                            int rank, int side, double* cells) {
+  const unsigned long long* w = res_words<NC>(a, round, rank, side);
+  u32_any* dst = (u32_any*)cells;
+  constexpr int N = RES_HALO * 2 * NC, M = (N + 63) / 64;
+  const int lane = threadIdx.x & 63;
+  int polls = 0;
+  long long since = 0;
+  for (;;) {
+    unsigned long long x[M];
+#pragma unroll
+    for (int k = 0; k < M; ++k) x[k] = res_load(w + (64 * k + lane < N ? 64 * k + lane : lane));
+    bool here = true;
+#pragma unroll
+    for (int k = 0; k < M; ++k) here = here && (unsigned)(x[k] >> 32) == tag;
+    if (__all(here)) {
+#pragma unroll
+      for (int k = 0; k < M; ++k)
+        if (64 * k + lane < N) dst[64 * k + lane] = (unsigned)x[k];
+      return true;
+    }
+    if (res_expired(a, polls, since)) return false;
+  }
+}
+
+// The run of one workgroup, single phase.  T: tiles of 64 lanes that a wave
+// holds (its registers); MAXG: the largest team it is built for (a multiple
+// of 64).  Per step the thermodynamic state of a cell is formed once, for its
+// flux and for its speed (k_step forms it twice, for the state it reads and
+// the one it writes); with one tile per wave and registers to keep it, the
+// flux, and always HLL's mid state, fall into the wait for the team's maximum.
+template <int FLUX, int FAST, int BLK, int T, int MAXG>
+__device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& mat) {
+  constexpr int NC = 14, W = BLK / 64, NT = W * T;
+  constexpr bool LATE_FLUX = T == 1 && BLK < 1024;
+  __shared__ double edge[2][NT][2][NC];  // new first and last updated cell of every tile, by parity
+  __shared__ double red[2][W];           // every wave's maximum, by parity
+  __shared__ double mine_out[2][RES_HALO][NC], theirs[2][RES_HALO][NC];
+  __shared__ double team_max, tnow[2];
+  __shared__ int dead;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long o0 = a.lo + (long long)a.rank * a.own;
+  const long long o1 = o0 + a.own < a.hi ? o0 + a.own : a.hi;
+  // positions are counted from the workgroup's first own cell
+  const int n_own = (int)(o1 - o0);
+  const int n_lo = o0 - a.lo < (1 << 24) ? (int)(a.lo - o0) : -(1 << 24);  // the problem's first cell
+  const int n_hi = a.hi - o0 < (1 << 24) ? (int)(a.hi - o0) : 1 << 24;     // and past its last
+  const int halo = a.G > 1 ? RES_HALO : 0;
+  auto cell = [&](int k) { return TILE * (w * T + k) + lane - halo; };
+  auto mine = [&](int k) {
+    const int tile = w * T + k, j = cell(k);
+    return (lane >= 1 || (tile == 0 && halo == 0)) && (lane <= TILE || (tile == NT - 1 && halo == 0)) &&
+           j >= 0 && j < n_own;
+  };
+  double q[T][NC], c[T];
+#pragma unroll
+  for (int k = 0; k < T; ++k) {
+    const int j = cell(k), jc = j < n_lo ? n_lo : (j >= n_hi ? n_hi - 1 : j);
+#pragma unroll
+    for (int r = 0; r < NC; ++r) q[k][r] = a.Qin[r * a.pitch + o0 + jc];
+  }
+  if (threadIdx.x == 0) dead = 0;
+  double t = a.t, lmax = 0.0;
+  long long s = 0;
+  int to_halo = RES_HALO;
+  int bad = 0;
+  bool ok = true;
+  for (;; ++s) {
+    double f[T][NC], u1[T], mn[T], mx[T], m = 0.0;
+    Thermo th;
+#pragma unroll
+    for (int k = 0; k < T; ++k) {
+      thermo<true, FAST>(mat, 1.0, q[k], th);
+      c[k] = sound_speed(mat, th);
+      u1[k] = th.u[0];
+      const bool own = mine(k);
+      bad |= own && (th.bad | !(c[k] < 1e300));
+      m = fmax(m, own ? fabs(u1[k]) + c[k] : 0.0);
+      if (!LATE_FLUX) phase_flux(mat, 1.0, th, q[k] + 5, f[k]);
+    }
+    m = wave_max_dpp(m);
+    if (lane == 0) red[s & 1][w] = m;
+    res_barrier();
+    lmax = wave_max_dpp(lane < W ? red[s & 1][lane] : 0.0);
+    if (a.G > 1 && w == 0) res_publish(a, s, lmax);
+    if (LATE_FLUX) phase_flux(mat, 1.0, th, q[0] + 5, f[0]);
+    if (FLUX == FLUX_HLL) {
+#pragma unroll
+      for (int k = 0; k < T; ++k) mid_range1<FAST>(mat, q[k], mn[k], mx[k]);
+    }
+    if (a.G > 1) {
+      if (w == 0) {
+        double lm = 0.0;
+        const bool got = res_collect<MAXG>(a, s, lm);
+        if (lane == 0) {
+          team_max = lm;
+          if (!got) dead = 1;
+        }
+      }
+      res_barrier();
+      lmax = team_max;
+      if (dead) {
+        ok = false;
+        break;
+      }
+    }
+    if (s >= a.kmax || !(t < a.t_end)) break;  // main.jl:202 `while t < T`
+    const double dtdx = a.cfl * rcp(lmax);
+    if (w == 0) {  // the time, by one wave
+      const double dt = a.cfl * a.dx / lmax;  // main.jl:212
+      if (lane == 0) {
+        if (a.dt_hist && a.rank == 0) a.dt_hist[s] = dt;
+        tnow[s & 1] = t + dt;
+      }
+    }
+    const bool renew = a.G > 1 && --to_halo == 0;  // uniform
+#pragma unroll
+    for (int k = 0; k < T; ++k) {
+      const double smin = u1[k] - c[k], smax = u1[k] + c[k];
+      double upd[NC];
+      if (FLUX == FLUX_RUSANOV)
+        update_rusanov1<true>(q[k], f[k], smin, smax, dtdx, a.lxf, upd);
+      else
+        update_hll1<true>(q[k], f[k], hll_coef(mn[k], mx[k], smin, lane_down(smax)), dtdx, upd);
+      // cells beyond the right halo stay as they are: copies that nothing renews
+      const int j = cell(k);
+      if (lane >= 1 && lane <= TILE && j > n_lo && j < n_hi - 1 && j < n_own + halo) {
+#pragma unroll
+        for (int r = 0; r < NC; ++r) q[k][r] = upd[r];
+      }
+      if (lane == 1 || lane == TILE) {
+        double* e = edge[s & 1][w * T + k][lane == 1 ? 0 : 1];
+#pragma unroll
+        for (int r = 0; r < NC; ++r) e[r] = q[k][r];
+      }
+      if (renew && mine(k)) {
+        if (j < RES_HALO) {
+#pragma unroll
+          for (int r = 0; r < NC; ++r) mine_out[0][j][r] = q[k][r];
+        }
+        if (j >= n_own - RES_HALO) {
+#pragma unroll
+          for (int r = 0; r < NC; ++r) mine_out[1][j - (n_own - RES_HALO)][r] = q[k][r];
+        }
+      }
+    }
+    res_barrier();
+    t = tnow[s & 1];
+#pragma unroll
+    for (int k = 0; k < T; ++k) {
+      const int tile = w * T + k;
+      if ((lane == 0 && tile > 0) || (lane == 63 && tile < NT - 1)) {
+        const double* e = edge[s & 1][lane == 0 ? tile - 1 : tile + 1][lane == 0 ? 1 : 0];
+#pragma unroll
+        for (int r = 0; r < NC; ++r) q[k][r] = e[r];
+      }
+    }
+    if (renew) {
+      to_halo = RES_HALO;
+      const long long round = (s + 1) / RES_HALO;
+      const unsigned tag = a.tag0 + (unsigned)s;
+      bool got = true;
+      if (w == 0 && a.rank > 0) {
+        res_send<NC>(a, round, tag, 0, &mine_out[0][0][0]);
+        got = res_receive<NC>(a, round, tag, a.rank - 1, 1, &theirs[0][0][0]);
+      }
+      if (w == W - 1 && a.rank < a.G - 1) {
+        res_send<NC>(a, round, tag, 1, &mine_out[1][0][0]);
+        got = res_receive<NC>(a, round, tag, a.rank + 1, 0, &theirs[1][0][0]);
+      }
+      if (!got) dead = 1;  // seen after the next step's barriers
+      res_barrier();
+#pragma unroll
+      for (int k = 0; k < T; ++k) {
+        const int j = cell(k);
+        const bool left = j < 0 && j >= n_lo;
+        if (left || (j >= n_own && j < n_own + RES_HALO && j < n_hi)) {
+          const double* e = left ? theirs[0][j + RES_HALO] : theirs[1][j - n_own];
+#pragma unroll
+          for (int r = 0; r < NC; ++r) q[k][r] = e[r];
+        }
+      }
+    }
+  }
+  if (ok) {
+#pragma unroll
+    for (int k = 0; k < T; ++k) {
+      if (mine(k)) {
+        const long long i = o0 + cell(k);
+#pragma unroll
+        for (int r = 0; r < NC; ++r) a.Qout[r * a.pitch + i] = q[k][r];
+        a.Cout[i] = c[k];
+      }
+    }
+    if (__any(bad) && lane == 0) atomicOr(a.status, 1);
+  }
+  return {s, t, lmax, ok};
+}
+
+}  // namespace hes

@@ -305,6 +305,83 @@ __device__ __forceinline__ void relax_pressure2(const MatDev* mat, double* q, do
   }
 }
 
+// One phase, Rusanov (or, with lxf, Lax-Friedrichs): the update of a lane's cell
+// from its own and its neighbour lanes' state q, flux f and speed bounds.
+// Rusanov face i+1/2: 1/2 (F_i + F_i+1) - 1/2 lam (Q_i+1 - Q_i) with
+// lam = max(lam_i, lam_i+1) (NumFluxes.jl:30, main.jl:47-48), split as
+// a_i + b_i+1 with a = F/2 + lam/2 Q and b = F/2 - lam/2 Q.  Each face sum
+// is formed from the same two rounded halves by both of its cells, so the
+// two cells see bit-identical face fluxes.  Every lane of the wave is active.
+template <bool PIN>
+__device__ __forceinline__ void update_rusanov1(const double* q, const double* f, double smin,
+                                                double smax, double dtdx, int lxf, double* upd) {
+  const double lam_c = fmax(fabs(smin), fabs(smax));  // maximum(abs.(eigvals))
+  // lambda = 1 / dtdx (main.jl:50), to about an ulp (dt itself stays exact)
+  const double hg = lxf ? 0.5 * rcp(dtdx) : 0.0;
+  const double lam_r = lane_down_z(lam_c), lam_l = lane_up_z(lam_c);
+  const double hr = lxf ? hg : 0.5 * fmax(lam_c, lam_r);
+  const double hl = lxf ? hg : 0.5 * fmax(lam_l, lam_c);
+#pragma unroll
+  for (int r = 0; r < 14; ++r) {
+    double fa = 0.5 * f[r] + hr * q[r];
+    double fb = 0.5 * f[r] - hl * q[r];
+    double Fr = fa + lane_down_z(fb);
+    double Fl = lane_up_z(fa) + fb;
+    upd[r] = q[r] - dtdx * (Fr - Fl);  // main.jl:59 with zero path integrals
+    if (PIN) pin(upd[r]);
+  }
+}
+
+// One component of the HLL update without path integrals: its state qr and
+// flux fr on this lane and its neighbours, every lane active.
+__device__ __forceinline__ double hll_component(double qr, double fr, const HllCoef& hc,
+                                                double dtdx) {
+  // one register holds the flux for both its uses (shifted to the left
+  // neighbour and local): left to itself the compiler may form the two
+  // from separate copies of the flux arithmetic, contracted differently,
+  // and a uniform state then moves by an ulp (F(Q) - F(Q) must be 0)
+  pin(fr);
+  // zero-filling shifts (every lane is active here): lane 63's face and
+  // lane 0's update read the zeros, and neither is stored
+  const double J = lane_down_z(fr) - fr;
+  const double dq = lane_down_z(qr) - qr;
+  // D- + D+ = J at every face (cl + cr = 1), so D-(i+1/2) + D+(i-1/2) =
+  // H(i+1/2) - H(i-1/2) with H = F_i + D-(i+1/2), the HLL flux: two
+  // fused products per face instead of four, and a uniform state still
+  // gives H = F_i exactly
+  const double h = fma(hc.cl, J, fma(hc.clr, dq, fr));
+  return qr - dtdx * (h - lane_up_z(h));  // conservative part is zero (NumFluxes.jl:82)
+}
+
+// One phase, HLL: the update of a lane's cell (all of NumFluxes.jl:70-132).
+template <bool PIN>
+__device__ __forceinline__ void update_hll1(const double* q, const double* f, const HllCoef& hc,
+                                            double dtdx, double* upd) {
+#pragma unroll
+  for (int r = 0; r < 14; ++r) {
+    upd[r] = hll_component(q[r], f[r], hc, dtdx);
+    if (PIN) pin(upd[r]);
+  }
+}
+
+// One phase, HLL: the eigenvalue range of face i+1/2's mid state.  The mid
+// state Q_m = (Q_i + Q_i+1) / 2 enters as the neighbours' sum S = 2 Q_m
+// (0.5 S is exact) with volume fraction 2: thermo's density takes det(S) / 2^3,
+// so every power of two scales out exactly and the range is Q_m's to the bit,
+// without the 14 halvings.
+template <int FAST>
+__device__ __forceinline__ void mid_range1(const MatDev& m, const double* q, double& mn,
+                                           double& mx) {
+  double qs[14];
+#pragma unroll
+  for (int r = 0; r < 14; ++r) qs[r] = q[r] + lane_down(q[r]);
+  Thermo t;
+  thermo<false, FAST>(m, 2.0, qs, t);
+  const double c = sound_speed(m, t);
+  mn = t.u[0] - c;
+  mx = t.u[0] + c;
+}
+
 // PIN (single phase): each updated component is pinned where it is computed
 // (see pin): Rusanov 102 instead of 160 VGPRs, HLL 106 instead of 136, four
 // waves per SIMD instead of three.  It pays on large grids (2^22 cells:
@@ -339,11 +416,8 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
   // (from u1 and the stored sound speeds), then each phase's flux is formed
   // and consumed by the update in turn, so only one phase's flux is live
   constexpr bool PHASED = NPH == 2 && PATHBUF;
-  // The mid state Q_m = (Q_i + Q_i+1) / 2 enters as the neighbours' sum
-  // S = 2 Q_m (0.5 S is exact) with volume fraction 2 a_m (one phase: 2):
-  // thermo's density takes det(S) / (2 a_m)^3, so every power of two scales
-  // out exactly and the thermodynamic state, sound speed and range are those
-  // of Q_m to the bit, without the 14 or 15 halvings per phase.
+  // The mid state enters as the neighbours' sum with volume fraction 2 a_m
+  // (see mid_range1).
   double mn_m = 0.0, mx_m = 0.0;
   if (HLL_STREAM && PHASED) {
 #pragma unroll
@@ -358,14 +432,7 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
       mx_m = p == 0 ? t.u[0] + c : fmax(mx_m, t.u[0] + c);
     }
   } else if (HLL_STREAM && NPH == 1) {
-    double qs[NC];
-#pragma unroll
-    for (int r = 0; r < NC; ++r) qs[r] = q[r] + lane_down(q[r]);
-    Thermo t;
-    thermo<false, FAST>(a.mat[0], 2.0, qs, t);
-    const double c = sound_speed(a.mat[0], t);
-    mn_m = t.u[0] - c;
-    mx_m = t.u[0] + c;
+    mid_range1<FAST>(a.mat[0], q, mn_m, mx_m);
   }
 
   double f[NC], smin, smax;
@@ -391,26 +458,7 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
 
   double upd[NC];
   if (FLUX == FLUX_RUSANOV && NPH == 1) {
-    // Rusanov face i+1/2: 1/2 (F_i + F_i+1) - 1/2 lam (Q_i+1 - Q_i) with
-    // lam = max(lam_i, lam_i+1) (NumFluxes.jl:30, main.jl:47-48), split as
-    // a_i + b_i+1 with a = F/2 + lam/2 Q and b = F/2 - lam/2 Q.  Each face sum
-    // is formed from the same two rounded halves by both of its cells, so the
-    // two cells see bit-identical face fluxes.
-    const double lam_c = fmax(fabs(smin), fabs(smax));  // maximum(abs.(eigvals))
-    // lambda = 1 / dtdx (main.jl:50), to about an ulp (dt itself stays exact)
-    const double hg = a.lxf ? 0.5 * rcp(dtdx) : 0.0;
-    const double lam_r = lane_down_z(lam_c), lam_l = lane_up_z(lam_c);
-    const double hr = a.lxf ? hg : 0.5 * fmax(lam_c, lam_r);
-    const double hl = a.lxf ? hg : 0.5 * fmax(lam_l, lam_c);
-#pragma unroll
-    for (int r = 0; r < NC; ++r) {
-      double fa = 0.5 * f[r] + hr * q[r];
-      double fb = 0.5 * f[r] - hl * q[r];
-      double Fr = fa + lane_down_z(fb);
-      double Fl = lane_up_z(fa) + fb;
-      upd[r] = q[r] - dtdx * (Fr - Fl);  // main.jl:59 with zero path integrals
-      if (PIN) pin(upd[r]);
-    }
+    update_rusanov1<PIN>(q, f, smin, smax, dtdx, a.lxf, upd);
   } else if (FLUX == FLUX_RUSANOV && NPH == 2 && PATHBUF) {
     // Two phases with the half path integrals precomputed (k_path2): each
     // component's face flux is formed (as face_rusanov forms it) and consumed
@@ -475,24 +523,6 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
       jump = !(((a0n - q[0]) == 0.0) & ((a1n - q[NPH == 2 ? 15 : 0]) == 0.0)) & (i >= a.lo) &
              (i < a.hi - 1);
     }
-    auto stream = [&](int r, double fr) {
-      // one register holds the flux for both its uses (shifted to the left
-      // neighbour and local): left to itself the compiler may form the two
-      // from separate copies of the flux arithmetic, contracted differently,
-      // and a uniform state then moves by an ulp (F(Q) - F(Q) must be 0)
-      pin(fr);
-      // zero-filling shifts (every lane is active here): lane 63's face and
-      // lane 0's update read the zeros, and neither is stored
-      const double J = lane_down_z(fr) - fr;
-      const double dq = lane_down_z(q[r]) - q[r];
-      // D- + D+ = J at every face (cl + cr = 1), so D-(i+1/2) + D+(i-1/2) =
-      // H(i+1/2) - H(i-1/2) with H = F_i + D-(i+1/2), the HLL flux: two
-      // fused products per face instead of four, and a uniform state still
-      // gives H = F_i exactly
-      const double h = fma(hc.cl, J, fma(hc.clr, dq, fr));
-      upd[r] = q[r] - dtdx * (h - lane_up_z(h));  // conservative part is zero (NumFluxes.jl:82)
-      if (PHASED || PIN) pin(upd[r]);
-    };
     if (PHASED) {
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
@@ -503,11 +533,14 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
         fp[0] = 0.0;
         phase_flux(a.mat[p], q[15 * p], t, q + 15 * p + 6, fp + 1);
 #pragma unroll
-        for (int k = 0; k < 15; ++k) stream(15 * p + k, fp[k]);
+        for (int k = 0; k < 15; ++k) {
+          const int r = 15 * p + k;
+          upd[r] = hll_component(q[r], fp[k], hc, dtdx);
+          pin(upd[r]);
+        }
       }
     } else {
-#pragma unroll
-      for (int r = 0; r < NC; ++r) stream(r, f[r]);
+      update_hll1<PIN>(q, f, hc, dtdx, upd);
     }
     if (NPH == 2 && __any(jump)) {  // loads and shifts as in the Rusanov branch, a phase at a time
 #pragma unroll

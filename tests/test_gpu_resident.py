@@ -1,0 +1,95 @@
+"""The time loop of a problem that fits the chip (one launch for all its steps)
+against the batched solver's one launch per step, bit for bit: the two share
+every cell's and face's arithmetic, so no tolerance enters."""
+import threading
+
+import numpy as np
+import pytest
+
+from hyperelasticsolver_amd.EquationsOfState import Barton2009
+from hyperelasticsolver_amd.batched import Batch
+from hyperelasticsolver_amd.initial import prim2cons, random_interfaces, random_phase_prims
+from hyperelasticsolver_amd.solver import Solver
+
+pytestmark = pytest.mark.gpu
+
+# the first and last size of every workgroup shape, teams of one and more, a
+# last workgroup of a few cells, and the first size that runs step by step
+SIZES = [3, 63, 65, 250, 251, 470, 1000, 59904, 59905, 123392, 123393, 250368, 250369, 377344, 377345]
+STEPS, MORE = 19, 12  # past two renewals of the halo cells; then on from there
+
+
+def _problem(eos, n, seed):
+    rng = np.random.default_rng(seed)
+    k = 6 if n > 60 else 2
+    return prim2cons(eos, random_phase_prims(rng, eos, k)), random_interfaces(rng, k - 1)
+
+
+def _stepwise(eos, n, flux, states, ifc, steps, t_end=None):
+    with Batch([eos], [n], flux=flux) as b:
+        if t_end is not None:
+            b.set_t_end(t_end)
+        b.set_piecewise([states], [ifc])
+        b.run(steps, mode="eager")
+        t, s = b.times()
+        return b.get_state(), t[0], s[0]
+
+
+@pytest.mark.parametrize("flux", ["rusanov", "hll", "lxf"])
+@pytest.mark.parametrize("n", SIZES)
+def test_resident_equals_stepwise(n, flux):
+    print(f"[resident] n={n} flux={flux}", flush=True)
+    eos = Barton2009() if n != 1000 else Barton2009(_beta=3.577, _gamma=2.088)
+    states, ifc = _problem(eos, n, n)
+    with Solver(eos, n, flux=flux) as s:
+        s.set_piecewise(states, ifc)
+        a = s.run(steps=STEPS, record_dt=True)
+        q1 = s.get_state()
+        dt = s.next_dt()
+        b = s.run(steps=MORE)
+        q2 = s.get_state()
+    r1, t1, _ = _stepwise(eos, n, flux, states, ifc, STEPS)
+    r2, t2, _ = _stepwise(eos, n, flux, states, ifc, STEPS + MORE)
+    assert np.array_equal(q1, r1) and np.array_equal(q2, r2)
+    assert (a["steps"], b["steps"]) == (STEPS, MORE) and (a["t"], b["t"]) == (t1, t2)
+    t = 0.0
+    for d in a["dt"]:
+        t += d
+    assert t == t1 and dt > 0.0
+
+
+@pytest.mark.parametrize("n", [200, 1000])
+def test_resident_end_time(n):
+    print(f"[resident t_end] n={n}", flush=True)
+    eos = Barton2009()
+    states, ifc = _problem(eos, n, 5)
+    with Solver(eos, n, flux="rusanov") as s:
+        s.set_piecewise(states, ifc)
+        r = s.run(t_end=10.5 * s.next_dt())
+        q = s.get_state()
+        again = s.run(steps=5, t_end=r["t"])  # already there: no step
+        assert again["steps"] == 0 and np.array_equal(s.get_state(), q)
+    ref, t, steps = _stepwise(eos, n, "rusanov", states, ifc, 40, t_end=r["t"])
+    assert np.array_equal(q, ref) and t == r["t"] and steps == r["steps"]
+
+
+def test_resident_teams_from_two_threads():
+    """Two teams that each need most of the chip: one waits for the other."""
+    n, eos = 200003, Barton2009()
+    states, ifc = _problem(eos, n, 9)
+    got = {}
+
+    def work(k):
+        with Solver(eos, n, flux="rusanov") as s:
+            s.set_piecewise(states, ifc)
+            for _ in range(5):
+                s.run(steps=40)
+            got[k] = s.get_state()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    ref, _, _ = _stepwise(eos, n, "rusanov", states, ifc, 200)
+    assert np.array_equal(got[0], ref) and np.array_equal(got[1], ref)
