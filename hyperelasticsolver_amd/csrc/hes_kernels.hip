@@ -159,36 +159,48 @@ struct ResArgs {
   unsigned long long* jcnt;
   ResOut* out;
   long long step0;
+  double relax, relax_p;       // two phases: 1 / tau of the sources (0: none)
   MatDev mat[2];
 };
 
-// Shape of a team's workgroups: threads, and tiles of 64 cells that a wave holds.
+// Shape of a team's workgroups: threads, and what a wave holds: tiles of 64
+// cells (one phase), or cells (two phases).
 struct ResShape {
   int block, tiles;
 };
 constexpr int RES_MAX_TEAM = 256;  // workgroups
+
+// The team's first workgroup leaves the handle's rings as k_step expects them.
+__device__ __forceinline__ void resident_end(const ResArgs& a, const ResTeam& tm, const ResOut& o) {
+  if (tm.rank != 0 || threadIdx.x != 0) return;
+  *a.out = o;
+  if (!o.ok) return;
+  const long long s = a.step0 + o.steps;
+  a.slots[s % 3] = (unsigned long long)__double_as_longlong(o.lmax);
+  a.slots[(s + 1) % 3] = 0ull;
+  a.slots[(s + 2) % 3] = 0ull;
+  a.tring[0] = o.t;
+  a.tring[1] = o.t;
+  if (a.jcnt) {
+    a.jcnt[0] = 0ull;
+    a.jcnt[1] = 0ull;
+  }
+}
 
 template <int FLUX, int FAST, int BLK, int T>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(BLK / 256)))
 void k_resident(ResArgs a) {
   ResTeam tm = a.team;
   tm.rank = (int)xcd_block();  // neighbours on one XCD
-  const ResOut o = resident_run1<FLUX, FAST, BLK, T, RES_MAX_TEAM>(tm, a.mat[0]);
-  if (tm.rank == 0 && threadIdx.x == 0) {
-    *a.out = o;
-    if (o.ok) {
-      const long long s = a.step0 + o.steps;
-      a.slots[s % 3] = (unsigned long long)__double_as_longlong(o.lmax);
-      a.slots[(s + 1) % 3] = 0ull;
-      a.slots[(s + 2) % 3] = 0ull;
-      a.tring[0] = o.t;
-      a.tring[1] = o.t;
-      if (a.jcnt) {
-        a.jcnt[0] = 0ull;
-        a.jcnt[1] = 0ull;
-      }
-    }
-  }
+  resident_end(a, tm, resident_run1<FLUX, FAST, BLK, T, RES_MAX_TEAM>(tm, a.mat[0]));
+}
+
+template <int FLUX, int FAST, int TW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
+void k_resident2(ResArgs a) {
+  ResTeam tm = a.team;
+  tm.rank = (int)xcd_block();
+  resident_end(a, tm, resident_run2<FLUX, FAST, TW, RES_MAX_TEAM>(tm, a.mat, a.relax, a.relax_p));
 }
 
 // Two phases: the faces with a volume-fraction jump of the step's input state,
@@ -763,13 +775,25 @@ constexpr long long RES_STEPS = 1LL << 16;  // steps of one launch at most
 // 7.6 / 8.2 against 9.3 / 11.8; the last against one launch per step, 300000:
 // 9.5 / 11.8 against 21.1 / 20.3).  Two tiles of 64 cells per wave and three
 // fill the registers of two waves per SIMD (200 to 256 VGPRs).
-constexpr ResShape RES_SHAPES[] = {{256, 1}, {512, 1}, {512, 2}, {512, 3}};
+constexpr ResShape RES_SHAPES[4] = {{256, 1}, {512, 1}, {512, 2}, {512, 3}};
+// Two phases: the narrowest tiles with which the team fits (resident_run2).
+// A face's path terms cost more than its cell, and the faces that jump sit
+// together around the interfaces, so a wave with 64 cells may work on all its
+// faces in turn while most of the chip has none; one launch per step spreads
+// them evenly.  us per step once the interfaces have spread, that against
+// this: HLL, 1000 cells 189 -> 21, 10007 60 -> 21, 27000 42 -> 31, but 59000
+// 38 -> 52, where it is left out; Rusanov 45 -> 14, 25 -> 14, 22 -> 14 and 26
+// -> 20.
+constexpr ResShape RES_SHAPES2[4] = {{256, 16}, {256, 32}, {256, 64}, {0, 0}};
+constexpr int RES_HLL2_MAX_TILE = 32;
 
 void plan_resident(hes_solver* h) {
   h->shape = {0, 0};
-  if (h->nph != 1) return;
-  for (const ResShape s : RES_SHAPES) {
-    const int cells = s.block / 64 * s.tiles * TILE + 2;  // of a team of one
+  for (const ResShape s : h->nph == 1 ? RES_SHAPES : RES_SHAPES2) {
+    if (s.block == 0) continue;
+    if (h->nph == 2 && h->flux == HES_FLUX_HLL && s.tiles > RES_HLL2_MAX_TILE) continue;
+    const int waves = s.block / 64;
+    const int cells = (h->nph == 1 ? waves * s.tiles * TILE : waves * (s.tiles - 2)) + 2;  // of a team of one
     const int per = cells - 2 * RES_HALO;
     const long long g = h->n <= cells ? 1 : (h->n + per - 1) / per;
     if (g > std::min(h->cus, RES_MAX_TEAM)) continue;
@@ -788,30 +812,39 @@ size_t comm_words(const hes_solver* h) {
 // idle: a team's workgroups ask for more LDS than half a unit has.
 constexpr unsigned RES_ALONE_LDS = 84 * 1024;
 
-template <int FLUX, int FAST, int BLK, int T>
-hipError_t launch_resident_t(const ResArgs& a, hipStream_t st) {
-  auto* k = k_resident<FLUX, FAST, BLK, T>;
-  const unsigned lds = a.team.G > 1 ? RES_ALONE_LDS : 0;
-  if (lds) {
-    const hipError_t e = hipFuncSetAttribute((const void*)k,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+hipError_t launch_resident_k(void (*k)(ResArgs), int block, const ResArgs& a, hipStream_t st) {
+  unsigned lds = 0;
+  if (a.team.G > 1) {
+    hipFuncAttributes fa;
+    hipError_t e = hipFuncGetAttributes(&fa, (const void*)k);
+    if (e == hipSuccess && fa.sharedSizeBytes < RES_ALONE_LDS) {
+      lds = RES_ALONE_LDS - (unsigned)fa.sharedSizeBytes;
+      e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    }
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k, dim3((unsigned)a.team.G), dim3(BLK), lds, st, a);
+  hipLaunchKernelGGL(k, dim3((unsigned)a.team.G), dim3((unsigned)block), lds, st, a);
   return hipGetLastError();
 }
 template <int FLUX, int FAST>
-hipError_t launch_resident_s(const hes_solver* h, const ResArgs& a) {
-  if (h->shape.block == 256) return launch_resident_t<FLUX, FAST, 256, 1>(a, h->stream);
-  if (h->shape.tiles == 1) return launch_resident_t<FLUX, FAST, 512, 1>(a, h->stream);
-  if (h->shape.tiles == 2) return launch_resident_t<FLUX, FAST, 512, 2>(a, h->stream);
-  return launch_resident_t<FLUX, FAST, 512, 3>(a, h->stream);
+auto resident_kernel(int nph, ResShape s) -> void (*)(ResArgs) {
+  if (nph == 2) {
+    if (s.tiles == 16) return k_resident2<FLUX, FAST, 16>;
+    if (s.tiles == 32) return k_resident2<FLUX, FAST, 32>;
+    if constexpr (FLUX == FLUX_RUSANOV) return k_resident2<FLUX, FAST, 64>;
+  }
+  if (s.block == 256) return k_resident<FLUX, FAST, 256, 1>;
+  return s.tiles == 1   ? k_resident<FLUX, FAST, 512, 1>
+         : s.tiles == 2 ? k_resident<FLUX, FAST, 512, 2>
+                        : k_resident<FLUX, FAST, 512, 3>;
 }
 hipError_t launch_resident(const hes_solver* h, const ResArgs& a) {
-  const bool fast = all_fast(h);
-  if (h->flux == HES_FLUX_HLL)
-    return fast ? launch_resident_s<FLUX_HLL, 1>(h, a) : launch_resident_s<FLUX_HLL, 0>(h, a);
-  return fast ? launch_resident_s<FLUX_RUSANOV, 1>(h, a) : launch_resident_s<FLUX_RUSANOV, 0>(h, a);
+  const bool fast = all_fast(h), hll = h->flux == HES_FLUX_HLL;
+  void (*k)(ResArgs) = hll ? (fast ? resident_kernel<FLUX_HLL, 1>(h->nph, h->shape)
+                                   : resident_kernel<FLUX_HLL, 0>(h->nph, h->shape))
+                           : (fast ? resident_kernel<FLUX_RUSANOV, 1>(h->nph, h->shape)
+                                   : resident_kernel<FLUX_RUSANOV, 0>(h->nph, h->shape));
+  return launch_resident_k(k, h->shape.block, a, h->stream);
 }
 
 // At most `steps` steps (<= RES_STEPS) in one launch.  *gave_up: no result
@@ -848,6 +881,8 @@ int run_resident(hes_solver* h, long long steps, double t_end, double* dt_hist, 
   a.jcnt = h->jcnt;
   a.out = &h->mail->out;
   a.step0 = s0;
+  a.relax = h->relax;
+  a.relax_p = h->relax_p;
   a.mat[0] = h->mat[0];
   a.mat[1] = h->mat[1];
   h->res_tag += (unsigned)steps + 1;

@@ -28,7 +28,7 @@
 // has: the launch then ends without a result and the caller's input is whole
 // (results go to another buffer, and only after the last wait).
 //
-// Measured, single phase, us per step, one launch per step against this:
+// Measured (two phases: see plan_resident), single phase, us per step, one launch per step against this:
 // 1000 cells 5.4 -> 3.4 (Rusanov) and 6.0 -> 3.7 (HLL), 30011 cells 7.2 -> 3.7
 // and 7.9 -> 3.5, 2^18 cells 20.4 -> 9.4 and 19.5 -> 11.8.  What is left: the
 // chain of dependent FP64 operations of one cell (2 us, a wave alone on its
@@ -374,6 +374,222 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
         for (int r = 0; r < NC; ++r) a.Qout[r * a.pitch + i] = q[k][r];
         a.Cout[i] = c[k];
       }
+    }
+    if (__any(bad) && lane == 0) atomicOr(a.status, 1);
+  }
+  return {s, t, lmax, ok};
+}
+
+// The run of one workgroup, two phases: four waves, one per SIMD, of TW cells
+// each (lanes TW and up repeat the last one in the stages of one lane per
+// cell).  The state's home is LDS, since the faces with a volume-fraction jump
+// are worked on by groups of GL lanes (face_path2, face_path2_hll) that need
+// the states of any face of the wave, and since their quadrature leaves no
+// registers for it.  A diffused interface soon makes every face of a small
+// problem such a face, and a face's 6 (Rusanov) or 18 (HLL) nodes are the
+// longest chain of a step: with TW = 16 all faces of a wave run at once, and a
+// problem of 1000 cells spreads over 24 workgroups; larger problems take wider
+// tiles (more of a problem on the chip, more faces per wave in turn).  GL is
+// that of the step-by-step kernels, whose sums over the nodes it orders.  All
+// face terms but Lax-Friedrichs' fall into the wait for the team's maximum.
+template <int FLUX, int FAST, int TW, int MAXG>
+__device__ __forceinline__ ResOut resident_run2(const ResTeam& a, const MatDev* mat, double relax,
+                                                double relax_p) {
+  constexpr int NC = 30, W = 4, STEP = TW - 2;
+  constexpr int GL = FLUX == FLUX_HLL ? HES_PATH_HLL_LANES : HES_PATH_LANES;
+  __shared__ double cells[W][NC][TW];   // the state
+  __shared__ double path[W][NC][TW];    // jump faces: flux difference (HLL), then the path terms
+  __shared__ double bound[W][3][TW];    // HLL: s_l, s_r, 1 / (s_r - s_l) of the faces
+  __shared__ unsigned char list[W][64]; // the wave's jump faces
+  __shared__ double red[2][W];
+  __shared__ double mine_out[2][RES_HALO][NC], theirs[2][RES_HALO][NC];
+  __shared__ double team_max, tnow[2];
+  __shared__ int dead;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lc = lane < TW ? lane : TW - 1;
+  const long long o0 = a.lo + (long long)a.rank * a.own;
+  const long long o1 = o0 + a.own < a.hi ? o0 + a.own : a.hi;
+  // positions are counted from the workgroup's first own cell
+  const int n_own = (int)(o1 - o0);
+  const int n_lo = o0 - a.lo < (1 << 24) ? (int)(a.lo - o0) : -(1 << 24);
+  const int n_hi = a.hi - o0 < (1 << 24) ? (int)(a.hi - o0) : 1 << 24;
+  const int halo = a.G > 1 ? RES_HALO : 0;
+  const int j = STEP * w + lc - halo;
+  const bool mine = lane < TW && (lc >= 1 || (w == 0 && halo == 0)) &&
+                    (lc <= STEP || (w == W - 1 && halo == 0)) && j >= 0 && j < n_own;
+  const bool moves = lane >= 1 && lane <= STEP && j > n_lo && j < n_hi - 1 && j < n_own + halo;
+  {
+    const int jc = j < n_lo ? n_lo : (j >= n_hi ? n_hi - 1 : j);
+    if (lane < TW) {
+#pragma unroll
+      for (int r = 0; r < NC; ++r) cells[w][r][lane] = a.Qin[r * a.pitch + o0 + jc];
+    }
+  }
+  if (threadIdx.x == 0) dead = 0;
+  double t = a.t, lmax = 0.0, c[2];
+  long long s = 0;
+  int to_halo = RES_HALO;
+  int bad = 0;
+  bool ok = true;
+  for (;; ++s) {
+    double q[NC];
+    auto load = [&]() {
+#pragma unroll
+      for (int r = 0; r < NC; ++r) q[r] = cells[w][r][lc];
+    };
+    load();
+    int b = 0;
+    const double lam = cell_speeds<2, FAST>(mat, q, c, b);
+    bad |= mine && b;
+    const double m = wave_max_dpp(mine ? lam : 0.0);
+    if (lane == 0) red[s & 1][w] = m;
+    res_barrier();
+    lmax = wave_max_dpp(lane < W ? red[s & 1][lane] : 0.0);
+    if (a.G > 1 && w == 0) res_publish(a, s, lmax);
+    // face i+1/2 of this lane: its jump as chunk_step tests it
+    const double a0n = lane_down(q[0]), a1n = lane_down(q[15]);
+    const bool jump = !(((a0n - q[0]) == 0.0) & ((a1n - q[15]) == 0.0)) & (lane < TW - 1) &
+                      (j >= n_lo) & (j < n_hi - 1);
+    const unsigned long long jumps = __ballot(jump);
+    const int faces = __popcll(jumps);
+    if (jump) list[w][__popcll(jumps & ((1ull << lane) - 1ull))] = (unsigned char)lane;
+    auto wait = [&]() {  // for the team's maximum
+      if (a.G == 1) return;
+      if (w == 0) {
+        double lm = 0.0;
+        const bool got = res_collect<MAXG>(a, s, lm);
+        if (lane == 0) {
+          team_max = lm;
+          if (!got) dead = 1;
+        }
+      }
+      res_barrier();
+      lmax = team_max;
+      ok = dead == 0;
+    };
+    // right minus left face flux of every component, without the path terms
+    double smin, smax, df[NC];
+    int b2 = 0;
+    HllCoef hc = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    speed_range2(mat, q, c, smin, smax);
+    if constexpr (FLUX == FLUX_RUSANOV) {
+      if (a.lxf) {  // the face speed dx / dt
+        wait();
+        if (!ok) break;
+      }
+      faces_rusanov2<FAST>(mat, q, smin, smax, a.cfl * rcp(lmax), a.lxf, b2,
+                           [&](int r, double d) { df[r] = d; });
+    } else {
+      double mn, mx;
+      mid_range2<FAST>(mat, q, mn, mx);
+      hc = hll_coef(mn, mx, smin, lane_down(smax));
+      if (lane < TW) {
+        bound[w][0][lane] = hc.s_l;
+        bound[w][1][lane] = hc.s_r;
+        bound[w][2][lane] = hc.isd;
+      }
+      faces_hll2<FAST>(mat, q, hc, b2, [&](int r, double d, double J) {
+        df[r] = d;
+        if (jump) path[w][r][lc] = J;
+      });
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+    for (int k = lane / GL; k < faces; k += 64 / GL) {
+      const int face = list[w][k];
+      if constexpr (FLUX == FLUX_RUSANOV)
+        face_path2<FAST, GL>(mat, &cells[w][0][0], &path[w][0][0], face, TW, lane & (GL - 1));
+      else
+        face_path2_hll_lds<FAST, GL>(mat, &cells[w][0][0], &bound[w][0][0], &path[w][0][0], face,
+                                     TW, lane & (GL - 1));
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (!(FLUX == FLUX_RUSANOV && a.lxf)) {
+      wait();
+      if (!ok) break;
+    }
+    if (s >= a.kmax || !(t < a.t_end)) break;  // main.jl:202 `while t < T`
+    const double dtdx = a.cfl * rcp(lmax);
+    if (w == 0) {  // the time, by one wave
+      const double dt = a.cfl * a.dx / lmax;  // main.jl:212
+      if (lane == 0) {
+        if (a.dt_hist && a.rank == 0) a.dt_hist[s] = dt;
+        tnow[s & 1] = t + dt;
+      }
+    }
+    double upd[NC];
+    load();
+#pragma unroll
+    for (int r = 0; r < NC; ++r) upd[r] = q[r] - dtdx * df[r];
+    if (faces) {
+#pragma unroll
+      for (int r = 0; r < NC; ++r) {
+        const double v = jump ? path[w][r][lc] : 0.0;
+        double dm = v, dp = v;
+        if constexpr (FLUX == FLUX_HLL) {  // the products k_path2_hll stores
+          dm = hc.cl * v;
+          dp = hc.cr * v;
+        }
+        upd[r] -= dtdx * (dm + lane_up_z(dp));  // D- of face i+1/2 + D+ of face i-1/2
+      }
+    }
+    if (moves) {
+      if (relax > 0.0 || relax_p > 0.0) {
+        const double dt = a.cfl * a.dx / lmax;
+        if (relax > 0.0) relax_velocity2(mat, upd, exp(-dt * relax));
+        if (relax_p > 0.0) relax_pressure2<FAST>(mat, upd, dt * relax_p);
+      }
+#pragma unroll
+      for (int r = 0; r < NC; ++r) cells[w][r][lane] = upd[r];
+    }
+    const bool renew = a.G > 1 && --to_halo == 0;  // uniform
+    if (renew && mine) {
+      if (j < RES_HALO) {
+#pragma unroll
+        for (int r = 0; r < NC; ++r) mine_out[0][j][r] = moves ? upd[r] : q[r];
+      }
+      if (j >= n_own - RES_HALO) {
+#pragma unroll
+        for (int r = 0; r < NC; ++r) mine_out[1][j - (n_own - RES_HALO)][r] = moves ? upd[r] : q[r];
+      }
+    }
+    res_barrier();
+    t = tnow[s & 1];
+    if ((lane == 0 && w > 0) || (lane == TW - 1 && w < W - 1)) {
+      const int nb = lane == 0 ? w - 1 : w + 1, nl = lane == 0 ? STEP : 1;
+#pragma unroll
+      for (int r = 0; r < NC; ++r) cells[w][r][lane] = cells[nb][r][nl];
+    }
+    if (renew) {
+      to_halo = RES_HALO;
+      const long long round = (s + 1) / RES_HALO;
+      const unsigned tag = a.tag0 + (unsigned)s;
+      bool got = true;
+      if (w == 0 && a.rank > 0) {
+        res_send<NC>(a, round, tag, 0, &mine_out[0][0][0]);
+        got = res_receive<NC>(a, round, tag, a.rank - 1, 1, &theirs[0][0][0]);
+      }
+      if (w == W - 1 && a.rank < a.G - 1) {
+        res_send<NC>(a, round, tag, 1, &mine_out[1][0][0]);
+        got = res_receive<NC>(a, round, tag, a.rank + 1, 0, &theirs[1][0][0]);
+      }
+      if (!got) dead = 1;  // seen after the next step's barriers
+      res_barrier();
+      const bool left = j < 0 && j >= n_lo;
+      if (lane < TW && (left || (j >= n_own && j < n_own + RES_HALO && j < n_hi))) {
+        const double* e = left ? theirs[0][j + RES_HALO] : theirs[1][j - n_own];
+#pragma unroll
+        for (int r = 0; r < NC; ++r) cells[w][r][lane] = e[r];
+      }
+    }
+  }
+  if (ok) {
+    if (mine) {
+#pragma unroll
+      for (int r = 0; r < NC; ++r) a.Qout[r * a.pitch + o0 + j] = cells[w][r][lc];
+      a.Cout[o0 + j] = c[0];
+      a.Cout[a.pitch + o0 + j] = c[1];
     }
     if (__any(bad) && lane == 0) atomicOr(a.status, 1);
   }

@@ -332,10 +332,11 @@ __device__ __forceinline__ void update_rusanov1(const double* q, const double* f
   }
 }
 
-// One component of the HLL update without path integrals: its state qr and
-// flux fr on this lane and its neighbours, every lane active.
-__device__ __forceinline__ double hll_component(double qr, double fr, const HllCoef& hc,
-                                                double dtdx) {
+// One component of the HLL face fluxes without path integrals, right face
+// minus left face, from its state qr and flux fr on this lane and its
+// neighbours (J: the flux difference of the right face), every lane active.
+__device__ __forceinline__ double hll_difference(double qr, double fr, const HllCoef& hc,
+                                                 double& J) {
   // one register holds the flux for both its uses (shifted to the left
   // neighbour and local): left to itself the compiler may form the two
   // from separate copies of the flux arithmetic, contracted differently,
@@ -343,14 +344,14 @@ __device__ __forceinline__ double hll_component(double qr, double fr, const HllC
   pin(fr);
   // zero-filling shifts (every lane is active here): lane 63's face and
   // lane 0's update read the zeros, and neither is stored
-  const double J = lane_down_z(fr) - fr;
+  J = lane_down_z(fr) - fr;
   const double dq = lane_down_z(qr) - qr;
   // D- + D+ = J at every face (cl + cr = 1), so D-(i+1/2) + D+(i-1/2) =
   // H(i+1/2) - H(i-1/2) with H = F_i + D-(i+1/2), the HLL flux: two
   // fused products per face instead of four, and a uniform state still
   // gives H = F_i exactly
   const double h = fma(hc.cl, J, fma(hc.clr, dq, fr));
-  return qr - dtdx * (h - lane_up_z(h));  // conservative part is zero (NumFluxes.jl:82)
+  return h - lane_up_z(h);
 }
 
 // One phase, HLL: the update of a lane's cell (all of NumFluxes.jl:70-132).
@@ -359,7 +360,9 @@ __device__ __forceinline__ void update_hll1(const double* q, const double* f, co
                                             double dtdx, double* upd) {
 #pragma unroll
   for (int r = 0; r < 14; ++r) {
-    upd[r] = hll_component(q[r], f[r], hc, dtdx);
+    double J;
+    const double d = hll_difference(q[r], f[r], hc, J);
+    upd[r] = q[r] - dtdx * d;  // conservative part is zero (NumFluxes.jl:82)
     if (PIN) pin(upd[r]);
   }
 }
@@ -380,6 +383,94 @@ __device__ __forceinline__ void mid_range1(const MatDev& m, const double* q, dou
   const double c = sound_speed(m, t);
   mn = t.u[0] - c;
   mx = t.u[0] + c;
+}
+
+// Two phases: [min_p(u1 - c_p), max_p(u1 + c_p)] of a cell from its sound
+// speeds, as cell_flux forms it.
+__device__ __forceinline__ void speed_range2(const MatDev* mat, const double* q, const double* cc,
+                                             double& smin, double& smax) {
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const double u1 = phase_u1<false>(mat[p], q[15 * p], q + 15 * p + 1);
+    smin = p == 0 ? u1 - cc[p] : fmin(smin, u1 - cc[p]);
+    smax = p == 0 ? u1 + cc[p] : fmax(smax, u1 + cc[p]);
+  }
+}
+
+// Two phases, HLL: the eigenvalue range of face i+1/2's mid state (the
+// neighbours' sum with volume fraction 2 a_m, see mid_range1).
+template <int FAST>
+__device__ __forceinline__ void mid_range2(const MatDev* mat, const double* q, double& mn,
+                                           double& mx) {
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    double qs[15];
+#pragma unroll
+    for (int r = 0; r < 15; ++r) qs[r] = q[15 * p + r] + lane_down(q[15 * p + r]);
+    Thermo t;
+    thermo<false, FAST>(mat[p], qs[0], qs + 1, t);
+    const double c = sound_speed(mat[p], t);
+    mn = p == 0 ? t.u[0] - c : fmin(mn, t.u[0] - c);
+    mx = p == 0 ? t.u[0] + c : fmax(mx, t.u[0] + c);
+  }
+}
+
+// Two phases, Rusanov without the path terms: out(r, d) receives component r's
+// conservative face fluxes, right face minus left face.  Each component's face
+// flux is formed (as face_rusanov forms it) and consumed in turn, so the
+// neighbour state and the face arrays are never all live at once.  Every lane
+// of the wave is active.
+template <int FAST, class Out>
+__device__ __forceinline__ void faces_rusanov2(const MatDev* mat, const double* q, double smin,
+                                               double smax, double dtdx, int lxf, int& bad,
+                                               Out out) {
+  const double lam_c = fmax(fabs(smin), fabs(smax));  // maximum(abs.(eigvals))
+  const double lam_n = fmax(fabs(lane_down(smin)), fabs(lane_down(smax)));
+  const double hl = lxf ? 0.5 * rcp(dtdx) : 0.5 * fmax(lam_c, lam_n);  // main.jl:47-50
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    Thermo t;
+    thermo<false, FAST>(mat[p], q[15 * p], q + 15 * p + 1, t);
+    bad |= t.bad;
+    double fp[15];
+    fp[0] = 0.0;
+    phase_flux(mat[p], q[15 * p], t, q + 15 * p + 6, fp + 1);
+#pragma unroll
+    for (int k = 0; k < 15; ++k) {
+      const int r = 15 * p + k;
+      // zero-filling shifts (every lane is active): only lane 63's face and
+      // lane 0's update see the zeros, and neither is stored
+      const double qn = lane_down_z(q[r]), fn = lane_down_z(fp[k]);
+      const double cons = 0.5 * (fp[k] + fn) - hl * (qn - q[r]);
+      out(r, cons - lane_up_z(cons));
+    }
+  }
+}
+
+// Two phases, HLL without the path terms (exact for faces without a
+// volume-fraction jump, where all three path integrals of
+// NumFluxes.jl:111-131 vanish), a phase's flux at a time: out(r, d, J)
+// receives component r's face fluxes, right face minus left face, and the
+// flux difference F_i+1 - F_i.
+template <int FAST, class Out>
+__device__ __forceinline__ void faces_hll2(const MatDev* mat, const double* q, const HllCoef& hc,
+                                           int& bad, Out out) {
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    Thermo t;
+    thermo<false, FAST>(mat[p], q[15 * p], q + 15 * p + 1, t);
+    bad |= t.bad;
+    double fp[15];
+    fp[0] = 0.0;
+    phase_flux(mat[p], q[15 * p], t, q + 15 * p + 6, fp + 1);
+#pragma unroll
+    for (int k = 0; k < 15; ++k) {
+      const int r = 15 * p + k;
+      double J;
+      const double d = hll_difference(q[r], fp[k], hc, J);
+      out(r, d, J);
+    }
+  }
 }
 
 // PIN (single phase): each updated component is pinned where it is computed
@@ -419,33 +510,17 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
   // The mid state enters as the neighbours' sum with volume fraction 2 a_m
   // (see mid_range1).
   double mn_m = 0.0, mx_m = 0.0;
-  if (HLL_STREAM && PHASED) {
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      double qs[15];
-#pragma unroll
-      for (int r = 0; r < 15; ++r) qs[r] = q[15 * p + r] + lane_down(q[15 * p + r]);
-      Thermo t;
-      thermo<false, FAST>(a.mat[p], qs[0], qs + 1, t);
-      const double c = sound_speed(a.mat[p], t);
-      mn_m = p == 0 ? t.u[0] - c : fmin(mn_m, t.u[0] - c);
-      mx_m = p == 0 ? t.u[0] + c : fmax(mx_m, t.u[0] + c);
-    }
-  } else if (HLL_STREAM && NPH == 1) {
+  if constexpr (HLL_STREAM && PHASED) {
+    mid_range2<FAST>(a.mat, q, mn_m, mx_m);
+  } else if constexpr (HLL_STREAM) {
     mid_range1<FAST>(a.mat[0], q, mn_m, mx_m);
   }
 
   double f[NC], smin, smax;
   int bad;
-  if (PHASED) {
-    // [min_p(u1 - c_p), max_p(u1 + c_p)] as cell_flux forms it
+  if constexpr (PHASED) {
     bad = 0;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const double u1 = phase_u1<false>(a.mat[p], q[15 * p], q + 15 * p + 1);
-      smin = p == 0 ? u1 - cc[p] : fmin(smin, u1 - cc[p]);
-      smax = p == 0 ? u1 + cc[p] : fmax(smax, u1 + cc[p]);
-    }
+    speed_range2(a.mat, q, cc, smin, smax);
   } else {
     cell_flux<NPH, FAST, NOC>(a.mat, q, cc, f, smin, smax, bad);
   }
@@ -457,41 +532,20 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
   const double dtdx = a.cfl * rcp(lmax);
 
   double upd[NC];
-  if (FLUX == FLUX_RUSANOV && NPH == 1) {
+  if constexpr (FLUX == FLUX_RUSANOV && NPH == 1) {
     update_rusanov1<PIN>(q, f, smin, smax, dtdx, a.lxf, upd);
-  } else if (FLUX == FLUX_RUSANOV && NPH == 2 && PATHBUF) {
-    // Two phases with the half path integrals precomputed (k_path2): each
-    // component's face flux is formed (as face_rusanov forms it) and consumed
-    // in turn, so the neighbour state and the face arrays are never all live
-    // at once; the path terms are added only in waves that have a face with a
-    // volume-fraction jump.
-    const double lam_c = fmax(fabs(smin), fabs(smax));  // maximum(abs.(eigvals))
-    const double lam_n = fmax(fabs(lane_down(smin)), fabs(lane_down(smax)));
-    const double hl = a.lxf ? 0.5 * rcp(dtdx) : 0.5 * fmax(lam_c, lam_n);  // main.jl:47-50
-    // the shifts run with every lane active (not under the lane-dependent
-    // conditions), so each lane sees its right neighbour's volume fractions
+  } else if constexpr (FLUX == FLUX_RUSANOV && PHASED) {
+    // the half path integrals are precomputed (k_path2) and added only in
+    // waves that have a face with a volume-fraction jump; the shifts run with
+    // every lane active (not under the lane-dependent conditions), so each
+    // lane sees its right neighbour's volume fractions
     const double a0n = lane_down(q[0]), a1n = lane_down(q[15]);
     const bool jump = !(((a0n - q[0]) == 0.0) & ((a1n - q[15]) == 0.0)) & (i >= a.lo) &
                       (i < a.hi - 1);
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      Thermo t;
-      thermo<false, FAST>(a.mat[p], q[15 * p], q + 15 * p + 1, t);
-      bad |= t.bad;
-      double fp[15];
-      fp[0] = 0.0;
-      phase_flux(a.mat[p], q[15 * p], t, q + 15 * p + 6, fp + 1);
-#pragma unroll
-      for (int k = 0; k < 15; ++k) {
-        const int r = 15 * p + k;
-        // zero-filling shifts (every lane is active): only lane 63's face and
-        // lane 0's update see the zeros, and neither is stored
-        const double qn = lane_down_z(q[r]), fn = lane_down_z(fp[k]);
-        const double cons = 0.5 * (fp[k] + fn) - hl * (qn - q[r]);
-        upd[r] = q[r] - dtdx * (cons - lane_up_z(cons));  // main.jl:59, conservative part
-        pin(upd[r]);
-      }
-    }
+    faces_rusanov2<FAST>(a.mat, q, smin, smax, dtdx, a.lxf, bad, [&](int r, double d) {
+      upd[r] = q[r] - dtdx * d;  // main.jl:59, conservative part
+      pin(upd[r]);
+    });
     if (__any(jump)) {
       // only the lanes of jump faces load, all 30 rows in one masked region
       // (so the loads issue together), and each touches only the cache lines
@@ -510,35 +564,19 @@ __device__ __forceinline__ double chunk_step(const ChunkCtx& a, long long i, con
         pin(upd[r]);
       }
     }
-  } else if (HLL_STREAM) {
-    // HLL: D-, D+ without path integrals, streamed per component (for one
-    // phase that is all of NumFluxes.jl:70-132; for two phases it is exact for
-    // faces without a volume-fraction jump, where all three path integrals of
-    // NumFluxes.jl:111-131 vanish, and faces with a jump add the difference to
-    // the full D-, D+ precomputed by k_path2_hll).
+  } else if constexpr (HLL_STREAM) {
+    // HLL: D-, D+ without path integrals, streamed per component; two-phase
+    // faces with a jump add the difference to the full D-, D+ precomputed by
+    // k_path2_hll
     const HllCoef hc = hll_coef(mn_m, mx_m, smin, lane_down(smax));
     bool jump = false;
-    if (NPH == 2) {  // shifts with every lane active, as in the Rusanov branch
-      const double a0n = lane_down(q[0]), a1n = lane_down(q[NPH == 2 ? 15 : 0]);
-      jump = !(((a0n - q[0]) == 0.0) & ((a1n - q[NPH == 2 ? 15 : 0]) == 0.0)) & (i >= a.lo) &
-             (i < a.hi - 1);
-    }
-    if (PHASED) {
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        Thermo t;
-        thermo<false, FAST>(a.mat[p], q[15 * p], q + 15 * p + 1, t);
-        bad |= t.bad;
-        double fp[15];
-        fp[0] = 0.0;
-        phase_flux(a.mat[p], q[15 * p], t, q + 15 * p + 6, fp + 1);
-#pragma unroll
-        for (int k = 0; k < 15; ++k) {
-          const int r = 15 * p + k;
-          upd[r] = hll_component(q[r], fp[k], hc, dtdx);
-          pin(upd[r]);
-        }
-      }
+    if constexpr (PHASED) {  // shifts with every lane active, as in the Rusanov branch
+      const double a0n = lane_down(q[0]), a1n = lane_down(q[15]);
+      jump = !(((a0n - q[0]) == 0.0) & ((a1n - q[15]) == 0.0)) & (i >= a.lo) & (i < a.hi - 1);
+      faces_hll2<FAST>(a.mat, q, hc, bad, [&](int r, double d, double) {
+        upd[r] = q[r] - dtdx * d;
+        pin(upd[r]);
+      });
     } else {
       update_hll1<PIN>(q, f, hc, dtdx, upd);
     }
@@ -697,14 +735,6 @@ __device__ __forceinline__ void bnode2(const MatDev* mat, const double* psi, dou
   }
 }
 
-// Sum of v[30] over the 16 lanes of a lane group (every lane of the group active).
-__device__ __forceinline__ void group16_sum(double* v) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1)
-#pragma unroll
-    for (int r = 0; r < 30; ++r) v[r] += __shfl_xor(v[r], o, 16);
-}
-
 // v[g] and v[g + 15] for lane g of a group (g < 15), by selects: indexing a
 // register array with a lane-dependent index would move it to scratch memory.
 __device__ __forceinline__ void rows_of_lane(const double* v, int g, double& lo, double& hi) {
@@ -721,6 +751,25 @@ __device__ __forceinline__ void rows_of_lane(const double* v, int g, double& lo,
 // g of the group), the quadrature nodes spread over the group's lanes: the
 // nodes evaluate the same code on different data, which a wave runs in
 // parallel for all its faces.
+
+// lane ^ O's v within a group of lanes: for O = 1, 2 a move within the quad
+// (DPP quad_perm), else through the LDS crossbar.
+template <int O, int GL>
+__device__ __forceinline__ double group_xor(double v) {
+  if constexpr (O == 1) return dpp_shift_z<0xB1>(v);       // quad_perm [1, 0, 3, 2]
+  else if constexpr (O == 2) return dpp_shift_z<0x4E>(v);  // quad_perm [2, 3, 0, 1]
+  else return __shfl_xor(v, O, GL);
+}
+
+// Sum of v[30] over the GL lanes of a lane group (every lane of the group active).
+template <int GL>
+__device__ __forceinline__ void group_sum(double* v) {
+  if constexpr (GL > 1) {
+#pragma unroll
+    for (int r = 0; r < 30; ++r) v[r] += group_xor<GL / 2, GL>(v[r]);
+    group_sum<GL / 2>(v);
+  }
+}
 
 // Number of lanes per jump face in the Rusanov path-term kernels.
 #ifndef HES_PATH_LANES
@@ -757,10 +806,7 @@ __device__ __forceinline__ void face_path2(const MatDev* mat, const double* __re
                          d);
     }
   }
-#pragma unroll
-  for (int o = GL / 2; o > 0; o >>= 1)
-#pragma unroll
-    for (int r = 0; r < 30; ++r) d[r] += __shfl_xor(d[r], o, GL);
+  group_sum<GL>(d);
 #pragma unroll
   for (int k = 0; k * GL < 30; ++k) {
     double v = 0.0;
@@ -770,15 +816,6 @@ __device__ __forceinline__ void face_path2(const MatDev* mat, const double* __re
     const int r = GL * k + g;
     if (r < 30) D[r * pitch + i] = 0.5 * v;
   }
-}
-
-// Sum of v[30] over the GL lanes of a lane group (every lane of the group active).
-template <int GL>
-__device__ __forceinline__ void group_sum(double* v) {
-#pragma unroll
-  for (int o = GL / 2; o > 0; o >>= 1)
-#pragma unroll
-    for (int r = 0; r < 30; ++r) v[r] += __shfl_xor(v[r], o, GL);
 }
 
 // Number of lanes per jump face in the HLL path-term kernels.
@@ -908,6 +945,83 @@ __device__ __forceinline__ void face_path2_hll(const MatDev* mat, const double* 
       D[r * pitch + i] = hc.cl * v;
       D[(30 + r) * pitch + i] = hc.cr * v;
     }
+  }
+}
+
+// The same two half-path integrals (their sum, rows 0..29 of D) from a state in
+// LDS, for a kernel whose lanes hold one cell each and have formed the face's
+// flux difference (D on entry) and wave-speed bounds (H: s_l, s_r and 1 / (s_r
+// - s_l)) already.  The states are read anew in every node round, behind an
+// offset that the compiler cannot see through, rather than held in registers.
+template <int FAST, int GL = HES_PATH_HLL_LANES>
+__device__ __forceinline__ void face_path2_hll_lds(const MatDev* mat, const double* Q,
+                                                   const double* H, double* D, int i, int pitch,
+                                                   int g) {
+  double bs[30];
+#pragma unroll
+  for (int r = 0; r < 30; ++r) bs[r] = 0.0;
+#pragma unroll 1
+  for (int round = 0; round * GL < 6; ++round) {
+    const int m = g + GL * round;
+    if (m < 6) {
+      int ofs = 0;
+      asm volatile("" : "+v"(ofs));
+      const double* ql = Q + i + ofs;
+      const double s = c_gl_s[m], oms = 1.0 - s;
+      double psi[30];
+#pragma unroll
+      for (int r = 0; r < 30; ++r) psi[r] = ql[r * pitch] * oms + ql[r * pitch + 1] * s;
+      bnode2<FAST, true>(mat, psi, c_gl_w[m], ql[1] - ql[0], ql[15 * pitch + 1] - ql[15 * pitch],
+                         bs);
+    }
+  }
+  group_sum<GL>(bs);
+  const double s_l = H[i], s_r = H[pitch + i], isd = H[2 * pitch + i];
+  double qh[30];
+  const double* ql = Q + i;
+#pragma unroll
+  for (int r = 0; r < 30; ++r) bs[r] = bs[r] + D[r * pitch + i];  // J = B_int + F_r - F_l
+#pragma unroll
+  for (int r = 0; r < 30; ++r)
+    qh[r] = (ql[r * pitch + 1] * s_r - ql[r * pitch] * s_l - bs[r]) * isd;
+  qh[0] = ql[0] + (s_r * (ql[1] - ql[0]) - bs[0]) * isd;
+  qh[15] = ql[15 * pitch] + (s_r * (ql[15 * pitch + 1] - ql[15 * pitch]) - bs[15]) * isd;
+  double bb[30];
+#pragma unroll
+  for (int r = 0; r < 30; ++r) bb[r] = 0.0;
+#pragma unroll 1
+  for (int round = 0; round * GL < 12; ++round) {
+    const int m = g + GL * round;
+    if (m < 12) {
+      const bool first = m < 6;
+      const int k = first ? m : m - 6;
+      // the cell at the segment's other end: Q_l, or Q_r one lane on
+      int ofs = first ? 0 : 1;
+      asm volatile("" : "+v"(ofs));
+      const double* qc = Q + i + ofs;
+      const double s = c_gl_s[k], oms = 1.0 - s;
+      double psi[30];
+#pragma unroll
+      for (int r = 0; r < 30; ++r) {
+        const double c = qc[r * pitch];
+        psi[r] = (first ? c : qh[r]) * oms + (first ? qh[r] : c) * s;
+      }
+      const double c0 = qc[0], c15 = qc[15 * pitch];
+      const double da0 = first ? qh[0] - c0 : c0 - qh[0];
+      const double da1 = first ? qh[15] - c15 : c15 - qh[15];
+      bnode2<FAST, true>(mat, psi, c_gl_w[k], da0, da1, bb);
+    }
+  }
+  group_sum<GL>(bb);
+  // lane g stores rows g, g + GL, g + 2 GL, ... (< 30)
+#pragma unroll
+  for (int k = 0; k * GL < 30; ++k) {
+    double v = 0.0;
+#pragma unroll
+    for (int j = 0; j < GL; ++j)
+      if (GL * k + j < 30) v = g == j ? bb[GL * k + j] : v;
+    const int r = GL * k + g;
+    if (r < 30) D[r * pitch + i] = v;
   }
 }
 

@@ -8,7 +8,8 @@ import pytest
 
 from hyperelasticsolver_amd.EquationsOfState import Barton2009
 from hyperelasticsolver_amd.batched import Batch
-from hyperelasticsolver_amd.initial import prim2cons, random_interfaces, random_phase_prims
+from hyperelasticsolver_amd.initial import (prim2cons, random_interfaces, random_phase_prims,
+                                            random_two_phase_prims)
 from hyperelasticsolver_amd.solver import Solver
 
 pytestmark = pytest.mark.gpu
@@ -56,6 +57,32 @@ def test_resident_equals_stepwise(n, flux):
     for d in a["dt"]:
         t += d
     assert t == t1 and dt > 0.0
+
+
+@pytest.mark.parametrize("flux", ["rusanov", "hll", "lxf"])
+@pytest.mark.parametrize("n", [3, 15, 58, 59, 1000, 10752, 10753, 27136, 27137, 59904, 59905])
+def test_resident_two_phase_equals_stepwise(n, flux):
+    """Rusanov and Lax-Friedrichs to the bit; for HLL the batch sums a face's
+    quadrature nodes in another order (two lanes per face, not four): 1e-13."""
+    print(f"[resident two-phase] n={n} flux={flux}", flush=True)
+    eos = (Barton2009(), Barton2009(_rho0=2.7, _b0=3.1))
+    if n == 1000:
+        eos = (Barton2009(_beta=3.577, _gamma=2.088), Barton2009(_rho0=2.7, _b0=3.1, _beta=3.577, _gamma=2.088))
+    rng = np.random.default_rng(n)
+    k = 6 if n > 60 else 2
+    states = prim2cons(eos, random_two_phase_prims(rng, eos, k))
+    ifc = random_interfaces(rng, k - 1)
+    with Solver(eos, n, flux=flux) as s:
+        s.set_piecewise(states, ifc)
+        a = s.run(steps=STEPS, record_dt=True)
+        s.run(steps=MORE)
+        q = s.get_state()
+    ref, t, _ = _stepwise(eos, n, flux, states, ifc, STEPS + MORE)
+    assert a["steps"] == STEPS and len(a["dt"]) == STEPS
+    if flux != "hll":
+        assert np.array_equal(q, ref)
+    else:
+        assert np.all(np.abs(q - ref).max(axis=1) <= 1e-13 * np.abs(ref).max(axis=1))
 
 
 @pytest.mark.parametrize("n", [200, 1000])
