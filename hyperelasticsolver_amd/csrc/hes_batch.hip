@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "hes_host.hpp"
+#include "hes_resident.hpp"
 #include "hes_step.hpp"
 #include "../../include/hes.h"
 
@@ -107,6 +108,21 @@ __device__ __forceinline__ void atomic_max_pos(unsigned long long* slot, double 
   if (m > 0.0) atomicMax(slot, (unsigned long long)__double_as_longlong(m));
 }
 
+// A material at a wave-uniform address into scalar registers (field by field,
+// through the constant address space).
+__device__ __forceinline__ MatDev uniform_mat(const MatDev* m) {
+  typedef const __attribute__((address_space(4))) MatDev cmat_t;
+  cmat_t* g = (cmat_t*)m;
+  MatDev d;
+  d.rho0 = g->rho0; d.irho0 = g->irho0; d.cv = g->cv; d.t0 = g->t0; d.b0sq = g->b0sq;
+  d.k0 = g->k0; d.alpha = g->alpha; d.beta = g->beta; d.gamma = g->gamma;
+  d.hk0a2 = g->hk0a2; d.k0_2a = g->k0_2a; d.k0_a = g->k0_a; d.cvt0 = g->cvt0;
+  d.icvt0 = g->icvt0; d.hb0sq = g->hb0sq; d.half_a = g->half_a; d.half_b = g->half_b;
+  d.half_g = g->half_g; d.ac_t = g->ac_t; d.ac_s = g->ac_s; d.ac_e = g->ac_e;
+  d.ac_w = g->ac_w; d.fast = g->fast; d.pad = 0;
+  return d;
+}
+
 // One step of one tile (wave-uniform `tile`).
 template <int NPH, int FLUX, int FAST, int PIN>
 __device__ __forceinline__ void batch_tile_step(const BatchArgs& a, int tile) {
@@ -122,18 +138,8 @@ __device__ __forceinline__ void batch_tile_step(const BatchArgs& a, int tile) {
   MatDev mloc[NPH];
   const MatDev* m = a.mats + NPH * p;
   if constexpr (NPH == 2) {
-    typedef const __attribute__((address_space(4))) MatDev cmat_t;
 #pragma unroll
-    for (int k = 0; k < NPH; ++k) {
-      cmat_t* g = (cmat_t*)(m + k);
-      MatDev& d = mloc[k];
-      d.rho0 = g->rho0; d.irho0 = g->irho0; d.cv = g->cv; d.t0 = g->t0; d.b0sq = g->b0sq;
-      d.k0 = g->k0; d.alpha = g->alpha; d.beta = g->beta; d.gamma = g->gamma;
-      d.hk0a2 = g->hk0a2; d.k0_2a = g->k0_2a; d.k0_a = g->k0_a; d.cvt0 = g->cvt0;
-      d.icvt0 = g->icvt0; d.hb0sq = g->hb0sq; d.half_a = g->half_a; d.half_b = g->half_b;
-      d.half_g = g->half_g; d.ac_t = g->ac_t; d.ac_s = g->ac_s; d.ac_e = g->ac_e;
-      d.ac_w = g->ac_w; d.fast = g->fast; d.pad = 0;
-    }
+    for (int k = 0; k < NPH; ++k) mloc[k] = uniform_mat(m + k);
     m = mloc;
   }
   const ChunkCtx ctx = {m,  a.Qin, a.Qout, a.Cin, a.Cout, a.status, a.pitch, lo, hi, cload(a.cfl + p),
@@ -494,6 +500,108 @@ __global__ void k_batch_carry_fin(unsigned long long* slots, long long* plaunch,
   plaunch[p] = launch;
 }
 
+// ---------------------------------------------------------------------------
+// The time loops of the whole batch in one launch, single phase
+// (hes_resident.hpp): a team of workgroups per problem
+// ---------------------------------------------------------------------------
+struct BResTeam {  // a problem's team
+  long long lo, hi;
+  long long slots, border;  // its words in the message buffer
+  int G, own;
+};
+struct BResItem {  // a workgroup's place: rank in the team of a problem
+  int p, rank;
+};
+struct BResOut {
+  double t, lmax;
+  int steps;
+};
+struct BResArgs {
+  const double* __restrict__ Qin;
+  double* __restrict__ Qout;
+  double* __restrict__ Cout;
+  const BResTeam* teams;
+  const BResItem* items;
+  const MatDev* mats;
+  const double* cfl;
+  const double* dx;
+  const double* t_end;
+  const double* tring;
+  unsigned long long* comm;
+  BResOut* out;
+  int* ticket;
+  int* status;
+  long long pitch;
+  int steps, lxf, step;
+  unsigned tag0;
+};
+
+// Workgroups take the teams' places in the order in which they start, not by
+// their block index: whoever waits for a team's missing workgroups then waits
+// for the ones that start next, and those find room because every earlier
+// team is complete and comes to its end.  Three workgroups share a compute
+// unit (one wave of each per SIMD, 168 VGPRs; with two tiles per wave the
+// fluxes wait in LDS, 52 KB of it per workgroup), so that one's waits are
+// filled by the others: the FP64 units are then busy 0.71 of the time (552 VALU
+// instructions per tile and step).  4096 problems of 256 .. 16384 cells, us per
+// step, one launch per step against this: Rusanov 780 -> 398, HLL 830 -> 564;
+// three tiles per wave at two waves per SIMD: 408 and 582; one tile: 516, 680.
+constexpr int BRES_BLOCK = 256, BRES_PER_CU = 3;
+constexpr int BRES_MAX_TEAM = 256;
+template <int FLUX, int FAST, int T>
+__global__ __launch_bounds__(BRES_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
+void k_batch_resident(BResArgs a) {
+  __shared__ int place;
+  if (threadIdx.x == 0) place = atomicAdd(a.ticket, 1);
+  __syncthreads();
+  const int item = __builtin_amdgcn_readfirstlane(place);
+  const int p = cload(&a.items[item].p);
+  const BResTeam* d = a.teams + p;
+  const MatDev mat = uniform_mat(a.mats + p);
+  ResTeam tm;
+  tm.Qin = a.Qin;
+  tm.Qout = a.Qout;
+  tm.Cout = a.Cout;
+  tm.pitch = a.pitch;
+  tm.lo = cload(&d->lo);
+  tm.hi = cload(&d->hi);
+  tm.G = cload(&d->G);
+  tm.rank = cload(&a.items[item].rank);
+  tm.own = cload(&d->own);
+  tm.cfl = cload(a.cfl + p);
+  tm.dx = cload(a.dx + p);
+  tm.t = cload(a.tring + 2 * p + (a.step & 1));
+  tm.t_end = cload(a.t_end + p);
+  tm.kmax = a.steps;
+  tm.dt_hist = nullptr;
+  tm.status = a.status;
+  tm.lxf = a.lxf;
+  tm.slots = a.comm + cload(&d->slots);
+  tm.border = a.comm + cload(&d->border);
+  tm.tag0 = a.tag0;
+  tm.gave_up = a.status + 2;
+  const ResOut o = resident_run1<FLUX, FAST, BRES_BLOCK, T, BRES_MAX_TEAM, (T > 1)>(tm, mat);
+  if (tm.rank == 0 && threadIdx.x == 0) a.out[p] = {o.t, o.lmax, (int)o.steps};
+}
+
+// After a launch in which every team came to its end: each problem's times,
+// step counts and CFL maximum as the step-by-step launches leave them, its
+// state being that of launch index `launch`.
+__global__ void k_batch_resident_end(const BResOut* out, const int* status, int P, long long launch,
+                                     double* tring, int* psteps, long long* plaunch,
+                                     unsigned long long* slots) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P || status[2]) return;
+  const BResOut o = out[p];
+  tring[2 * p] = o.t;
+  tring[2 * p + 1] = o.t;
+  psteps[p] += o.steps;
+  plaunch[p] = launch;
+  slots[3 * p + launch % 3] = (unsigned long long)__double_as_longlong(o.lmax);
+  slots[3 * p + (launch + 1) % 3] = 0ull;
+  slots[3 * p + (launch + 2) % 3] = 0ull;
+}
+
 __global__ void k_soa_to_aos_b(const double* __restrict__ in, double* __restrict__ out, int nc,
                                long long n, long long pitch) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -533,6 +641,18 @@ struct hes_batch {
   hipStream_t stream;
   hipEvent_t ev0, ev1;
   bool has_state;
+  bool ends;  // end times are set: problems may have stopped at earlier launches
+  // the whole loop in one launch (run_batch_resident)
+  int dev, cus;
+  int res_tiles;             // tiles per wave; 0: one launch per step
+  int res_groups;            // workgroups
+  bool res_waits;            // some problem has more than one
+  unsigned res_tag;          // the last tag in its message buffer
+  BResTeam* teams;
+  BResItem* items;
+  BResOut* res_out;
+  unsigned long long* comm;  // a ticket counter, all slots, all halo words
+  long long comm_clear;      // leading words to clear before a launch
 };
 
 namespace {
@@ -654,6 +774,154 @@ int batch_carry(hes_batch* h) {
   return HES_OK;
 }
 
+// ---- the whole loop in one launch ------------------------------------------------
+
+constexpr long long BRES_STEPS = 1LL << 16;  // steps of one launch at most
+
+// Teams for every problem, with one tile per wave or two.  One has the shorter
+// chain of work per step and wastes less of a short problem's last wave, two
+// need fewer exchanges and, the chip full, 1.27 times less time per tile (516
+// against 398 us above).  So one when all its workgroups are on the chip at
+// once (64 problems of 100 .. 3000 cells: 3.7 against 5.0 us per step) or when
+// its tiles are that many fewer (1000 of 60 .. 700 cells: 12.5 against 14.5),
+// else two, the largest problems first.  None if a problem does not fit.
+hipError_t plan_batch_resident(hes_batch* h) {
+  h->res_tiles = 0;
+  if (h->nph != 1) return hipSuccess;
+  std::vector<BResTeam> teams(h->P);
+  int most = 0;
+  auto fit = [&](int t) -> long long {  // workgroups with t tiles per wave
+    const long long one = BRES_BLOCK / 64 * t * TILE + 2, per = one - 2 * RES_HALO;
+    long long groups = 0;
+    most = 0;
+    for (int p = 0; p < h->P; ++p) {
+      const long long n = h->offsets_h[p + 1] - h->offsets_h[p];
+      const long long g = n <= one ? 1 : (n + per - 1) / per;
+      if (g > std::min(h->cus, BRES_MAX_TEAM)) return -1;
+      teams[p].lo = h->offsets_h[p];
+      teams[p].hi = h->offsets_h[p + 1];
+      teams[p].G = (int)g;
+      teams[p].own = (int)((n + g - 1) / g);
+      most = std::max(most, (int)g);
+      groups += g;
+    }
+    return groups;
+  };
+  const long long groups2 = fit(2), groups1 = fit(1);
+  const bool one = groups1 >= 0 && (groups1 <= BRES_PER_CU * h->cus || 1.27 * groups1 < 2.0 * groups2);
+  const long long groups = one ? groups1 : fit(2);
+  const int tiles = one ? 1 : 2;
+  if (groups < 0 || groups > 0x7fffffffLL) return hipSuccess;
+  h->res_waits = most > 1;
+  std::vector<int> order(h->P);
+  for (int p = 0; p < h->P; ++p) order[p] = p;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    return teams[x].hi - teams[x].lo > teams[y].hi - teams[y].lo;
+  });
+  std::vector<BResItem> items;
+  items.reserve((size_t)groups);
+  long long at = 1;  // after the ticket counter
+  for (int p : order) {
+    for (int r = 0; r < teams[p].G; ++r) items.push_back({p, r});
+    teams[p].slots = at;
+    if (teams[p].G > 1) at += 2LL * teams[p].G * RES_SLOT;
+  }
+  h->comm_clear = at;
+  for (int p : order) {
+    teams[p].border = at;
+    if (teams[p].G > 1) at += 2LL * teams[p].G * 2 * RES_HALO * 2 * h->nc;
+  }
+  hipError_t e = hipMalloc((void**)&h->teams, sizeof(BResTeam) * teams.size());
+  if (e == hipSuccess) e = hipMalloc((void**)&h->items, sizeof(BResItem) * items.size());
+  if (e == hipSuccess) e = hipMalloc((void**)&h->res_out, sizeof(BResOut) * (size_t)h->P);
+  if (e == hipSuccess) e = hipMalloc((void**)&h->comm, sizeof(unsigned long long) * (size_t)at);
+  if (e == hipSuccess) e = hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * (size_t)at, h->stream);
+  if (e == hipSuccess)
+    e = copy_on(h->stream, h->teams, teams.data(), sizeof(BResTeam) * teams.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = copy_on(h->stream, h->items, items.data(), sizeof(BResItem) * items.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    h->res_tiles = tiles;
+    h->res_groups = (int)groups;
+  }
+  return e;
+}
+
+template <int FLUX, int FAST>
+void launch_batch_resident(const hes_batch* h, const BResArgs& a) {
+  const dim3 grid((unsigned)h->res_groups), block(BRES_BLOCK);
+  if (h->res_tiles == 1)
+    hipLaunchKernelGGL((k_batch_resident<FLUX, FAST, 1>), grid, block, 0, h->stream, a);
+  else
+    hipLaunchKernelGGL((k_batch_resident<FLUX, FAST, 2>), grid, block, 0, h->stream, a);
+}
+
+// `steps` (<= BRES_STEPS) steps of every problem in one launch.  *gave_up: no
+// result (a team's workgroups were not on the chip together), the batch is as
+// before.  Adds to *ms the launch's time.
+int run_batch_resident(hes_batch* h, long long steps, float* ms, bool* gave_up) {
+  if (h->ends) {  // problems that stopped at an earlier launch
+    const int rc = batch_carry(h);
+    if (rc != HES_OK) return rc;
+  }
+  const long long s0 = h->step;
+  BResArgs a;
+  a.Qin = h->Q[s0 & 1];
+  a.Qout = h->Q[(s0 + 1) & 1];
+  a.Cout = h->C[(s0 + 1) & 1];
+  a.teams = h->teams;
+  a.items = h->items;
+  a.mats = h->mats;
+  a.cfl = h->cfl;
+  a.dx = h->dx;
+  a.t_end = h->t_end;
+  a.tring = h->tring;
+  a.comm = h->comm;
+  a.out = h->res_out;
+  a.ticket = (int*)h->comm;
+  a.status = h->status;
+  a.pitch = h->pitch;
+  a.steps = (int)steps;
+  a.lxf = h->flux == HES_FLUX_LXF;
+  a.step = (int)(s0 & 1);
+  a.tag0 = h->res_tag + 1;
+  h->res_tag += (unsigned)steps + 1;
+  int st[4] = {0, 0, 0, 0};
+  {
+    ComputeUnits units(h->dev, h->cus, h->res_waits ? h->cus : 0);
+    HIP_TRY(hipEventRecord(h->ev0, h->stream));
+    HIP_TRY(hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * (size_t)h->comm_clear, h->stream));
+    if (h->flux == HES_FLUX_HLL)
+      h->fast ? launch_batch_resident<FLUX_HLL, 1>(h, a) : launch_batch_resident<FLUX_HLL, 0>(h, a);
+    else
+      h->fast ? launch_batch_resident<FLUX_RUSANOV, 1>(h, a)
+              : launch_batch_resident<FLUX_RUSANOV, 0>(h, a);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_batch_resident_end, dim3((unsigned)((h->P + 127) / 128)), dim3(128), 0,
+                       h->stream, h->res_out, h->status, h->P, s0 + steps, h->tring, h->psteps,
+                       h->plaunch, h->slots);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipEventRecord(h->ev1, h->stream));
+    HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
+  }
+  *gave_up = st[2] != 0;
+  if (*gave_up) {
+    h->res_tiles = 0;  // step by step from here on
+    HIP_TRY(zero_on(h->stream, h->status + 2, sizeof(int)));
+    return HES_OK;
+  }
+  float one = 0.f;
+  HIP_TRY(hipEventElapsedTime(&one, h->ev0, h->ev1));
+  *ms += one;
+  h->step = s0 + steps;
+  if ((steps & 1) == 0) {  // the result is where an odd number of steps would have left it
+    std::swap(h->Q[0], h->Q[1]);
+    std::swap(h->C[0], h->C[1]);
+  }
+  if (st[0]) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
+  return HES_OK;
+}
+
 int batch_init_speeds(hes_batch* h) {
   long long s = h->step;
   HIP_TRY(hipMemsetAsync(h->slots, 0, sizeof(unsigned long long) * 3 * h->P, h->stream));
@@ -697,7 +965,7 @@ int hes_batch_destroy(hes_batch* h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   void* ptrs[] = {h->Q[0], h->Q[1], h->C[0], h->C[1], h->tiles, h->offsets, h->mats, h->cfl,
                   h->dx, h->t_end, h->tring, h->slots, h->psteps, h->status, h->dpath, h->jcnt,
-                  h->jlist, h->jprob, h->plaunch};
+                  h->jlist, h->jprob, h->plaunch, h->teams, h->items, h->res_out, h->comm};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
@@ -715,7 +983,12 @@ int hes_batch_create(hes_batch** out, int nphase, int flux, int nproblems, const
   if (flux != HES_FLUX_RUSANOV && flux != HES_FLUX_HLL && flux != HES_FLUX_LXF)
     return fail(HES_ERR_ARG, "unknown flux");
   if (nproblems < 1 || !ncells || !materials) return fail(HES_ERR_ARG, "null argument");
+  int dev = 0, cus = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   hes_batch* h = new hes_batch();
+  h->dev = dev;
+  h->cus = cus;
   h->nph = nphase;
   h->flux = flux;
   h->nc = nphase == 1 ? 14 : 30;
@@ -789,6 +1062,7 @@ int hes_batch_create(hes_batch** out, int nphase, int flux, int nproblems, const
   up((void**)&h->psteps, nullptr, sizeof(int) * nproblems);
   up((void**)&h->plaunch, nullptr, sizeof(long long) * nproblems);
   up((void**)&h->status, nullptr, sizeof(int) * 4);
+  if (e == hipSuccess) e = plan_batch_resident(h);
   if (e == hipSuccess) e = hipEventCreate(&h->ev0);
   if (e == hipSuccess) e = hipEventCreate(&h->ev1);
   if (e != hipSuccess) {
@@ -819,6 +1093,7 @@ int hes_batch_set_t_end(hes_batch* h, const double* t_end) {
     if (rc != HES_OK) return rc;
   }
   std::vector<double> v(h->P, INFINITY);
+  h->ends = t_end != nullptr;
   if (t_end)
     for (int p = 0; p < h->P; ++p) v[p] = t_end[p];
   HIP_TRY(copy_on(h->stream, h->t_end, v.data(), sizeof(double) * h->P, hipMemcpyHostToDevice));
@@ -929,12 +1204,28 @@ int hes_batch_set_launch(hes_batch* h, int block, int xcd, int tiles_per_wave) {
   return HES_OK;
 }
 
-// mode 0: one batched launch per step; 1: the whole step loop captured in one
-// hipGraph and launched once; 2: one launch per problem per step.
+// mode 0: one batched launch per step; 1: the whole step loop in one launch
+// (single phase, problems that fit the chip), else captured in one hipGraph
+// and launched once; 2: one launch per problem per step.
 int hes_batch_run(hes_batch* h, long long steps, int mode, float* elapsed_ms) {
   if (!h) return fail(HES_ERR_ARG, "null handle");
   if (!h->has_state) return fail(HES_ERR_ARG, "no state set");
   if (steps < 0 || mode < 0 || mode > 2) return fail(HES_ERR_ARG, "bad argument");
+  float before = 0.f;
+  if (mode == 1) {
+    while (steps > 0 && h->res_tiles) {
+      const long long k = std::min(steps, BRES_STEPS);
+      bool gave_up = false;
+      const int rc = run_batch_resident(h, k, &before, &gave_up);
+      if (rc != HES_OK) return rc;
+      if (gave_up) break;
+      steps -= k;
+    }
+    if (steps == 0) {
+      if (elapsed_ms) *elapsed_ms = before;
+      return HES_OK;
+    }
+  }
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   if (mode == 1 && steps > 0) {
@@ -974,7 +1265,7 @@ int hes_batch_run(hes_batch* h, long long steps, int mode, float* elapsed_ms) {
   }
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
-  if (elapsed_ms) *elapsed_ms = ms;
+  if (elapsed_ms) *elapsed_ms = before + ms;
   h->step += steps;
   int st = 0;
   HIP_TRY(copy_on(h->stream, &st, h->status, sizeof(int), hipMemcpyDeviceToHost));

@@ -211,13 +211,15 @@ __device__ __forceinline__ bool res_receive(const ResTeam& a, long long round, u
 // flux and for its speed (k_step forms it twice, for the state it reads and
 // the one it writes); with one tile per wave and registers to keep it, the
 // flux, and always HLL's mid state, fall into the wait for the team's maximum.
-template <int FLUX, int FAST, int BLK, int T, int MAXG>
+template <int FLUX, int FAST, int BLK, int T, int MAXG, bool FLUX_LDS = false>
 __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& mat) {
   constexpr int NC = 14, W = BLK / 64, NT = W * T;
   constexpr bool LATE_FLUX = T == 1 && BLK < 1024;
   __shared__ double edge[2][NT][2][NC];  // new first and last updated cell of every tile, by parity
   __shared__ double red[2][W];           // every wave's maximum, by parity
   __shared__ double mine_out[2][RES_HALO][NC], theirs[2][RES_HALO][NC];
+  // FLUX_LDS: the 11 components of every cell's flux that are not zero
+  __shared__ double flux[FLUX_LDS ? NT : 1][FLUX_LDS ? 11 : 1][64];
   __shared__ double team_max, tnow[2];
   __shared__ int dead;
   const int lane = threadIdx.x & 63;
@@ -260,6 +262,11 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
       bad |= own && (th.bad | !(c[k] < 1e300));
       m = fmax(m, own ? fabs(u1[k]) + c[k] : 0.0);
       if (!LATE_FLUX) phase_flux(mat, 1.0, th, q[k] + 5, f[k]);
+      if (FLUX_LDS) {
+#pragma unroll
+        for (int r = 0, z = 0; r < NC; ++r)
+          if (r < 5 || (r - 5) % 3) flux[w * T + k][z++][lane] = f[k][r];
+      }
     }
     m = wave_max_dpp(m);
     if (lane == 0) red[s & 1][w] = m;
@@ -300,6 +307,10 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
 #pragma unroll
     for (int k = 0; k < T; ++k) {
       const double smin = u1[k] - c[k], smax = u1[k] + c[k];
+      if (FLUX_LDS) {
+#pragma unroll
+        for (int r = 0, z = 0; r < NC; ++r) f[k][r] = r < 5 || (r - 5) % 3 ? flux[w * T + k][z++][lane] : 0.0;
+      }
       double upd[NC];
       if (FLUX == FLUX_RUSANOV)
         update_rusanov1<true>(q[k], f[k], smin, smax, dtdx, a.lxf, upd);

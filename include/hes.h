@@ -77,8 +77,11 @@ int hes_solver_time(hes_solver* h, double* t, long long* steps);
 int hes_solver_next_dt(hes_solver* h, double* dt);
 
 /* Advance while steps < max_steps and t < t_end (main.jl:202 `while t < T`;
- * pass INFINITY for a fixed step count).  use_graph replays the launches of
- * each 60-step chunk from a captured hipGraph.  Outputs may be NULL:
+ * pass INFINITY for a fixed step count).  A problem that fits the chip (up to
+ * about 377000 cells, two phases 59000, HLL 27000) runs in one launch for all
+ * its steps; a larger one takes one launch (sequence) per step, and use_graph
+ * replays those of each 60-step chunk from a captured hipGraph.  Outputs may
+ * be NULL:
  * steps_done, t_now, elapsed_ms (HIP events on the solver stream around the
  * whole run) and dt_out (max_steps doubles: the dt of every executed step). */
 int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_graph,
@@ -147,7 +150,9 @@ int hes_batch_set_t_end(hes_batch* h, const double* t_end);
  * many cells). */
 int hes_batch_set_launch(hes_batch* h, int block, int xcd, int tiles_per_wave);
 /* Advance every problem by `steps` steps.  mode 0: one launch per step;
- * 1: the whole step loop captured in one hipGraph and launched once;
+ * 1: the whole step loop at once: one launch in which a team of workgroups
+ * holds each problem on the chip (one phase, problems of up to about 60000
+ * cells), else captured in one hipGraph and launched once;
  * 2: one launch per problem per step (the per-problem loop). */
 int hes_batch_run(hes_batch* h, long long steps, int mode, float* elapsed_ms);
 /* Time every launch shape (block 64/256 x XCD order on/off x 1, 2 or 4 tiles

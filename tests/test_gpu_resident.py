@@ -120,3 +120,35 @@ def test_resident_teams_from_two_threads():
         t.join()
     ref, _, _ = _stepwise(eos, n, "rusanov", states, ifc, 200)
     assert np.array_equal(got[0], ref) and np.array_equal(got[1], ref)
+
+
+# lengths around what one workgroup holds (one and two tiles per wave), teams,
+# and a last workgroup of a few cells
+LENGTHS = [3, 64, 250, 251, 498, 499, 702, 965, 1000, 5000]
+
+
+@pytest.mark.parametrize("flux", ["rusanov", "hll", "lxf"])
+@pytest.mark.parametrize("copies", [1, 160])  # one tile per wave; two (more than the chip at once)
+def test_resident_batch_equals_stepwise(flux, copies):
+    print(f"[resident batch] flux={flux} copies={copies}", flush=True)
+    n = LENGTHS * copies
+    general = flux == "hll" and copies == 1
+    eos = [Barton2009(_b0=2.1 * (1 + 0.01 * (p % 7)), **({"_beta": 3.577, "_gamma": 2.088} if general else {}))
+           for p in range(len(n))]
+    data = [_problem(e, m, p % 40) for p, (e, m) in enumerate(zip(eos, n))]
+    got = []
+    for mode in ("eager", "graph"):
+        with Batch(eos, n, flux=flux) as b:
+            b.set_piecewise([d[0] for d in data], [d[1] for d in data])
+            b.run(STEPS, mode=mode)
+            first = b.get_state()
+            t, _ = b.times()
+            end = np.where(np.arange(len(n)) % 3 == 0, 1.2 * t, np.inf)  # some stop, at their own steps
+            b.set_t_end(end)
+            b.run(MORE, mode=mode)
+            b.run(1, mode="eager")  # and on, a launch per step
+            b.run(MORE, mode=mode)
+            got.append((first, b.get_state(), *b.times()))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    assert got[0][3].min() < STEPS + 2 * MORE + 1 == got[0][3].max()
