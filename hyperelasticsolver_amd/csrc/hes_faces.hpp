@@ -140,6 +140,95 @@ __device__ __forceinline__ void bcol2(const MatDev* mat, const double* q, BCol& 
   }
 }
 
+// Neighbour values within a wave: lane_down(v) is lane + 1's v (lane 63 keeps
+// its own), lane_up(v) is lane - 1's v (lane 0 keeps its own), as
+// __shfl_down / __shfl_up by 1.  By default they are the wave-wide DPP shifts
+// (wave_shl:1 / wave_shr:1, plain VALU moves); HES_DPP_SHIFT=0 selects the LDS
+// crossbar (ds_bpermute) instead.
+#ifndef HES_DPP_SHIFT
+#define HES_DPP_SHIFT 1
+#endif
+#if HES_DPP_SHIFT
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift(double v) {
+  const long long b = __double_as_longlong(v);
+  int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+  lo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
+  hi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double lane_down(double v) { return dpp_shift<0x130>(v); }  // wave_shl:1
+__device__ __forceinline__ double lane_up(double v) { return dpp_shift<0x138>(v); }    // wave_shr:1
+// The same shifts writing zero into the lane that has no source (lane 63 for
+// lane_down_z, lane 0 for lane_up_z) or whose source lane is inactive, so
+// they are only used where every lane of the wave is active: never under a
+// lane-dependent condition (a && or ?: whose other operand varies by lane).  With no old value to keep, the shifted
+// copy goes straight into a new register: one DPP move per half, where
+// lane_down / lane_up first copy the value (the original stays live).  For
+// values whose boundary-lane result only reaches the halo lanes' own face and
+// update, which are never stored.
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift_z(double v) {
+  const long long b = __double_as_longlong(v);
+  int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+  lo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true);
+  hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double lane_down_z(double v) { return dpp_shift_z<0x130>(v); }
+__device__ __forceinline__ double lane_up_z(double v) { return dpp_shift_z<0x138>(v); }
+#else
+__device__ __forceinline__ double lane_down(double v) { return __shfl_down(v, 1); }
+__device__ __forceinline__ double lane_up(double v) { return __shfl_up(v, 1); }
+__device__ __forceinline__ double lane_down_z(double v) { return __shfl_down(v, 1); }
+__device__ __forceinline__ double lane_up_z(double v) { return __shfl_up(v, 1); }
+#endif
+
+// lane ^ O's v within a group of lanes: for O = 1, 2 a move within the quad
+// (DPP quad_perm), else through the LDS crossbar.
+template <int O, int GL>
+__device__ __forceinline__ double group_xor(double v) {
+  if constexpr (O == 1) return dpp_shift_z<0xB1>(v);       // quad_perm [1, 0, 3, 2]
+  else if constexpr (O == 2) return dpp_shift_z<0x4E>(v);  // quad_perm [2, 3, 0, 1]
+  else return __shfl_xor(v, O, GL);
+}
+
+// Sum of v[30] over the GL lanes of a lane group (every lane of the group active).
+template <int GL>
+__device__ __forceinline__ void group_sum(double* v) {
+  if constexpr (GL > 1) {
+#pragma unroll
+    for (int r = 0; r < 30; ++r) v[r] += group_xor<GL / 2, GL>(v[r]);
+    group_sum<GL / 2>(v);
+  }
+}
+
+// One quadrature node's share of a path integral (NumFluxes.jl:39-47, 97-107):
+// w b^p(psi) da_p in the rows of phase block p, where psi is the state at the
+// node, b^p the non-zero column of B's block p and da_p the volume-fraction
+// jump of the path.  The integral is the sum over the nodes.
+// ACC: add the share to out instead of writing it.
+template <int FAST, bool ACC = false>
+__device__ __forceinline__ void bnode2(const MatDev* mat, const double* psi, double w, double da0,
+                                       double da1, double* out) {
+  BCol b;
+  bcol2<FAST>(mat, psi, b);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const double wd = w * (p == 0 ? da0 : da1);
+    double* o = out + 15 * p;
+    auto put = [&](int r, double v) { o[r] = ACC ? o[r] + v : v; };
+    put(0, wd * b.uI0);
+    if (!ACC) o[1] = 0.0;
+    put(2, wd * b.sI[0]);
+    put(3, wd * b.sI[1]);
+    put(4, wd * b.sI[2]);
+    put(5, wd * b.sIu);
+#pragma unroll
+    for (int r = 0; r < 9; ++r) put(6 + r, wd * b.a[p][r]);
+  }
+}
+
 // Integral of B(psi) dpsi/ds along psi(s) = qa (1 - s) + qb s over [0,1]
 // (NumFluxes.jl:97-107 / 39-47).  B has one non-zero column per phase block,
 // so the integral is (sum_q w_q b^p(psi_q)) times the volume-fraction jump.
@@ -191,9 +280,30 @@ __device__ void bint2(const MatDev* mat, const double* qa, const double* qb, dou
   }
 }
 
+// The same integral by a group of GL lanes that all hold qa and qb, the nodes
+// spread over the lanes (node m on lane m mod GL): every lane receives it.
+template <bool LOBATTO, int FAST, int GL>
+__device__ __forceinline__ void bint2_group(const MatDev* mat, const double* qa, const double* qb,
+                                            double* out) {
+  const int g = threadIdx.x & (GL - 1);
+#pragma unroll
+  for (int r = 0; r < 30; ++r) out[r] = 0.0;
+  if (qb[0] - qa[0] == 0.0 && qb[15] - qa[15] == 0.0) return;  // the whole group
+#pragma unroll 1
+  for (int m = g; m < 6; m += GL) {
+    const double s = LOBATTO ? c_lo_s[m] : c_gl_s[m], oms = 1.0 - s;
+    double psi[30];
+#pragma unroll
+    for (int r = 0; r < 30; ++r) psi[r] = qa[r] * oms + qb[r] * s;
+    bnode2<FAST, true>(mat, psi, LOBATTO ? c_lo_w[m] : c_gl_w[m], qb[0] - qa[0], qb[15] - qa[15], out);
+  }
+  group_sum<GL>(out);
+}
+
 // Rusanov / LxF face (NumFluxes.jl:25-60): conservative flux and the common
 // half path integral D- = D+.
-template <int NPH, int FAST = -1>
+// GL: lanes of a group that evaluate the same face.
+template <int NPH, int FAST = -1, int GL = 1>
 __device__ __forceinline__ void face_rusanov(const MatDev* mat, const double* ql, const double* qr,
                                              const double* fl, const double* fr, double lam,
                                              double* cons, double* dmp) {
@@ -202,7 +312,8 @@ __device__ __forceinline__ void face_rusanov(const MatDev* mat, const double* ql
 #pragma unroll
   for (int r = 0; r < NC; ++r) cons[r] = 0.5 * (fl[r] + fr[r]) - hl * (qr[r] - ql[r]);
   if (NPH == 2) {
-    bint2<true, FAST>(mat, ql, qr, dmp);
+    if constexpr (GL == 1) bint2<true, FAST>(mat, ql, qr, dmp);
+    else bint2_group<true, FAST, GL>(mat, ql, qr, dmp);
 #pragma unroll
     for (int r = 0; r < NC; ++r) dmp[r] = 0.5 * dmp[r];
   }
@@ -253,8 +364,8 @@ __device__ __forceinline__ void mid_speed_range(const MatDev* mat, const double*
 
 // HLL face (NumFluxes.jl:70-132): D- and D+ (the conservative part is zero).
 // smin_l = min eig of the left cell, smax_r = max eig of the right cell.  When
-// coef is given it receives the coefficients used.
-template <int NPH, int FAST = -1>
+// coef is given it receives the coefficients used.  GL as for face_rusanov.
+template <int NPH, int FAST = -1, int GL = 1>
 __device__ __forceinline__ void face_hll(const MatDev* mat, const double* ql, const double* qr,
                                          const double* fl, const double* fr, double smin_l,
                                          double smax_r, double* dm, double* dp,
@@ -275,8 +386,12 @@ __device__ __forceinline__ void face_hll(const MatDev* mat, const double* ql, co
     }
   } else {
     // path_int = B_int(Q_l, Q_r) + F(Q_r) - F(Q_l)
+    auto integral = [&](const double* qa, const double* qb, double* out) {
+      if constexpr (GL == 1) bint2<false, FAST>(mat, qa, qb, out);
+      else bint2_group<false, FAST, GL>(mat, qa, qb, out);
+    };
     double J[NC];
-    bint2<false, FAST>(mat, ql, qr, J);
+    integral(ql, qr, J);
 #pragma unroll
     for (int r = 0; r < NC; ++r) J[r] = J[r] + (fr[r] - fl[r]);
     // Q_hll; the volume-fraction rows are written as a_l + (s_r (a_r - a_l) - P)/(s_r - s_l),
@@ -289,10 +404,10 @@ __device__ __forceinline__ void face_hll(const MatDev* mat, const double* ql, co
     double b[NC];
 #pragma unroll
     for (int r = 0; r < NC; ++r) J[r] = fr[r] - fl[r];
-    bint2<false, FAST>(mat, ql, qh, b);
+    integral(ql, qh, b);
 #pragma unroll
     for (int r = 0; r < NC; ++r) J[r] = J[r] + b[r];
-    bint2<false, FAST>(mat, qh, qr, b);
+    integral(qh, qr, b);
 #pragma unroll
     for (int r = 0; r < NC; ++r) {
       double Jr = J[r] + b[r];

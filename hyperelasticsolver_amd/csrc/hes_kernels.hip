@@ -410,7 +410,7 @@ __global__ __launch_bounds__(64) void k_point(int op, const double* __restrict__
     double cc[NPH];
     out[i] = cell_speeds<NPH>(mat, q, cc, bad);
   }
-  if (bad) atomicOr(status, 1);
+  if (bad) *status = 1;  // may be host memory: a store, not an atomic
 }
 
 // EquationsOfState point functions: energy / entropy / stress / acoustic.
@@ -486,18 +486,24 @@ __global__ __launch_bounds__(64) void k_eos(int op, MatDev m, const double* __re
   } else if (op == EOS_INVARIANTS) {  // Strains.jl:46-52
     invariants_gen(v9 + 9 * i, out + 3 * i);
   }
-  if (bad) atomicOr(status, 1);
+  if (bad) *status = 1;
 }
 
-// Face fluxes for arrays of face states (NumFluxes.lxf / hll).
-template <int NPH, int FLUX>
+// Face fluxes for arrays of face states (NumFluxes.lxf / hll), a group of GL
+// lanes per face.  A two-phase face is a chain of 6 (lxf) or 18 (hll)
+// quadrature nodes on one lane (k_face<2, 1>: 31 us for a single face); with 16
+// lanes per face a segment's six nodes run at once.  All lanes of a group do the rest
+// of the face's work alike, which a chip full of faces would pay for: see
+// FACE_GROUP_MAX.
+template <int NPH, int FLUX, int GL>
 __global__ __launch_bounds__(64) void k_face(const double* __restrict__ QL, const double* __restrict__ QR,
                        const double* __restrict__ aux, double* __restrict__ cons,
                        double* __restrict__ dm, double* __restrict__ dp, long long n, MatDev m0,
                        MatDev m1) {
   constexpr int NC = NComp<NPH>::value;
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / GL;
+  if (i >= n) return;  // whole groups
+  const int g = threadIdx.x & (GL - 1);
   MatDev mat[2] = {m0, m1};
   double ql[NC], qr[NC], fl[NC], fr[NC];
 #pragma unroll
@@ -509,23 +515,26 @@ __global__ __launch_bounds__(64) void k_face(const double* __restrict__ QL, cons
   int bad;
   cell_flux<NPH>(mat, ql, cc, fl, s0, s1, bad);
   cell_flux<NPH>(mat, qr, cc, fr, s0, s1, bad);
+  double c[NC], a[NC], b[NC];
   if (FLUX == FLUX_RUSANOV) {
-    double c[NC], d[NC];
-    face_rusanov<NPH>(mat, ql, qr, fl, fr, aux[i], c, d);
+    face_rusanov<NPH, -1, GL>(mat, ql, qr, fl, fr, aux[i], c, a);
+#pragma unroll
     for (int r = 0; r < NC; ++r) {
-      cons[i * NC + r] = c[r];
-      dm[i * NC + r] = NPH == 2 ? d[r] : 0.0;
-      dp[i * NC + r] = NPH == 2 ? d[r] : 0.0;
+      if (NPH == 1) a[r] = 0.0;
+      b[r] = a[r];
     }
   } else {
     // aux holds [min eig of left, max eig of right] per face
-    double a[NC], b[NC];
-    face_hll<NPH>(mat, ql, qr, fl, fr, aux[2 * i], aux[2 * i + 1], a, b);
-    for (int r = 0; r < NC; ++r) {
-      cons[i * NC + r] = 0.0;
-      dm[i * NC + r] = a[r];
-      dp[i * NC + r] = b[r];
-    }
+    face_hll<NPH, -1, GL>(mat, ql, qr, fl, fr, aux[2 * i], aux[2 * i + 1], a, b);
+#pragma unroll
+    for (int r = 0; r < NC; ++r) c[r] = 0.0;
+  }
+#pragma unroll
+  for (int r = 0; r < NC; ++r) {
+    if ((r & (GL - 1)) != g) continue;  // lane g stores rows g, g + GL, ...
+    cons[i * NC + r] = c[r];
+    dm[i * NC + r] = a[r];
+    dp[i * NC + r] = b[r];
   }
 }
 
@@ -1293,27 +1302,134 @@ int hes_copy_bandwidth(long long bytes, int reps, double* gbs) {
   return HES_OK;
 }
 
+}  // extern "C"
+
 // ---------------------------------------------------------------------------
 // Point-wise API (host arrays, synchronous)
 // ---------------------------------------------------------------------------
 namespace {
 
-struct DevBuf {
-  double* p = nullptr;
-  ~DevBuf() { if (p) (void)hipFree(p); }
-  hipError_t alloc(size_t n) { return hipMalloc(&p, n * sizeof(double) + 8); }
+// What a call works in: page-locked host memory that the kernels read and
+// write themselves (small calls: no copies), device memory (larger ones), and
+// a stream of its own.  Allocated for every call they cost one on a single
+// state 90 of its 100 us.  One per call that is under way; at most SPACES_KEPT
+// wait for the next, per device, with at most Space::DEVICE bytes each.
+struct Space {
+  static constexpr size_t HOST = 128 * 1024, DEVICE = 96 << 20;
+  int dev = 0;
+  char* host = nullptr;
+  char* device = nullptr;
+  size_t device_bytes = 0;
+  hipStream_t stream = nullptr;
 };
+constexpr size_t SPACES_KEPT = 4;
+std::mutex& spaces_mutex() {
+  static std::mutex m;
+  return m;
+}
+std::vector<Space>& spaces() {
+  static auto* v = new std::vector<Space>();  // outlives the runtime's own end
+  return *v;
+}
+void space_free(Space& s) {
+  if (s.stream) (void)hipStreamDestroy(s.stream);
+  if (s.host) (void)hipHostFree(s.host);
+  if (s.device) (void)hipFree(s.device);
+}
+hipError_t space_take(Space* s) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  {
+    std::lock_guard<std::mutex> lock(spaces_mutex());
+    auto& v = spaces();
+    for (size_t k = 0; k < v.size(); ++k)
+      if (v[k].dev == dev) {
+        *s = v[k];
+        v.erase(v.begin() + (long)k);
+        return hipSuccess;
+      }
+  }
+  s->dev = dev;
+  e = hipHostMalloc((void**)&s->host, Space::HOST);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
+  if (e != hipSuccess) {
+    space_free(*s);
+    *s = Space();
+  }
+  return e;
+}
+void space_give(Space& s, bool keep) {
+  if (keep && s.device_bytes <= Space::DEVICE) {
+    std::lock_guard<std::mutex> lock(spaces_mutex());
+    size_t here = 0;
+    for (const Space& o : spaces()) here += o.dev == s.dev;
+    if (here < SPACES_KEPT) {
+      spaces().push_back(s);
+      return;
+    }
+  }
+  space_free(s);
+}
 
-struct DevStatus {
-  int* p = nullptr;
-  ~DevStatus() { if (p) (void)hipFree(p); }
+// A point-wise call: up to four input and three output arrays of doubles on
+// the host.  launch(in, out, status, stream) gets arrays the device can use.
+struct PointIo {
+  const double* in[4] = {nullptr, nullptr, nullptr, nullptr};
+  size_t nin[4] = {0, 0, 0, 0};
+  double* out[3] = {nullptr, nullptr, nullptr};
+  size_t nout[3] = {0, 0, 0};
 };
-
-int finish_status(DevStatus& st) {
-  int v = 0;
-  HIP_TRY(hipDeviceSynchronize());
-  HIP_TRY(hipMemcpy(&v, st.p, sizeof(int), hipMemcpyDeviceToHost));
-  if (v) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
+template <class Launch>
+int run_points(const PointIo& io, Launch launch) {
+  const double* in[4] = {nullptr, nullptr, nullptr, nullptr};
+  double* out[3] = {nullptr, nullptr, nullptr};
+  auto padded = [](size_t n) { return (n * sizeof(double) + 63) / 64 * 64; };
+  size_t total = 64;  // the status word
+  for (size_t n : io.nin) total += padded(n);
+  for (size_t n : io.nout) total += padded(n);
+  Space s;
+  HIP_TRY(space_take(&s));
+  // the status word is the page-locked one either way
+  int* status = (int*)s.host;
+  *status = 0;
+  const bool small = total <= Space::HOST;
+  hipError_t e = hipSuccess;
+  if (!small && s.device_bytes < total) {
+    if (s.device) e = hipFree(s.device);
+    s.device = nullptr;
+    s.device_bytes = 0;
+    if (e == hipSuccess) e = hipMalloc((void**)&s.device, total);
+    if (e == hipSuccess) s.device_bytes = total;
+  }
+  char* at = (small ? s.host : s.device) + 64;
+  for (int k = 0; k < 4 && e == hipSuccess; ++k) {
+    if (!io.in[k]) continue;
+    if (small) std::memcpy(at, io.in[k], io.nin[k] * sizeof(double));
+    else e = hipMemcpyAsync(at, io.in[k], io.nin[k] * sizeof(double), hipMemcpyHostToDevice, s.stream);
+    in[k] = (const double*)at;
+    at += padded(io.nin[k]);
+  }
+  for (int k = 0; k < 3; ++k) {
+    if (!io.out[k]) continue;
+    out[k] = (double*)at;
+    at += padded(io.nout[k]);
+  }
+  if (e == hipSuccess) {
+    launch(in, out, status, s.stream);
+    e = hipGetLastError();
+  }
+  for (int k = 0; k < 3 && e == hipSuccess && !small; ++k)
+    if (io.out[k])
+      e = hipMemcpyAsync(io.out[k], out[k], io.nout[k] * sizeof(double), hipMemcpyDeviceToHost, s.stream);
+  const hipError_t es = hipStreamSynchronize(s.stream);
+  if (e == hipSuccess) e = es;
+  const int st = e == hipSuccess ? *(volatile int*)status : 0;
+  for (int k = 0; k < 3 && e == hipSuccess && small; ++k)
+    if (io.out[k]) std::memcpy(io.out[k], out[k], io.nout[k] * sizeof(double));
+  space_give(s, e == hipSuccess);
+  HIP_TRY(e);
+  if (st) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
   return HES_OK;
 }
 
@@ -1325,26 +1441,22 @@ int point_call(int op, int nph, const double* mats, const double* in, double* ou
     if (!mat_ok(mats + 8 * p)) return fail(HES_ERR_ARG, "invalid material constants");
   if (n == 0) return HES_OK;
   MatDev m0 = make_mat(mats), m1 = make_mat(nph == 2 ? mats + 8 : mats);
-  DevBuf di, dout;
-  DevStatus st;
-  HIP_TRY(di.alloc((size_t)n * in_w));
-  HIP_TRY(dout.alloc((size_t)n * out_w));
-  HIP_TRY(hipMalloc(&st.p, sizeof(int)));
-  HIP_TRY(hipMemset(st.p, 0, sizeof(int)));
-  HIP_TRY(hipMemcpy(di.p, in, sizeof(double) * (size_t)n * in_w, hipMemcpyHostToDevice));
   unsigned nb = (unsigned)((n + 63) / 64);
   double nv[3] = {1.0, 0.0, 0.0};
   if (nvec) { nv[0] = nvec[0]; nv[1] = nvec[1]; nv[2] = nvec[2]; }
-  if (nph == 1)
-    hipLaunchKernelGGL(k_point<1>, dim3(nb), dim3(64), 0, 0, op, di.p, dout.p, n, m0, m1, nv[0],
-                       nv[1], nv[2], st.p);
-  else
-    hipLaunchKernelGGL(k_point<2>, dim3(nb), dim3(64), 0, 0, op, di.p, dout.p, n, m0, m1, nv[0],
-                       nv[1], nv[2], st.p);
-  HIP_TRY(hipGetLastError());
-  int rc = finish_status(st);
-  HIP_TRY(hipMemcpy(out, dout.p, sizeof(double) * (size_t)n * out_w, hipMemcpyDeviceToHost));
-  return rc;
+  PointIo io;
+  io.in[0] = in;
+  io.nin[0] = (size_t)n * in_w;
+  io.out[0] = out;
+  io.nout[0] = (size_t)n * out_w;
+  return run_points(io, [&](const double* const* i, double* const* o, int* status, hipStream_t s) {
+    if (nph == 1)
+      hipLaunchKernelGGL(k_point<1>, dim3(nb), dim3(64), 0, s, op, i[0], o[0], n, m0, m1, nv[0],
+                         nv[1], nv[2], status);
+    else
+      hipLaunchKernelGGL(k_point<2>, dim3(nb), dim3(64), 0, s, op, i[0], o[0], n, m0, m1, nv[0],
+                         nv[1], nv[2], status);
+  });
 }
 
 int eos_call(int op, const double* mat, const double* s, const double* s2, const double* v,
@@ -1353,24 +1465,34 @@ int eos_call(int op, const double* mat, const double* s, const double* s2, const
   if (!mat_ok(mat)) return fail(HES_ERR_ARG, "invalid material constants");
   if (n == 0) return HES_OK;
   MatDev m = make_mat(mat);
-  DevBuf ds, ds2, dv, dn, dout;
-  DevStatus st;
-  HIP_TRY(hipMalloc(&st.p, sizeof(int)));
-  HIP_TRY(hipMemset(st.p, 0, sizeof(int)));
-  if (s) { HIP_TRY(ds.alloc(n)); HIP_TRY(hipMemcpy(ds.p, s, sizeof(double) * n, hipMemcpyHostToDevice)); }
-  if (s2) { HIP_TRY(ds2.alloc(n)); HIP_TRY(hipMemcpy(ds2.p, s2, sizeof(double) * n, hipMemcpyHostToDevice)); }
-  if (v) { HIP_TRY(dv.alloc((size_t)n * vw)); HIP_TRY(hipMemcpy(dv.p, v, sizeof(double) * n * vw, hipMemcpyHostToDevice)); }
-  if (nv) { HIP_TRY(dn.alloc((size_t)n * 3)); HIP_TRY(hipMemcpy(dn.p, nv, sizeof(double) * n * 3, hipMemcpyHostToDevice)); }
-  HIP_TRY(dout.alloc((size_t)n * ow));
   unsigned nb = (unsigned)((n + 63) / 64);
-  hipLaunchKernelGGL(k_eos, dim3(nb), dim3(64), 0, 0, op, m, ds.p, ds2.p, dv.p, dn.p, dout.p, n, st.p);
-  HIP_TRY(hipGetLastError());
-  int rc = finish_status(st);
-  HIP_TRY(hipMemcpy(out, dout.p, sizeof(double) * (size_t)n * ow, hipMemcpyDeviceToHost));
-  return rc;
+  PointIo io;
+  const double* in[4] = {s, s2, v, nv};
+  const size_t w[4] = {1, 1, (size_t)vw, 3};
+  for (int k = 0; k < 4; ++k) {
+    io.in[k] = in[k];
+    io.nin[k] = in[k] ? (size_t)n * w[k] : 0;
+  }
+  io.out[0] = out;
+  io.nout[0] = (size_t)n * ow;
+  return run_points(io, [&](const double* const* i, double* const* o, int* status, hipStream_t st) {
+    hipLaunchKernelGGL(k_eos, dim3(nb), dim3(64), 0, st, op, m, i[0], i[1], i[2], i[3], o[0], n, status);
+  });
+}
+
+// Two-phase faces of up to this many take 16 lanes each.
+constexpr long long FACE_GROUP_MAX = 4096;
+
+template <int NPH, int FLUX, int GL>
+void launch_face(const double* const* i, double* const* o, long long n, const MatDev& m0,
+                 const MatDev& m1, hipStream_t s) {
+  hipLaunchKernelGGL((k_face<NPH, FLUX, GL>), dim3((unsigned)((n * GL + 63) / 64)), dim3(64), 0, s,
+                     i[0], i[1], i[2], o[0], o[1], o[2], n, m0, m1);
 }
 
 }  // namespace
+
+extern "C" {
 
 int hes_cons2prim(int nph, const double* mats, const double* Q, double* P, long long n) {
   int w = nph == 1 ? 14 : 30;
@@ -1452,31 +1574,24 @@ int hes_face_flux(int nph, int flux, const double* mats, const double* QL, const
   int w = nph == 1 ? 14 : 30;
   int aw = flux == HES_FLUX_HLL ? 2 : 1;
   MatDev m0 = make_mat(mats), m1 = make_mat(nph == 2 ? mats + 8 : mats);
-  DevBuf dl, dr, da, dc, ddm, ddp;
-  HIP_TRY(dl.alloc((size_t)n * w));
-  HIP_TRY(dr.alloc((size_t)n * w));
-  HIP_TRY(da.alloc((size_t)n * aw));
-  HIP_TRY(dc.alloc((size_t)n * w));
-  HIP_TRY(ddm.alloc((size_t)n * w));
-  HIP_TRY(ddp.alloc((size_t)n * w));
-  HIP_TRY(hipMemcpy(dl.p, QL, sizeof(double) * n * w, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(dr.p, QR, sizeof(double) * n * w, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(da.p, aux, sizeof(double) * n * aw, hipMemcpyHostToDevice));
-  unsigned nb = (unsigned)((n + 63) / 64);
-  if (nph == 1 && flux == HES_FLUX_RUSANOV)
-    hipLaunchKernelGGL((k_face<1, FLUX_RUSANOV>), dim3(nb), dim3(64), 0, 0, dl.p, dr.p, da.p, dc.p, ddm.p, ddp.p, n, m0, m1);
-  else if (nph == 1)
-    hipLaunchKernelGGL((k_face<1, FLUX_HLL>), dim3(nb), dim3(64), 0, 0, dl.p, dr.p, da.p, dc.p, ddm.p, ddp.p, n, m0, m1);
-  else if (flux == HES_FLUX_RUSANOV)
-    hipLaunchKernelGGL((k_face<2, FLUX_RUSANOV>), dim3(nb), dim3(64), 0, 0, dl.p, dr.p, da.p, dc.p, ddm.p, ddp.p, n, m0, m1);
-  else
-    hipLaunchKernelGGL((k_face<2, FLUX_HLL>), dim3(nb), dim3(64), 0, 0, dl.p, dr.p, da.p, dc.p, ddm.p, ddp.p, n, m0, m1);
-  HIP_TRY(hipGetLastError());
-  HIP_TRY(hipDeviceSynchronize());
-  HIP_TRY(hipMemcpy(cons, dc.p, sizeof(double) * n * w, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(dm, ddm.p, sizeof(double) * n * w, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(dp, ddp.p, sizeof(double) * n * w, hipMemcpyDeviceToHost));
-  return HES_OK;
+  PointIo io;
+  const double* in[3] = {QL, QR, aux};
+  double* out[3] = {cons, dm, dp};
+  for (int k = 0; k < 3; ++k) {
+    io.in[k] = in[k];
+    io.nin[k] = (size_t)n * (k < 2 ? w : aw);
+    io.out[k] = out[k];
+    io.nout[k] = (size_t)n * w;
+  }
+  const bool hll = flux == HES_FLUX_HLL, few = n <= FACE_GROUP_MAX;
+  return run_points(io, [&](const double* const* i, double* const* o, int*, hipStream_t s) {
+    if (nph == 1 && !hll) launch_face<1, FLUX_RUSANOV, 1>(i, o, n, m0, m1, s);
+    else if (nph == 1) launch_face<1, FLUX_HLL, 1>(i, o, n, m0, m1, s);
+    else if (!hll && few) launch_face<2, FLUX_RUSANOV, 16>(i, o, n, m0, m1, s);
+    else if (!hll) launch_face<2, FLUX_RUSANOV, 1>(i, o, n, m0, m1, s);
+    else if (few) launch_face<2, FLUX_HLL, 16>(i, o, n, m0, m1, s);
+    else launch_face<2, FLUX_HLL, 1>(i, o, n, m0, m1, s);
+  });
 }
 
 // ---- Hyperelasticity (the single-phase module, Hyperelasticity.jl:25-114):

@@ -47,50 +47,6 @@ __device__ __forceinline__ void st_stream(double v, double* p) {
 #endif
 }
 
-// Neighbour values within a wave: lane_down(v) is lane + 1's v (lane 63 keeps
-// its own), lane_up(v) is lane - 1's v (lane 0 keeps its own), as
-// __shfl_down / __shfl_up by 1.  By default they are the wave-wide DPP shifts
-// (wave_shl:1 / wave_shr:1, plain VALU moves); HES_DPP_SHIFT=0 selects the LDS
-// crossbar (ds_bpermute) instead.
-#ifndef HES_DPP_SHIFT
-#define HES_DPP_SHIFT 1
-#endif
-#if HES_DPP_SHIFT
-template <int CTRL>
-__device__ __forceinline__ double dpp_shift(double v) {
-  const long long b = __double_as_longlong(v);
-  int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
-  lo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
-  hi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ double lane_down(double v) { return dpp_shift<0x130>(v); }  // wave_shl:1
-__device__ __forceinline__ double lane_up(double v) { return dpp_shift<0x138>(v); }    // wave_shr:1
-// The same shifts writing zero into the lane that has no source (lane 63 for
-// lane_down_z, lane 0 for lane_up_z) or whose source lane is inactive, so
-// they are only used where every lane of the wave is active: never under a
-// lane-dependent condition (a && or ?: whose other operand varies by lane).  With no old value to keep, the shifted
-// copy goes straight into a new register: one DPP move per half, where
-// lane_down / lane_up first copy the value (the original stays live).  For
-// values whose boundary-lane result only reaches the halo lanes' own face and
-// update, which are never stored.
-template <int CTRL>
-__device__ __forceinline__ double dpp_shift_z(double v) {
-  const long long b = __double_as_longlong(v);
-  int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
-  lo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true);
-  hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ double lane_down_z(double v) { return dpp_shift_z<0x130>(v); }
-__device__ __forceinline__ double lane_up_z(double v) { return dpp_shift_z<0x138>(v); }
-#else
-__device__ __forceinline__ double lane_down(double v) { return __shfl_down(v, 1); }
-__device__ __forceinline__ double lane_up(double v) { return __shfl_up(v, 1); }
-__device__ __forceinline__ double lane_down_z(double v) { return __shfl_down(v, 1); }
-__device__ __forceinline__ double lane_up_z(double v) { return __shfl_up(v, 1); }
-#endif
-
 // Block order across the 8 XCDs: the hardware deals consecutive blocks to
 // XCDs round-robin; remap so each XCD walks a contiguous stretch of cells and
 // the cache lines two neighbouring tiles share stay in one L2.
@@ -709,67 +665,10 @@ __device__ __forceinline__ unsigned long long block_append(bool flag, unsigned l
   return base + share[w] + (unsigned long long)__popcll(m & ((1ull << lane) - 1ull));
 }
 
-// One quadrature node's share of a path integral (NumFluxes.jl:39-47, 97-107):
-// w b^p(psi) da_p in the rows of phase block p, where psi is the state at the
-// node, b^p the non-zero column of B's block p and da_p the volume-fraction
-// jump of the path.  The integral is the sum over the nodes.
-// ACC: add the share to out instead of writing it.
-template <int FAST, bool ACC = false>
-__device__ __forceinline__ void bnode2(const MatDev* mat, const double* psi, double w, double da0,
-                                       double da1, double* out) {
-  BCol b;
-  bcol2<FAST>(mat, psi, b);
-#pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const double wd = w * (p == 0 ? da0 : da1);
-    double* o = out + 15 * p;
-    auto put = [&](int r, double v) { o[r] = ACC ? o[r] + v : v; };
-    put(0, wd * b.uI0);
-    if (!ACC) o[1] = 0.0;
-    put(2, wd * b.sI[0]);
-    put(3, wd * b.sI[1]);
-    put(4, wd * b.sI[2]);
-    put(5, wd * b.sIu);
-#pragma unroll
-    for (int r = 0; r < 9; ++r) put(6 + r, wd * b.a[p][r]);
-  }
-}
-
-// v[g] and v[g + 15] for lane g of a group (g < 15), by selects: indexing a
-// register array with a lane-dependent index would move it to scratch memory.
-__device__ __forceinline__ void rows_of_lane(const double* v, int g, double& lo, double& hi) {
-  lo = 0.0;
-  hi = 0.0;
-#pragma unroll
-  for (int r = 0; r < 15; ++r) {
-    lo = g == r ? v[r] : lo;
-    hi = g == r ? v[r + 15] : hi;
-  }
-}
-
 // The jump faces' path terms are computed by a group of lanes per face (lane
 // g of the group), the quadrature nodes spread over the group's lanes: the
 // nodes evaluate the same code on different data, which a wave runs in
 // parallel for all its faces.
-
-// lane ^ O's v within a group of lanes: for O = 1, 2 a move within the quad
-// (DPP quad_perm), else through the LDS crossbar.
-template <int O, int GL>
-__device__ __forceinline__ double group_xor(double v) {
-  if constexpr (O == 1) return dpp_shift_z<0xB1>(v);       // quad_perm [1, 0, 3, 2]
-  else if constexpr (O == 2) return dpp_shift_z<0x4E>(v);  // quad_perm [2, 3, 0, 1]
-  else return __shfl_xor(v, O, GL);
-}
-
-// Sum of v[30] over the GL lanes of a lane group (every lane of the group active).
-template <int GL>
-__device__ __forceinline__ void group_sum(double* v) {
-  if constexpr (GL > 1) {
-#pragma unroll
-    for (int r = 0; r < 30; ++r) v[r] += group_xor<GL / 2, GL>(v[r]);
-    group_sum<GL / 2>(v);
-  }
-}
 
 // Number of lanes per jump face in the Rusanov path-term kernels.
 #ifndef HES_PATH_LANES
