@@ -17,6 +17,7 @@
 #include "hes_host.hpp"
 #include "hes_resident.hpp"
 #include "hes_step.hpp"
+#include "hes_transfer.hpp"
 #include "../../include/hes.h"
 
 using namespace hes;
@@ -602,12 +603,6 @@ __global__ void k_batch_resident_end(const BResOut* out, const int* status, int 
   slots[3 * p + (launch + 2) % 3] = 0ull;
 }
 
-__global__ void k_soa_to_aos_b(const double* __restrict__ in, double* __restrict__ out, int nc,
-                               long long n, long long pitch) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  for (int r = 0; r < nc; ++r) out[i * nc + r] = in[r * pitch + i];
-}
 __global__ void k_aos_to_soa_b(const double* __restrict__ in, double* __restrict__ out, int nc,
                                long long n, long long pitch) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1165,15 +1160,8 @@ int hes_batch_get_state(hes_batch* h, double* Q) {
   if (!h->has_state) return fail(HES_ERR_ARG, "no state set");
   const int rc = batch_carry(h);  // problems that stopped early into the current buffer
   if (rc != HES_OK) return rc;
-  size_t bytes = sizeof(double) * (size_t)h->nc * h->N;
-  double* tmp = nullptr;
-  HIP_TRY(hipMalloc(&tmp, bytes));
-  hipLaunchKernelGGL(k_soa_to_aos_b, dim3((unsigned)((h->N + 255) / 256)), dim3(256), 0, h->stream,
-                     h->Q[h->step & 1], tmp, h->nc, h->N, h->pitch);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(Q, tmp, bytes, hipMemcpyDeviceToHost, h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  (void)hipFree(tmp);
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  const hipError_t e = download_state(h->Q[h->step & 1], Q, h->nc, h->N, h->pitch);
   if (e != hipSuccess) {
     g_err = std::string("batch get_state: ") + hipGetErrorString(e);
     return HES_ERR_HIP;

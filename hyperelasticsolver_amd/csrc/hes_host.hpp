@@ -8,6 +8,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "hes_device.hpp"
 #include "../../include/hes.h"
@@ -119,5 +120,80 @@ class ComputeUnits {
   }
   int dev_, need_;
 };
+
+// What a call works in: page-locked host memory that the kernels read and
+// write themselves (small calls: no copies), device memory (larger ones), and
+// a stream of its own.  Allocated for every call they cost one on a single
+// state 90 of its 100 us.  One per call that is under way; at most SPACES_KEPT
+// wait for the next, per device, with at most Space::DEVICE bytes each.
+struct Space {
+  static constexpr size_t HOST = 128 * 1024, DEVICE = 96 << 20;
+  int dev = 0;
+  char* host = nullptr;
+  char* device = nullptr;
+  size_t device_bytes = 0;
+  hipStream_t stream = nullptr;
+};
+inline constexpr size_t SPACES_KEPT = 4;
+inline std::mutex& spaces_mutex() {
+  static std::mutex m;
+  return m;
+}
+inline std::vector<Space>& spaces() {
+  static auto* v = new std::vector<Space>();  // outlives the runtime's own end
+  return *v;
+}
+inline void space_free(Space& s) {
+  if (s.stream) (void)hipStreamDestroy(s.stream);
+  if (s.host) (void)hipHostFree(s.host);
+  if (s.device) (void)hipFree(s.device);
+}
+inline hipError_t space_take(Space* s) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  {
+    std::lock_guard<std::mutex> lock(spaces_mutex());
+    auto& v = spaces();
+    for (size_t k = 0; k < v.size(); ++k)
+      if (v[k].dev == dev) {
+        *s = v[k];
+        v.erase(v.begin() + (long)k);
+        return hipSuccess;
+      }
+  }
+  s->dev = dev;
+  e = hipHostMalloc((void**)&s->host, Space::HOST);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
+  if (e != hipSuccess) {
+    space_free(*s);
+    *s = Space();
+  }
+  return e;
+}
+inline void space_give(Space& s, bool keep) {
+  if (keep && s.device_bytes <= Space::DEVICE) {
+    std::lock_guard<std::mutex> lock(spaces_mutex());
+    size_t here = 0;
+    for (const Space& o : spaces()) here += o.dev == s.dev;
+    if (here < SPACES_KEPT) {
+      spaces().push_back(s);
+      return;
+    }
+  }
+  space_free(s);
+}
+
+
+// Device memory of at least `bytes` in s (its contents are lost when it grows).
+inline hipError_t space_device(Space& s, size_t bytes) {
+  if (s.device_bytes >= bytes) return hipSuccess;
+  hipError_t e = s.device ? hipFree(s.device) : hipSuccess;
+  s.device = nullptr;
+  s.device_bytes = 0;
+  if (e == hipSuccess) e = hipMalloc((void**)&s.device, bytes);
+  if (e == hipSuccess) s.device_bytes = bytes;
+  return e;
+}
 
 }  // namespace hes

@@ -26,6 +26,7 @@
 #include "hes_host.hpp"
 #include "hes_resident.hpp"
 #include "hes_step.hpp"
+#include "hes_transfer.hpp"
 #include "../../include/hes.h"
 
 using namespace hes;
@@ -273,20 +274,13 @@ __global__ __launch_bounds__(BLOCK) void k_speeds(const double* __restrict__ Q,
   block_max_to_slot(lam, slot);
 }
 
-// AoS (component fastest, the Julia Matrix layout) <-> SoA.
+// AoS (component fastest, the Julia Matrix layout) -> SoA (back: hes_transfer.hpp).
 __global__ void k_aos_to_soa(const double* __restrict__ in, double* __restrict__ out, int nc,
                              long long n, long long pitch) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   for (int r = 0; r < nc; ++r) out[r * pitch + i] = in[i * nc + r];
 }
-__global__ void k_soa_to_aos(const double* __restrict__ in, double* __restrict__ out, int nc,
-                             long long n, long long pitch) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  for (int r = 0; r < nc; ++r) out[i * nc + r] = in[r * pitch + i];
-}
-
 // Piecewise-constant initial state: cell i (0-based, centre x = (i + 1/2) / n)
 // takes state k = #{j : x > s_j} for sorted interfaces s_j.  With one interface
 // at 1/2 this is main.jl:103 (cell i is left iff i < n/2).
@@ -554,7 +548,7 @@ struct hes_solver {
   long long* jlist;          // two phases: jump-face list (n entries)
   double* Q[2];
   double* C[2];
-  unsigned long long* slots;
+  unsigned long long* slots;  // with it, in one allocation: tring, jcnt, status, comm
   double* tring;
   int* status;
   double* dt_hist;
@@ -570,10 +564,12 @@ struct hes_solver {
   int res_g, res_own;        // workgroups and cells of each
   unsigned long long* comm;  // their slots, then their halo words
   unsigned res_tag;          // the last tag written there
-  struct ResMail {           // page-locked, written by the launch
-    ResOut out;
-    int status[4];
-  }* mail;
+};
+
+// What a launch of the whole loop leaves in page-locked memory.
+struct ResMail {
+  ResOut out;
+  int status[4];
 };
 
 namespace {
@@ -670,16 +666,35 @@ StepArgs make_args(hes_solver* h, long long s, double t_end, double* hist, int h
   return a;
 }
 
+// A new state's bookkeeping (one block): rings, counters and, if fresh, the
+// status word; and the end cells, which never change, into the other buffer
+// (56 or 120 copies of 8 bytes cost 150 us when each was one of its own).
+__global__ __launch_bounds__(64) void k_begin(const double* __restrict__ Q, double* __restrict__ other,
+                                              int nc, long long n, long long pitch,
+                                              unsigned long long* slots, double* tring, double t,
+                                              unsigned long long* jcnt, int* status, int fresh) {
+  const int r = threadIdx.x;
+  if (r < nc) {
+    other[r * pitch] = Q[r * pitch];
+    other[r * pitch + n - 1] = Q[r * pitch + n - 1];
+  }
+  if (r < 3) slots[r] = 0ull;
+  if (r < 2) {
+    tring[r] = t;
+    if (jcnt) jcnt[r] = 0ull;
+  }
+  if (fresh && r < 4) status[r] = 0;
+}
+
 // Recompute sound speeds and the CFL max of the current state; reset rings.
-int init_speeds(hes_solver* h) {
-  long long s = h->step;
-  HIP_TRY(hipMemsetAsync(h->slots, 0, 3 * sizeof(unsigned long long), h->stream));
-  if (h->jcnt) HIP_TRY(hipMemsetAsync(h->jcnt, 0, 2 * sizeof(unsigned long long), h->stream));
-  double tr[2] = {h->t, h->t};
-  HIP_TRY(hipMemcpyAsync(h->tring, tr, sizeof(tr), hipMemcpyHostToDevice, h->stream));
-  long long nb = (h->n + BLOCK - 1) / BLOCK;
+// The status word comes back through `mail` (page-locked).
+int init_speeds(hes_solver* h, bool fresh, int* mail) {
+  const long long s = h->step;
   const double* Qs = h->Q[s & 1];
   double* Cs = h->C[s & 1];
+  hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, h->stream, Qs, h->Q[(s + 1) & 1], h->nc, h->n,
+                     h->pitch, h->slots, h->tring, h->t, h->jcnt, h->status, (int)fresh);
+  const long long nb = (h->n + BLOCK - 1) / BLOCK;
   if (h->nph == 1)
     hipLaunchKernelGGL(k_speeds<1>, dim3((unsigned)nb), dim3(BLOCK), 0, h->stream, Qs, Cs, h->n,
                        h->pitch, h->mat[0], h->mat[1], h->slots + (s % 3), h->status);
@@ -687,18 +702,9 @@ int init_speeds(hes_solver* h) {
     hipLaunchKernelGGL(k_speeds<2>, dim3((unsigned)nb), dim3(BLOCK), 0, h->stream, Qs, Cs, h->n,
                        h->pitch, h->mat[0], h->mat[1], h->slots + (s % 3), h->status);
   HIP_TRY(hipGetLastError());
-  // the end cells never change: copy their state and speeds into the other buffer
-  for (int r = 0; r < h->nc; ++r) {
-    HIP_TRY(hipMemcpyAsync(h->Q[(s + 1) & 1] + r * h->pitch, h->Q[s & 1] + r * h->pitch,
-                           sizeof(double), hipMemcpyDeviceToDevice, h->stream));
-    HIP_TRY(hipMemcpyAsync(h->Q[(s + 1) & 1] + r * h->pitch + h->n - 1,
-                           h->Q[s & 1] + r * h->pitch + h->n - 1, sizeof(double),
-                           hipMemcpyDeviceToDevice, h->stream));
-  }
+  HIP_TRY(hipMemcpyAsync(mail, h->status, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
-  int st[2];
-  HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
-  if (st[0]) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
+  if (*mail) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
   return HES_OK;
 }
 
@@ -860,7 +866,10 @@ hipError_t launch_resident(const hes_solver* h, const ResArgs& a) {
 // (the launch's workgroups were not on the chip together), the handle's state
 // is as before.  Adds to *ms the launch's time.
 int run_resident(hes_solver* h, long long steps, double t_end, double* dt_hist, long long* done,
-                 float* ms, bool* gave_up) {
+                 float* ms, int* bad, bool* gave_up) {
+  Space sp;
+  HIP_TRY(space_take(&sp));
+  ResMail* mail = (ResMail*)sp.host;
   ResArgs a;
   std::memset((void*)&a, 0, sizeof(a));
   const long long s0 = h->step;
@@ -888,35 +897,44 @@ int run_resident(hes_solver* h, long long steps, double t_end, double* dt_hist, 
   a.slots = h->slots;
   a.tring = h->tring;
   a.jcnt = h->jcnt;
-  a.out = &h->mail->out;
+  a.out = &mail->out;
   a.step0 = s0;
   a.relax = h->relax;
   a.relax_p = h->relax_p;
   a.mat[0] = h->mat[0];
   a.mat[1] = h->mat[1];
   h->res_tag += (unsigned)steps + 1;
+  hipError_t e;
   {
     ComputeUnits units(h->dev, h->cus, h->res_g > 1 ? h->res_g : 0);
-    HIP_TRY(hipEventRecord(h->ev0, h->stream));
-    HIP_TRY(hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * 2 * h->res_g * RES_SLOT, h->stream));
-    HIP_TRY(launch_resident(h, a));
-    HIP_TRY(hipEventRecord(h->ev1, h->stream));
-    HIP_TRY(hipMemcpyAsync(h->mail->status, h->status, sizeof(h->mail->status), hipMemcpyDeviceToHost,
-                           h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    e = hipEventRecord(h->ev0, h->stream);
+    if (e == hipSuccess)
+      e = hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * 2 * h->res_g * RES_SLOT, h->stream);
+    if (e == hipSuccess) e = launch_resident(h, a);
+    if (e == hipSuccess) e = hipEventRecord(h->ev1, h->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(mail->status, h->status, sizeof(mail->status), hipMemcpyDeviceToHost, h->stream);
+    const hipError_t es = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess) e = es;
   }
-  *gave_up = h->mail->status[2] != 0;
+  const ResMail got = *mail;
+  int rc = HES_OK;
+  *gave_up = e == hipSuccess && got.status[2] != 0;
   if (*gave_up) {
     h->shape = {0, 0};  // step by step from here on
-    HIP_TRY(zero_on(h->stream, h->status + 2, sizeof(int)));
-    return init_speeds(h);
+    e = zero_on(h->stream, h->status + 2, sizeof(int));
+    if (e == hipSuccess) rc = init_speeds(h, false, mail->status);
   }
+  space_give(sp, e == hipSuccess);
+  HIP_TRY(e);
+  if (*gave_up || rc != HES_OK) return rc;
   float one = 0.f;
   HIP_TRY(hipEventElapsedTime(&one, h->ev0, h->ev1));
   *ms += one;
-  *done = h->mail->out.steps;
+  *bad = got.status[0];
+  *done = got.out.steps;
   h->step = s0 + *done;
-  h->t = h->mail->out.t;
+  h->t = got.out.t;
   if ((*done & 1) == 0) {  // the result is where an odd number of steps would have left it
     std::swap(h->Q[0], h->Q[1]);
     std::swap(h->C[0], h->C[1]);
@@ -986,21 +1004,21 @@ int hes_solver_create(hes_solver** out, int nphase, int flux, long long ncells,
     if (e == hipSuccess) e = hipMalloc(&h->C[b], cbytes);
   }
   if (e == hipSuccess && nphase == 2) e = hipMalloc(&h->dpath, 2 * qbytes);  // D-, D+ rows
-  if (e == hipSuccess && nphase == 2) e = hipMalloc(&h->jcnt, 2 * sizeof(unsigned long long));
   if (e == hipSuccess && nphase == 2) e = hipMalloc(&h->jlist, sizeof(long long) * (size_t)ncells);
-  if (e == hipSuccess) e = hipMalloc(&h->slots, 4 * sizeof(unsigned long long));
-  if (e == hipSuccess) e = hipMalloc(&h->tring, 2 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&h->status, 4 * sizeof(int));
+  // the small words in one allocation: CFL ring, time ring, jump-face counts,
+  // status, then the team's messages, each on a line of its own
+  const size_t words = 4 * 16 + (h->shape.block ? comm_words(h) : 0);
+  if (e == hipSuccess) e = hipMalloc(&h->slots, sizeof(unsigned long long) * words);
+  if (e == hipSuccess) {
+    h->tring = (double*)(h->slots + 16);
+    if (nphase == 2) h->jcnt = h->slots + 32;
+    h->status = (int*)(h->slots + 48);
+    h->comm = h->slots + 64;
+  }
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&h->ev0);
   if (e == hipSuccess) e = hipEventCreate(&h->ev1);
-  if (e == hipSuccess) e = zero_on(h->stream, h->status, 4 * sizeof(int));
-  if (h->shape.block) {
-    const size_t bytes = sizeof(unsigned long long) * comm_words(h);
-    if (e == hipSuccess) e = hipMalloc(&h->comm, bytes);
-    if (e == hipSuccess) e = hipMemsetAsync(h->comm, 0, bytes, h->stream);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&h->mail, sizeof(*h->mail));
-  }
+  if (e == hipSuccess) e = zero_on(h->stream, h->slots, sizeof(unsigned long long) * words);
   if (e != hipSuccess) {
     g_err = std::string("allocation failed: ") + hipGetErrorString(e);
     hes_solver_destroy(h);
@@ -1035,13 +1053,8 @@ int hes_solver_destroy(hes_solver* h) {
   }
   if (h->slots) (void)hipFree(h->slots);
   if (h->dpath) (void)hipFree(h->dpath);
-  if (h->jcnt) (void)hipFree(h->jcnt);
   if (h->jlist) (void)hipFree(h->jlist);
-  if (h->tring) (void)hipFree(h->tring);
-  if (h->status) (void)hipFree(h->status);
   if (h->dt_hist) (void)hipFree(h->dt_hist);
-  if (h->comm) (void)hipFree(h->comm);
-  if (h->mail) (void)hipHostFree(h->mail);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1049,28 +1062,35 @@ int hes_solver_destroy(hes_solver* h) {
   return HES_OK;
 }
 
+// The end of setting a state: its speeds and bookkeeping, unless e has failed.
+static int state_set(hes_solver* h, Space& sp, hipError_t e, const char* what) {
+  int rc = HES_ERR_HIP;
+  if (e == hipSuccess) {
+    h->has_state = true;
+    rc = init_speeds(h, true, (int*)sp.host);
+  } else {
+    g_err = std::string(what) + hipGetErrorString(e);
+  }
+  const hipError_t es = hipStreamSynchronize(h->stream);  // sp is in use until here
+  space_give(sp, e == hipSuccess && es == hipSuccess);
+  return rc;
+}
+
 static int set_state_common(hes_solver* h, const double* src, hipMemcpyKind kind, double t0) {
   size_t bytes = sizeof(double) * (size_t)h->nc * (size_t)h->n;
-  double* tmp = nullptr;
-  HIP_TRY(hipMalloc(&tmp, bytes));
-  hipError_t e = hipMemcpyAsync(tmp, src, bytes, kind, h->stream);
+  Space sp;
+  HIP_TRY(space_take(&sp));
+  hipError_t e = space_device(sp, bytes);
+  if (e == hipSuccess) e = hipMemcpyAsync(sp.device, src, bytes, kind, h->stream);
   if (e == hipSuccess) {
     h->step = 0;
     h->t = t0;
     long long nb = (h->n + 255) / 256;
-    hipLaunchKernelGGL(k_aos_to_soa, dim3((unsigned)nb), dim3(256), 0, h->stream, tmp, h->Q[0],
-                       h->nc, h->n, h->pitch);
+    hipLaunchKernelGGL(k_aos_to_soa, dim3((unsigned)nb), dim3(256), 0, h->stream,
+                       (const double*)sp.device, h->Q[0], h->nc, h->n, h->pitch);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  (void)hipFree(tmp);
-  if (e != hipSuccess) {
-    g_err = std::string("set_state: ") + hipGetErrorString(e);
-    return HES_ERR_HIP;
-  }
-  HIP_TRY(zero_on(h->stream, h->status, 4 * sizeof(int)));
-  h->has_state = true;
-  return init_speeds(h);
+  return state_set(h, sp, e, "set_state: ");
 }
 
 int hes_solver_set_state(hes_solver* h, const double* Q, double t0) {
@@ -1084,32 +1104,31 @@ int hes_solver_set_piecewise(hes_solver* h, int nstates, const double* states,
     return fail(HES_ERR_ARG, "null argument");
   for (int j = 0; j + 1 < nstates - 1; ++j)
     if (!(interfaces[j] <= interfaces[j + 1])) return fail(HES_ERR_ARG, "interfaces not sorted");
-  double *ds = nullptr, *di = nullptr;
-  HIP_TRY(hipMalloc(&ds, sizeof(double) * (size_t)nstates * h->nc));
-  HIP_TRY(hipMalloc(&di, sizeof(double) * (size_t)(nstates > 1 ? nstates - 1 : 1)));
-  hipError_t e = copy_on(h->stream, ds, states, sizeof(double) * (size_t)nstates * h->nc,
-                          hipMemcpyHostToDevice);
-  if (e == hipSuccess && nstates > 1)
-    e = copy_on(h->stream, di, interfaces, sizeof(double) * (size_t)(nstates - 1),
-                hipMemcpyHostToDevice);
+  const size_t ns = (size_t)nstates * h->nc, ni = (size_t)(nstates - 1);
+  Space sp;
+  HIP_TRY(space_take(&sp));
+  // the states, then the interfaces: page-locked if they fit beside the status word
+  hipError_t e = space_device(sp, sizeof(double) * (ns + ni));
+  double* dev = (double*)sp.device;
+  if (e == hipSuccess && sizeof(double) * (ns + ni) + 64 <= Space::HOST) {
+    double* at = (double*)(sp.host + 64);
+    std::memcpy(at, states, sizeof(double) * ns);
+    if (ni) std::memcpy(at + ns, interfaces, sizeof(double) * ni);
+    e = hipMemcpyAsync(dev, at, sizeof(double) * (ns + ni), hipMemcpyHostToDevice, h->stream);
+  } else if (e == hipSuccess) {
+    e = hipMemcpyAsync(dev, states, sizeof(double) * ns, hipMemcpyHostToDevice, h->stream);
+    if (e == hipSuccess && ni)
+      e = hipMemcpyAsync(dev + ns, interfaces, sizeof(double) * ni, hipMemcpyHostToDevice, h->stream);
+  }
   if (e == hipSuccess) {
     h->step = 0;
     h->t = t0;
     long long nb = (h->n + 255) / 256;
-    hipLaunchKernelGGL(k_piecewise, dim3((unsigned)nb), dim3(256), 0, h->stream, ds, di,
+    hipLaunchKernelGGL(k_piecewise, dim3((unsigned)nb), dim3(256), 0, h->stream, dev, dev + ns,
                        nstates - 1, h->nc, h->Q[0], h->n, h->pitch);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  (void)hipFree(ds);
-  (void)hipFree(di);
-  if (e != hipSuccess) {
-    g_err = std::string("set_piecewise: ") + hipGetErrorString(e);
-    return HES_ERR_HIP;
-  }
-  HIP_TRY(zero_on(h->stream, h->status, 4 * sizeof(int)));
-  h->has_state = true;
-  return init_speeds(h);
+  return state_set(h, sp, e, "set_piecewise: ");
 }
 
 int hes_solver_set_state_device(hes_solver* h, const double* dQ, double t0) {
@@ -1120,16 +1139,8 @@ int hes_solver_set_state_device(hes_solver* h, const double* dQ, double t0) {
 int hes_solver_get_state(hes_solver* h, double* Q) {
   if (!h || !Q) return fail(HES_ERR_ARG, "null argument");
   if (!h->has_state) return fail(HES_ERR_ARG, "no state set");
-  size_t bytes = sizeof(double) * (size_t)h->nc * (size_t)h->n;
-  double* tmp = nullptr;
-  HIP_TRY(hipMalloc(&tmp, bytes));
-  long long nb = (h->n + 255) / 256;
-  hipLaunchKernelGGL(k_soa_to_aos, dim3((unsigned)nb), dim3(256), 0, h->stream, h->Q[h->step & 1],
-                     tmp, h->nc, h->n, h->pitch);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(Q, tmp, bytes, hipMemcpyDeviceToHost, h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  (void)hipFree(tmp);
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  const hipError_t e = download_state(h->Q[h->step & 1], Q, h->nc, h->n, h->pitch);
   if (e != hipSuccess) {
     g_err = std::string("get_state: ") + hipGetErrorString(e);
     return HES_ERR_HIP;
@@ -1197,11 +1208,10 @@ int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_gra
     const long long k = std::min(max_steps - done, RES_STEPS);
     long long now = 0;
     bool gave_up = false;
-    const int rc = run_resident(h, k, t_end, hist ? hist + done : nullptr, &now, &ms, &gave_up);
+    const int rc = run_resident(h, k, t_end, hist ? hist + done : nullptr, &now, &ms, &bad, &gave_up);
     if (rc != HES_OK) return rc;
     if (gave_up) break;
     done += now;
-    bad = h->mail->status[0];
     ended = now < k || done == max_steps;  // t reached t_end, or all steps done
   }
   if (!ended) {
@@ -1309,69 +1319,6 @@ int hes_copy_bandwidth(long long bytes, int reps, double* gbs) {
 // ---------------------------------------------------------------------------
 namespace {
 
-// What a call works in: page-locked host memory that the kernels read and
-// write themselves (small calls: no copies), device memory (larger ones), and
-// a stream of its own.  Allocated for every call they cost one on a single
-// state 90 of its 100 us.  One per call that is under way; at most SPACES_KEPT
-// wait for the next, per device, with at most Space::DEVICE bytes each.
-struct Space {
-  static constexpr size_t HOST = 128 * 1024, DEVICE = 96 << 20;
-  int dev = 0;
-  char* host = nullptr;
-  char* device = nullptr;
-  size_t device_bytes = 0;
-  hipStream_t stream = nullptr;
-};
-constexpr size_t SPACES_KEPT = 4;
-std::mutex& spaces_mutex() {
-  static std::mutex m;
-  return m;
-}
-std::vector<Space>& spaces() {
-  static auto* v = new std::vector<Space>();  // outlives the runtime's own end
-  return *v;
-}
-void space_free(Space& s) {
-  if (s.stream) (void)hipStreamDestroy(s.stream);
-  if (s.host) (void)hipHostFree(s.host);
-  if (s.device) (void)hipFree(s.device);
-}
-hipError_t space_take(Space* s) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  {
-    std::lock_guard<std::mutex> lock(spaces_mutex());
-    auto& v = spaces();
-    for (size_t k = 0; k < v.size(); ++k)
-      if (v[k].dev == dev) {
-        *s = v[k];
-        v.erase(v.begin() + (long)k);
-        return hipSuccess;
-      }
-  }
-  s->dev = dev;
-  e = hipHostMalloc((void**)&s->host, Space::HOST);
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
-  if (e != hipSuccess) {
-    space_free(*s);
-    *s = Space();
-  }
-  return e;
-}
-void space_give(Space& s, bool keep) {
-  if (keep && s.device_bytes <= Space::DEVICE) {
-    std::lock_guard<std::mutex> lock(spaces_mutex());
-    size_t here = 0;
-    for (const Space& o : spaces()) here += o.dev == s.dev;
-    if (here < SPACES_KEPT) {
-      spaces().push_back(s);
-      return;
-    }
-  }
-  space_free(s);
-}
-
 // A point-wise call: up to four input and three output arrays of doubles on
 // the host.  launch(in, out, status, stream) gets arrays the device can use.
 struct PointIo {
@@ -1395,13 +1342,7 @@ int run_points(const PointIo& io, Launch launch) {
   *status = 0;
   const bool small = total <= Space::HOST;
   hipError_t e = hipSuccess;
-  if (!small && s.device_bytes < total) {
-    if (s.device) e = hipFree(s.device);
-    s.device = nullptr;
-    s.device_bytes = 0;
-    if (e == hipSuccess) e = hipMalloc((void**)&s.device, total);
-    if (e == hipSuccess) s.device_bytes = total;
-  }
+  if (!small) e = space_device(s, total);
   char* at = (small ? s.host : s.device) + 64;
   for (int k = 0; k < 4 && e == hipSuccess; ++k) {
     if (!io.in[k]) continue;

@@ -1,0 +1,161 @@
+// hes_transfer.hpp -- a state on its way to the host: structure-of-arrays rows
+// on the device, one state after another (component fastest) in host memory.
+//
+// A copy into pageable memory runs at the rate of one host thread that copies
+// out of the runtime's staging memory and takes the page faults of a fresh
+// array (9 GB/s; 52 ms for 2^22 cells of 14 components, whose 400 Rusanov
+// steps take 72).  A large state is therefore cut into pieces, and several
+// threads each let a kernel write a piece into page-locked memory of their
+// own, in the host's order, and copy it out.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+#include "hes_host.hpp"
+
+namespace hes {
+
+// Cells [first, first + cells) of the rows Q in the host's order into out
+// (device or page-locked host memory), a block per GATHER_CELLS of them by way
+// of LDS, so that both sides move whole lines.
+constexpr int GATHER_CELLS = 128, GATHER_BLOCK = 256;
+static __global__ __launch_bounds__(GATHER_BLOCK) void k_gather(const double* __restrict__ Q,
+                                                               double* __restrict__ out, int nc,
+                                                               long long first, long long cells,
+                                                               long long pitch) {
+  extern __shared__ double tile[];
+  const long long c0 = (long long)blockIdx.x * GATHER_CELLS;
+  const int here = (int)(cells - c0 < GATHER_CELLS ? cells - c0 : GATHER_CELLS);
+  const int c = threadIdx.x % GATHER_CELLS;
+  if (c < here)
+    for (int r = threadIdx.x / GATHER_CELLS; r < nc; r += GATHER_BLOCK / GATHER_CELLS)
+      tile[c * nc + r] = __builtin_nontemporal_load(Q + r * pitch + first + c0 + c);
+  __syncthreads();
+  for (int t = threadIdx.x; t < here * nc; t += GATHER_BLOCK) out[c0 * nc + t] = tile[t];
+}
+
+inline hipError_t gather(const double* Q, double* out, int nc, long long first, long long cells,
+                         long long pitch, hipStream_t s) {
+  hipLaunchKernelGGL(k_gather, dim3((unsigned)((cells + GATHER_CELLS - 1) / GATHER_CELLS)),
+                     dim3(GATHER_BLOCK), sizeof(double) * GATHER_CELLS * nc, s, Q, out, nc, first,
+                     cells, pitch);
+  return hipGetLastError();
+}
+
+// Page-locked pieces of memory with a stream each, for the threads of large
+// downloads; at most PIECES_KEPT wait for the next one, per device.
+struct Piece {
+  static constexpr size_t BYTES = 4 << 20;
+  int dev = 0;
+  char* p = nullptr;
+  hipStream_t stream = nullptr;
+};
+inline constexpr int DOWNLOAD_THREADS = 8;
+inline constexpr size_t PIECES_KEPT = DOWNLOAD_THREADS;
+inline std::vector<Piece>& pieces() {  // under spaces_mutex()
+  static auto* v = new std::vector<Piece>();
+  return *v;
+}
+inline void piece_free(Piece& b) {
+  if (b.stream) (void)hipStreamDestroy(b.stream);
+  if (b.p) (void)hipHostFree(b.p);
+}
+inline hipError_t piece_take(int dev, Piece* b) {
+  {
+    std::lock_guard<std::mutex> lock(spaces_mutex());
+    auto& v = pieces();
+    for (size_t k = 0; k < v.size(); ++k)
+      if (v[k].dev == dev) {
+        *b = v[k];
+        v.erase(v.begin() + (long)k);
+        return hipSuccess;
+      }
+  }
+  b->dev = dev;
+  hipError_t e = hipHostMalloc((void**)&b->p, Piece::BYTES);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
+  if (e != hipSuccess) {
+    piece_free(*b);
+    *b = Piece();
+  }
+  return e;
+}
+inline void piece_give(Piece& b, bool keep) {
+  if (keep) {
+    std::lock_guard<std::mutex> lock(spaces_mutex());
+    size_t here = 0;
+    for (const Piece& o : pieces()) here += o.dev == b.dev;
+    if (here < PIECES_KEPT) {
+      pieces().push_back(b);
+      return;
+    }
+  }
+  piece_free(b);
+}
+
+// From this size on a download is shared by threads: below it their start and
+// the pieces' faults cost what they save.
+constexpr size_t DOWNLOAD_SHARED_MIN = 6 << 20;
+
+// The n states of rows Q (written by work that has been waited for) into `out`.
+inline hipError_t download_state(const double* Q, double* out, int nc, long long n,
+                                 long long pitch) {
+  const size_t bytes = sizeof(double) * (size_t)nc * (size_t)n;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (bytes < DOWNLOAD_SHARED_MIN) {
+    Space s;
+    e = space_take(&s);
+    if (e != hipSuccess) return e;
+    const bool small = bytes <= Space::HOST;
+    if (!small) e = space_device(s, bytes);
+    double* at = (double*)(small ? s.host : s.device);
+    if (e == hipSuccess) e = gather(Q, at, nc, 0, n, pitch, s.stream);
+    if (e == hipSuccess && !small) e = hipMemcpyAsync(out, at, bytes, hipMemcpyDeviceToHost, s.stream);
+    const hipError_t es = hipStreamSynchronize(s.stream);
+    if (e == hipSuccess) e = es;
+    if (e == hipSuccess && small) std::memcpy(out, at, bytes);
+    space_give(s, e == hipSuccess);
+    return e;
+  }
+  // cells of a piece: a share of a small state, a whole piece of a large one
+  const size_t piece = std::max<size_t>(std::min(Piece::BYTES, bytes / DOWNLOAD_THREADS), 1 << 20);
+  const long long per = (long long)(piece / (sizeof(double) * nc));
+  const long long parts = (n + per - 1) / per;
+  std::atomic<long long> next{0};
+  std::atomic<int> failed{(int)hipSuccess};
+  auto work = [&]() {
+    Piece b;
+    hipError_t we = hipSetDevice(dev);
+    if (we == hipSuccess) we = piece_take(dev, &b);
+    while (we == hipSuccess && failed.load() == (int)hipSuccess) {
+      const long long k = next.fetch_add(1);
+      if (k >= parts) break;
+      const long long c0 = k * per, cells = std::min(per, n - c0);
+      we = gather(Q, (double*)b.p, nc, c0, cells, pitch, b.stream);
+      const hipError_t es = b.stream ? hipStreamSynchronize(b.stream) : hipSuccess;
+      if (we == hipSuccess) we = es;
+      if (we == hipSuccess)
+        std::memcpy(out + c0 * nc, b.p, sizeof(double) * (size_t)nc * (size_t)cells);
+    }
+    if (we != hipSuccess) failed.store((int)we);
+    if (b.p) piece_give(b, we == hipSuccess);
+  };
+  std::vector<std::thread> threads;
+  try {
+    for (long long k = 1; k < std::min<long long>(DOWNLOAD_THREADS, parts); ++k)
+      threads.emplace_back(work);
+  } catch (const std::system_error&) {  // fewer threads share the work
+  }
+  work();
+  for (std::thread& t : threads) t.join();
+  return (hipError_t)failed.load();
+}
+
+}  // namespace hes
