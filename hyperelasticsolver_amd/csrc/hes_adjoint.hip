@@ -22,10 +22,9 @@
 // its conserved state and of b0, c0) is generated code (hes_adjoint_gen.hpp).
 //
 // Storage: every `every`-th state is kept (with its sound speeds); a backward
-// segment recomputes the states in between with the forward kernel (bit-identical
-// to the first pass), then runs the reverse steps over them.  The recompute of
-// the next (earlier) segment runs on a second stream into the other of two
-// segment buffers while the reverse steps of the current one run.  The lmax term of
+// segment recomputes the states in between with the first pass's arithmetic
+// and time steps (the same bits), then runs the reverse steps over them (see
+// record_backward for how the two share the GPU).  The lmax term of
 // step s needs the global sum dtdxbar_s, so it is applied when step s-1 loads
 // Qbar_s: the one or two waves holding the argmax cell reduce the block
 // partials of step s and add lmaxbar_s * dlam/d(Q, b0, c0) of that cell
@@ -129,7 +128,6 @@ struct AdjFwdArgs {
   unsigned long long* lmax;  // lmax[s] = max CFL speed of state s (double bits)
   double* blk_val;           // FWD_RECORD: per-block argmax of the CFL speed of state s + 1
   long long* blk_idx;
-  long long* istar;          // FWD_FIND: argmax cell of every state
   int* status;
   long long n, pitch, s;
   double cfl, dx;
@@ -137,13 +135,11 @@ struct AdjFwdArgs {
 };
 
 // What a forward step records of the new state s + 1's CFL speeds:
-//   FWD_MAX     the first pass: their max, into lmax[s + 1]
-//   FWD_RECORD  the first pass at a checkpoint state: also the per-block argmax
-//   FWD_FIND    a recompute of the reverse pass: the argmax cell (smallest
-//               index) of the max that the first pass recorded, into istar[s + 1]
+//   FWD_MAX     their max, into lmax[s + 1]
+//   FWD_RECORD  into a checkpoint state: also the per-block argmax
 // The argmax of the states between checkpoints is found while the reverse
-// pass recomputes them, so the first pass does no more than a plain run's max.
-enum { FWD_MAX = 0, FWD_RECORD = 1, FWD_FIND = 2 };
+// pass recomputes them, so this pass does no more than a plain run's max.
+enum { FWD_MAX = 0, FWD_RECORD = 1 };
 
 // One time step: the solver's chunk step (so states match a plain run bit for
 // bit) plus the bookkeeping of the reverse pass.
@@ -159,19 +155,7 @@ __global__ __launch_bounds__(ABLK) __attribute__((amdgpu_waves_per_eu(3))) void 
   const double lmax = lmax_of(a.lmax, a.s);
   const double lam = chunk_step<1, FLUX_RUSANOV, 1>(ctx, i, q, cc, lmax);
   const bool owned = i >= 0 && i < a.n && lane >= 1 && lane <= TILE;
-  if constexpr (MODE == FWD_FIND) {
-    // The recomputed speeds are those of the first pass, bit for bit.  Where
-    // the maximum is that of a uniform region, every cell of it attains it:
-    // one atomic per wave that lies before the smallest index found so far,
-    // not one per cell (half of 2^18 cells tied: 34 us per step, all of it
-    // the atomics on one word; 20 us with this).
-    const unsigned long long hits = __ballot(owned && lam == lmax_of(a.lmax, a.s + 1));
-    if (hits != 0ull && lane == 0) {
-      unsigned long long* slot = (unsigned long long*)(a.istar + a.s + 1);
-      const unsigned long long at = (unsigned long long)(i + (long long)__builtin_ctzll(hits));
-      if (at < __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(slot, at);
-    }
-  } else if constexpr (MODE == FWD_RECORD) {
+  if constexpr (MODE == FWD_RECORD) {
     const long long row = (a.s + 1) * (long long)gridDim.x;
     record_speeds<ABLK>(lam, owned, i, a.lmax + a.s + 1, a.blk_val + row, a.blk_idx + row);
   } else {
@@ -184,6 +168,57 @@ __global__ __launch_bounds__(ABLK) __attribute__((amdgpu_waves_per_eu(3))) void 
         atomicMax(slot, bits);
     }
   }
+}
+
+// The whole first pass in one launch, for a problem that fits the chip.
+struct AdjResArgs {
+  ResTeam team;
+  AdjHook hook;
+  MatDev mat;
+};
+template <int BLK, int T>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(BLK / 256)))
+void k_adj_resident(AdjResArgs a) {
+  ResTeam tm = a.team;
+  tm.rank = (int)xcd_block();
+  AdjHook hook = a.hook;
+  hook.first = tm.rank == 0 && threadIdx.x == 0;
+  (void)resident_run1<FLUX_RUSANOV, 1, BLK, T, RES_MAX_TEAM>(tm, a.mat, hook);
+}
+__global__ void k_adj_nocell(long long* __restrict__ istar, long long m) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < m) istar[t] = NO_CELL;
+}
+
+// States s + 1 .. s + steps from state s (segment_run).  With zin (the zero
+// flags of Qbar of state `end`, a segment's last), only workgroups whose
+// states the reverse steps down to state s can read run: those within reach of
+// a tile with a cotangent or of an argmax cell, which moves one cell per step
+// and is read a tile to either side.
+struct AdjSegArgs {
+  SegCtx c;
+  const int* zin;
+  const long long* istar;
+  long long s, end, nsteps;
+  int nw;
+  MatDev mat;
+};
+__global__ __launch_bounds__(SEG_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
+void k_adj_segment(AdjSegArgs a) {
+  SegCtx c = a.c;
+  c.o0 = xcd_block() * (c.halo ? SEG_OWN : SEG_CELLS);
+  c.o1 = min(c.o0 + (c.halo ? SEG_OWN : SEG_CELLS), c.hi);
+  if (a.zin) {
+    const long long reach = a.end - a.s + 2 * TILE + 2;
+    const long long lo = max(c.o0 - reach, 0LL), hi = min(c.o1 + reach, c.hi);  // [lo, hi)
+    bool needed = false;
+    for (long long t = lo / TILE + threadIdx.x; t < a.nw && t * TILE < hi; t += SEG_BLOCK)
+      needed |= a.zin[t] == 0;
+    for (long long s = a.s + threadIdx.x; s <= a.end && s < a.nsteps; s += SEG_BLOCK)
+      needed |= a.istar[s] >= lo && a.istar[s] < hi;
+    if (!__syncthreads_or(needed)) return;
+  }
+  segment_run(c, a.mat);
 }
 
 // Argmax cell of the CFL speed of the checkpoint states from the per-block
@@ -588,6 +623,9 @@ __global__ __launch_bounds__(64) void k_adj_final(
 // ---------------------------------------------------------------------------
 struct hes_adjoint {
   long long n, pitch, nsteps, every, nck;
+  int dev = 0, cus = 0;
+  ResPlan res = {{0, 0}, 0, 0};        // the first pass in one launch; block 0: a launch per step
+  unsigned long long* comm = nullptr;  // its team's messages
   int nb;    // blocks of the tiled kernels
   int nbr;   // blocks of the reverse step: one per CU (persistent waves)
   int nbl;   // blocks of the one-cell-per-thread kernels
@@ -668,7 +706,6 @@ AdjFwdArgs fwd_args(hes_adjoint* h, long long s, const double* qi, double* qo, c
   a.lmax = h->lmax;
   a.blk_val = h->blk_val;
   a.blk_idx = h->blk_idx;
-  a.istar = h->istar;
   a.status = h->status;
   a.n = h->n;
   a.pitch = h->pitch;
@@ -679,14 +716,58 @@ AdjFwdArgs fwd_args(hes_adjoint* h, long long s, const double* qi, double* qo, c
   return a;
 }
 
-hipError_t record_forward(hes_adjoint* h) {
+long long comm_words(const hes_adjoint* h) { return (long long)res_words_of(h->res.G, NQ); }
+
+// The first pass from checkpoint 0 (the initial state) in one launch.
+hipError_t record_resident(hes_adjoint* h) {
+  hipStream_t st = h->stream;
+  const long long words = comm_words(h);
+  hipLaunchKernelGGL(k_adj_zero, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
+                     (double*)h->comm, words);
+  hipLaunchKernelGGL(k_adj_nocell, dim3((unsigned)((h->nsteps + 255) / 256)), dim3(256), 0, st,
+                     h->istar, h->nsteps);
+  AdjResArgs a;
+  std::memset((void*)&a, 0, sizeof(a));
+  double *qn, *cn;
+  fwd_slot(h, h->nsteps, &qn, &cn);
+  ResTeam& tm = a.team;
+  tm.Qin = ck_q(h, 0);
+  tm.Qout = qn;
+  tm.Cout = cn;
+  tm.pitch = h->pitch;
+  tm.hi = h->n;
+  tm.G = h->res.G;
+  tm.own = h->res.own;
+  tm.cfl = h->cfl;
+  tm.dx = h->dx;
+  tm.t_end = INFINITY;
+  tm.kmax = h->nsteps;
+  tm.status = h->status;
+  tm.slots = h->comm;
+  tm.border = h->comm + (size_t)2 * h->res.G * RES_SLOT;
+  tm.tag0 = 1;  // the buffer was cleared above
+  tm.gave_up = h->status + 2;
+  a.hook.ck = ck_q(h, 0);
+  a.hook.lmax = h->lmax;
+  a.hook.istar = h->istar;
+  a.hook.every = h->every;
+  a.hook.nsteps = h->nsteps;
+  a.hook.pitch = h->pitch;
+  a.hook.stride = 1;
+  a.mat = h->mat;
+  const ResShape& sh = h->res.shape;
+  void (*k)(AdjResArgs) = sh.block == 256  ? k_adj_resident<256, 1>
+                          : sh.tiles == 1 ? k_adj_resident<512, 1>
+                          : sh.tiles == 2 ? k_adj_resident<512, 2>
+                                          : k_adj_resident<512, 3>;
+  return res_launch(k, sh.block, h->res.G, a, st);
+}
+
+// The first pass from checkpoint 0, a launch per step.
+void record_steps(hes_adjoint* h) {
   hipStream_t st = h->stream;
   const long long n = h->n;
   const unsigned nbl = (unsigned)h->nbl;
-  hipLaunchKernelGGL(k_adj_p2c, dim3((h->nst + 63) / 64), dim3(64), 0, st, h->prims, h->gin,
-                     h->states, h->nst);
-  hipLaunchKernelGGL(k_adj_fill, dim3(nbl), dim3(LBLK), 0, st, h->states, h->bounds, h->nst,
-                     ck_q(h, 0), n, h->pitch);
   hipLaunchKernelGGL(k_adj_ends, dim3((h->nslots * 2 * NQ + 63) / 64), dim3(64), 0, st,
                      ck_q(h, 0), h->slots, h->nslots, n, h->pitch);
   hipLaunchKernelGGL(k_adj_zero, dim3((unsigned)((h->nsteps + 1 + 255) / 256)), dim3(256), 0, st,
@@ -708,6 +789,22 @@ hipError_t record_forward(hes_adjoint* h) {
   }
   hipLaunchKernelGGL(k_adj_argmax, dim3((unsigned)h->nsteps), dim3(64), 0, st, h->blk_val,
                      h->blk_idx, h->nb, h->nbl, h->every, h->istar);
+}
+
+hipError_t record_forward(hes_adjoint* h) {
+  hipStream_t st = h->stream;
+  const long long n = h->n;
+  const unsigned nbl = (unsigned)h->nbl;
+  hipLaunchKernelGGL(k_adj_p2c, dim3((h->nst + 63) / 64), dim3(64), 0, st, h->prims, h->gin,
+                     h->states, h->nst);
+  hipLaunchKernelGGL(k_adj_fill, dim3(nbl), dim3(LBLK), 0, st, h->states, h->bounds, h->nst,
+                     ck_q(h, 0), n, h->pitch);
+  if (h->res.shape.block) {
+    const hipError_t e = record_resident(h);
+    if (e != hipSuccess) return e;
+  } else {
+    record_steps(h);
+  }
   double *qn, *cn;
   fwd_slot(h, h->nsteps, &qn, &cn);
   hipLaunchKernelGGL(k_adj_loss, dim3(nbl), dim3(LBLK), 0, st, qn, h->rho_t, h->u_t, h->mat8[0],
@@ -732,46 +829,78 @@ hipError_t record_backward(hes_adjoint* h) {
                      h->zf + (long long)fin * h->nw, h->n, h->pitch, h->nw);
   hipLaunchKernelGGL(k_adj_izero, dim3((unsigned)((h->nw + 255) / 256)), dim3(256), 0, st,
                      h->zf + (long long)(1 - fin) * h->nw, (long long)h->nw);
-  // Segment c's states are recomputed into segment buffer c & 1 on stream2
-  // (the k_adj_fwd steps and k_adj_lam, which read only the checkpoints and
-  // the first pass's CFL records), while the reverse steps of segment c + 1
-  // run on `st` from the other buffer.  Events order the two: the reverse of
-  // segment c waits for its buffer to be ready, and the recompute of segment
-  // c - 1 waits until the reverse of segment c + 1 (the last reader of the
-  // buffer it overwrites) is done.  Both streams are in the capture: stream2
-  // forks from `st` and joins it at the end.
-  hipStream_t st2 = h->stream2;
-  HIP_TRY_E(hipEventRecord(h->ev_fork, st));
-  HIP_TRY_E(hipStreamWaitEvent(st2, h->ev_fork, 0));
+  // Segment c's states are recomputed into segment buffer c & 1 (k_adj_segment
+  // and k_adj_lam, which read only the checkpoints and the first pass's CFL
+  // records).  Where zero tiles are skipped, that follows the reverse steps of
+  // segment c + 1 on `st`, whose zero flags say which states are needed (at
+  // 2^18 cells a few hundredths).  Otherwise it runs on stream2 while the
+  // reverse steps of segment c + 1 run on `st` from the other buffer, and
+  // events order the two: the reverse of segment c waits for its buffer to be
+  // ready, and the recompute of segment c - 1 waits until the reverse of
+  // segment c + 1 (the last reader of the buffer it overwrites) is done.  Both
+  // streams are in the capture: stream2 forks from `st` and joins it at the end.
+  // (A first pass step by step leaves the argmax cells between checkpoints to
+  // be found here, on every cell.)
+  const bool find = h->res.shape.block == 0;
+  // Small problems keep the overlap: their recompute is short, and all of it is
+  // soon needed (us per reverse step, overlapped and skipping: 1000 cells 9.4
+  // and 10.5, 30000 10.3 and 10.6, 50000 11.0 and 10.5, 131072 14.1 and 12.3,
+  // 2^18 18.1 and 13.3; 34.5 with one launch per recomputed step).
+  const bool skip = h->sparse && !find && h->nw > 3 * h->cus;
+  hipStream_t st2 = skip ? st : h->stream2;
+  if (!skip) {
+    HIP_TRY_E(hipEventRecord(h->ev_fork, st));
+    HIP_TRY_E(hipStreamWaitEvent(st2, h->ev_fork, 0));
+  }
   auto recompute = [&](long long c) -> hipError_t {
     const long long s0 = c * h->every;
     const long long end = std::min(s0 + h->every, h->nsteps);
     const int buf = (int)(c & 1);
-    for (long long s = s0; s + 1 < end; ++s) {
-      // each recomputed state keeps its sound speeds in row 14 of its slot,
-      // as the checkpoints do: the reverse step reads its face speeds there
-      const double* ci = seg_slot(h, s, s0, buf) + 14 * h->pitch;
-      double* co = seg_slot(h, s + 1, s0, buf) + 14 * h->pitch;
-      hipLaunchKernelGGL(k_adj_fwd<FWD_FIND>, dim3((unsigned)h->nb), dim3(ABLK), 0, st2,
-                         fwd_args(h, s, seg_slot(h, s, s0, buf), seg_slot(h, s + 1, s0, buf), ci,
-                                  co));
+    for (long long s = s0; s + 1 < end; s += SEG_STEPS) {
+      AdjSegArgs a;
+      std::memset((void*)&a, 0, sizeof(a));
+      a.c.Q = seg_slot(h, s, s0, buf);
+      a.c.out = seg_slot(h, s + 1, s0, buf);
+      a.c.lmax = h->lmax + s;
+      a.c.istar = h->istar + s;
+      a.c.stride = 1;
+      a.c.pitch = h->pitch;
+      a.c.hi = h->n;
+      a.c.halo = h->n > SEG_CELLS ? SEG_STEPS : 0;
+      a.c.steps = (int)std::min<long long>(SEG_STEPS, end - 1 - s);
+      a.c.find = find;
+      a.c.cfl = h->cfl;
+      a.zin = skip ? h->zf + (end & 1) * h->nw : nullptr;
+      a.istar = h->istar;
+      a.s = s;
+      a.end = end;
+      a.nsteps = h->nsteps;
+      a.nw = h->nw;
+      a.mat = h->mat;
+      const long long per = a.c.halo ? SEG_OWN : SEG_CELLS;
+      hipLaunchKernelGGL(k_adj_segment, dim3((unsigned)((h->n + per - 1) / per)), dim3(SEG_BLOCK),
+                         0, st2, a);
     }
     const int cnt = (int)(end - s0);
     hipLaunchKernelGGL(k_adj_lam, dim3((cnt + 63) / 64), dim3(64), 0, st2, ck_q(h, c),
                        h->seg[buf], 15 * h->pitch, h->pitch, h->istar, h->gin, s0, cnt, h->n,
                        h->Jlam);
-    return hipEventRecord(h->ev_ready[buf], st2);
+    return skip ? hipSuccess : hipEventRecord(h->ev_ready[buf], st2);
   };
-  HIP_TRY_E(recompute(h->nck - 1));
+  if (!skip) HIP_TRY_E(recompute(h->nck - 1));
   for (long long c = h->nck - 1; c >= 0; --c) {
     const long long s0 = c * h->every;
     const long long end = std::min(s0 + h->every, h->nsteps);
     const int buf = (int)(c & 1);
-    if (c >= 1) {
-      if (c + 1 < h->nck) HIP_TRY_E(hipStreamWaitEvent(st2, h->ev_done[(c + 1) & 1], 0));
-      HIP_TRY_E(recompute(c - 1));
+    if (skip) {
+      HIP_TRY_E(recompute(c));
+    } else {
+      if (c >= 1) {
+        if (c + 1 < h->nck) HIP_TRY_E(hipStreamWaitEvent(st2, h->ev_done[(c + 1) & 1], 0));
+        HIP_TRY_E(recompute(c - 1));
+      }
+      HIP_TRY_E(hipStreamWaitEvent(st, h->ev_ready[buf], 0));
     }
-    HIP_TRY_E(hipStreamWaitEvent(st, h->ev_ready[buf], 0));
     for (long long s = end - 1; s >= s0; --s) {
       AdjStepArgs a;
       a.Q = seg_slot(h, s, s0, buf);
@@ -801,10 +930,12 @@ hipError_t record_backward(hes_adjoint* h) {
       a.gin[4] = h->mat8[3];
       hipLaunchKernelGGL(k_adj_step, dim3((unsigned)h->nbr), dim3(ABLK), 0, st, a);
     }
-    HIP_TRY_E(hipEventRecord(h->ev_done[buf], st));
+    if (!skip) HIP_TRY_E(hipEventRecord(h->ev_done[buf], st));
   }
-  HIP_TRY_E(hipEventRecord(h->ev_join, st2));
-  HIP_TRY_E(hipStreamWaitEvent(st, h->ev_join, 0));
+  if (!skip) {
+    HIP_TRY_E(hipEventRecord(h->ev_join, st2));
+    HIP_TRY_E(hipStreamWaitEvent(st, h->ev_join, 0));
+  }
   hipLaunchKernelGGL(k_adj_q0sum, dim3((unsigned)h->nbl), dim3(LBLK), 0, st, h->qb[0], h->bounds,
                      h->nst, h->part, h->n, h->pitch);
   hipLaunchKernelGGL(k_adj_final, dim3(1), dim3(64), 0, st, h->part, h->nbl, h->thb, h->nbr,
@@ -853,6 +984,9 @@ int hes_adjoint_create(hes_adjoint** out, long long ncells, const double* materi
       cus < 1)
     return fail(HES_ERR_HIP, "cannot read the device's compute-unit count");
   hes_adjoint* h = new hes_adjoint();
+  h->dev = dev;
+  h->cus = cus;
+  h->res = res_plan1(ncells, cus);
   h->n = ncells;
   h->pitch = (ncells + 63) / 64 * 64 + 256;  // rows padded off a power-of-two stride, as the solver's
   h->nsteps = nsteps;
@@ -898,6 +1032,7 @@ int hes_adjoint_create(hes_adjoint** out, long long ncells, const double* materi
   if (e == hipSuccess) e = dalloc(&h->rho_t, P);
   if (e == hipSuccess) e = dalloc(&h->u_t, P);
   if (e == hipSuccess) e = dalloc(&h->status, 4);
+  if (e == hipSuccess && h->res.shape.block) e = dalloc(&h->comm, (size_t)comm_words(h));
   if (e == hipSuccess) e = zero_on(h->stream, h->status, 4 * sizeof(int));
   if (e == hipSuccess) {
     // gin = (b0, c0, rho0, cv, t0): the inputs of the generated routines
@@ -905,11 +1040,9 @@ int hes_adjoint_create(hes_adjoint** out, long long ncells, const double* materi
     e = copy_on(h->stream, h->gin, g, sizeof(g), hipMemcpyHostToDevice);
   }
   if (e == hipSuccess) {
-    // every state slot whose end cells must be filled
+    // the state slots whose end cells a pass step by step does not write
     std::vector<double*> sl;
     for (long long c = 1; c < h->nck; ++c) sl.push_back(ck_q(h, c));
-    for (int b = 0; b < 2; ++b)
-      for (long long j = 0; j + 1 < h->every; ++j) sl.push_back(h->seg[b] + j * 15 * P);
     sl.push_back(h->fq[0]);
     sl.push_back(h->fq[1]);
     h->nslots = (int)sl.size();
@@ -936,7 +1069,7 @@ int hes_adjoint_destroy(hes_adjoint* h) {
   void* bufs[] = {h->ck, h->seg[0], h->seg[1], h->fq[0], h->fq[1], h->fc[0], h->fc[1], h->qb[0], h->qb[1], h->zf,
                   h->lmax, h->blk_val, h->blk_idx, h->istar, h->Jlam, h->dtp, h->thb, h->lossp,
                   h->part, h->sums, h->gout, h->gin, h->prims, h->states, h->bounds, h->rho_t,
-                  h->u_t, h->slots, h->status};
+                  h->u_t, h->slots, h->status, h->comm};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   hipEvent_t evs[] = {h->ev0, h->ev1, h->ev_fork, h->ev_join, h->ev_ready[0], h->ev_ready[1],
@@ -1026,16 +1159,25 @@ int hes_adjoint_forward(hes_adjoint* h, double* loss, float* elapsed_ms) {
       return HES_ERR_HIP;
     }
   }
-  HIP_TRY(hipEventRecord(h->ev0, h->stream));
-  if (h->use_graph) HIP_TRY(hipGraphLaunch(h->gf, h->stream));
-  else HIP_TRY(record_forward(h));
-  HIP_TRY(hipEventRecord(h->ev1, h->stream));
-  HIP_TRY(hipEventSynchronize(h->ev1));
+  int st[4];
+  {
+    ComputeUnits units(h->dev, h->cus, h->res.shape.block && h->res.G > 1 ? h->res.G : 0);
+    HIP_TRY(hipEventRecord(h->ev0, h->stream));
+    if (h->use_graph) HIP_TRY(hipGraphLaunch(h->gf, h->stream));
+    else HIP_TRY(record_forward(h));
+    HIP_TRY(hipEventRecord(h->ev1, h->stream));
+    HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
+  }
+  if (st[2]) {  // the team was not on the chip together: a launch per step from here on
+    h->res.shape = {0, 0};
+    if (h->gf) (void)hipGraphExecDestroy(h->gf);
+    if (h->gb) (void)hipGraphExecDestroy(h->gb);
+    h->gf = h->gb = nullptr;
+    return hes_adjoint_forward(h, loss, elapsed_ms);
+  }
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   if (elapsed_ms) *elapsed_ms = ms;
-  int st[2];
-  HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
   if (st[0]) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
   std::vector<double> lp(h->nbl);
   HIP_TRY(copy_on(h->stream, lp.data(), h->lossp, sizeof(double) * h->nbl, hipMemcpyDeviceToHost));
@@ -1137,6 +1279,7 @@ int hes_adjoint_info(hes_adjoint* h, long long* device_bytes, long long* checkpo
   const long long P = h->pitch;
   long long b = h->nck * 15 * P + 2 * (h->every - 1) * 15 * P + 2 * (14 + 1 + 14) * P;
   b = b * 8 + (h->nsteps + 1) * 8 + h->nsteps * (long long)h->nb * 16 + h->nsteps * (8 + JL * 8);
+  if (h->comm) b += 8 * comm_words(h);
   if (device_bytes) *device_bytes = b;
   if (checkpoints) *checkpoints = h->nck;
   return HES_OK;

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "hes_adjoint_gen.hpp"
+#include "hes_resident.hpp"
 #include "hes_step.hpp"
 
 // A batch and a single problem must evolve bit for bit alike, so both
@@ -214,6 +215,130 @@ __device__ __forceinline__ void reverse_chunk(const double* q, double* qb, bool 
     for (int k = 0; k < 6; ++k) ob[NQ + k] = lbar * gO[k];
   };
   hes_gen::cell_fwd_vjp(in, out, seed, seed_acoustic, ib);
+}
+
+// The argmax cell of a state's CFL speed (smallest index): the cells of this
+// wave that attain the recorded maximum lmax, lane 0 holding cell i0.  Where
+// the maximum is that of a uniform region, every cell of it attains it: one
+// atomic per wave that lies before the smallest index found so far, not one
+// per cell (half of 2^18 cells tied: 34 us per step, all of it the atomics on
+// one word; 20 us with this).
+__device__ __forceinline__ void note_argmax(bool own, double lam, double lmax, long long i0,
+                                            long long* istar) {
+  const unsigned long long hits = __ballot(own && lam == lmax);
+  if (hits != 0ull && (threadIdx.x & 63) == 0) {
+    unsigned long long* slot = (unsigned long long*)istar;
+    const unsigned long long at = (unsigned long long)(i0 + (long long)__builtin_ctzll(hits));
+    if (at < __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin(slot, at);
+  }
+}
+
+// What the forward pass keeps of a state while it stays on the chip
+// (resident_run1's hook): its CFL maximum and argmax cell, and every
+// `every`-th state with its sound speeds.
+struct AdjHook {
+  double* ck;  // the next checkpoint's slot: 14 rows of the state, then the speeds
+  unsigned long long* lmax;  // of state s at lmax[s * stride]
+  long long* istar;
+  long long next, every, nsteps, pitch, stride;
+  bool first;  // this thread records the maximum
+  __device__ __forceinline__ void tile(long long s, double lm, bool own, bool lead, long long i,
+                                       const double* q, double c, double u1) {
+    // its first workgroup has the smallest index
+    if (s < nsteps && lead) {
+      const unsigned long long hits = __ballot(own && fabs(u1) + c == lm);
+      if (hits != 0ull && (threadIdx.x & 63) == 0)
+        atomicMin((unsigned long long*)(istar + s * stride),
+                  (unsigned long long)(i + (long long)__builtin_ctzll(hits)));
+    }
+    if (s == next && s < nsteps && own) {
+      if (s > 0) {
+#pragma unroll
+        for (int r = 0; r < NQ; ++r) ck[r * pitch + i] = q[r];
+      }
+      ck[NQ * pitch + i] = c;
+    }
+  }
+  __device__ __forceinline__ void end(long long s, double lm) {
+    if (first) lmax[s * stride] = (unsigned long long)__double_as_longlong(lm);
+    if (s == next) {
+      next += every;
+      ck += 15 * pitch;
+    }
+  }
+};
+
+// Recompute of the states between checkpoints.  Their time steps are known
+// from the first pass, so nothing has to be exchanged between workgroups: each
+// takes SEG_STEPS steps with its cells in registers and SEG_STEPS halo cells
+// on either side, which lose one valid cell per step at their outer end, and
+// writes every state on the way (a launch per step read and wrote each state,
+// 20 us per step at 2^18 cells; here 5 us).  The halo costs 25% more
+// arithmetic; 25 steps make two launches of the usual 50-step segment.
+constexpr int SEG_BLOCK = 256;
+constexpr int SEG_STEPS = 25;
+constexpr int SEG_CELLS = SEG_BLOCK / 64 * TILE + 2;    // cells of a workgroup
+constexpr int SEG_OWN = SEG_CELLS - 2 * SEG_STEPS;      // without the halos
+struct SegCtx {
+  const double* Q;   // state s (14 rows)
+  double* out;       // states s + 1, s + 2, ..: slots of 15 rows
+  const unsigned long long* lmax;  // of state s + k at lmax[k * stride]
+  long long* istar;  // of state s + k at istar[k * stride] (find)
+  long long stride, pitch, lo, hi, o0, o1;  // the problem's cells, this workgroup's
+  int halo, steps, find;
+  double cfl;
+};
+__device__ __forceinline__ void segment_run(const SegCtx& a, const MatDev& mat) {
+  constexpr int W = SEG_BLOCK / 64;
+  __shared__ double edge[2][W][2][NQ];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long i = a.o0 - a.halo + TILE * w + lane;
+  const long long ic = i < a.lo ? a.lo : (i >= a.hi ? a.hi - 1 : i);
+  const bool whole = a.halo == 0;
+  const bool own = i >= a.o0 && i < a.o1 && (lane >= 1 || (whole && w == 0)) &&
+                   (lane <= TILE || (whole && w == W - 1));
+  const bool moves = lane >= 1 && lane <= TILE && i > a.lo && i < a.hi - 1;
+  double q[NQ];
+#pragma unroll
+  for (int r = 0; r < NQ; ++r) q[r] = a.Q[r * a.pitch + ic];
+  double* out = a.out - 15 * a.pitch;
+#pragma unroll 1
+  for (int k = 0;; ++k, out += 15 * a.pitch) {
+    Thermo th;
+    thermo<true, 1>(mat, 1.0, q, th);
+    const double c = sound_speed(mat, th);
+    if (k > 0) {
+      if (own) {
+#pragma unroll
+        for (int r = 0; r < NQ; ++r) out[r * a.pitch + i] = q[r];
+        out[NQ * a.pitch + i] = c;
+      }
+      if (a.find)
+        note_argmax(own, fabs(th.u[0]) + c, lmax_of(a.lmax, k * a.stride), i - lane,
+                    a.istar + k * a.stride);
+    }
+    if (k == a.steps) return;
+    double f[NQ], upd[NQ];
+    phase_flux(mat, 1.0, th, q + 5, f);
+    const double dtdx = a.cfl * rcp(lmax_of(a.lmax, k * a.stride));
+    update_rusanov1<true>(q, f, th.u[0] - c, th.u[0] + c, dtdx, 0, upd);
+    if (moves) {
+#pragma unroll
+      for (int r = 0; r < NQ; ++r) q[r] = upd[r];
+    }
+    if (lane == 1 || lane == TILE) {
+#pragma unroll
+      for (int r = 0; r < NQ; ++r) edge[k & 1][w][lane == 1 ? 0 : 1][r] = q[r];
+    }
+    res_barrier();
+    if ((lane == 0 && w > 0) || (lane == 63 && w < W - 1)) {
+      const double* e = edge[k & 1][lane == 0 ? w - 1 : w + 1][lane == 0 ? 1 : 0];
+#pragma unroll
+      for (int r = 0; r < NQ; ++r) q[r] = e[r];
+    }
+  }
 }
 
 }  // namespace hes_adj

@@ -164,13 +164,6 @@ struct ResArgs {
   MatDev mat[2];
 };
 
-// Shape of a team's workgroups: threads, and what a wave holds: tiles of 64
-// cells (one phase), or cells (two phases).
-struct ResShape {
-  int block, tiles;
-};
-constexpr int RES_MAX_TEAM = 256;  // workgroups
-
 // The team's first workgroup leaves the handle's rings as k_step expects them.
 __device__ __forceinline__ void resident_end(const ResArgs& a, const ResTeam& tm, const ResOut& o) {
   if (tm.rank != 0 || threadIdx.x != 0) return;
@@ -781,16 +774,6 @@ int run_launches(hes_solver* h, long long max_steps, double t_end, int use_graph
 
 constexpr long long RES_STEPS = 1LL << 16;  // steps of one launch at most
 
-// How a problem is laid on the chip (block 0: it is not, and runs step by
-// step): the first of these shapes whose team has a compute unit for every
-// workgroup.  Fewer waves per SIMD come first, since a step's chain of
-// dependent FP64 operations is what a team of few waves waits for (us per
-// step, Rusanov / HLL, this shape against the next at the same cells, 59000:
-// 4.4 / 3.8 against 4.9 / 4.9; 123000: 5.3 / 5.1 against 7.1 / 8.2; 250000:
-// 7.6 / 8.2 against 9.3 / 11.8; the last against one launch per step, 300000:
-// 9.5 / 11.8 against 21.1 / 20.3).  Two tiles of 64 cells per wave and three
-// fill the registers of two waves per SIMD (200 to 256 VGPRs).
-constexpr ResShape RES_SHAPES[4] = {{256, 1}, {512, 1}, {512, 2}, {512, 3}};
 // Two phases: the narrowest tiles with which the team fits (resident_run2).
 // A face's path terms cost more than its cell, and the faces that jump sit
 // together around the interfaces, so a wave with 64 cells may work on all its
@@ -799,48 +782,17 @@ constexpr ResShape RES_SHAPES[4] = {{256, 1}, {512, 1}, {512, 2}, {512, 3}};
 // this: HLL, 1000 cells 189 -> 21, 10007 60 -> 21, 27000 42 -> 31, but 59000
 // 38 -> 52, where it is left out; Rusanov 45 -> 14, 25 -> 14, 22 -> 14 and 26
 // -> 20.
-constexpr ResShape RES_SHAPES2[4] = {{256, 16}, {256, 32}, {256, 64}, {0, 0}};
-constexpr int RES_HLL2_MAX_TILE = 32;
+constexpr ResShape RES_SHAPES2[3] = {{256, 16}, {256, 32}, {256, 64}};  // HLL: the first two
 
 void plan_resident(hes_solver* h) {
-  h->shape = {0, 0};
-  for (const ResShape s : h->nph == 1 ? RES_SHAPES : RES_SHAPES2) {
-    if (s.block == 0) continue;
-    if (h->nph == 2 && h->flux == HES_FLUX_HLL && s.tiles > RES_HLL2_MAX_TILE) continue;
-    const int waves = s.block / 64;
-    const int cells = (h->nph == 1 ? waves * s.tiles * TILE : waves * (s.tiles - 2)) + 2;  // of a team of one
-    const int per = cells - 2 * RES_HALO;
-    const long long g = h->n <= cells ? 1 : (h->n + per - 1) / per;
-    if (g > std::min(h->cus, RES_MAX_TEAM)) continue;
-    h->shape = s;
-    h->res_g = (int)g;
-    h->res_own = (int)((h->n + g - 1) / g);
-    return;
-  }
+  const ResPlan p = h->nph == 1 ? res_plan1(h->n, h->cus)
+                                : res_plan(h->n, h->cus, RES_SHAPES2, h->flux == HES_FLUX_HLL ? 2 : 3,
+                                           [](ResShape s) { return s.block / 64 * (s.tiles - 2) + 2; });
+  h->shape = p.shape;
+  h->res_g = p.G;
+  h->res_own = p.own;
 }
 
-size_t comm_words(const hes_solver* h) {
-  return (size_t)2 * h->res_g * RES_SLOT + (size_t)2 * h->res_g * 2 * RES_HALO * 2 * h->nc;
-}
-
-// Two workgroups on one compute unit would share its SIMDs while other units
-// idle: a team's workgroups ask for more LDS than half a unit has.
-constexpr unsigned RES_ALONE_LDS = 84 * 1024;
-
-hipError_t launch_resident_k(void (*k)(ResArgs), int block, const ResArgs& a, hipStream_t st) {
-  unsigned lds = 0;
-  if (a.team.G > 1) {
-    hipFuncAttributes fa;
-    hipError_t e = hipFuncGetAttributes(&fa, (const void*)k);
-    if (e == hipSuccess && fa.sharedSizeBytes < RES_ALONE_LDS) {
-      lds = RES_ALONE_LDS - (unsigned)fa.sharedSizeBytes;
-      e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    }
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(k, dim3((unsigned)a.team.G), dim3((unsigned)block), lds, st, a);
-  return hipGetLastError();
-}
 template <int FLUX, int FAST>
 auto resident_kernel(int nph, ResShape s) -> void (*)(ResArgs) {
   if (nph == 2) {
@@ -859,7 +811,7 @@ hipError_t launch_resident(const hes_solver* h, const ResArgs& a) {
                                    : resident_kernel<FLUX_HLL, 0>(h->nph, h->shape))
                            : (fast ? resident_kernel<FLUX_RUSANOV, 1>(h->nph, h->shape)
                                    : resident_kernel<FLUX_RUSANOV, 0>(h->nph, h->shape));
-  return launch_resident_k(k, h->shape.block, a, h->stream);
+  return res_launch(k, h->shape.block, a.team.G, a, h->stream);
 }
 
 // At most `steps` steps (<= RES_STEPS) in one launch.  *gave_up: no result
@@ -1007,7 +959,7 @@ int hes_solver_create(hes_solver** out, int nphase, int flux, long long ncells,
   if (e == hipSuccess && nphase == 2) e = hipMalloc(&h->jlist, sizeof(long long) * (size_t)ncells);
   // the small words in one allocation: CFL ring, time ring, jump-face counts,
   // status, then the team's messages, each on a line of its own
-  const size_t words = 4 * 16 + (h->shape.block ? comm_words(h) : 0);
+  const size_t words = 4 * 16 + (h->shape.block ? res_words_of(h->res_g, h->nc) : 0);
   if (e == hipSuccess) e = hipMalloc(&h->slots, sizeof(unsigned long long) * words);
   if (e == hipSuccess) {
     h->tring = (double*)(h->slots + 16);

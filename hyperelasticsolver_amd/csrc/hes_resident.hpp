@@ -35,6 +35,8 @@
 // SIMD), the team's maximum (1.3 us for 5 workgroups, 2.1 us for 256), and
 // from two waves per SIMD on the FP64 issue rate (0.95 us per tile and SIMD).
 #pragma once
+#include <algorithm>
+#include <type_traits>
 #include "hes_step.hpp"
 
 namespace hes {
@@ -126,8 +128,10 @@ __device__ __forceinline__ void res_publish(const ResTeam& a, long long s, doubl
   if ((threadIdx.x & 63) == 0)
     res_store(a.slots + ((s & 1) * a.G + a.rank) * (long long)RES_SLOT, bits | sign);
 }
-template <int MAXG>
-__device__ __forceinline__ bool res_collect(const ResTeam& a, long long s, double& lmax) {
+// LEAD: leader receives the first workgroup that attains it.
+template <int MAXG, bool LEAD = false>
+__device__ __forceinline__ bool res_collect(const ResTeam& a, long long s, double& lmax,
+                                            int* leader = nullptr) {
   const int lane = threadIdx.x & 63;
   const unsigned long long sign = (unsigned long long)((s >> 1) & 1) << 63;
   const unsigned long long* sl = a.slots + (s & 1) * a.G * (long long)RES_SLOT;
@@ -152,6 +156,16 @@ __device__ __forceinline__ bool res_collect(const ResTeam& a, long long s, doubl
     }
     if (__all(here)) {
       lmax = wave_max_dpp(m);
+      if constexpr (LEAD) {
+        *leader = 0;
+#pragma unroll
+        for (int k = MAXG / 64 - 1; k >= 0; --k) {
+          const unsigned long long at = __ballot(
+              64 * k + lane < a.G &&
+              __longlong_as_double((long long)(x[k] & 0x7fffffffffffffffull)) == lmax);
+          if (at) *leader = 64 * k + (int)__builtin_ctzll(at);
+        }
+      }
       return true;
     }
     if (res_expired(a, polls, since)) return false;
@@ -211,9 +225,16 @@ __device__ __forceinline__ bool res_receive(const ResTeam& a, long long round, u
 // flux and for its speed (k_step forms it twice, for the state it reads and
 // the one it writes); with one tile per wave and registers to keep it, the
 // flux, and always HLL's mid state, fall into the wait for the team's maximum.
-template <int FLUX, int FAST, int BLK, int T, int MAXG, bool FLUX_LDS = false>
-__device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& mat) {
+// hook: told of every state s that the run passes through, once its maximum
+// lmax is known: hook.tile for each of a wave's tiles (every lane active; own:
+// the lane's cell i belongs to this workgroup; lead: this is the team's first
+// workgroup with a cell of speed lmax), then hook.end.
+struct ResNoHook {};
+template <int FLUX, int FAST, int BLK, int T, int MAXG, bool FLUX_LDS = false, class Hook = ResNoHook>
+__device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& mat,
+                                                Hook hook = Hook()) {
   constexpr int NC = 14, W = BLK / 64, NT = W * T;
+  constexpr bool HOOK = !std::is_same<Hook, ResNoHook>::value;
   constexpr bool LATE_FLUX = T == 1 && BLK < 1024;
   __shared__ double edge[2][NT][2][NC];  // new first and last updated cell of every tile, by parity
   __shared__ double red[2][W];           // every wave's maximum, by parity
@@ -221,7 +242,7 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
   // FLUX_LDS: the 11 components of every cell's flux that are not zero
   __shared__ double flux[FLUX_LDS ? NT : 1][FLUX_LDS ? 11 : 1][64];
   __shared__ double team_max, tnow[2];
-  __shared__ int dead;
+  __shared__ int dead, leader;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long long o0 = a.lo + (long long)a.rank * a.own;
@@ -244,7 +265,10 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
 #pragma unroll
     for (int r = 0; r < NC; ++r) q[k][r] = a.Qin[r * a.pitch + o0 + jc];
   }
-  if (threadIdx.x == 0) dead = 0;
+  if (threadIdx.x == 0) {
+    dead = 0;
+    leader = 0;
+  }
   double t = a.t, lmax = 0.0;
   long long s = 0;
   int to_halo = RES_HALO;
@@ -281,9 +305,11 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
     if (a.G > 1) {
       if (w == 0) {
         double lm = 0.0;
-        const bool got = res_collect<MAXG>(a, s, lm);
+        int lead = 0;
+        const bool got = res_collect<MAXG, HOOK>(a, s, lm, &lead);
         if (lane == 0) {
           team_max = lm;
+          if (HOOK) leader = lead;
           if (!got) dead = 1;
         }
       }
@@ -293,6 +319,12 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
         ok = false;
         break;
       }
+    }
+    if constexpr (HOOK) {
+#pragma unroll
+      for (int k = 0; k < T; ++k)
+        hook.tile(s, lmax, mine(k), leader == a.rank, o0 + cell(k), q[k], c[k], u1[k]);
+      hook.end(s, lmax);
     }
     if (s >= a.kmax || !(t < a.t_end)) break;  // main.jl:202 `while t < T`
     const double dtdx = a.cfl * rcp(lmax);
@@ -607,4 +639,68 @@ __device__ __forceinline__ ResOut resident_run2(const ResTeam& a, const MatDev* 
   return {s, t, lmax, ok};
 }
 
+// ---- host side --------------------------------------------------------------
+
+// Shape of a team's workgroups: threads, and what a wave holds: tiles of 64
+// cells (one phase), or cells (two phases).
+struct ResShape {
+  int block, tiles;
+};
+inline constexpr int RES_MAX_TEAM = 256;  // workgroups
+
+// How a problem is laid on the chip (block 0: it is not, and runs step by
+// step): the first of these shapes whose team has a compute unit for every
+// workgroup.  Fewer waves per SIMD come first, since a step's chain of
+// dependent FP64 operations is what a team of few waves waits for (us per
+// step, Rusanov / HLL, this shape against the next at the same cells, 59000:
+// 4.4 / 3.8 against 4.9 / 4.9; 123000: 5.3 / 5.1 against 7.1 / 8.2; 250000:
+// 7.6 / 8.2 against 9.3 / 11.8; the last against one launch per step, 300000:
+// 9.5 / 11.8 against 21.1 / 20.3).  Two tiles of 64 cells per wave and three
+// fill the registers of two waves per SIMD (200 to 256 VGPRs).
+inline constexpr ResShape RES_SHAPES[4] = {{256, 1}, {512, 1}, {512, 2}, {512, 3}};
+
+struct ResPlan {
+  ResShape shape;
+  int G, own;  // workgroups, and cells of each
+};
+// The first of `count` shapes (whose single workgroup holds cells_of cells)
+// whose team fits.
+template <class Cells>
+ResPlan res_plan(long long n, int cus, const ResShape* shapes, int count, Cells cells_of) {
+  for (int k = 0; k < count; ++k) {
+    const int cells = cells_of(shapes[k]), per = cells - 2 * RES_HALO;
+    const long long g = n <= cells ? 1 : (n + per - 1) / per;
+    if (g <= std::min(cus, RES_MAX_TEAM)) return {shapes[k], (int)g, (int)((n + g - 1) / g)};
+  }
+  return {{0, 0}, 0, 0};
+}
+inline ResPlan res_plan1(long long n, int cus) {
+  return res_plan(n, cus, RES_SHAPES, 4,
+                  [](ResShape s) { return s.block / 64 * s.tiles * TILE + 2; });
+}
+
+// 64-bit words of a team's message buffer: slots, then halo words.
+inline size_t res_words_of(int G, int nc) {
+  return (size_t)2 * G * RES_SLOT + (size_t)2 * G * 2 * RES_HALO * 2 * nc;
+}
+
+// Two workgroups on one compute unit would share its SIMDs while other units
+// idle: a team's workgroups ask for more LDS than half a unit has.
+inline constexpr unsigned RES_ALONE_LDS = 84 * 1024;
+
+template <class Args>
+hipError_t res_launch(void (*k)(Args), int block, int G, const Args& a, hipStream_t st) {
+  unsigned lds = 0;
+  if (G > 1) {
+    hipFuncAttributes fa;
+    hipError_t e = hipFuncGetAttributes(&fa, (const void*)k);
+    if (e == hipSuccess && fa.sharedSizeBytes < RES_ALONE_LDS) {
+      lds = RES_ALONE_LDS - (unsigned)fa.sharedSizeBytes;
+      e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    }
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)G), dim3((unsigned)block), lds, st, a);
+  return hipGetLastError();
+}
 }  // namespace hes

@@ -1,0 +1,86 @@
+"""The adjoint's first pass in one launch and its recompute of whole segments,
+at the edges of their workgroups: the forward pass against the batched solver's
+one launch per step, and gradients with the states between checkpoints
+recomputed against gradients with every state kept, bit for bit (the same
+arithmetic, so no tolerance enters)."""
+import numpy as np
+import pytest
+
+from hyperelasticsolver_amd.EquationsOfState import Barton2009
+from hyperelasticsolver_amd.adjoint import Adjoint, phase_prims_to_adjoint
+from hyperelasticsolver_amd.batched import Batch
+from hyperelasticsolver_amd.initial import prim2cons, random_interfaces, random_phase_prims
+
+pytestmark = pytest.mark.gpu
+
+# one workgroup of the recompute and several (250 cells alone, 200 each), the
+# first pass's workgroup shapes, both sides of the size from which only states
+# near a cotangent are recomputed (on 256 compute units), and a first pass
+# step by step
+SIZES = [3, 250, 251, 400, 401, 1000, 59905, 47616, 47617, 123393, 250369, 377345]
+STEPS = 53  # two full launches of the recompute and a part of one
+
+
+def _problem(n):
+    rng = np.random.default_rng(n)
+    eos = Barton2009()
+    k = 5 if n > 60 else 2
+    prims14 = random_phase_prims(rng, eos, k)
+    ifc = random_interfaces(rng, k - 1)
+    return eos, prims14, phase_prims_to_adjoint(prims14), list(ifc)
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_first_pass_equals_stepwise(n):
+    print(f"[adjoint passes] forward n={n}", flush=True)
+    eos, prims14, prims, ifc = _problem(n)
+    zero = np.zeros(n)
+    with Adjoint(eos, n, STEPS, every=20) as a:
+        a.set_initial(prims, ifc)
+        a.set_target(zero, zero)
+        a.forward()
+        q = a.final_state()
+        a.forward()
+        assert np.array_equal(q, a.final_state())
+    with Batch([eos], [n], flux="rusanov") as b:
+        b.set_piecewise([prim2cons(eos, prims14)], [ifc])
+        b.run(STEPS, mode="eager")
+        r = b.get_state()
+    # the initial states come from two routines that may differ in the last
+    # bits, which 53 steps carry along
+    scale = np.abs(r).max(axis=1, keepdims=True) + 1e-300
+    assert np.all(np.abs(q - r) <= 1e-10 * scale)
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_recomputed_states_change_nothing(n):
+    print(f"[adjoint passes] gradients n={n}", flush=True)
+    eos, _, prims, ifc = _problem(n)
+    # a misfit on a few cells, so that most tiles stay without a cotangent
+    with Adjoint(eos, n, STEPS, every=STEPS) as a:
+        a.set_initial(prims, ifc)
+        a.set_target(np.zeros(n), np.zeros(n))
+        a.forward()
+        rho, u = a.profiles()
+    rho = rho.copy()
+    rho[n // 3:n // 3 + 5] *= 1.01
+
+    def gradient(every, sparse, graph=True):
+        with Adjoint(eos, n, STEPS, every=every) as a:
+            a.set_sparse(sparse)
+            a.set_launch(graph)
+            a.set_initial(prims, ifc)
+            a.set_target(rho, u)
+            out = []
+            for _ in range(2):  # a captured pass replays
+                loss = a.forward()
+                g, gm = a.backward()
+                out.append(np.concatenate([[loss], g.ravel(), gm]))
+            assert np.array_equal(out[0], out[1])
+            return out[0]
+
+    ref = gradient(1, False)
+    assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0.0
+    for every, sparse, graph in ((2, True, True), (26, False, True), (27, True, True),
+                                 (STEPS, True, False), (STEPS, False, True)):
+        assert np.array_equal(gradient(every, sparse, graph), ref), (every, sparse)
