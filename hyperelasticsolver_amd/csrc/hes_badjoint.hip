@@ -12,15 +12,17 @@
 // owns cells [off_p, off_p+1)); one wave works on one tile of TILE cells of
 // one problem, as in the batched solver, so a launch covers the whole batch.
 //
-// Per problem and step the forward pass records the CFL maximum (an atomic
-// max per wave) and, per tile, the argmax (value, smallest index) of the new
-// state's speeds.  The reverse step is the one-problem reverse step
-// (reverse_chunk) on each tile.  Every reduction of a problem's dtdxbar and
-// (b0bar, c0bar) runs over its tiles in tile order, so results do not depend
-// on scheduling.  Storage, recompute and the overlap of the recompute with the
-// reverse steps follow hes_adjoint.hip: every `every`-th state is kept, and a
-// backward segment's states are recomputed on a second stream into one of two
-// segment buffers while the reverse steps of the previous segment run.
+// The forward pass of a batch whose problems fit the chip is one launch (a
+// team of workgroups per problem); else a launch per step, which records the
+// CFL maximum (an atomic max per wave) and, per tile, the argmax (value,
+// smallest index) of the new state's speeds.  The reverse step is the
+// one-problem reverse step (reverse_chunk) on each tile.  Every reduction of a
+// problem's dtdxbar and (b0bar, c0bar) runs over its tiles in tile order, so
+// results do not depend on scheduling.  Storage, recompute and the overlap of
+// the recompute with the reverse steps follow hes_adjoint.hip: every
+// `every`-th state is kept, and a backward segment's states are recomputed on
+// a second stream into one of two segment buffers while the reverse steps of
+// the previous segment run.
 // the secular-function eigenvalue iteration throughout (see sym3_extreme);
 // set before any include
 #define HES_EIG_SECULAR 1
@@ -177,7 +179,6 @@ struct BAdjFwdArgs {
   long long pitch, s;
   double cfl;
   int P, ntiles;
-  int write_lmax;            // max-reduce the new state's speeds into lmax[(s + 1) P + p]
 };
 
 // One time step of every problem: the solver's chunk step (so states match a
@@ -195,12 +196,85 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
   load_chunk<1>(ctx, i, q, cc);
   const double lmax = lmax_of(a.lmax, a.s * a.P + p);
   const double lam = chunk_step<1, FLUX_RUSANOV, 1>(ctx, i, q, cc, lmax);
-  if (a.write_lmax) {
-    const bool owned = lane >= 1 && lane <= TILE && i < td.hi;
-    const long long row = (a.s + 1) * (long long)a.ntiles;
-    record_tile(lam, owned, i, a.lmax + (a.s + 1) * a.P + p, a.blk_val ? a.blk_val + row : nullptr,
-                a.blk_idx ? a.blk_idx + row : nullptr, tile);
-  }
+  const bool owned = lane >= 1 && lane <= TILE && i < td.hi;
+  const long long row = (a.s + 1) * (long long)a.ntiles;
+  record_tile(lam, owned, i, a.lmax + (a.s + 1) * a.P + p, a.blk_val ? a.blk_val + row : nullptr,
+              a.blk_idx ? a.blk_idx + row : nullptr, tile);
+}
+
+// The whole first pass of every problem in one launch (a team of workgroups
+// per problem, hes_resident.hpp), for problems that fit the chip.  us per step,
+// one launch per step against this: 256 problems of 1024 .. 8192 cells 51 ->
+// 28, 1000 of 100 .. 900 cells 23 -> 15, 16 of them 5.5 -> 3.8.
+struct BAdjResArgs {
+  const BResTeam* teams;
+  const BResItem* items;
+  unsigned long long* comm;
+  const MatDev* mats;
+  const double* dx;
+  const double* Qin;
+  double* Qout;
+  double* Cout;
+  AdjHook hook;
+  int* status;
+  double cfl;
+};
+template <int T>
+__global__ __launch_bounds__(BRES_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
+void k_badj_resident(BAdjResArgs a) {
+  ResTeam tm;
+  const int p = bres_place((int*)a.comm, a.items, a.teams, a.comm, tm);
+  const MatDev mat = uniform_mat(a.mats + p);
+  tm.Qin = a.Qin;
+  tm.Qout = a.Qout;
+  tm.Cout = a.Cout;
+  tm.pitch = a.hook.pitch;
+  tm.cfl = a.cfl;
+  tm.dx = cload(a.dx + p);
+  tm.t = 0.0;
+  tm.t_end = INFINITY;
+  tm.kmax = a.hook.nsteps;
+  tm.dt_hist = nullptr;
+  tm.status = a.status;
+  tm.lxf = 0;
+  tm.tag0 = 1;  // the buffer is cleared before the launch
+  tm.gave_up = a.status + 2;
+  AdjHook hook = a.hook;
+  hook.lmax += p;
+  hook.istar += p;
+  hook.first = tm.rank == 0 && threadIdx.x == 0;
+  (void)resident_run1<FLUX_RUSANOV, 1, BRES_BLOCK, T, RES_MAX_TEAM, (T > 1)>(tm, mat, hook);
+}
+__global__ void k_badj_nocell(long long* __restrict__ istar, long long m) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < m) istar[t] = NO_CELL;
+}
+
+// States s + 1 .. s + steps of every problem from state s (segment_run), a
+// workgroup per entry of the table.  Reverse pass of 256 problems of 1024 ..
+// 8192 cells, the recompute in a launch per step against this: 249 -> 240 ms
+// (the reverse steps, one wave per SIMD, are what it waits for).
+struct BSeg {
+  long long lo, hi, o0, o1;  // the problem's cells, the workgroup's
+  int p, halo;
+};
+struct BAdjSegArgs {
+  const BSeg* segs;
+  const MatDev* mats;
+  SegCtx c;
+};
+__global__ __launch_bounds__(SEG_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
+void k_badj_segment(BAdjSegArgs a) {
+  const BSeg* g = a.segs + __builtin_amdgcn_readfirstlane((int)xcd_block());
+  SegCtx c = a.c;
+  c.lo = cload(&g->lo);
+  c.hi = cload(&g->hi);
+  c.o0 = cload(&g->o0);
+  c.o1 = cload(&g->o1);
+  c.halo = cload(&g->halo);
+  const int p = cload(&g->p);
+  c.lmax += p;
+  segment_run(c, uniform_mat(a.mats + p));
 }
 
 // Argmax cell of the CFL speed of every (state, problem) from the per-tile
@@ -646,6 +720,16 @@ struct hes_badjoint {
   std::vector<long long> offs_h;
   std::vector<int> tfirst_h, tprob_h, poff_h;
   std::vector<double> mats_h;  // 8 x P
+  int dev = 0, cus = 0;
+  // the first pass in one launch (tiles 0: a launch per step)
+  int res_tiles = 0, res_groups = 0;
+  bool res_waits = false;
+  size_t res_words = 0;
+  BResTeam* teams = nullptr;
+  BResItem* items = nullptr;
+  unsigned long long* comm = nullptr;
+  BSeg* segs = nullptr;  // the recompute's workgroups
+  int nsegs = 0;
   BTile* tiles = nullptr;
   int* tfirst = nullptr;
   long long* offs = nullptr;
@@ -709,7 +793,7 @@ double* bseg_slot(hes_badjoint* h, long long s, long long s0, int buf) {
 }
 
 BAdjFwdArgs bfwd_args(hes_badjoint* h, long long s, const double* qi, double* qo, const double* ci,
-                      double* co, bool first_pass) {
+                      double* co) {
   BAdjFwdArgs a;
   a.tiles = h->tiles;
   a.mats = h->mats;
@@ -719,7 +803,7 @@ BAdjFwdArgs bfwd_args(hes_badjoint* h, long long s, const double* qi, double* qo
   a.Cin = ci;
   a.Cout = co;
   a.lmax = h->lmax;
-  const bool rec = first_pass && s + 1 < h->nsteps;  // the final state needs no argmax
+  const bool rec = s + 1 < h->nsteps;  // the final state needs no argmax
   a.blk_val = rec ? h->blk_val : nullptr;
   a.blk_idx = rec ? h->blk_idx : nullptr;
   a.status = h->status;
@@ -728,19 +812,45 @@ BAdjFwdArgs bfwd_args(hes_badjoint* h, long long s, const double* qi, double* qo
   a.cfl = h->cfl;
   a.P = h->P;
   a.ntiles = h->ntiles;
-  a.write_lmax = first_pass ? 1 : 0;
   return a;
 }
 
 unsigned blocks_of(long long m, int per) { return (unsigned)((m + per - 1) / per); }
 
-hipError_t brecord_forward(hes_badjoint* h) {
+// The first pass from checkpoint 0 (the initial states) in one launch.
+void brecord_resident(hes_badjoint* h) {
+  hipStream_t st = h->stream;
+  const long long words = (long long)h->res_words, pairs = h->nsteps * h->P;
+  hipLaunchKernelGGL(k_badj_zero, dim3(blocks_of(words, LBLK)), dim3(LBLK), 0, st,
+                     (double*)h->comm, words);
+  hipLaunchKernelGGL(k_badj_nocell, dim3(blocks_of(pairs, LBLK)), dim3(LBLK), 0, st, h->istar, pairs);
+  BAdjResArgs a;
+  std::memset((void*)&a, 0, sizeof(a));
+  a.teams = h->teams;
+  a.items = h->items;
+  a.comm = h->comm;
+  a.mats = h->mats;
+  a.dx = h->dx;
+  a.Qin = bck_q(h, 0);
+  bfwd_slot(h, h->nsteps, &a.Qout, &a.Cout);
+  a.hook.ck = bck_q(h, 0);
+  a.hook.lmax = h->lmax;
+  a.hook.istar = h->istar;
+  a.hook.every = h->every;
+  a.hook.nsteps = h->nsteps;
+  a.hook.pitch = h->pitch;
+  a.hook.stride = h->P;
+  a.status = h->status;
+  a.cfl = h->cfl;
+  const dim3 grid((unsigned)h->res_groups), block(BRES_BLOCK);
+  if (h->res_tiles == 1) hipLaunchKernelGGL(k_badj_resident<1>, grid, block, 0, st, a);
+  else hipLaunchKernelGGL(k_badj_resident<2>, grid, block, 0, st, a);
+}
+
+// The first pass from checkpoint 0, a launch per step.
+void brecord_steps(hes_badjoint* h) {
   hipStream_t st = h->stream;
   const unsigned nt = (unsigned)h->ntiles;
-  hipLaunchKernelGGL(k_badj_p2c, dim3(blocks_of(h->npieces, 64)), dim3(64), 0, st, h->prims,
-                     h->gin, h->piece_prob, h->states, h->npieces);
-  hipLaunchKernelGGL(k_badj_fill, dim3(blocks_of(h->N, LBLK)), dim3(LBLK), 0, st, h->states,
-                     h->bounds, h->npieces, bck_q(h, 0), h->N, h->pitch);
   hipLaunchKernelGGL(k_badj_ends, dim3(blocks_of((long long)h->nslots * h->P * 2 * NQ, LBLK)),
                      dim3(LBLK), 0, st, bck_q(h, 0), h->slots, h->nslots, h->offs, h->P, h->pitch);
   hipLaunchKernelGGL(k_badj_zero, dim3(blocks_of((h->nsteps + 1) * h->P, LBLK)), dim3(LBLK), 0, st,
@@ -751,11 +861,22 @@ hipError_t brecord_forward(hes_badjoint* h) {
     double *qi, *ci, *qo, *co;
     bfwd_slot(h, s, &qi, &ci);
     bfwd_slot(h, s + 1, &qo, &co);
-    hipLaunchKernelGGL(k_badj_fwd, dim3(nt), dim3(64), 0, st, bfwd_args(h, s, qi, qo, ci, co, true));
+    hipLaunchKernelGGL(k_badj_fwd, dim3(nt), dim3(64), 0, st, bfwd_args(h, s, qi, qo, ci, co));
   }
   const long long npairs = h->nsteps * h->P;
   hipLaunchKernelGGL(k_badj_argmax, dim3(blocks_of(npairs, 4)), dim3(256), 0, st, h->blk_val,
                      h->blk_idx, h->tfirst, h->ntiles, h->P, npairs, h->istar);
+}
+
+hipError_t brecord_forward(hes_badjoint* h) {
+  hipStream_t st = h->stream;
+  const unsigned nt = (unsigned)h->ntiles;
+  hipLaunchKernelGGL(k_badj_p2c, dim3(blocks_of(h->npieces, 64)), dim3(64), 0, st, h->prims,
+                     h->gin, h->piece_prob, h->states, h->npieces);
+  hipLaunchKernelGGL(k_badj_fill, dim3(blocks_of(h->N, LBLK)), dim3(LBLK), 0, st, h->states,
+                     h->bounds, h->npieces, bck_q(h, 0), h->N, h->pitch);
+  if (h->res_tiles) brecord_resident(h);
+  else brecord_steps(h);
   double *qn, *cn;
   bfwd_slot(h, h->nsteps, &qn, &cn);
   hipLaunchKernelGGL(k_badj_loss, dim3(nt), dim3(64), 0, st, h->tiles, qn, h->rho_t, h->u_t, h->gin,
@@ -789,14 +910,21 @@ hipError_t brecord_backward(hes_badjoint* h) {
     const long long s0 = c * h->every;
     const long long end = std::min(s0 + h->every, h->nsteps);
     const int buf = (int)(c & 1);
-    for (long long s = s0; s + 1 < end; ++s) {
-      // each recomputed state keeps its sound speeds in row 14 of its slot,
-      // as the checkpoints do: the reverse step reads its face speeds there
-      const double* ci = bseg_slot(h, s, s0, buf) + 14 * h->pitch;
-      double* co = bseg_slot(h, s + 1, s0, buf) + 14 * h->pitch;
-      hipLaunchKernelGGL(k_badj_fwd, dim3(nt), dim3(64), 0, st2,
-                         bfwd_args(h, s, bseg_slot(h, s, s0, buf), bseg_slot(h, s + 1, s0, buf), ci,
-                                   co, false));
+    // each recomputed state keeps its sound speeds in row 14 of its slot,
+    // as the checkpoints do: the reverse step reads its face speeds there
+    for (long long s = s0; s + 1 < end; s += SEG_STEPS) {
+      BAdjSegArgs a;
+      std::memset((void*)&a, 0, sizeof(a));
+      a.segs = h->segs;
+      a.mats = h->mats;
+      a.c.Q = bseg_slot(h, s, s0, buf);
+      a.c.out = bseg_slot(h, s + 1, s0, buf);
+      a.c.lmax = h->lmax + s * h->P;
+      a.c.stride = h->P;
+      a.c.pitch = h->pitch;
+      a.c.steps = (int)std::min<long long>(SEG_STEPS, end - 1 - s);
+      a.c.cfl = h->cfl;
+      hipLaunchKernelGGL(k_badj_segment, dim3((unsigned)h->nsegs), dim3(SEG_BLOCK), 0, st2, a);
     }
     const int cnt = (int)(end - s0);
     hipLaunchKernelGGL(k_badj_lam, dim3(blocks_of((long long)cnt * h->P, 64)), dim3(64), 0, st2,
@@ -937,7 +1065,19 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
       return fail(HES_ERR_HIP, "cannot read the device's compute-unit count");
     }
     h->nbr = std::min(h->ntiles, 4 * cus);  // one reverse wave per SIMD
+    h->dev = dev;
+    h->cus = cus;
   }
+  std::vector<BSeg> segs;
+  for (int p = 0; p < nproblems; ++p) {
+    const long long lo = h->offs_h[p], hi = h->offs_h[p + 1];
+    const bool whole = hi - lo <= SEG_CELLS;
+    for (long long c = lo; c < hi; c += whole ? SEG_CELLS : SEG_OWN)
+      segs.push_back({lo, hi, c, std::min(c + (whole ? SEG_CELLS : SEG_OWN), hi), p,
+                      whole ? 0 : SEG_STEPS});
+  }
+  h->nsegs = (int)segs.size();
+  const BResPlan pl = bres_plan(h->offs_h, h->cus, NQ);
   h->pitch = (h->N + 63) / 64 * 64 + 256;  // rows padded off a power-of-two stride, as the solver's
   const size_t Pt = (size_t)h->pitch;
   hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
@@ -979,12 +1119,20 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
   up(&h->u_t, nullptr, Pt);
   up(&h->gmat, nullptr, 2 * (size_t)nproblems);
   up(&h->status, nullptr, 4);
+  up(&h->segs, segs.data(), segs.size());
+  if (pl.tiles) {
+    up(&h->teams, pl.teams.data(), pl.teams.size());
+    up(&h->items, pl.items.data(), pl.items.size());
+    up(&h->comm, nullptr, pl.words);
+    h->res_tiles = pl.tiles;
+    h->res_groups = (int)pl.items.size();
+    h->res_waits = pl.waits;
+    h->res_words = pl.words;
+  }
   if (e == hipSuccess) e = zero_on(h->stream, h->status, 4 * sizeof(int));
   if (e == hipSuccess) {
     std::vector<double*> sl;
     for (long long c = 1; c < h->nck; ++c) sl.push_back(bck_q(h, c));
-    for (int b = 0; b < 2; ++b)
-      for (long long j = 0; j + 1 < h->every; ++j) sl.push_back(h->seg[b] + j * 15 * Pt);
     sl.push_back(h->fq[0]);
     sl.push_back(h->fq[1]);
     h->nslots = (int)sl.size();
@@ -1008,7 +1156,8 @@ int hes_badjoint_destroy(hes_badjoint* h) {
                   h->seg[1], h->fq[0], h->fq[1], h->fc[0], h->fc[1], h->qb[0], h->qb[1], h->zf,
                   h->lmax, h->blk_val, h->blk_idx, h->istar, h->Jlam, h->dtp, h->thb, h->lossp,
                   h->rho_t, h->u_t, h->slots, h->status, h->poff, h->piece_prob, h->bounds,
-                  h->prims, h->states, h->sums, h->gstates, h->gmat};
+                  h->prims, h->states, h->sums, h->gstates, h->gmat, h->teams, h->items, h->comm,
+                  h->segs};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   hipEvent_t evs[] = {h->ev0, h->ev1, h->ev_fork, h->ev_join, h->ev_ready[0], h->ev_ready[1],
@@ -1121,16 +1270,23 @@ int hes_badjoint_forward(hes_badjoint* h, double* losses, double* total, float* 
       return HES_ERR_HIP;
     }
   }
-  HIP_TRY(hipEventRecord(h->ev0, h->stream));
-  if (h->use_graph) HIP_TRY(hipGraphLaunch(h->gf, h->stream));
-  else HIP_TRY(brecord_forward(h));
-  HIP_TRY(hipEventRecord(h->ev1, h->stream));
-  HIP_TRY(hipEventSynchronize(h->ev1));
+  int st[4];
+  {
+    ComputeUnits units(h->dev, h->cus, h->res_tiles && h->res_waits ? h->cus : 0);
+    HIP_TRY(hipEventRecord(h->ev0, h->stream));
+    if (h->use_graph) HIP_TRY(hipGraphLaunch(h->gf, h->stream));
+    else HIP_TRY(brecord_forward(h));
+    HIP_TRY(hipEventRecord(h->ev1, h->stream));
+    HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
+  }
+  if (st[2]) {  // a team was not on the chip together: a launch per step from here on
+    h->res_tiles = 0;
+    drop_graphs(h);
+    return hes_badjoint_forward(h, losses, total, elapsed_ms);
+  }
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   if (elapsed_ms) *elapsed_ms = ms;
-  int st[2];
-  HIP_TRY(copy_on(h->stream, st, h->status, sizeof(st), hipMemcpyDeviceToHost));
   if (st[0]) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
   std::vector<double> lp(h->ntiles);
   HIP_TRY(copy_on(h->stream, lp.data(), h->lossp, sizeof(double) * lp.size(), hipMemcpyDeviceToHost));
@@ -1237,6 +1393,7 @@ int hes_badjoint_info(hes_badjoint* h, long long* total_cells, long long* device
   long long b = h->nck * 15 * Pt + 2 * (h->every - 1) * 15 * Pt + 2 * (14 + 1 + 14) * Pt + 2 * Pt;
   b = b * 8 + (h->nsteps + 1) * P * 8 + h->nsteps * T * 16 + h->nsteps * P * (8 + JL * 8) +
       T * (2 * 4 + 2 * 8 + 2 * 8 + 8);
+  b += 8 * (long long)h->res_words + h->nsegs * (long long)sizeof(BSeg);
   if (total_cells) *total_cells = h->N;
   if (device_bytes) *device_bytes = b;
   if (checkpoints) *checkpoints = h->nck;

@@ -109,21 +109,6 @@ __device__ __forceinline__ void atomic_max_pos(unsigned long long* slot, double 
   if (m > 0.0) atomicMax(slot, (unsigned long long)__double_as_longlong(m));
 }
 
-// A material at a wave-uniform address into scalar registers (field by field,
-// through the constant address space).
-__device__ __forceinline__ MatDev uniform_mat(const MatDev* m) {
-  typedef const __attribute__((address_space(4))) MatDev cmat_t;
-  cmat_t* g = (cmat_t*)m;
-  MatDev d;
-  d.rho0 = g->rho0; d.irho0 = g->irho0; d.cv = g->cv; d.t0 = g->t0; d.b0sq = g->b0sq;
-  d.k0 = g->k0; d.alpha = g->alpha; d.beta = g->beta; d.gamma = g->gamma;
-  d.hk0a2 = g->hk0a2; d.k0_2a = g->k0_2a; d.k0_a = g->k0_a; d.cvt0 = g->cvt0;
-  d.icvt0 = g->icvt0; d.hb0sq = g->hb0sq; d.half_a = g->half_a; d.half_b = g->half_b;
-  d.half_g = g->half_g; d.ac_t = g->ac_t; d.ac_s = g->ac_s; d.ac_e = g->ac_e;
-  d.ac_w = g->ac_w; d.fast = g->fast; d.pad = 0;
-  return d;
-}
-
 // One step of one tile (wave-uniform `tile`).
 template <int NPH, int FLUX, int FAST, int PIN>
 __device__ __forceinline__ void batch_tile_step(const BatchArgs& a, int tile) {
@@ -505,14 +490,6 @@ __global__ void k_batch_carry_fin(unsigned long long* slots, long long* plaunch,
 // The time loops of the whole batch in one launch, single phase
 // (hes_resident.hpp): a team of workgroups per problem
 // ---------------------------------------------------------------------------
-struct BResTeam {  // a problem's team
-  long long lo, hi;
-  long long slots, border;  // its words in the message buffer
-  int G, own;
-};
-struct BResItem {  // a workgroup's place: rank in the team of a problem
-  int p, rank;
-};
 struct BResOut {
   double t, lmax;
   int steps;
@@ -537,38 +514,16 @@ struct BResArgs {
   unsigned tag0;
 };
 
-// Workgroups take the teams' places in the order in which they start, not by
-// their block index: whoever waits for a team's missing workgroups then waits
-// for the ones that start next, and those find room because every earlier
-// team is complete and comes to its end.  Three workgroups share a compute
-// unit (one wave of each per SIMD, 168 VGPRs; with two tiles per wave the
-// fluxes wait in LDS, 52 KB of it per workgroup), so that one's waits are
-// filled by the others: the FP64 units are then busy 0.71 of the time (552 VALU
-// instructions per tile and step).  4096 problems of 256 .. 16384 cells, us per
-// step, one launch per step against this: Rusanov 780 -> 398, HLL 830 -> 564;
-// three tiles per wave at two waves per SIMD: 408 and 582; one tile: 516, 680.
-constexpr int BRES_BLOCK = 256, BRES_PER_CU = 3;
-constexpr int BRES_MAX_TEAM = 256;
 template <int FLUX, int FAST, int T>
 __global__ __launch_bounds__(BRES_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
 void k_batch_resident(BResArgs a) {
-  __shared__ int place;
-  if (threadIdx.x == 0) place = atomicAdd(a.ticket, 1);
-  __syncthreads();
-  const int item = __builtin_amdgcn_readfirstlane(place);
-  const int p = cload(&a.items[item].p);
-  const BResTeam* d = a.teams + p;
-  const MatDev mat = uniform_mat(a.mats + p);
   ResTeam tm;
+  const int p = bres_place(a.ticket, a.items, a.teams, a.comm, tm);
+  const MatDev mat = uniform_mat(a.mats + p);
   tm.Qin = a.Qin;
   tm.Qout = a.Qout;
   tm.Cout = a.Cout;
   tm.pitch = a.pitch;
-  tm.lo = cload(&d->lo);
-  tm.hi = cload(&d->hi);
-  tm.G = cload(&d->G);
-  tm.rank = cload(&a.items[item].rank);
-  tm.own = cload(&d->own);
   tm.cfl = cload(a.cfl + p);
   tm.dx = cload(a.dx + p);
   tm.t = cload(a.tring + 2 * p + (a.step & 1));
@@ -577,11 +532,9 @@ void k_batch_resident(BResArgs a) {
   tm.dt_hist = nullptr;
   tm.status = a.status;
   tm.lxf = a.lxf;
-  tm.slots = a.comm + cload(&d->slots);
-  tm.border = a.comm + cload(&d->border);
   tm.tag0 = a.tag0;
   tm.gave_up = a.status + 2;
-  const ResOut o = resident_run1<FLUX, FAST, BRES_BLOCK, T, BRES_MAX_TEAM, (T > 1)>(tm, mat);
+  const ResOut o = resident_run1<FLUX, FAST, BRES_BLOCK, T, RES_MAX_TEAM, (T > 1)>(tm, mat);
   if (tm.rank == 0 && threadIdx.x == 0) a.out[p] = {o.t, o.lmax, (int)o.steps};
 }
 
@@ -773,72 +726,27 @@ int batch_carry(hes_batch* h) {
 
 constexpr long long BRES_STEPS = 1LL << 16;  // steps of one launch at most
 
-// Teams for every problem, with one tile per wave or two.  One has the shorter
-// chain of work per step and wastes less of a short problem's last wave, two
-// need fewer exchanges and, the chip full, 1.27 times less time per tile (516
-// against 398 us above).  So one when all its workgroups are on the chip at
-// once (64 problems of 100 .. 3000 cells: 3.7 against 5.0 us per step) or when
-// its tiles are that many fewer (1000 of 60 .. 700 cells: 12.5 against 14.5),
-// else two, the largest problems first.  None if a problem does not fit.
 hipError_t plan_batch_resident(hes_batch* h) {
   h->res_tiles = 0;
   if (h->nph != 1) return hipSuccess;
-  std::vector<BResTeam> teams(h->P);
-  int most = 0;
-  auto fit = [&](int t) -> long long {  // workgroups with t tiles per wave
-    const long long one = BRES_BLOCK / 64 * t * TILE + 2, per = one - 2 * RES_HALO;
-    long long groups = 0;
-    most = 0;
-    for (int p = 0; p < h->P; ++p) {
-      const long long n = h->offsets_h[p + 1] - h->offsets_h[p];
-      const long long g = n <= one ? 1 : (n + per - 1) / per;
-      if (g > std::min(h->cus, BRES_MAX_TEAM)) return -1;
-      teams[p].lo = h->offsets_h[p];
-      teams[p].hi = h->offsets_h[p + 1];
-      teams[p].G = (int)g;
-      teams[p].own = (int)((n + g - 1) / g);
-      most = std::max(most, (int)g);
-      groups += g;
-    }
-    return groups;
-  };
-  const long long groups2 = fit(2), groups1 = fit(1);
-  const bool one = groups1 >= 0 && (groups1 <= BRES_PER_CU * h->cus || 1.27 * groups1 < 2.0 * groups2);
-  const long long groups = one ? groups1 : fit(2);
-  const int tiles = one ? 1 : 2;
-  if (groups < 0 || groups > 0x7fffffffLL) return hipSuccess;
-  h->res_waits = most > 1;
-  std::vector<int> order(h->P);
-  for (int p = 0; p < h->P; ++p) order[p] = p;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-    return teams[x].hi - teams[x].lo > teams[y].hi - teams[y].lo;
-  });
-  std::vector<BResItem> items;
-  items.reserve((size_t)groups);
-  long long at = 1;  // after the ticket counter
-  for (int p : order) {
-    for (int r = 0; r < teams[p].G; ++r) items.push_back({p, r});
-    teams[p].slots = at;
-    if (teams[p].G > 1) at += 2LL * teams[p].G * RES_SLOT;
-  }
-  h->comm_clear = at;
-  for (int p : order) {
-    teams[p].border = at;
-    if (teams[p].G > 1) at += 2LL * teams[p].G * 2 * RES_HALO * 2 * h->nc;
-  }
-  hipError_t e = hipMalloc((void**)&h->teams, sizeof(BResTeam) * teams.size());
-  if (e == hipSuccess) e = hipMalloc((void**)&h->items, sizeof(BResItem) * items.size());
+  const BResPlan pl = bres_plan(h->offsets_h, h->cus, h->nc);
+  if (pl.tiles == 0) return hipSuccess;
+  hipError_t e = hipMalloc((void**)&h->teams, sizeof(BResTeam) * pl.teams.size());
+  if (e == hipSuccess) e = hipMalloc((void**)&h->items, sizeof(BResItem) * pl.items.size());
   if (e == hipSuccess) e = hipMalloc((void**)&h->res_out, sizeof(BResOut) * (size_t)h->P);
-  if (e == hipSuccess) e = hipMalloc((void**)&h->comm, sizeof(unsigned long long) * (size_t)at);
-  if (e == hipSuccess) e = hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * (size_t)at, h->stream);
+  if (e == hipSuccess) e = hipMalloc((void**)&h->comm, sizeof(unsigned long long) * pl.words);
   if (e == hipSuccess)
-    e = copy_on(h->stream, h->teams, teams.data(), sizeof(BResTeam) * teams.size(), hipMemcpyHostToDevice);
+    e = hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * pl.words, h->stream);
   if (e == hipSuccess)
-    e = copy_on(h->stream, h->items, items.data(), sizeof(BResItem) * items.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) {
-    h->res_tiles = tiles;
-    h->res_groups = (int)groups;
-  }
+    e = copy_on(h->stream, h->teams, pl.teams.data(), sizeof(BResTeam) * pl.teams.size(),
+                hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = copy_on(h->stream, h->items, pl.items.data(), sizeof(BResItem) * pl.items.size(),
+                hipMemcpyHostToDevice);
+  h->comm_clear = (long long)pl.clear;
+  h->res_waits = pl.waits;
+  h->res_groups = (int)pl.items.size();
+  if (e == hipSuccess) h->res_tiles = pl.tiles;
   return e;
 }
 

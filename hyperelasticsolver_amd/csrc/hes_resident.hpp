@@ -37,6 +37,7 @@
 #pragma once
 #include <algorithm>
 #include <type_traits>
+#include <vector>
 #include "hes_step.hpp"
 
 namespace hes {
@@ -639,6 +640,62 @@ __device__ __forceinline__ ResOut resident_run2(const ResTeam& a, const MatDev* 
   return {s, t, lmax, ok};
 }
 
+// A material at a wave-uniform address into scalar registers (field by field,
+// through the constant address space).
+__device__ __forceinline__ MatDev uniform_mat(const MatDev* m) {
+  typedef const __attribute__((address_space(4))) MatDev cmat_t;
+  cmat_t* g = (cmat_t*)m;
+  MatDev d;
+  d.rho0 = g->rho0; d.irho0 = g->irho0; d.cv = g->cv; d.t0 = g->t0; d.b0sq = g->b0sq;
+  d.k0 = g->k0; d.alpha = g->alpha; d.beta = g->beta; d.gamma = g->gamma;
+  d.hk0a2 = g->hk0a2; d.k0_2a = g->k0_2a; d.k0_a = g->k0_a; d.cvt0 = g->cvt0;
+  d.icvt0 = g->icvt0; d.hb0sq = g->hb0sq; d.half_a = g->half_a; d.half_b = g->half_b;
+  d.half_g = g->half_g; d.ac_t = g->ac_t; d.ac_s = g->ac_s; d.ac_e = g->ac_e;
+  d.ac_w = g->ac_w; d.fast = g->fast; d.pad = 0;
+  return d;
+}
+
+// ---- the time loops of a batch (one phase): a team per problem ---------------
+
+struct BResTeam {  // a problem's team
+  long long lo, hi;
+  long long slots, border;  // its words in the message buffer
+  int G, own;
+};
+struct BResItem {  // a workgroup's place: rank in the team of a problem
+  int p, rank;
+};
+// Workgroups take the teams' places in the order in which they start, not by
+// their block index: whoever waits for a team's missing workgroups then waits
+// for the ones that start next, and those find room because every earlier
+// team is complete and comes to its end.  Three workgroups share a compute
+// unit (one wave of each per SIMD, 168 VGPRs; with two tiles per wave the
+// fluxes wait in LDS, 52 KB of it per workgroup), so that one's waits are
+// filled by the others: the FP64 units are then busy 0.71 of the time (552 VALU
+// instructions per tile and step).  4096 problems of 256 .. 16384 cells, us per
+// step, one launch per step against this: Rusanov 780 -> 398, HLL 830 -> 564;
+// three tiles per wave at two waves per SIMD: 408 and 582; one tile: 516, 680.
+inline constexpr int BRES_BLOCK = 256, BRES_PER_CU = 3;
+// This workgroup's problem, and its place in the problem's team (tm's cells and
+// messages).
+__device__ __forceinline__ int bres_place(int* ticket, const BResItem* items, const BResTeam* teams,
+                                          unsigned long long* comm, ResTeam& tm) {
+  __shared__ int place;
+  if (threadIdx.x == 0) place = atomicAdd(ticket, 1);
+  __syncthreads();
+  const int item = __builtin_amdgcn_readfirstlane(place);
+  const int p = cload(&items[item].p);
+  const BResTeam* d = teams + p;
+  tm.lo = cload(&d->lo);
+  tm.hi = cload(&d->hi);
+  tm.G = cload(&d->G);
+  tm.rank = cload(&items[item].rank);
+  tm.own = cload(&d->own);
+  tm.slots = comm + cload(&d->slots);
+  tm.border = comm + cload(&d->border);
+  return p;
+}
+
 // ---- host side --------------------------------------------------------------
 
 // Shape of a team's workgroups: threads, and what a wave holds: tiles of 64
@@ -703,4 +760,67 @@ hipError_t res_launch(void (*k)(Args), int block, int G, const Args& a, hipStrea
   hipLaunchKernelGGL(k, dim3((unsigned)G), dim3((unsigned)block), lds, st, a);
   return hipGetLastError();
 }
+// Teams for every problem of a batch (cells [offsets[p], offsets[p + 1])), with
+// one tile per wave or two.  One has the shorter chain of work per step and
+// wastes less of a short problem's last wave, two need fewer exchanges and, the
+// chip full, 1.27 times less time per tile (516 against 398 us above).  So one
+// when all its workgroups are on the chip at once (64 problems of 100 .. 3000
+// cells: 3.7 against 5.0 us per step) or when its tiles are that many fewer
+// (1000 of 60 .. 700 cells: 12.5 against 14.5), else two, the largest problems
+// first.  tiles = 0 if a problem does not fit.
+struct BResPlan {
+  int tiles = 0;
+  bool waits = false;  // some problem has more than one workgroup
+  std::vector<BResTeam> teams;
+  std::vector<BResItem> items;
+  // 64-bit words of the message buffer: the ticket counter and all slots (to be
+  // cleared before a launch), then the halo words
+  size_t clear = 0, words = 0;
+};
+inline BResPlan bres_plan(const std::vector<long long>& offsets, int cus, int nc) {
+  const int P = (int)offsets.size() - 1;
+  BResPlan pl;
+  pl.teams.resize(P);
+  auto fit = [&](int t) -> long long {  // workgroups with t tiles per wave
+    const long long one = BRES_BLOCK / 64 * t * TILE + 2, per = one - 2 * RES_HALO;
+    long long groups = 0;
+    pl.waits = false;
+    for (int p = 0; p < P; ++p) {
+      const long long n = offsets[p + 1] - offsets[p];
+      const long long g = n <= one ? 1 : (n + per - 1) / per;
+      if (g > std::min(cus, RES_MAX_TEAM)) return -1;
+      pl.teams[p] = {offsets[p], offsets[p + 1], 0, 0, (int)g, (int)((n + g - 1) / g)};
+      pl.waits = pl.waits || g > 1;
+      groups += g;
+    }
+    return groups;
+  };
+  const long long groups2 = fit(2), groups1 = fit(1);
+  const bool one = groups1 >= 0 && (groups1 <= BRES_PER_CU * cus || 1.27 * groups1 < 2.0 * groups2);
+  const long long groups = one ? groups1 : fit(2);
+  if (groups < 0 || groups > 0x7fffffffLL) return pl;
+  std::vector<int> order(P);
+  for (int p = 0; p < P; ++p) order[p] = p;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    return pl.teams[x].hi - pl.teams[x].lo > pl.teams[y].hi - pl.teams[y].lo;
+  });
+  pl.items.reserve((size_t)groups);
+  size_t at = 1;  // after the ticket counter
+  for (int p : order) {
+    BResTeam& t = pl.teams[p];
+    for (int r = 0; r < t.G; ++r) pl.items.push_back({p, r});
+    t.slots = (long long)at;
+    if (t.G > 1) at += (size_t)2 * t.G * RES_SLOT;
+  }
+  pl.clear = at;
+  for (int p : order) {
+    BResTeam& t = pl.teams[p];
+    t.border = (long long)at;
+    if (t.G > 1) at += (size_t)2 * t.G * 2 * RES_HALO * 2 * nc;
+  }
+  pl.words = at;
+  pl.tiles = one ? 1 : 2;
+  return pl;
+}
+
 }  // namespace hes

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from hyperelasticsolver_amd.EquationsOfState import Barton2009
-from hyperelasticsolver_amd.adjoint import Adjoint, phase_prims_to_adjoint
+from hyperelasticsolver_amd.adjoint import Adjoint, BatchAdjoint, phase_prims_to_adjoint
 from hyperelasticsolver_amd.batched import Batch
 from hyperelasticsolver_amd.initial import prim2cons, random_interfaces, random_phase_prims
 
@@ -84,3 +84,50 @@ def test_recomputed_states_change_nothing(n):
     for every, sparse, graph in ((2, True, True), (26, False, True), (27, True, True),
                                  (STEPS, True, False), (STEPS, False, True)):
         assert np.array_equal(gradient(every, sparse, graph), ref), (every, sparse)
+
+
+# few workgroups (a tile per wave), more than the chip holds at once (two), a
+# problem that does not fit and runs step by step
+BATCHES = [[3, 62, 250, 251, 400, 401, 498, 499, 1000, 9000], [8000] * 40 + [5, 700], [123393, 300]]
+
+
+@pytest.mark.parametrize("which", range(len(BATCHES)))
+def test_batch_passes(which):
+    """Forward states and gradients of a batch: the one-problem adjoint's
+    states to the bit, and the same gradients whatever is recomputed."""
+    cells = BATCHES[which]
+    print(f"[adjoint passes] batch of {len(cells)}, up to {max(cells)} cells", flush=True)
+    rng = np.random.default_rng(which)
+    eos = [Barton2009(_rho0=8.93 * x, _b0=2.1 * y) for x, y in rng.uniform(0.9, 1.1, (len(cells), 2))]
+    prims = [phase_prims_to_adjoint(random_phase_prims(rng, e, 2)) for e in eos]
+    ifc = [[0.5]] * len(cells)
+    off = np.concatenate([[0], np.cumsum(cells)])
+    zero = np.zeros(off[-1])
+
+    def run(every, sparse, graph=True, target=None):
+        with BatchAdjoint(eos, cells, STEPS, every=every) as b:
+            b.set_sparse(sparse)
+            b.set_launch(graph)
+            b.set_initial(prims, ifc)
+            b.set_target(*(target or (zero, zero)))
+            out = []
+            for _ in range(2):
+                loss = b.forward()
+                out.append(np.concatenate([np.ravel(loss)] + [np.ravel(x) for g in b.backward() for x in g]))
+            assert np.array_equal(out[0], out[1])
+            return out[0], b.final_state(), b.profiles()
+
+    _, state, (rho, u) = run(STEPS, True)
+    for p in {0, len(cells) // 2, len(cells) - 1}:
+        n, sl = cells[p], slice(off[p], off[p + 1])
+        with Adjoint(eos[p], n, STEPS, every=STEPS) as a:
+            a.set_initial(prims[p], ifc[p])
+            a.set_target(zero[sl], zero[sl])
+            a.forward()
+            assert np.array_equal(a.final_state(), state[:, sl]), p
+    rho = rho.copy()
+    rho[off[:-1] + np.array(cells) // 3] *= 1.01  # one observed cell per problem
+    ref = run(1, False, target=(rho, u))[0]
+    assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0.0
+    for every, sparse, graph in ((2, True, True), (26, False, True), (27, True, False), (STEPS, True, True)):
+        assert np.array_equal(run(every, sparse, graph, (rho, u))[0], ref), (every, sparse, graph)
