@@ -886,12 +886,7 @@ int hes_batch_create(hes_batch** out, int nphase, int flux, int nproblems, const
   if (flux != HES_FLUX_RUSANOV && flux != HES_FLUX_HLL && flux != HES_FLUX_LXF)
     return fail(HES_ERR_ARG, "unknown flux");
   if (nproblems < 1 || !ncells || !materials) return fail(HES_ERR_ARG, "null argument");
-  int dev = 0, cus = 0;
-  HIP_TRY(hipGetDevice(&dev));
-  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   hes_batch* h = new hes_batch();
-  h->dev = dev;
-  h->cus = cus;
   h->nph = nphase;
   h->flux = flux;
   h->nc = nphase == 1 ? 14 : 30;
@@ -930,7 +925,10 @@ int hes_batch_create(hes_batch** out, int nphase, int flux, int nproblems, const
   h->N = h->offsets_h[nproblems];
   h->pitch = (h->N + 63) / 64 * 64 + 256;  // rows padded off a power-of-two stride, as the solver's
   size_t qb = sizeof(double) * (size_t)h->nc * h->pitch, cb = sizeof(double) * (size_t)nphase * h->pitch;
-  hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
+  hipError_t e = hipGetDevice(&h->dev);
+  if (e == hipSuccess)
+    e = hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, h->dev);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   for (int b = 0; b < 2 && e == hipSuccess; ++b) {
     e = hipMalloc(&h->Q[b], qb);
     if (e == hipSuccess) e = hipMalloc(&h->C[b], cb);
