@@ -142,7 +142,7 @@ class Adjoint:
 
 class BatchAdjoint:
     """Reverse mode of a batch of independent fixed-length single-phase
-    Rusanov runs (one launch per step covers every problem).  Problem p has
+    Rusanov runs (every launch covers all problems).  Problem p has
     its own material, cell count, dx (default 1 / ncells[p]), pieces and
     target; every problem takes `steps` steps.  `backward()` returns, per
     problem, the gradient of its own misfit L_p with respect to its pieces'

@@ -1,9 +1,11 @@
-"""Batched solves: thousands of independent 1D problems in one launch per step.
+"""Batched solves: thousands of independent 1D problems advanced together.
 
 Each problem has its own length, materials, CFL number and dx, hence its own
 time step (main.jl:204-214 applied per problem).  The state of all problems is
 packed (ncomp x total cells, problems one after another) and lives on the GPU.
-`run(steps, mode="graph")` captures the whole step loop in one hipGraph;
+`run(steps, mode="graph")` runs the whole step loop at once: in one launch
+(one phase, problems that fit the chip) or as one captured hipGraph;
+`mode="eager"` takes one launch per step;
 `mode="loop"` is the one-problem-per-launch baseline; `autotune()` picks the
 launch shape by timing each candidate on the actual problem set.
 """

@@ -1,5 +1,6 @@
 // hes_batch.hip -- many independent 1D problems of uneven length advanced
-// together: one launch per time step covers every problem.
+// together: one launch per time step covers every problem, or one launch all
+// time steps of them (one phase, hes_resident.hpp).
 //
 // All cells of all problems are packed into one structure-of-arrays state
 // (problem p owns cells [offsets[p], offsets[p+1])).  Work is cut into tiles of

@@ -1,7 +1,8 @@
 // hes_kernels.hip -- gfx950 kernels of the finite-volume time step and the
 // C-ABI of libhes.so (declared in include/hes.h).
 //
-// Time step (main.jl:202-241).  One launch per step:
+// Time step (main.jl:202-241).  Problems that fit the chip take all their steps
+// in one launch (hes_resident.hpp), larger ones one launch per step:
 //   k_step<NPH,FLUX>  reads Q^n and the per-cell sound speeds c^n, takes
 //                     dt^n = cfl dx / max lambda^n from a ring slot written by
 //                     the previous launch, evaluates each cell's flux once and

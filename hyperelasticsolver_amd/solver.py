@@ -1,9 +1,10 @@
 """Time stepping on the GPU: the loop of main.jl:202-241 behind libhes.so.
 
 `Solver` owns the device state of one 1D problem (structure-of-arrays FP64 in
-HBM) and advances it with one fused kernel launch per step.  The state crosses
-the host boundary only in `set_state` / `get_state`, in the reference's Julia
-layout (ncomp x nx, component fastest).
+HBM) and advances it with one fused kernel launch per step, or, if it fits the
+chip, with one launch for all steps.  The state crosses the host boundary only
+in `set_state` / `get_state`, in the reference's Julia layout (ncomp x nx,
+component fastest).
 """
 import ctypes
 import math
