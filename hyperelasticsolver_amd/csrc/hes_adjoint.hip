@@ -203,22 +203,24 @@ struct AdjSegArgs {
   int nw;
   MatDev mat;
 };
-__global__ __launch_bounds__(SEG_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
+template <int BLK>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(3)))
 void k_adj_segment(AdjSegArgs a) {
   SegCtx c = a.c;
-  c.o0 = xcd_block() * (c.halo ? SEG_OWN : SEG_CELLS);
-  c.o1 = min(c.o0 + (c.halo ? SEG_OWN : SEG_CELLS), c.hi);
+  const int per = c.halo ? seg_own(BLK) : seg_cells(BLK);
+  c.o0 = xcd_block() * per;
+  c.o1 = min(c.o0 + per, c.hi);
   if (a.zin) {
     const long long reach = a.end - a.s + 2 * TILE + 2;
     const long long lo = max(c.o0 - reach, 0LL), hi = min(c.o1 + reach, c.hi);  // [lo, hi)
     bool needed = false;
-    for (long long t = lo / TILE + threadIdx.x; t < a.nw && t * TILE < hi; t += SEG_BLOCK)
+    for (long long t = lo / TILE + threadIdx.x; t < a.nw && t * TILE < hi; t += BLK)
       needed |= a.zin[t] == 0;
-    for (long long s = a.s + threadIdx.x; s <= a.end && s < a.nsteps; s += SEG_BLOCK)
+    for (long long s = a.s + threadIdx.x; s <= a.end && s < a.nsteps; s += BLK)
       needed |= a.istar[s] >= lo && a.istar[s] < hi;
     if (!__syncthreads_or(needed)) return;
   }
-  segment_run(c, a.mat);
+  segment_run<BLK>(c, a.mat);
 }
 
 // Argmax cell of the CFL speed of the checkpoint states from the per-block
@@ -844,9 +846,12 @@ hipError_t record_backward(hes_adjoint* h) {
   const bool find = h->res.shape.block == 0;
   // Small problems keep the overlap: their recompute is short, and all of it is
   // soon needed (us per reverse step, overlapped and skipping: 1000 cells 9.4
-  // and 10.5, 30000 10.3 and 10.6, 50000 11.0 and 10.5, 131072 14.1 and 12.3,
-  // 2^18 18.1 and 13.3; 34.5 with one launch per recomputed step).
+  // and 10.5, 30000 9.6 and 10.6, 50000 at most 11.0 and 10.5, 131072 at most
+  // 14.1 and 12.3, 2^18 at most 18.1 and 13.3; "at most": with 256 threads)
   const bool skip = h->sparse && !find && h->nw > 3 * h->cus;
+  const int blk = skip || find ? SEG_BLOCK : SEG_BLOCK_BESIDE;
+  void (*segment)(AdjSegArgs) =
+      blk == SEG_BLOCK ? k_adj_segment<SEG_BLOCK> : k_adj_segment<SEG_BLOCK_BESIDE>;
   hipStream_t st2 = skip ? st : h->stream2;
   if (!skip) {
     HIP_TRY_E(hipEventRecord(h->ev_fork, st));
@@ -866,7 +871,7 @@ hipError_t record_backward(hes_adjoint* h) {
       a.c.stride = 1;
       a.c.pitch = h->pitch;
       a.c.hi = h->n;
-      a.c.halo = h->n > SEG_CELLS ? SEG_STEPS : 0;
+      a.c.halo = h->n > seg_cells(blk) ? SEG_STEPS : 0;
       a.c.steps = (int)std::min<long long>(SEG_STEPS, end - 1 - s);
       a.c.find = find;
       a.c.cfl = h->cfl;
@@ -877,9 +882,8 @@ hipError_t record_backward(hes_adjoint* h) {
       a.nsteps = h->nsteps;
       a.nw = h->nw;
       a.mat = h->mat;
-      const long long per = a.c.halo ? SEG_OWN : SEG_CELLS;
-      hipLaunchKernelGGL(k_adj_segment, dim3((unsigned)((h->n + per - 1) / per)), dim3(SEG_BLOCK),
-                         0, st2, a);
+      const long long per = a.c.halo ? seg_own(blk) : seg_cells(blk);
+      hipLaunchKernelGGL(segment, dim3((unsigned)((h->n + per - 1) / per)), dim3(blk), 0, st2, a);
     }
     const int cnt = (int)(end - s0);
     hipLaunchKernelGGL(k_adj_lam, dim3((cnt + 63) / 64), dim3(64), 0, st2, ck_q(h, c),

@@ -274,12 +274,19 @@ struct AdjHook {
 // takes SEG_STEPS steps with its cells in registers and SEG_STEPS halo cells
 // on either side, which lose one valid cell per step at their outer end, and
 // writes every state on the way (a launch per step read and wrote each state,
-// 20 us per step at 2^18 cells; here 5 us).  The halo costs 25% more
-// arithmetic; 25 steps make two launches of the usual 50-step segment.
-constexpr int SEG_BLOCK = 256;
+// 20 us per step at 2^18 cells; here 5 us).  25 steps make two launches of the
+// usual 50-step segment.
 constexpr int SEG_STEPS = 25;
-constexpr int SEG_CELLS = SEG_BLOCK / 64 * TILE + 2;    // cells of a workgroup
-constexpr int SEG_OWN = SEG_CELLS - 2 * SEG_STEPS;      // without the halos
+constexpr int seg_cells(int block) { return block / 64 * TILE + 2; }  // of a workgroup
+constexpr int seg_own(int block) { return seg_cells(block) - 2 * SEG_STEPS; }  // without the halos
+// Threads of a workgroup: beside the reverse steps the larger one, whose halos
+// cost 11% (reverse pass, ms, 256 / 512 threads: 2^18 cells without skipping
+// 70.8 / 69.3, 30000 cells 5.14 / 4.76, 16 small problems 5.66 / 5.32, 256
+// larger ones 239 / 234, 1000 small ones 18.4 / 18.5); the smaller one where
+// workgroups without a cotangent near them end at once (2^18 cells 26.6 /
+// 27.8) and above the chip's size (500000 cells 7.0 / 7.3); 1024 is no better
+// than 512 and slower for many small problems (20.3).
+constexpr int SEG_BLOCK = 256, SEG_BLOCK_BESIDE = 512;
 struct SegCtx {
   const double* Q;   // state s (14 rows)
   double* out;       // states s + 1, s + 2, ..: slots of 15 rows
@@ -289,8 +296,9 @@ struct SegCtx {
   int halo, steps, find;
   double cfl;
 };
+template <int BLK>
 __device__ __forceinline__ void segment_run(const SegCtx& a, const MatDev& mat) {
-  constexpr int W = SEG_BLOCK / 64;
+  constexpr int W = BLK / 64;
   __shared__ double edge[2][W][2][NQ];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

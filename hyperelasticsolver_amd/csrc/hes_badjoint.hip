@@ -252,7 +252,7 @@ __global__ void k_badj_nocell(long long* __restrict__ istar, long long m) {
 
 // States s + 1 .. s + steps of every problem from state s (segment_run), a
 // workgroup per entry of the table.  Reverse pass of 256 problems of 1024 ..
-// 8192 cells, the recompute in a launch per step against this: 249 -> 240 ms
+// 8192 cells, the recompute in a launch per step against this: 249 -> 234 ms
 // (the reverse steps, one wave per SIMD, are what it waits for).
 struct BSeg {
   long long lo, hi, o0, o1;  // the problem's cells, the workgroup's
@@ -263,7 +263,7 @@ struct BAdjSegArgs {
   const MatDev* mats;
   SegCtx c;
 };
-__global__ __launch_bounds__(SEG_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ __launch_bounds__(SEG_BLOCK_BESIDE) __attribute__((amdgpu_waves_per_eu(3)))
 void k_badj_segment(BAdjSegArgs a) {
   const BSeg* g = a.segs + __builtin_amdgcn_readfirstlane((int)xcd_block());
   SegCtx c = a.c;
@@ -274,7 +274,7 @@ void k_badj_segment(BAdjSegArgs a) {
   c.halo = cload(&g->halo);
   const int p = cload(&g->p);
   c.lmax += p;
-  segment_run(c, uniform_mat(a.mats + p));
+  segment_run<SEG_BLOCK_BESIDE>(c, uniform_mat(a.mats + p));
 }
 
 // Argmax cell of the CFL speed of every (state, problem) from the per-tile
@@ -924,7 +924,8 @@ hipError_t brecord_backward(hes_badjoint* h) {
       a.c.pitch = h->pitch;
       a.c.steps = (int)std::min<long long>(SEG_STEPS, end - 1 - s);
       a.c.cfl = h->cfl;
-      hipLaunchKernelGGL(k_badj_segment, dim3((unsigned)h->nsegs), dim3(SEG_BLOCK), 0, st2, a);
+      hipLaunchKernelGGL(k_badj_segment, dim3((unsigned)h->nsegs), dim3(SEG_BLOCK_BESIDE), 0, st2,
+                         a);
     }
     const int cnt = (int)(end - s0);
     hipLaunchKernelGGL(k_badj_lam, dim3(blocks_of((long long)cnt * h->P, 64)), dim3(64), 0, st2,
@@ -1071,10 +1072,10 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
   std::vector<BSeg> segs;
   for (int p = 0; p < nproblems; ++p) {
     const long long lo = h->offs_h[p], hi = h->offs_h[p + 1];
-    const bool whole = hi - lo <= SEG_CELLS;
-    for (long long c = lo; c < hi; c += whole ? SEG_CELLS : SEG_OWN)
-      segs.push_back({lo, hi, c, std::min(c + (whole ? SEG_CELLS : SEG_OWN), hi), p,
-                      whole ? 0 : SEG_STEPS});
+    const bool whole = hi - lo <= seg_cells(SEG_BLOCK_BESIDE);
+    const int per = whole ? seg_cells(SEG_BLOCK_BESIDE) : seg_own(SEG_BLOCK_BESIDE);
+    for (long long c = lo; c < hi; c += per)
+      segs.push_back({lo, hi, c, std::min(c + per, hi), p, whole ? 0 : SEG_STEPS});
   }
   h->nsegs = (int)segs.size();
   const BResPlan pl = bres_plan(h->offs_h, h->cus, NQ);
