@@ -847,7 +847,7 @@ hipError_t record_backward(hes_adjoint* h) {
   // Small problems keep the overlap: their recompute is short, and all of it is
   // soon needed (us per reverse step, overlapped and skipping: 1000 cells 9.4
   // and 10.5, 30000 9.6 and 10.6, 50000 at most 11.0 and 10.5, 131072 at most
-  // 14.1 and 12.3, 2^18 at most 18.1 and 13.3; "at most": with 256 threads)
+  // 14.1 and 12.3, 2^18 at most 18.1 and 13.3; "at most": with 256 threads).
   const bool skip = h->sparse && !find && h->nw > 3 * h->cus;
   const int blk = skip || find ? SEG_BLOCK : SEG_BLOCK_BESIDE;
   void (*segment)(AdjSegArgs) =
