@@ -1156,8 +1156,8 @@ int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_gra
   long long done = 0;
   float ms = 0.f;
   int bad = 0;
-  bool ended = max_steps == 0;
-  while (h->shape.block && !ended) {
+  bool ended = false;
+  while (h->shape.block && max_steps > 0 && !ended) {
     const long long k = std::min(max_steps - done, RES_STEPS);
     long long now = 0;
     bool gave_up = false;
@@ -1167,7 +1167,7 @@ int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_gra
     done += now;
     ended = now < k || done == max_steps;  // t reached t_end, or all steps done
   }
-  if (!ended) {
+  if (!ended) {  // also for no step at all: a bad state is reported
     long long now = 0;
     const int rc = run_launches(h, max_steps - done, t_end, use_graph, hist ? hist + done : nullptr,
                                 &now, &ms, &bad);
