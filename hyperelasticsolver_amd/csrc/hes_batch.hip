@@ -762,8 +762,8 @@ void launch_batch_resident(const hes_batch* h, const BResArgs& a) {
 
 // `steps` (<= BRES_STEPS) steps of every problem in one launch.  *gave_up: no
 // result (a team's workgroups were not on the chip together), the batch is as
-// before.  Adds to *ms the launch's time.
-int run_batch_resident(hes_batch* h, long long steps, float* ms, bool* gave_up) {
+// before.  Adds to *ms the launch's time; *bad: a state has left the domain.
+int run_batch_resident(hes_batch* h, long long steps, float* ms, int* bad, bool* gave_up) {
   if (h->ends) {  // problems that stopped at an earlier launch
     const int rc = batch_carry(h);
     if (rc != HES_OK) return rc;
@@ -822,7 +822,7 @@ int run_batch_resident(hes_batch* h, long long steps, float* ms, bool* gave_up) 
     std::swap(h->Q[0], h->Q[1]);
     std::swap(h->C[0], h->C[1]);
   }
-  if (st[0]) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
+  *bad = st[0];
   return HES_OK;
 }
 
@@ -1107,17 +1107,18 @@ int hes_batch_run(hes_batch* h, long long steps, int mode, float* elapsed_ms) {
   if (!h->has_state) return fail(HES_ERR_ARG, "no state set");
   if (steps < 0 || mode < 0 || mode > 2) return fail(HES_ERR_ARG, "bad argument");
   float before = 0.f;
-  if (mode == 1) {
-    while (steps > 0 && h->res_tiles) {
+  if (mode == 1 && steps > 0 && h->res_tiles) {
+    int bad = 0;
+    bool gave_up = false;
+    while (steps > 0 && !gave_up) {
       const long long k = std::min(steps, BRES_STEPS);
-      bool gave_up = false;
-      const int rc = run_batch_resident(h, k, &before, &gave_up);
+      const int rc = run_batch_resident(h, k, &before, &bad, &gave_up);
       if (rc != HES_OK) return rc;
-      if (gave_up) break;
-      steps -= k;
+      if (!gave_up) steps -= k;
     }
     if (steps == 0) {
       if (elapsed_ms) *elapsed_ms = before;
+      if (bad) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
       return HES_OK;
     }
   }

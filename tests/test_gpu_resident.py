@@ -172,3 +172,28 @@ def test_resident_batch_equals_stepwise(flux, copies):
     for a, b in zip(*got):
         assert np.array_equal(a, b)
     assert got[0][3].min() < STEPS + 2 * MORE + 1 == got[0][3].max()
+
+
+@pytest.mark.parametrize("mode", ["eager", "graph"])
+def test_batch_goes_on_beside_a_bad_problem(mode):
+    """One problem of two is outside the domain: every run says so, also one of
+    no steps, and the other problem takes all its steps, in one launch or
+    several."""
+    print(f"[resident batch] bad problem, {mode}", flush=True)
+    n, steps, eos = 20, 66000, Barton2009()
+    states, ifc = _problem(eos, n, 5)
+    bad = np.array(states, order="F")
+    bad[5:14] *= -1.0
+    with Batch([eos] * 2, [n] * 2, flux="rusanov") as b:
+        with pytest.raises(DomainError):
+            b.set_piecewise([states, bad], [ifc, ifc])
+        for k in (0, steps, 0):
+            with pytest.raises(DomainError):
+                b.run(k, mode=mode)
+        t, done = b.times()
+        got = b.get_state()[:, :n]
+    with Batch([eos], [n], flux="rusanov") as b:
+        b.set_piecewise([states], [ifc])
+        b.run(steps, mode="eager")
+        assert done[0] == steps and t[0] == b.times()[0][0]
+        assert np.array_equal(got, b.get_state())
