@@ -140,15 +140,13 @@ __device__ __forceinline__ void bcol2(const MatDev* mat, const double* q, BCol& 
   }
 }
 
-// Neighbour values within a wave: lane_down(v) is lane + 1's v (lane 63 keeps
-// its own), lane_up(v) is lane - 1's v (lane 0 keeps its own), as
-// __shfl_down / __shfl_up by 1.  By default they are the wave-wide DPP shifts
-// (wave_shl:1 / wave_shr:1, plain VALU moves); HES_DPP_SHIFT=0 selects the LDS
-// crossbar (ds_bpermute) instead.
-#ifndef HES_DPP_SHIFT
-#define HES_DPP_SHIFT 1
-#endif
-#if HES_DPP_SHIFT
+// v moved between the lanes of a wave by a DPP control (plain VALU moves).
+// dpp_shift: a lane without a source keeps its own value.  dpp_shift_z: it
+// gets zero, also where the source lane is inactive, so it is only used where
+// every source lane is active: never under a lane-dependent condition (a && or
+// ?: whose other operand varies by lane).  With no old value to keep, the
+// shifted copy goes straight into a new register: one DPP move per half, where
+// dpp_shift first copies the value (the original stays live).
 template <int CTRL>
 __device__ __forceinline__ double dpp_shift(double v) {
   const long long b = __double_as_longlong(v);
@@ -157,16 +155,6 @@ __device__ __forceinline__ double dpp_shift(double v) {
   hi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-__device__ __forceinline__ double lane_down(double v) { return dpp_shift<0x130>(v); }  // wave_shl:1
-__device__ __forceinline__ double lane_up(double v) { return dpp_shift<0x138>(v); }    // wave_shr:1
-// The same shifts writing zero into the lane that has no source (lane 63 for
-// lane_down_z, lane 0 for lane_up_z) or whose source lane is inactive, so
-// they are only used where every lane of the wave is active: never under a
-// lane-dependent condition (a && or ?: whose other operand varies by lane).  With no old value to keep, the shifted
-// copy goes straight into a new register: one DPP move per half, where
-// lane_down / lane_up first copy the value (the original stays live).  For
-// values whose boundary-lane result only reaches the halo lanes' own face and
-// update, which are never stored.
 template <int CTRL>
 __device__ __forceinline__ double dpp_shift_z(double v) {
   const long long b = __double_as_longlong(v);
@@ -175,6 +163,21 @@ __device__ __forceinline__ double dpp_shift_z(double v) {
   hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
+
+// Neighbour values within a wave: lane_down(v) is lane + 1's v (lane 63 keeps
+// its own), lane_up(v) is lane - 1's v (lane 0 keeps its own), as
+// __shfl_down / __shfl_up by 1.  The _z forms write zero into the lane that has
+// no source (lane 63 or lane 0), every lane being active: for values whose
+// boundary-lane result only reaches the halo lanes' own face and update, which
+// are never stored.  By default they are the wave-wide DPP shifts (wave_shl:1
+// / wave_shr:1); HES_DPP_SHIFT=0 selects the LDS crossbar (ds_bpermute)
+// instead.
+#ifndef HES_DPP_SHIFT
+#define HES_DPP_SHIFT 1
+#endif
+#if HES_DPP_SHIFT
+__device__ __forceinline__ double lane_down(double v) { return dpp_shift<0x130>(v); }  // wave_shl:1
+__device__ __forceinline__ double lane_up(double v) { return dpp_shift<0x138>(v); }    // wave_shr:1
 __device__ __forceinline__ double lane_down_z(double v) { return dpp_shift_z<0x130>(v); }
 __device__ __forceinline__ double lane_up_z(double v) { return dpp_shift_z<0x138>(v); }
 #else
