@@ -57,6 +57,7 @@ _SIGS = {
     "hes_solver_next_dt": [_vp, _dp],
     "hes_solver_run": [_vp, _ll, _d, _i, ctypes.POINTER(_ll), _dp,
                        ctypes.POINTER(ctypes.c_float), _dp],
+    "hes_solver_team": [_vp, ctypes.POINTER(_ll), ctypes.POINTER(_i)],
     "hes_solver_time_steps": [_vp, _ll, ctypes.POINTER(ctypes.c_float)],
     "hes_solver_set_relaxation": [_vp, _d],
     "hes_solver_set_pressure_relaxation": [_vp, _d],
@@ -69,6 +70,7 @@ _SIGS = {
     "hes_adjoint_backward": [_vp, _dp, _dp, ctypes.POINTER(ctypes.c_float)],
     "hes_adjoint_set_sparse": [_vp, _i],
     "hes_adjoint_set_launch": [_vp, _i],
+    "hes_adjoint_team": [_vp, ctypes.POINTER(_ll), ctypes.POINTER(_i)],
     "hes_adjoint_get_state": [_vp, _dp],
     "hes_adjoint_get_profiles": [_vp, _dp, _dp],
     "hes_adjoint_info": [_vp, ctypes.POINTER(_ll), ctypes.POINTER(_ll)],
@@ -80,6 +82,7 @@ _SIGS = {
     "hes_badjoint_backward": [_vp, _dp, _dp, ctypes.POINTER(ctypes.c_float)],
     "hes_badjoint_set_sparse": [_vp, _i],
     "hes_badjoint_set_launch": [_vp, _i],
+    "hes_badjoint_team": [_vp, ctypes.POINTER(_ll), ctypes.POINTER(_i)],
     "hes_badjoint_get_state": [_vp, _dp],
     "hes_badjoint_get_profiles": [_vp, _dp, _dp],
     "hes_badjoint_info": [_vp, ctypes.POINTER(_ll), ctypes.POINTER(_ll), ctypes.POINTER(_ll)],
@@ -93,6 +96,7 @@ _SIGS = {
     "hes_batch_get_times": [_vp, _dp, ctypes.POINTER(_ll)],
     "hes_batch_set_t_end": [_vp, _dp],
     "hes_batch_set_launch": [_vp, _i, _i, _i],
+    "hes_batch_team": [_vp, ctypes.POINTER(_ll), ctypes.POINTER(_i)],
     "hes_batch_run": [_vp, _ll, _i, ctypes.POINTER(ctypes.c_float)],
     "hes_batch_autotune": [_vp, _i, ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_i),
                            ctypes.POINTER(ctypes.c_float)],
@@ -155,6 +159,14 @@ def check(rc):
     if rc == HES_ERR_DOMAIN:
         raise DomainError(msg)
     raise HesError(f"libhes error {rc}: {msg}")
+
+
+def team(fn, handle, wait_us):
+    """Call a `hes_*_team` entry; returns the team's workgroups."""
+    w = None if wait_us is None else ctypes.byref(ctypes.c_longlong(int(wait_us)))
+    n = ctypes.c_int()
+    check(fn(handle, w, ctypes.byref(n)))
+    return n.value
 
 
 def ptr(a):

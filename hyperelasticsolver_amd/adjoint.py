@@ -21,7 +21,7 @@ import ctypes
 
 import numpy as np
 
-from ._lib import check, lib, ptr
+from ._lib import check, lib, ptr, team
 from .solver import materials_array, nphase_of
 
 NPRIM = 13  # u(3), vec(A) column-major (9), S
@@ -119,6 +119,13 @@ class Adjoint:
     def set_launch(self, use_graph=True):
         """Replay each pass as one hipGraph (default) or launch its kernels one by one."""
         check(lib().hes_adjoint_set_launch(self._h, 1 if use_graph else 0))
+
+    def team(self, wait_us=None):
+        """Workgroups of the forward run's launch (0: a launch per step).  With
+        wait_us: how long they wait for one another before a launch per step
+        takes over for good (4 s unless set; 0: at once; negative: a launch per
+        step always).  The results are the same bits either way."""
+        return team(lib().hes_adjoint_team, self._h, wait_us)
 
     def final_state(self):
         Q = np.empty((14, self.n), order="F")
@@ -253,6 +260,13 @@ class BatchAdjoint:
 
     def set_launch(self, use_graph=True):
         check(lib().hes_badjoint_set_launch(self._h, 1 if use_graph else 0))
+
+    def team(self, wait_us=None):
+        """Workgroups of the forward run's launch (0: a launch per step).  With
+        wait_us: how long they wait for one another before a launch per step
+        takes over for good (4 s unless set; 0: at once; negative: a launch per
+        step always).  The results are the same bits either way."""
+        return team(lib().hes_badjoint_team, self._h, wait_us)
 
     def final_state(self):
         Q = np.empty((14, self.N), order="F")

@@ -13,7 +13,7 @@ import ctypes
 
 import numpy as np
 
-from ._lib import check, columns, lib, ptr
+from ._lib import check, columns, lib, ptr, team
 from .solver import FLUXES, materials_array, ncomp_of, nphase_of
 
 MODES = {"eager": 0, "graph": 1, "loop": 2}
@@ -120,6 +120,13 @@ class Batch:
         ms = ctypes.c_float()
         check(lib().hes_batch_run(self._h, int(steps), MODES[mode], ctypes.byref(ms)))
         return ms.value
+
+    def team(self, wait_us=None):
+        """Workgroups of the launch that takes all steps of a `graph` run (0: a launch per step).  With
+        wait_us: how long they wait for one another before a launch per step
+        takes over for good (4 s unless set; 0: at once; negative: a launch per
+        step always).  The results are the same bits either way."""
+        return team(lib().hes_batch_team, self._h, wait_us)
 
     def autotune(self, steps=3):
         """Time every launch shape (block, XCD order, tiles per wave) on the

@@ -626,7 +626,9 @@ __global__ __launch_bounds__(64) void k_adj_final(
 struct hes_adjoint {
   long long n, pitch, nsteps, every, nck;
   int dev = 0, cus = 0;
-  ResPlan res = {{0, 0}, 0, 0};        // the first pass in one launch; block 0: a launch per step
+  ResPlan plan = {{0, 0}, 0, 0};       // the first pass in one launch; block 0: it does not fit
+  ResPlan res = {{0, 0}, 0, 0};        // the same, or block 0: a launch per step
+  long long res_wait = res_ticks(RES_WAIT_US);  // ticks that its workgroups wait for one another
   unsigned long long* comm = nullptr;  // its team's messages
   int nb;    // blocks of the tiled kernels
   int nbr;   // blocks of the reverse step: one per CU (persistent waves)
@@ -749,6 +751,7 @@ hipError_t record_resident(hes_adjoint* h) {
   tm.border = h->comm + (size_t)2 * h->res.G * RES_SLOT;
   tm.tag0 = 1;  // the buffer was cleared above
   tm.gave_up = h->status + 2;
+  tm.wait = h->res_wait;
   a.hook.ck = ck_q(h, 0);
   a.hook.lmax = h->lmax;
   a.hook.istar = h->istar;
@@ -965,6 +968,11 @@ hipError_t dalloc(T** p, size_t count) {
   return hipMalloc((void**)p, sizeof(T) * (count > 0 ? count : 1));
 }
 
+void drop_graphs(hes_adjoint* h) {
+  if (h->gf) { (void)hipGraphExecDestroy(h->gf); h->gf = nullptr; }
+  if (h->gb) { (void)hipGraphExecDestroy(h->gb); h->gb = nullptr; }
+}
+
 }  // namespace
 
 extern "C" {
@@ -990,7 +998,7 @@ int hes_adjoint_create(hes_adjoint** out, long long ncells, const double* materi
   hes_adjoint* h = new hes_adjoint();
   h->dev = dev;
   h->cus = cus;
-  h->res = res_plan1(ncells, cus);
+  h->plan = h->res = res_plan1(ncells, cus);
   h->n = ncells;
   h->pitch = (ncells + 63) / 64 * 64 + 256;  // rows padded off a power-of-two stride, as the solver's
   h->nsteps = nsteps;
@@ -1068,8 +1076,7 @@ int hes_adjoint_destroy(hes_adjoint* h) {
   if (!h) return HES_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   if (h->stream2) (void)hipStreamSynchronize(h->stream2);
-  if (h->gf) (void)hipGraphExecDestroy(h->gf);
-  if (h->gb) (void)hipGraphExecDestroy(h->gb);
+  drop_graphs(h);
   void* bufs[] = {h->ck, h->seg[0], h->seg[1], h->fq[0], h->fq[1], h->fc[0], h->fc[1], h->qb[0], h->qb[1], h->zf,
                   h->lmax, h->blk_val, h->blk_idx, h->istar, h->Jlam, h->dtp, h->thb, h->lossp,
                   h->part, h->sums, h->gout, h->gin, h->prims, h->states, h->bounds, h->rho_t,
@@ -1114,8 +1121,7 @@ int hes_adjoint_set_initial(hes_adjoint* h, int nstates, const double* prims,
     h->has_init = false;
     h->fwd_done = false;
     (void)hipStreamSynchronize(h->stream);
-    if (h->gf) { (void)hipGraphExecDestroy(h->gf); h->gf = nullptr; }
-    if (h->gb) { (void)hipGraphExecDestroy(h->gb); h->gb = nullptr; }
+    drop_graphs(h);
     void* old[] = {h->prims, h->states, h->bounds, h->part, h->sums, h->gout};
     for (void* p : old)
       if (p) (void)hipFree(p);
@@ -1174,9 +1180,7 @@ int hes_adjoint_forward(hes_adjoint* h, double* loss, float* elapsed_ms) {
   }
   if (st[2]) {  // the team was not on the chip together: a launch per step from here on
     h->res.shape = {0, 0};
-    if (h->gf) (void)hipGraphExecDestroy(h->gf);
-    if (h->gb) (void)hipGraphExecDestroy(h->gb);
-    h->gf = h->gb = nullptr;
+    drop_graphs(h);
     return hes_adjoint_forward(h, loss, elapsed_ms);
   }
   float ms = 0.f;
@@ -1239,6 +1243,18 @@ int hes_adjoint_set_sparse(hes_adjoint* h, int on) {
 int hes_adjoint_set_launch(hes_adjoint* h, int use_graph) {
   if (!h) return fail(HES_ERR_ARG, "null handle");
   h->use_graph = use_graph != 0;
+  return HES_OK;
+}
+
+int hes_adjoint_team(hes_adjoint* h, const long long* wait_us, int* workgroups) {
+  if (!h) return fail(HES_ERR_ARG, "null handle");
+  if (wait_us) {
+    h->res_wait = res_ticks(*wait_us);
+    h->res.shape = *wait_us < 0 ? ResShape{0, 0} : h->plan.shape;
+    drop_graphs(h);
+    h->fwd_done = false;  // a reverse pass goes by how its first pass ran
+  }
+  if (workgroups) *workgroups = h->res.shape.block ? h->res.G : 0;
   return HES_OK;
 }
 

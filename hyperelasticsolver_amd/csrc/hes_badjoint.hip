@@ -218,6 +218,7 @@ struct BAdjResArgs {
   AdjHook hook;
   int* status;
   double cfl;
+  long long wait;
 };
 template <int T>
 __global__ __launch_bounds__(BRES_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
@@ -239,6 +240,7 @@ void k_badj_resident(BAdjResArgs a) {
   tm.lxf = 0;
   tm.tag0 = 1;  // the buffer is cleared before the launch
   tm.gave_up = a.status + 2;
+  tm.wait = a.wait;
   AdjHook hook = a.hook;
   hook.lmax += p;
   hook.istar += p;
@@ -721,8 +723,10 @@ struct hes_badjoint {
   std::vector<int> tfirst_h, tprob_h, poff_h;
   std::vector<double> mats_h;  // 8 x P
   int dev = 0, cus = 0;
-  // the first pass in one launch (tiles 0: a launch per step)
-  int res_tiles = 0, res_groups = 0;
+  // the first pass in one launch (plan_tiles 0: no such launch; res_tiles 0: a
+  // launch per step)
+  int plan_tiles = 0, res_tiles = 0, res_groups = 0;
+  long long res_wait = res_ticks(RES_WAIT_US);  // ticks that a team's workgroups wait for one another
   bool res_waits = false;
   size_t res_words = 0;
   BResTeam* teams = nullptr;
@@ -842,6 +846,7 @@ void brecord_resident(hes_badjoint* h) {
   a.hook.stride = h->P;
   a.status = h->status;
   a.cfl = h->cfl;
+  a.wait = h->res_wait;
   const dim3 grid((unsigned)h->res_groups), block(BRES_BLOCK);
   if (h->res_tiles == 1) hipLaunchKernelGGL(k_badj_resident<1>, grid, block, 0, st, a);
   else hipLaunchKernelGGL(k_badj_resident<2>, grid, block, 0, st, a);
@@ -1125,7 +1130,7 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
     up(&h->teams, pl.teams.data(), pl.teams.size());
     up(&h->items, pl.items.data(), pl.items.size());
     up(&h->comm, nullptr, pl.words);
-    h->res_tiles = pl.tiles;
+    h->plan_tiles = h->res_tiles = pl.tiles;
     h->res_groups = (int)pl.items.size();
     h->res_waits = pl.waits;
     h->res_words = pl.words;
@@ -1348,6 +1353,18 @@ int hes_badjoint_set_sparse(hes_badjoint* h, int on) {
 int hes_badjoint_set_launch(hes_badjoint* h, int use_graph) {
   if (!h) return fail(HES_ERR_ARG, "null handle");
   h->use_graph = use_graph != 0;
+  return HES_OK;
+}
+
+int hes_badjoint_team(hes_badjoint* h, const long long* wait_us, int* workgroups) {
+  if (!h) return fail(HES_ERR_ARG, "null handle");
+  if (wait_us) {
+    h->res_wait = res_ticks(*wait_us);
+    h->res_tiles = *wait_us < 0 ? 0 : h->plan_tiles;
+    drop_graphs(h);
+    h->fwd_done = false;  // as hes_adjoint_team
+  }
+  if (workgroups) *workgroups = h->res_tiles ? h->res_groups : 0;
   return HES_OK;
 }
 

@@ -513,6 +513,7 @@ struct BResArgs {
   long long pitch;
   int steps, lxf, step;
   unsigned tag0;
+  long long wait;
 };
 
 template <int FLUX, int FAST, int T>
@@ -535,6 +536,7 @@ void k_batch_resident(BResArgs a) {
   tm.lxf = a.lxf;
   tm.tag0 = a.tag0;
   tm.gave_up = a.status + 2;
+  tm.wait = a.wait;
   const ResOut o = resident_run1<FLUX, FAST, BRES_BLOCK, T, RES_MAX_TEAM, (T > 1)>(tm, mat);
   if (tm.rank == 0 && threadIdx.x == 0) a.out[p] = {o.t, o.lmax, (int)o.steps};
 }
@@ -593,7 +595,9 @@ struct hes_batch {
   bool ends;  // end times are set: problems may have stopped at earlier launches
   // the whole loop in one launch (run_batch_resident)
   int dev, cus;
-  int res_tiles;             // tiles per wave; 0: one launch per step
+  int plan_tiles;            // tiles per wave; 0: no such launch
+  int res_tiles;             // the same, or 0: one launch per step
+  long long res_wait;        // ticks that a team's workgroups wait for one another
   int res_groups;            // workgroups
   bool res_waits;            // some problem has more than one
   unsigned res_tag;          // the last tag in its message buffer
@@ -728,7 +732,8 @@ int batch_carry(hes_batch* h) {
 constexpr long long BRES_STEPS = 1LL << 16;  // steps of one launch at most
 
 hipError_t plan_batch_resident(hes_batch* h) {
-  h->res_tiles = 0;
+  h->plan_tiles = h->res_tiles = 0;
+  h->res_wait = res_ticks(RES_WAIT_US);
   if (h->nph != 1) return hipSuccess;
   const BResPlan pl = bres_plan(h->offsets_h, h->cus, h->nc);
   if (pl.tiles == 0) return hipSuccess;
@@ -747,7 +752,7 @@ hipError_t plan_batch_resident(hes_batch* h) {
   h->comm_clear = (long long)pl.clear;
   h->res_waits = pl.waits;
   h->res_groups = (int)pl.items.size();
-  if (e == hipSuccess) h->res_tiles = pl.tiles;
+  if (e == hipSuccess) h->plan_tiles = h->res_tiles = pl.tiles;
   return e;
 }
 
@@ -789,6 +794,7 @@ int run_batch_resident(hes_batch* h, long long steps, float* ms, int* bad, bool*
   a.lxf = h->flux == HES_FLUX_LXF;
   a.step = (int)(s0 & 1);
   a.tag0 = h->res_tag + 1;
+  a.wait = h->res_wait;
   h->res_tag += (unsigned)steps + 1;
   int st[4] = {0, 0, 0, 0};
   {
@@ -1096,6 +1102,16 @@ int hes_batch_set_launch(hes_batch* h, int block, int xcd, int tiles_per_wave) {
   h->block = block;
   h->xcd = xcd ? 1 : 0;
   h->tpw = tiles_per_wave;
+  return HES_OK;
+}
+
+int hes_batch_team(hes_batch* h, const long long* wait_us, int* workgroups) {
+  if (!h) return fail(HES_ERR_ARG, "null handle");
+  if (wait_us) {
+    h->res_wait = res_ticks(*wait_us);
+    h->res_tiles = *wait_us < 0 ? 0 : h->plan_tiles;
+  }
+  if (workgroups) *workgroups = h->res_tiles ? h->res_groups : 0;
   return HES_OK;
 }
 

@@ -554,7 +554,9 @@ struct hes_solver {
   bool has_state;
   // the time loop in one launch (run_resident), for problems that fit the chip
   int dev, cus;
-  ResShape shape;            // block 0: one launch per step
+  ResShape plan;             // of its workgroups; block 0: it does not fit
+  ResShape shape;            // the same, or block 0: one launch per step
+  long long res_wait;        // ticks that the team's workgroups wait for one another
   int res_g, res_own;        // workgroups and cells of each
   unsigned long long* comm;  // their slots, then their halo words
   unsigned res_tag;          // the last tag written there
@@ -789,7 +791,8 @@ void plan_resident(hes_solver* h) {
   const ResPlan p = h->nph == 1 ? res_plan1(h->n, h->cus)
                                 : res_plan(h->n, h->cus, RES_SHAPES2, h->flux == HES_FLUX_HLL ? 2 : 3,
                                            [](ResShape s) { return s.block / 64 * (s.tiles - 2) + 2; });
-  h->shape = p.shape;
+  h->plan = h->shape = p.shape;
+  h->res_wait = res_ticks(RES_WAIT_US);
   h->res_g = p.G;
   h->res_own = p.own;
 }
@@ -847,6 +850,7 @@ int run_resident(hes_solver* h, long long steps, double t_end, double* dt_hist, 
   tm.border = h->comm + (size_t)2 * h->res_g * RES_SLOT;
   tm.tag0 = h->res_tag + 1;
   tm.gave_up = h->status + 2;
+  tm.wait = h->res_wait;
   a.slots = h->slots;
   a.tring = h->tring;
   a.jcnt = h->jcnt;
@@ -1181,6 +1185,16 @@ int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_gra
     HIP_TRY(copy_on(h->stream, dt_out, h->dt_hist, sizeof(double) * (size_t)done,
                     hipMemcpyDeviceToHost));
   if (bad) return fail(HES_ERR_DOMAIN, "non-positive det(rho A) or non-finite state");
+  return HES_OK;
+}
+
+int hes_solver_team(hes_solver* h, const long long* wait_us, int* workgroups) {
+  if (!h) return fail(HES_ERR_ARG, "null handle");
+  if (wait_us) {
+    h->res_wait = res_ticks(*wait_us);
+    h->shape = *wait_us < 0 ? ResShape{0, 0} : h->plan;
+  }
+  if (workgroups) *workgroups = h->shape.block ? h->res_g : 0;
   return HES_OK;
 }
 

@@ -24,7 +24,7 @@
 // written again only after every workgroup has published the step between,
 // i.e. has read it.
 //
-// Every wait gives up after HES_RES_WAIT_TICKS, or at once when another workgroup
+// Every wait gives up after ResTeam::wait, or at once when another workgroup
 // has: the launch then ends without a result and the caller's input is whole
 // (results go to another buffer, and only after the last wait).
 //
@@ -44,12 +44,8 @@ namespace hes {
 
 constexpr int RES_SLOT = 8;  // 64-bit words per slot: one per 64 B (stores of many
                              // workgroups into one line serialise; 256 workgroups: 3.1 -> 2.1 us)
-#ifndef HES_RES_WAIT_TICKS
-#define HES_RES_WAIT_TICKS 400000000LL  // of the 100 MHz counter: 4 s
-#endif
-#ifndef HES_RES_POLLS
-#define HES_RES_POLLS 64  // polls between two looks at the time
-#endif
+constexpr long long RES_WAIT_US = 4000000;  // the longest wait for a message, unless the user sets it
+constexpr int RES_POLLS = 64;               // polls between two looks at the time
 constexpr int RES_HALO = 8;  // halo cells on either side of a workgroup (a team of one has none)
 
 // wave_max by DPP shifts instead of the LDS crossbar (a dependent chain of 6
@@ -87,6 +83,8 @@ struct ResTeam {
   unsigned long long* border;  // halo words: 2 G 2 RES_HALO 2 NC
   unsigned tag0;               // larger than every tag in `border`
   int* gave_up;                // nonzero: a wait ended without its message
+  long long wait;              // ticks of the 100 MHz counter; 0: the team's last workgroup
+                               // gives up at its first wait
 };
 
 struct ResOut {
@@ -111,11 +109,11 @@ __device__ __forceinline__ void res_barrier() {
 // One check of a wait's end, every few polls: true when the wait is over
 // without its message (the time is up here, or another workgroup gave up).
 __device__ __forceinline__ bool res_expired(const ResTeam& a, int& polls, long long& since) {
-  if (++polls % HES_RES_POLLS) return false;
+  if (++polls % RES_POLLS) return false;
   const long long now = wall_clock64();
   if (since == 0) since = now;
   if (__hip_atomic_load(a.gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return true;
-  if (now - since < HES_RES_WAIT_TICKS) return false;
+  if (now - since < a.wait) return false;
   __hip_atomic_store(a.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return true;
 }
@@ -138,6 +136,10 @@ __device__ __forceinline__ bool res_collect(const ResTeam& a, long long s, doubl
   const unsigned long long* sl = a.slots + (s & 1) * a.G * (long long)RES_SLOT;
   int polls = 0;
   long long since = 0;
+  if (a.wait == 0 && a.rank == a.G - 1) {
+    __hip_atomic_store(a.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+  }
   for (;;) {
     unsigned long long x[MAXG / 64];
 #pragma unroll
@@ -704,6 +706,11 @@ struct ResShape {
   int block, tiles;
 };
 inline constexpr int RES_MAX_TEAM = 256;  // workgroups
+
+// Ticks of the device's 100 MHz counter in a time to wait (0 if it is negative).
+inline long long res_ticks(long long microseconds) {
+  return std::min(std::max(microseconds, 0LL), 1LL << 40) * 100;
+}
 
 // How a problem is laid on the chip (block 0: it is not, and runs step by
 // step): the first of these shapes whose team has a compute unit for every

@@ -12,7 +12,7 @@ import math
 import numpy as np
 
 from . import _lib
-from ._lib import FLUX_HLL, FLUX_LXF, FLUX_RUSANOV, check, columns, lib, ptr
+from ._lib import FLUX_HLL, FLUX_LXF, FLUX_RUSANOV, check, columns, lib, ptr, team
 
 # flux kinds of the time step: the face speed of NumFluxes.lxf as main.jl:46-50
 # chooses it (Rusanov: max over the face's two cells; Lax-Friedrichs: dx / dt),
@@ -173,6 +173,13 @@ class Solver:
         if record_dt:
             res["dt"] = dts[: done.value]
         return res
+
+    def team(self, wait_us=None):
+        """Workgroups of the launch that takes all steps of a run (0: a launch per step).  With
+        wait_us: how long they wait for one another before a launch per step
+        takes over for good (4 s unless set; 0: at once; negative: a launch per
+        step always).  The results are the same bits either way."""
+        return team(lib().hes_solver_team, self._h, wait_us)
 
     def time_steps(self, reps):
         """GPU time (ms) of `reps` back-to-back steps, replayed from one captured graph."""

@@ -107,6 +107,16 @@ int hes_solver_set_relaxation(hes_solver* h, double tau);
  * tau = INFINITY switches it off (the default). */
 int hes_solver_set_pressure_relaxation(hes_solver* h, double tau);
 
+/* The workgroups of a run in one launch, a team, wait for one another.  If they
+ * do not meet within *wait_us microseconds (4 s unless set; another program may
+ * hold a part of the GPU), the launch ends without a result and the run goes on
+ * with a launch per step, as do all later runs until this is called with a time
+ * again.  0: a team of several workgroups gives up at its first wait; negative:
+ * a launch per step always.  wait_us may be NULL (no change).  *workgroups (may
+ * be NULL) is the team's size, 0 where a launch per step is taken.  The results
+ * are the same bits either way. */
+int hes_solver_team(hes_solver* h, const long long* wait_us, int* workgroups);
+
 /* Time `reps` back-to-back steps (the step kernels and nothing else) with HIP
  * events on the solver stream; the state advances by reps steps.  The steps
  * are captured into one graph before the first event (as hes_solver_run
@@ -155,6 +165,8 @@ int hes_batch_set_launch(hes_batch* h, int block, int xcd, int tiles_per_wave);
  * cells), else captured in one hipGraph and launched once;
  * 2: one launch per problem per step (the per-problem loop). */
 int hes_batch_run(hes_batch* h, long long steps, int mode, float* elapsed_ms);
+/* As hes_solver_team, for mode 1; *workgroups counts all problems' teams. */
+int hes_batch_team(hes_batch* h, const long long* wait_us, int* workgroups);
 /* Time every launch shape (block 64/256 x XCD order on/off x 1, 2 or 4 tiles
  * per wave) for `steps` steps on the current state (which is restored
  * afterwards) and keep the fastest. */
@@ -198,6 +210,9 @@ int hes_adjoint_set_sparse(hes_adjoint* h, int on);
 /* use_graph != 0 (the default): each pass is one captured hipGraph, replayed;
  * 0: the kernels of a pass are launched one by one. */
 int hes_adjoint_set_launch(hes_adjoint* h, int use_graph);
+/* As hes_solver_team, for the forward run.  After a call with a time the
+ * forward run has to be made again before a reverse pass. */
+int hes_adjoint_team(hes_adjoint* h, const long long* wait_us, int* workgroups);
 /* Final state of the forward run (14 x ncells, Julia layout). */
 int hes_adjoint_get_state(hes_adjoint* h, double* Q_host);
 /* rho and u1 of every cell of the final state, computed exactly as the misfit
@@ -238,9 +253,10 @@ int hes_badjoint_forward(hes_badjoint* h, double* losses, double* total, float* 
  * [2p + 1] = (dL_p/db0_p, dL_p/dc0_p). */
 int hes_badjoint_backward(hes_badjoint* h, double* grad_states, double* grad_material,
                           float* elapsed_ms);
-/* As hes_adjoint_set_sparse / hes_adjoint_set_launch. */
+/* As hes_adjoint_set_sparse / hes_adjoint_set_launch / hes_adjoint_team. */
 int hes_badjoint_set_sparse(hes_badjoint* h, int on);
 int hes_badjoint_set_launch(hes_badjoint* h, int use_graph);
+int hes_badjoint_team(hes_badjoint* h, const long long* wait_us, int* workgroups);
 /* Final packed state (14 x total cells, Julia layout) and its rho, u1 profiles
  * as the misfit computes them. */
 int hes_badjoint_get_state(hes_badjoint* h, double* Q_host);
