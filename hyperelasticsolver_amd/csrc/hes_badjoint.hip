@@ -1083,7 +1083,7 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
       segs.push_back({lo, hi, c, std::min(c + per, hi), p, whole ? 0 : SEG_STEPS});
   }
   h->nsegs = (int)segs.size();
-  const BResPlan pl = bres_plan(h->offs_h, h->cus, NQ);
+  const BResPlan pl = bres_plan(h->offs_h, h->cus, NQ, false, true);
   h->pitch = (h->N + 63) / 64 * 64 + 256;  // rows padded off a power-of-two stride, as the solver's
   const size_t Pt = (size_t)h->pitch;
   hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);

@@ -735,7 +735,7 @@ hipError_t plan_batch_resident(hes_batch* h) {
   h->plan_tiles = h->res_tiles = 0;
   h->res_wait = res_ticks(RES_WAIT_US);
   if (h->nph != 1) return hipSuccess;
-  const BResPlan pl = bres_plan(h->offsets_h, h->cus, h->nc);
+  const BResPlan pl = bres_plan(h->offsets_h, h->cus, h->nc, h->flux == HES_FLUX_HLL, h->fast);
   if (pl.tiles == 0) return hipSuccess;
   hipError_t e = hipMalloc((void**)&h->teams, sizeof(BResTeam) * pl.teams.size());
   if (e == hipSuccess) e = hipMalloc((void**)&h->items, sizeof(BResItem) * pl.items.size());

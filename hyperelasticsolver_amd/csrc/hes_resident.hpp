@@ -774,7 +774,8 @@ hipError_t res_launch(void (*k)(Args), int block, int G, const Args& a, hipStrea
 // when all its workgroups are on the chip at once (64 problems of 100 .. 3000
 // cells: 3.7 against 5.0 us per step) or when its tiles are that many fewer
 // (1000 of 60 .. 700 cells: 12.5 against 14.5), else two, the largest problems
-// first.  tiles = 0 if a problem does not fit.
+// first.  tiles = 0 if a problem does not fit, or if a launch per step is faster
+// (bres_pays).
 struct BResPlan {
   int tiles = 0;
   bool waits = false;  // some problem has more than one workgroup
@@ -784,7 +785,27 @@ struct BResPlan {
   // cleared before a launch), then the halo words
   size_t clear = 0, words = 0;
 };
-inline BResPlan bres_plan(const std::vector<long long>& offsets, int cus, int nc) {
+// Many problems of a few cells: a workgroup's four waves all work, however few
+// cells its problem has, where a launch per step takes a wave per tile.  So once
+// the chip is full, one launch for all steps pays only if it takes less time than
+// a launch per step; both by us per step as measured on 256 compute units (the
+// latter in a captured graph, its capture and launch included), in the order
+// Rusanov, HLL, then with general exponents.  A launch per step against this,
+// us per step: 16384 problems of 3 cells 43 and 71 (HLL 45 and 106), of 62 cells
+// 57 and 71 (58 and 106), of 100 cells 94 and 71 (102 and 106), of 124 cells 110
+// and 72 (114 and 106); 4096 of 3 cells 15 and 18, of 62 cells 20 and 18 (19 and
+// 27); 2048 of 3 cells 11 and 10 (12 and 14), of 62 cells 17 and 10 (18 and 14).
+inline bool bres_pays(long long groups, int tiles_per_wave, long long tiles, long long cells,
+                      int cus, bool hll, bool fast) {
+  if (groups <= (long long)BRES_PER_CU * cus) return true;
+  constexpr double group_ns[4][2] = {{4.5, 7.9}, {6.45, 11.7}, {5.5, 10.1}, {8.65, 15.9}};
+  constexpr double step[4] = {1.0, 1.04, 1.10, 1.22};
+  const int k = (hll ? 1 : 0) + (fast ? 0 : 2);
+  const double once = 0.8 + 1e-3 * group_ns[k][tiles_per_wave - 1] * (double)groups;
+  const double each = step[k] * (8.0 + 2.1e-3 * (double)tiles + 15.5e-6 * (double)cells);
+  return once <= each;
+}
+inline BResPlan bres_plan(const std::vector<long long>& offsets, int cus, int nc, bool hll, bool fast) {
   const int P = (int)offsets.size() - 1;
   BResPlan pl;
   pl.teams.resize(P);
@@ -806,6 +827,9 @@ inline BResPlan bres_plan(const std::vector<long long>& offsets, int cus, int nc
   const bool one = groups1 >= 0 && (groups1 <= BRES_PER_CU * cus || 1.27 * groups1 < 2.0 * groups2);
   const long long groups = one ? groups1 : fit(2);
   if (groups < 0 || groups > 0x7fffffffLL) return pl;
+  long long tiles = 0;
+  for (int p = 0; p < P; ++p) tiles += (offsets[p + 1] - offsets[p] + TILE - 1) / TILE;
+  if (!bres_pays(groups, one ? 1 : 2, tiles, offsets[P] - offsets[0], cus, hll, fast)) return pl;
   std::vector<int> order(P);
   for (int p = 0; p < P; ++p) order[p] = p;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) {

@@ -1,0 +1,65 @@
+"""The library's host code without a GPU: libhes.so over a stand-in for the HIP
+runtime (fake_hip.cpp) in a process of its own, which plans routes, allocates
+and moves states; no kernel of the scheme runs."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes, sys
+sys.path.insert(0, {root!r})
+fake = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
+fake.fake_device_cap.argtypes = fake.fake_device_fail_from.argtypes = [ctypes.c_size_t]
+fake.fake_host_fail_from.argtypes = [ctypes.c_size_t, ctypes.c_longlong]
+fake.fake_device_used.restype = ctypes.c_size_t
+NONE = 2 ** 64 - 1  # no limit
+import numpy as np
+from hyperelasticsolver_amd._lib import HesError
+from hyperelasticsolver_amd.EquationsOfState import Barton2009
+from hyperelasticsolver_amd.adjoint import Adjoint, BatchAdjoint
+from hyperelasticsolver_amd.batched import Batch
+from hyperelasticsolver_amd.solver import Solver
+EOS = Barton2009()
+GENERAL = Barton2009(_beta=3.577, _gamma=2.088)
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC",
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", so], check=True)
+
+    def run(script):
+        r = subprocess.run([sys.executable, "-c", PRELUDE.format(root=ROOT, so=so) + textwrap.dedent(script)],
+                           cwd=ROOT, capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-3000:]
+
+    return run
+
+
+def test_route_of_a_batch(host):
+    """One launch for all steps where it is measured to pay, else a launch per
+    step: many problems of a few cells fill one wave of a workgroup's four."""
+    host("""
+    def team(P, n, flux="rusanov", eos=EOS):
+        with Batch([eos] * P, [n] * P, flux=flux) as b:
+            return b.team()
+    for n in (3, 32, 62):
+        assert team(16384, n) == team(16384, n, "hll") == team(16384, n, eos=GENERAL) == 0, n
+    assert team(4096, 3) == team(4096, 32, "hll") == team(16384, 100, "hll") == 0
+    assert team(16384, 124, "hll", GENERAL) == 0
+    # the chip is not full, or the waves have work
+    assert team(256, 3) == team(256, 3, "hll") == 256 and team(768, 3, "hll", GENERAL) == 768
+    assert team(16384, 124) == team(16384, 186, "hll") == team(16384, 250, "hll", GENERAL) == 16384
+    assert team(4096, 434) == 4096 and team(4096, 980, "hll") == 3 * 4096
+    with BatchAdjoint([EOS] * 8192, [40] * 8192, 4) as b:
+        assert b.team() == 0
+    with BatchAdjoint([EOS] * 200, [40] * 200, 4) as b:
+        assert b.team() == 200
+    """)
