@@ -302,7 +302,13 @@ __device__ __forceinline__ void segment_run(const SegCtx& a, const MatDev& mat) 
   __shared__ double edge[2][W][2][NQ];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const long long i = a.o0 - a.halo + TILE * w + lane;
+  // waves past the problem's last cell end here (a barrier waits for the waves
+  // that have not): of a short problem's workgroup only its own tiles work
+  const long long i0 = a.o0 - a.halo;
+  const long long past = a.hi - i0;  // cells from the first one on
+  const int last = past - 2 < (long long)TILE * (W - 1) ? (int)((past - 2) / TILE) : W - 1;
+  if (w > last) return;
+  const long long i = i0 + TILE * w + lane;
   const long long ic = i < a.lo ? a.lo : (i >= a.hi ? a.hi - 1 : i);
   const bool whole = a.halo == 0;
   const bool own = i >= a.o0 && i < a.o1 && (lane >= 1 || (whole && w == 0)) &&
@@ -341,7 +347,7 @@ __device__ __forceinline__ void segment_run(const SegCtx& a, const MatDev& mat) 
       for (int r = 0; r < NQ; ++r) edge[k & 1][w][lane == 1 ? 0 : 1][r] = q[r];
     }
     res_barrier();
-    if ((lane == 0 && w > 0) || (lane == 63 && w < W - 1)) {
+    if ((lane == 0 && w > 0) || (lane == 63 && w < last)) {
       const double* e = edge[k & 1][lane == 0 ? w - 1 : w + 1][lane == 0 ? 1 : 0];
 #pragma unroll
       for (int r = 0; r < NQ; ++r) q[r] = e[r];

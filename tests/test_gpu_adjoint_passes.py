@@ -87,8 +87,12 @@ def test_recomputed_states_change_nothing(n):
 
 
 # few workgroups (a tile per wave), more than the chip holds at once (two), a
-# problem that does not fit and runs step by step
-BATCHES = [[3, 62, 250, 251, 498, 499, 896, 897, 1000, 9000], [8000] * 40 + [5, 700], [123393, 300]]
+# problem that does not fit and runs step by step; then the last lengths that
+# each size of the recompute's workgroups holds, and waves past a short
+# problem's end (its last cell in a wave's first or last lane)
+BATCHES = [[3, 62, 250, 251, 498, 499, 896, 897, 1000, 9000], [8000] * 40 + [5, 700], [123393, 300],
+           [3, 62, 63, 64], [3, 65, 125, 126], [64, 127, 187, 188, 189, 250], [63, 125, 126, 497, 498],
+           [510, 511, 512, 513, 899, 946, 947]]
 
 
 @pytest.mark.parametrize("which", range(len(BATCHES)))
@@ -127,6 +131,8 @@ def test_batch_passes(which):
             assert np.array_equal(a.final_state(), state[:, sl]), p
     rho = rho.copy()
     rho[off[:-1] + np.array(cells) // 3] *= 1.01  # one observed cell per problem
+    u = u.copy()
+    u[off[1:] - 1 - (np.array(cells) > 9)] += 0.01  # and one at its end
     ref = run(1, False, target=(rho, u))[0]
     assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0.0
     for every, sparse, graph in ((2, True, True), (26, False, True), (27, True, False), (STEPS, True, True)):
