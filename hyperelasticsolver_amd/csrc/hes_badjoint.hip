@@ -202,8 +202,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
               a.blk_idx ? a.blk_idx + row : nullptr, tile);
 }
 
-// The whole first pass of every problem in one launch (a team of workgroups
-// per problem, hes_resident.hpp), for problems that fit the chip.  us per step,
+// The first pass of every problem in one launch (a team of workgroups per
+// problem, hes_resident.hpp), for problems that fit the chip.  us per step,
 // one launch per step against this: 256 problems of 1024 .. 8192 cells 51 ->
 // 28, 1000 of 100 .. 900 cells 23 -> 15, 16 of them 5.5 -> 3.8.
 struct BAdjResArgs {
@@ -218,7 +218,7 @@ struct BAdjResArgs {
   AdjHook hook;
   int* status;
   double cfl;
-  long long wait;
+  long long wait, steps;
 };
 template <int T>
 __global__ __launch_bounds__(BRES_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
@@ -234,7 +234,7 @@ void k_badj_resident(BAdjResArgs a) {
   tm.dx = cload(a.dx + p);
   tm.t = 0.0;
   tm.t_end = INFINITY;
-  tm.kmax = a.hook.nsteps;
+  tm.kmax = a.steps;
   tm.dt_hist = nullptr;
   tm.status = a.status;
   tm.lxf = 0;
@@ -836,12 +836,11 @@ BAdjFwdArgs bfwd_args(hes_badjoint* h, long long s, const double* qi, double* qo
 
 unsigned blocks_of(long long m, int per) { return (unsigned)((m + per - 1) / per); }
 
-// The first pass from checkpoint 0 (the initial states) in one launch.
+// The first pass from checkpoint 0 (the initial states), BRES_STEPS steps a
+// launch.  A state on the border of two launches is recorded by both, alike.
 void brecord_resident(hes_badjoint* h) {
   hipStream_t st = h->stream;
   const long long words = (long long)h->res_words, pairs = h->nsteps * h->P;
-  hipLaunchKernelGGL(k_badj_zero, dim3(blocks_of(words, LBLK)), dim3(LBLK), 0, st,
-                     (double*)h->comm, words);
   hipLaunchKernelGGL(k_badj_nocell, dim3(blocks_of(pairs, LBLK)), dim3(LBLK), 0, st, h->istar, pairs);
   BAdjResArgs a;
   std::memset((void*)&a, 0, sizeof(a));
@@ -850,21 +849,32 @@ void brecord_resident(hes_badjoint* h) {
   a.comm = h->comm;
   a.mats = h->mats;
   a.dx = h->dx;
-  a.Qin = bck_q(h, 0);
-  bfwd_slot(h, h->nsteps, &a.Qout, &a.Cout);
-  a.hook.ck = bck_q(h, 0);
-  a.hook.lmax = h->lmax;
-  a.hook.istar = h->istar;
   a.hook.every = h->every;
-  a.hook.nsteps = h->nsteps;
   a.hook.pitch = h->pitch;
   a.hook.stride = h->P;
   a.status = h->status;
   a.cfl = h->cfl;
   a.wait = h->res_wait;
   const dim3 grid((unsigned)h->res_groups), block(BRES_BLOCK);
-  if (h->res_tiles == 1) hipLaunchKernelGGL(k_badj_resident<1>, grid, block, 0, st, a);
-  else hipLaunchKernelGGL(k_badj_resident<2>, grid, block, 0, st, a);
+  a.Qout = bck_q(h, 0);
+  for (long long s = 0; s < h->nsteps; s += BRES_STEPS) {
+    hipLaunchKernelGGL(k_badj_zero, dim3(blocks_of(words, LBLK)), dim3(LBLK), 0, st,
+                       (double*)h->comm, words);
+    const long long left = h->nsteps - s, after = (left - 1) / BRES_STEPS;  // steps, launches
+    const int to = (int)((h->nsteps + after) & 1);  // in turn, the last one where it is looked for
+    a.Qin = a.Qout;
+    a.Qout = h->fq[to];
+    a.Cout = h->fc[to];
+    a.steps = std::min(left, BRES_STEPS);
+    const long long c = (s + h->every - 1) / h->every;  // the first checkpoint from state s on
+    a.hook.ck = bck_q(h, c);
+    a.hook.next = c * h->every - s;
+    a.hook.lmax = h->lmax + s * h->P;
+    a.hook.istar = h->istar + s * h->P;
+    a.hook.nsteps = left;
+    if (h->res_tiles == 1) hipLaunchKernelGGL(k_badj_resident<1>, grid, block, 0, st, a);
+    else hipLaunchKernelGGL(k_badj_resident<2>, grid, block, 0, st, a);
+  }
 }
 
 // The first pass from checkpoint 0, a launch per step.

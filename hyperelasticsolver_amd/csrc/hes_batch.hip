@@ -729,8 +729,6 @@ int batch_carry(hes_batch* h) {
 
 // ---- the whole loop in one launch ------------------------------------------------
 
-constexpr long long BRES_STEPS = 1LL << 16;  // steps of one launch at most
-
 hipError_t plan_batch_resident(hes_batch* h) {
   h->plan_tiles = h->res_tiles = 0;
   h->res_wait = res_ticks(RES_WAIT_US);

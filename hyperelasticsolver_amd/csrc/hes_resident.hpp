@@ -678,6 +678,11 @@ struct BResItem {  // a workgroup's place: rank in the team of a problem
 // step, one launch per step against this: Rusanov 780 -> 398, HLL 830 -> 564;
 // three tiles per wave at two waves per SIMD: 408 and 582; one tile: 516, 680.
 inline constexpr int BRES_BLOCK = 256, BRES_PER_CU = 3;
+// Steps of one launch at most.  The first workgroups of a team that is next in
+// line wait until an earlier team has taken all its steps, which has to stay
+// well below the time after which a wait gives up: a step of a full chip takes
+// 9 to 16 us, this many 0.15 to 0.3 s, and a launch more costs 30 us.
+inline constexpr long long BRES_STEPS = 1LL << 14;
 // This workgroup's problem, and its place in the problem's team (tm's cells and
 // messages).
 __device__ __forceinline__ int bres_place(int* ticket, const BResItem* items, const BResTeam* teams,

@@ -14,6 +14,7 @@ namespace {
 constexpr int OK = 0, OUT_OF_MEMORY = 2;
 std::mutex mutex;
 std::map<const void*, std::string> kernels;
+std::map<std::string, long long> launches;
 std::map<void*, size_t> device;
 size_t device_used = 0, device_cap = ~(size_t)0, device_fail_min = ~(size_t)0;
 size_t host_fail_min = ~(size_t)0;
@@ -41,6 +42,13 @@ void fake_device_fail_from(size_t bytes) { device_fail_min = bytes; }  // alloca
 void fake_host_fail_from(size_t bytes, long long allowed) {
   host_fail_min = bytes;
   host_allowed = allowed;
+}
+long long fake_launches(const char* name) {  // of kernels whose name contains this
+  std::lock_guard<std::mutex> lock(mutex);
+  long long n = 0;
+  for (auto& k : launches)
+    if (k.first.find(name) != std::string::npos) n += k.second;
+  return n;
 }
 size_t fake_device_used() { return device_used; }
 
@@ -85,6 +93,12 @@ const char* hipGetErrorString(int e) { return e == OUT_OF_MEMORY ? "out of memor
 int hipStreamCreateWithFlags(void** s, unsigned) { *s = std::malloc(1); return OK; }
 int hipStreamDestroy(void* s) { std::free(s); return OK; }
 int hipStreamSynchronize(void*) { return OK; }
+int hipStreamBeginCapture(void*, int) { return OK; }
+int hipStreamEndCapture(void*, void** g) { *g = std::malloc(1); return OK; }
+int hipGraphInstantiate(void** x, void*, void*, char*, size_t) { *x = std::malloc(1); return OK; }
+int hipGraphLaunch(void*, void*) { return OK; }
+int hipGraphDestroy(void* g) { std::free(g); return OK; }
+int hipGraphExecDestroy(void* x) { std::free(x); return OK; }
 int hipStreamWaitEvent(void*, void*, unsigned) { return OK; }
 int hipEventCreate(void** e) { *e = std::malloc(1); return OK; }
 int hipEventCreateWithFlags(void** e, unsigned) { return hipEventCreate(e); }
@@ -120,6 +134,7 @@ int hipLaunchKernel(const void* f, Dim3, Dim3, void** a, size_t, void*) {
   {
     std::lock_guard<std::mutex> lock(mutex);
     name = kernels[f];
+    ++launches[name];
   }
   auto ll = [&](int k) { return *(long long*)a[k]; };
   if (name.find("k_aos_to_soa") != std::string::npos) {  // in, out, nc, n, pitch

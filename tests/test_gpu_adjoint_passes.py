@@ -137,3 +137,29 @@ def test_batch_passes(which):
     assert np.all(np.isfinite(ref)) and np.abs(ref).max() > 0.0
     for every, sparse, graph in ((2, True, True), (26, False, True), (27, True, False), (STEPS, True, True)):
         assert np.array_equal(run(every, sparse, graph, (rho, u))[0], ref), (every, sparse, graph)
+
+
+@pytest.mark.parametrize("every", [4096, 5000])  # a checkpoint where two launches meet, and none
+def test_batch_first_pass_in_two_launches(every):
+    """More steps than one launch of the first pass takes: the losses, states
+    and gradients of a launch per step."""
+    cells, steps = [300, 20, 3], 16384 + 50
+    print(f"[adjoint passes] batch, {steps} steps, every {every}", flush=True)
+    eos = [Barton2009()] * len(cells)
+    rng = np.random.default_rng(every)
+    prims = [phase_prims_to_adjoint(random_phase_prims(rng, e, 2)) for e in eos]
+
+    def run(wait):
+        with BatchAdjoint(eos, cells, steps, every=every) as b:
+            b.team(wait)
+            b.set_initial(prims, [[0.5]] * len(cells))
+            b.set_target(np.full(sum(cells), 8.9), np.zeros(sum(cells)))
+            losses = b.forward()
+            out = [losses, b.final_state()] + [x for g in b.backward() for x in g]
+            assert (b.team() > 0) == (wait > 0)
+            return out
+
+    ref = run(-1)
+    assert np.all(np.isfinite(ref[0])) and np.all(np.isfinite(ref[1]))
+    for x, y in zip(run(4_000_000), ref):
+        assert np.array_equal(x, y, equal_nan=True)

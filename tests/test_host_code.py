@@ -17,6 +17,7 @@ fake = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
 fake.fake_device_cap.argtypes = fake.fake_device_fail_from.argtypes = [ctypes.c_size_t]
 fake.fake_host_fail_from.argtypes = [ctypes.c_size_t, ctypes.c_longlong]
 fake.fake_device_used.restype = ctypes.c_size_t
+fake.fake_launches.restype = ctypes.c_longlong
 NONE = 2 ** 64 - 1  # no limit
 import numpy as np
 from hyperelasticsolver_amd._lib import HesError
@@ -62,4 +63,22 @@ def test_route_of_a_batch(host):
         assert b.team() == 0
     with BatchAdjoint([EOS] * 200, [40] * 200, 4) as b:
         assert b.team() == 200
+    """)
+
+
+def test_long_batches_take_several_launches(host):
+    """The workgroups of a team next in line wait for an earlier team's last
+    step: no launch takes so many steps that this could pass for a team that
+    does not meet."""
+    host("""
+    with Batch([EOS] * 2000, [980] * 2000) as b:
+        b.set_state(np.ones((14, b.N), order="F"))
+        b.run(40000)
+        assert fake.fake_launches(b"k_batch_resident_end") == 3
+    cells, steps = [700, 20], 40000
+    with BatchAdjoint([EOS] * 2, cells, steps, every=1000) as b:
+        b.set_initial([np.ones((13, 1))] * 2, [[], []])
+        b.set_target(np.zeros(720), np.zeros(720))
+        b.forward()
+        assert fake.fake_launches(b"k_badj_resident") == 3
     """)
