@@ -1171,7 +1171,7 @@ int hes_adjoint_forward(hes_adjoint* h, double* loss, float* elapsed_ms) {
   }
   int st[4];
   {
-    ComputeUnits units(h->dev, h->cus, h->res.shape.block && h->res.G > 1 ? h->res.G : 0);
+    ComputeUnits units(h->dev, h->cus, h->res.shape.block ? h->res.G : 0, h->res.G > 1);
     HIP_TRY(hipEventRecord(h->ev0, h->stream));
     if (h->use_graph) HIP_TRY(hipGraphLaunch(h->gf, h->stream));
     else HIP_TRY(record_forward(h));

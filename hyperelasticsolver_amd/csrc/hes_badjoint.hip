@@ -1308,7 +1308,8 @@ int hes_badjoint_forward(hes_badjoint* h, double* losses, double* total, float* 
   }
   int st[4];
   {
-    ComputeUnits units(h->dev, h->cus, h->res_tiles && h->res_waits ? h->cus : 0);
+    ComputeUnits units(h->dev, h->cus, h->res_tiles == 0 ? 0 : h->res_waits ? h->cus : h->res_groups,
+                       h->res_waits);
     HIP_TRY(hipEventRecord(h->ev0, h->stream));
     if (h->use_graph) HIP_TRY(hipGraphLaunch(h->gf, h->stream));
     else HIP_TRY(brecord_forward(h));

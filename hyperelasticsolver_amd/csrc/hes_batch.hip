@@ -796,7 +796,7 @@ int run_batch_resident(hes_batch* h, long long steps, float* ms, int* bad, bool*
   h->res_tag += (unsigned)steps + 1;
   int st[4] = {0, 0, 0, 0};
   {
-    ComputeUnits units(h->dev, h->cus, h->res_waits ? h->cus : 0);
+    ComputeUnits units(h->dev, h->cus, h->res_waits ? h->cus : h->res_groups, h->res_waits);
     HIP_TRY(hipEventRecord(h->ev0, h->stream));
     HIP_TRY(hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * (size_t)h->comm_clear, h->stream));
     if (h->flux == HES_FLUX_HLL)

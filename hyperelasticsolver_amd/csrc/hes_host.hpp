@@ -3,14 +3,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cmath>
-#include <condition_variable>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
 
 #include "hes_device.hpp"
+#include "hes_units.hpp"
 #include "../../include/hes.h"
 
 namespace hes {
@@ -84,42 +83,6 @@ inline hipError_t zero_on(hipStream_t s, void* dst, size_t bytes) {
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   return e;
 }
-
-// Compute units for a launch whose workgroups wait for one another: two such
-// launches may only run at once if both fit, or each could hold units that the
-// other's missing workgroups need.  Held from before the launch until its
-// stream has been waited for.  (Other launches end by themselves.)
-class ComputeUnits {
- public:
-  ComputeUnits(int device, int total, int need) : dev_(device), need_(need) {
-    std::unique_lock<std::mutex> lock(mutex());
-    State& s = state(dev_);
-    s.cv.wait(lock, [&] { return s.used == 0 || s.used + need_ <= total; });
-    s.used += need_;
-  }
-  ~ComputeUnits() {
-    std::lock_guard<std::mutex> lock(mutex());
-    state(dev_).used -= need_;
-    state(dev_).cv.notify_all();
-  }
-  ComputeUnits(const ComputeUnits&) = delete;
-  ComputeUnits& operator=(const ComputeUnits&) = delete;
-
- private:
-  struct State {
-    int used = 0;
-    std::condition_variable cv;
-  };
-  static std::mutex& mutex() {
-    static std::mutex m;
-    return m;
-  }
-  static State& state(int device) {  // entries stay where they are
-    static std::map<int, State> s;
-    return s[device];
-  }
-  int dev_, need_;
-};
 
 // What a call works in: page-locked host memory that the kernels read and
 // write themselves (small calls: no copies), device memory (larger ones), and

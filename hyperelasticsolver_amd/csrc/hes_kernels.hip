@@ -863,7 +863,7 @@ int run_resident(hes_solver* h, long long steps, double t_end, double* dt_hist, 
   h->res_tag += (unsigned)steps + 1;
   hipError_t e;
   {
-    ComputeUnits units(h->dev, h->cus, h->res_g > 1 ? h->res_g : 0);
+    ComputeUnits units(h->dev, h->cus, h->res_g, h->res_g > 1);
     e = hipEventRecord(h->ev0, h->stream);
     if (e == hipSuccess)
       e = hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * 2 * h->res_g * RES_SLOT, h->stream);

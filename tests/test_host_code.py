@@ -82,3 +82,14 @@ def test_long_batches_take_several_launches(host):
         b.forward()
         assert fake.fake_launches(b"k_badj_resident") == 3
     """)
+
+
+def test_which_launches_run_together(tmp_path):
+    """Launches whose workgroups wait for one another and launches that only
+    hold compute units for long: who may enter beside whom, and in which order."""
+    exe = str(tmp_path / "units")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread",
+                    "-I" + os.path.join(ROOT, "hyperelasticsolver_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "units_host.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
