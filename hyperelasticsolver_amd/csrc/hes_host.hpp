@@ -6,7 +6,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <vector>
+#include <type_traits>
 
 #include "hes_device.hpp"
 #include "hes_units.hpp"
@@ -87,8 +87,8 @@ inline hipError_t zero_on(hipStream_t s, void* dst, size_t bytes) {
 // What a call works in: page-locked host memory that the kernels read and
 // write themselves (small calls: no copies), device memory (larger ones), and
 // a stream of its own.  Allocated for every call they cost one on a single
-// state 90 of its 100 us.  One per call that is under way; at most SPACES_KEPT
-// wait for the next, per device, with at most Space::DEVICE bytes each.
+// state 90 of its 100 us.  One per call that is under way; a few are kept for
+// the next, with at most Space::DEVICE bytes each.
 struct Space {
   static constexpr size_t HOST = 128 * 1024, DEVICE = 96 << 20;
   int dev = 0;
@@ -97,15 +97,43 @@ struct Space {
   size_t device_bytes = 0;
   hipStream_t stream = nullptr;
 };
-inline constexpr size_t SPACES_KEPT = 4;
-inline std::mutex& spaces_mutex() {
-  static std::mutex m;
-  return m;
+// What finished calls leave for the next ones, at most PER_DEVICE of it for each
+// device (T::dev).  A fixed array: taking and giving allocate nothing.
+template <class T, int PER_DEVICE>
+class Kept {
+ public:
+  bool take(int dev, T* t) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (int k = 0; k < n_; ++k)
+      if (kept_[k].dev == dev) {
+        *t = kept_[k];
+        kept_[k] = kept_[--n_];
+        return true;
+      }
+    return false;
+  }
+  bool give(const T& t) {  // false: there is enough of it
+    std::lock_guard<std::mutex> lock(mutex_);
+    int here = 0;
+    for (int k = 0; k < n_; ++k) here += kept_[k].dev == t.dev;
+    if (here == PER_DEVICE || n_ == ROOM) return false;
+    kept_[n_++] = t;
+    return true;
+  }
+
+ private:
+  static constexpr int ROOM = 8 * PER_DEVICE;
+  std::mutex mutex_;
+  T kept_[ROOM];
+  int n_ = 0;
+};
+using KeptSpaces = Kept<Space, 4>;
+inline KeptSpaces& spaces() {
+  static KeptSpaces s;
+  static_assert(std::is_trivially_destructible<KeptSpaces>::value, "outlives the runtime's own end");
+  return s;
 }
-inline std::vector<Space>& spaces() {
-  static auto* v = new std::vector<Space>();  // outlives the runtime's own end
-  return *v;
-}
+
 inline void space_free(Space& s) {
   if (s.stream) (void)hipStreamDestroy(s.stream);
   if (s.host) (void)hipHostFree(s.host);
@@ -115,16 +143,7 @@ inline hipError_t space_take(Space* s) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  {
-    std::lock_guard<std::mutex> lock(spaces_mutex());
-    auto& v = spaces();
-    for (size_t k = 0; k < v.size(); ++k)
-      if (v[k].dev == dev) {
-        *s = v[k];
-        v.erase(v.begin() + (long)k);
-        return hipSuccess;
-      }
-  }
+  if (spaces().take(dev, s)) return hipSuccess;
   s->dev = dev;
   e = hipHostMalloc((void**)&s->host, Space::HOST);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
@@ -135,18 +154,8 @@ inline hipError_t space_take(Space* s) {
   return e;
 }
 inline void space_give(Space& s, bool keep) {
-  if (keep && s.device_bytes <= Space::DEVICE) {
-    std::lock_guard<std::mutex> lock(spaces_mutex());
-    size_t here = 0;
-    for (const Space& o : spaces()) here += o.dev == s.dev;
-    if (here < SPACES_KEPT) {
-      spaces().push_back(s);
-      return;
-    }
-  }
-  space_free(s);
+  if (!keep || s.device_bytes > Space::DEVICE || !spaces().give(s)) space_free(s);
 }
-
 
 // Device memory of at least `bytes` in s (its contents are lost when it grows).
 inline hipError_t space_device(Space& s, size_t bytes) {

@@ -12,9 +12,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
-#include <vector>
 
 #include "hes_host.hpp"
 
@@ -48,7 +47,7 @@ inline hipError_t gather(const double* Q, double* out, int nc, long long first, 
 }
 
 // Page-locked pieces of memory with a stream each, for the threads of large
-// downloads; at most PIECES_KEPT wait for the next one, per device.
+// downloads; those of one download are kept for the next.
 struct Piece {
   static constexpr size_t BYTES = 4 << 20;
   int dev = 0;
@@ -56,26 +55,18 @@ struct Piece {
   hipStream_t stream = nullptr;
 };
 inline constexpr int DOWNLOAD_THREADS = 8;
-inline constexpr size_t PIECES_KEPT = DOWNLOAD_THREADS;
-inline std::vector<Piece>& pieces() {  // under spaces_mutex()
-  static auto* v = new std::vector<Piece>();
-  return *v;
+using KeptPieces = Kept<Piece, DOWNLOAD_THREADS>;
+inline KeptPieces& pieces() {
+  static KeptPieces p;
+  static_assert(std::is_trivially_destructible<KeptPieces>::value, "outlives the runtime's own end");
+  return p;
 }
 inline void piece_free(Piece& b) {
   if (b.stream) (void)hipStreamDestroy(b.stream);
   if (b.p) (void)hipHostFree(b.p);
 }
 inline hipError_t piece_take(int dev, Piece* b) {
-  {
-    std::lock_guard<std::mutex> lock(spaces_mutex());
-    auto& v = pieces();
-    for (size_t k = 0; k < v.size(); ++k)
-      if (v[k].dev == dev) {
-        *b = v[k];
-        v.erase(v.begin() + (long)k);
-        return hipSuccess;
-      }
-  }
+  if (pieces().take(dev, b)) return hipSuccess;
   b->dev = dev;
   hipError_t e = hipHostMalloc((void**)&b->p, Piece::BYTES);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
@@ -86,16 +77,7 @@ inline hipError_t piece_take(int dev, Piece* b) {
   return e;
 }
 inline void piece_give(Piece& b, bool keep) {
-  if (keep) {
-    std::lock_guard<std::mutex> lock(spaces_mutex());
-    size_t here = 0;
-    for (const Piece& o : pieces()) here += o.dev == b.dev;
-    if (here < PIECES_KEPT) {
-      pieces().push_back(b);
-      return;
-    }
-  }
-  piece_free(b);
+  if (!keep || !pieces().give(b)) piece_free(b);
 }
 
 // From this size on a download is shared by threads: below it their start and
@@ -147,14 +129,15 @@ inline hipError_t download_state(const double* Q, double* out, int nc, long long
     if (we != hipSuccess) failed.store((int)we);
     if (b.p) piece_give(b, we == hipSuccess);
   };
-  std::vector<std::thread> threads;
+  std::thread threads[DOWNLOAD_THREADS - 1];
   try {
     for (long long k = 1; k < std::min<long long>(DOWNLOAD_THREADS, parts); ++k)
-      threads.emplace_back(work);
-  } catch (const std::system_error&) {  // fewer threads share the work
+      threads[k - 1] = std::thread(work);
+  } catch (const std::exception&) {  // fewer threads share the work
   }
   work();
-  for (std::thread& t : threads) t.join();
+  for (std::thread& t : threads)
+    if (t.joinable()) t.join();
   return (hipError_t)failed.load();
 }
 

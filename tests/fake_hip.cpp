@@ -1,13 +1,15 @@
 // A HIP runtime on host memory, for tests of the library's host code without a
 // GPU: loaded before libhes.so, its functions stand in for the runtime's.
 // Device memory is host memory, a launch runs nothing except the kernels that
-// move a state in and out (named below), and allocations can be made to fail.
+// move a state in and out (named below), and allocations can be made to fail,
+// the library's own of host memory among them.
 #include <atomic>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 
 namespace {
@@ -19,6 +21,13 @@ std::map<void*, size_t> device;
 size_t device_used = 0, device_cap = ~(size_t)0, device_fail_min = ~(size_t)0;
 size_t host_fail_min = ~(size_t)0;
 long long host_allowed = 0;  // host allocations of at least host_fail_min that still succeed
+std::atomic<bool> new_fails{false};
+thread_local int inside = 0;  // this file's own allocations always succeed
+struct Lock {
+  std::lock_guard<std::mutex> lock{mutex};
+  Lock() { ++inside; }
+  ~Lock() { --inside; }
+};
 thread_local int last_error = OK;
 int result(int e) {
   if (e != OK) last_error = e;
@@ -35,8 +44,17 @@ struct Config {
 thread_local Config config;
 }  // namespace
 
+void* operator new(size_t n) {
+  void* p = new_fails && !inside ? nullptr : std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 extern "C" {
 // ---- what a test sets and reads
+void fake_new_fails(int on) { new_fails = on != 0; }  // the library's own allocations of host memory
 void fake_device_cap(size_t bytes) { device_cap = bytes; }
 void fake_device_fail_from(size_t bytes) { device_fail_min = bytes; }  // allocations this large fail
 void fake_host_fail_from(size_t bytes, long long allowed) {
@@ -44,7 +62,7 @@ void fake_host_fail_from(size_t bytes, long long allowed) {
   host_allowed = allowed;
 }
 long long fake_launches(const char* name) {  // of kernels whose name contains this
-  std::lock_guard<std::mutex> lock(mutex);
+  Lock lock;
   long long n = 0;
   for (auto& k : launches)
     if (k.first.find(name) != std::string::npos) n += k.second;
@@ -54,7 +72,7 @@ size_t fake_device_used() { return device_used; }
 
 // ---- the runtime
 int hipMalloc(void** p, size_t n) {
-  std::lock_guard<std::mutex> lock(mutex);
+  Lock lock;
   if (n >= device_fail_min || device_used + n > device_cap) return result(OUT_OF_MEMORY);
   *p = std::calloc(1, n ? n : 1);
   device[*p] = n;
@@ -62,7 +80,7 @@ int hipMalloc(void** p, size_t n) {
   return OK;
 }
 int hipFree(void* p) {
-  std::lock_guard<std::mutex> lock(mutex);
+  Lock lock;
   if (p) {
     device_used -= device[p];
     device.erase(p);
@@ -71,7 +89,7 @@ int hipFree(void* p) {
   return OK;
 }
 int hipHostMalloc(void** p, size_t n, unsigned) {
-  std::lock_guard<std::mutex> lock(mutex);
+  Lock lock;
   if (n >= host_fail_min && host_allowed-- <= 0) return result(OUT_OF_MEMORY);
   *p = std::calloc(1, n);
   return OK;
@@ -114,7 +132,7 @@ void** __hipRegisterFatBinary(const void*) {
 void __hipUnregisterFatBinary(void**) {}
 void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, void*,
                            void*, int*) {
-  std::lock_guard<std::mutex> lock(mutex);
+  Lock lock;
   kernels[f] = name;
 }
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
@@ -132,7 +150,7 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* shared, void** st
 int hipLaunchKernel(const void* f, Dim3, Dim3, void** a, size_t, void*) {
   std::string name;
   {
-    std::lock_guard<std::mutex> lock(mutex);
+    Lock lock;
     name = kernels[f];
     ++launches[name];
   }

@@ -93,3 +93,26 @@ def test_which_launches_run_together(tmp_path):
                     os.path.join(ROOT, "tests", "units_host.cpp"), "-o", exe], check=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+def test_no_exception_leaves_a_call(host):
+    """Calls on a handle and point-wise calls work, or report an error, when host
+    memory is short: nothing is thrown across the C interface."""
+    host("""
+    from hyperelasticsolver_amd.initial import prim2cons
+    n = 120000  # a download shared by threads
+    q = np.asfortranarray(np.arange(14.0 * n).reshape(14, n, order="F"))
+    out = np.empty_like(q)
+    with Solver(EOS, n) as s, Solver(EOS, 300000) as t, Batch([EOS] * 2, [900] * 2) as b:
+        t.set_state(np.ones((14, 300000), order="F"))
+        b.set_state(np.ones((14, 1800), order="F"))
+        fake.fake_new_fails(1)
+        s.set_state(q)
+        got = s.get_state()
+        prim2cons(EOS, q[:, :3])
+        s.run(steps=4)
+        t.run(steps=4)
+        b.run(4)
+        fake.fake_new_fails(0)
+        assert np.array_equal(got, q)
+    """)
