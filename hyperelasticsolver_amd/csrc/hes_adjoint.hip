@@ -965,7 +965,7 @@ hipError_t capture(hes_adjoint* h, bool fwd, hipGraphExec_t* out) {
 
 template <class T>
 hipError_t dalloc(T** p, size_t count) {
-  return hipMalloc((void**)p, sizeof(T) * (count > 0 ? count : 1));
+  return device_alloc(p, sizeof(T) * (count > 0 ? count : 1));
 }
 
 void drop_graphs(hes_adjoint* h) {

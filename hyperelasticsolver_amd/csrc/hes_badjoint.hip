@@ -1028,7 +1028,7 @@ hipError_t bcapture(hes_badjoint* h, bool fwd, hipGraphExec_t* out) {
 
 template <class T>
 hipError_t balloc(T** p, size_t count) {
-  return hipMalloc((void**)p, sizeof(T) * (count > 0 ? count : 1));
+  return device_alloc(p, sizeof(T) * (count > 0 ? count : 1));
 }
 
 void drop_graphs(hes_badjoint* h) {

@@ -735,10 +735,10 @@ hipError_t plan_batch_resident(hes_batch* h) {
   if (h->nph != 1) return hipSuccess;
   const BResPlan pl = bres_plan(h->offsets_h, h->cus, h->nc, h->flux == HES_FLUX_HLL, h->fast);
   if (pl.tiles == 0) return hipSuccess;
-  hipError_t e = hipMalloc((void**)&h->teams, sizeof(BResTeam) * pl.teams.size());
-  if (e == hipSuccess) e = hipMalloc((void**)&h->items, sizeof(BResItem) * pl.items.size());
-  if (e == hipSuccess) e = hipMalloc((void**)&h->res_out, sizeof(BResOut) * (size_t)h->P);
-  if (e == hipSuccess) e = hipMalloc((void**)&h->comm, sizeof(unsigned long long) * pl.words);
+  hipError_t e = device_alloc(&h->teams, sizeof(BResTeam) * pl.teams.size());
+  if (e == hipSuccess) e = device_alloc(&h->items, sizeof(BResItem) * pl.items.size());
+  if (e == hipSuccess) e = device_alloc(&h->res_out, sizeof(BResOut) * (size_t)h->P);
+  if (e == hipSuccess) e = device_alloc(&h->comm, sizeof(unsigned long long) * pl.words);
   if (e == hipSuccess)
     e = hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * pl.words, h->stream);
   if (e == hipSuccess)
@@ -935,11 +935,11 @@ int hes_batch_create(hes_batch** out, int nphase, int flux, int nproblems, const
     e = hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, h->dev);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   for (int b = 0; b < 2 && e == hipSuccess; ++b) {
-    e = hipMalloc(&h->Q[b], qb);
-    if (e == hipSuccess) e = hipMalloc(&h->C[b], cb);
+    e = device_alloc(&h->Q[b], qb);
+    if (e == hipSuccess) e = device_alloc(&h->C[b], cb);
   }
   auto up = [&](void** d, const void* src, size_t bytes) {
-    if (e == hipSuccess) e = hipMalloc(d, bytes);
+    if (e == hipSuccess) e = device_alloc(d, bytes);
     if (e == hipSuccess && src) e = copy_on(h->stream, *d, src, bytes, hipMemcpyHostToDevice);
   };
   std::vector<TileDesc> tdesc(tstart.size());
@@ -1010,7 +1010,7 @@ int hes_batch_set_state(hes_batch* h, const double* Q, const double* t0) {
   if (!h || !Q) return fail(HES_ERR_ARG, "null argument");
   size_t bytes = sizeof(double) * (size_t)h->nc * h->N;
   double* tmp = nullptr;
-  HIP_TRY(hipMalloc(&tmp, bytes));
+  HIP_TRY(device_alloc(&tmp, bytes));
   hipError_t e = copy_on(h->stream, tmp, Q, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_aos_to_soa_b, dim3((unsigned)((h->N + 255) / 256)), dim3(256), 0, h->stream,
@@ -1041,9 +1041,9 @@ int hes_batch_set_piecewise(hes_batch* h, const int* nstates, const double* stat
       if (!(interfaces[k] <= interfaces[k + 1])) return fail(HES_ERR_ARG, "interfaces not sorted");
   int *dso = nullptr;
   double *dst = nullptr, *dif = nullptr;
-  HIP_TRY(hipMalloc(&dso, sizeof(int) * (h->P + 1)));
-  hipError_t e = hipMalloc(&dst, sizeof(double) * (size_t)S * h->nc);
-  if (e == hipSuccess) e = hipMalloc(&dif, sizeof(double) * (size_t)(I > 0 ? I : 1));
+  HIP_TRY(device_alloc(&dso, sizeof(int) * (h->P + 1)));
+  hipError_t e = device_alloc(&dst, sizeof(double) * (size_t)S * h->nc);
+  if (e == hipSuccess) e = device_alloc(&dif, sizeof(double) * (size_t)(I > 0 ? I : 1));
   if (e == hipSuccess)
     e = copy_on(h->stream, dso, soff.data(), sizeof(int) * (h->P + 1), hipMemcpyHostToDevice);
   if (e == hipSuccess)
@@ -1201,12 +1201,12 @@ int hes_batch_autotune(hes_batch* h, int steps, int* best_block, int* best_xcd, 
   long long* pl0 = nullptr;
   const hipMemcpyKind dd = hipMemcpyDeviceToDevice;
   // every buffer is freed on every path: the first failure skips the rest
-  hipError_t e = hipMalloc(&q0, qb);
-  if (e == hipSuccess) e = hipMalloc(&c0, cb);
-  if (e == hipSuccess) e = hipMalloc(&t0, sizeof(double) * 2 * h->P);
-  if (e == hipSuccess) e = hipMalloc(&sl0, sizeof(unsigned long long) * 3 * h->P);
-  if (e == hipSuccess) e = hipMalloc(&ps0, sizeof(int) * h->P);
-  if (e == hipSuccess) e = hipMalloc(&pl0, sizeof(long long) * h->P);
+  hipError_t e = device_alloc(&q0, qb);
+  if (e == hipSuccess) e = device_alloc(&c0, cb);
+  if (e == hipSuccess) e = device_alloc(&t0, sizeof(double) * 2 * h->P);
+  if (e == hipSuccess) e = device_alloc(&sl0, sizeof(unsigned long long) * 3 * h->P);
+  if (e == hipSuccess) e = device_alloc(&ps0, sizeof(int) * h->P);
+  if (e == hipSuccess) e = device_alloc(&pl0, sizeof(long long) * h->P);
   if (e == hipSuccess) e = copy_on(h->stream, q0, h->Q[s0 & 1], qb, dd);
   if (e == hipSuccess) e = copy_on(h->stream, c0, h->C[s0 & 1], cb, dd);
   if (e == hipSuccess) e = copy_on(h->stream, t0, h->tring, sizeof(double) * 2 * h->P, dd);

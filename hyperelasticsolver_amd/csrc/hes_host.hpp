@@ -120,6 +120,11 @@ class Kept {
     kept_[n_++] = t;
     return true;
   }
+  template <class F>
+  void each(F f) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (int k = 0; k < n_; ++k) f(kept_[k]);
+  }
 
  private:
   static constexpr int ROOM = 8 * PER_DEVICE;
@@ -132,6 +137,24 @@ inline KeptSpaces& spaces() {
   static KeptSpaces s;
   static_assert(std::is_trivially_destructible<KeptSpaces>::value, "outlives the runtime's own end");
   return s;
+}
+
+// Device memory.  Where it is short, that of kept spaces is given back first.
+template <class T>
+hipError_t device_alloc(T** p, size_t bytes) {
+  hipError_t e = hipMalloc((void**)p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  bool freed = false;
+  spaces().each([&](Space& s) {
+    if (!s.device) return;
+    freed = true;
+    (void)hipFree(s.device);
+    s.device = nullptr;
+    s.device_bytes = 0;
+  });
+  if (!freed) return e;
+  (void)hipGetLastError();  // of the first attempt
+  return hipMalloc((void**)p, bytes);
 }
 
 inline void space_free(Space& s) {
@@ -163,7 +186,7 @@ inline hipError_t space_device(Space& s, size_t bytes) {
   hipError_t e = s.device ? hipFree(s.device) : hipSuccess;
   s.device = nullptr;
   s.device_bytes = 0;
-  if (e == hipSuccess) e = hipMalloc((void**)&s.device, bytes);
+  if (e == hipSuccess) e = device_alloc(&s.device, bytes);
   if (e == hipSuccess) s.device_bytes = bytes;
   return e;
 }

@@ -957,15 +957,15 @@ int hes_solver_create(hes_solver** out, int nphase, int flux, long long ncells,
   size_t cbytes = sizeof(double) * (size_t)nphase * (size_t)h->pitch;
   hipError_t e = hipSuccess;
   for (int b = 0; b < 2 && e == hipSuccess; ++b) {
-    e = hipMalloc(&h->Q[b], qbytes);
-    if (e == hipSuccess) e = hipMalloc(&h->C[b], cbytes);
+    e = device_alloc(&h->Q[b], qbytes);
+    if (e == hipSuccess) e = device_alloc(&h->C[b], cbytes);
   }
-  if (e == hipSuccess && nphase == 2) e = hipMalloc(&h->dpath, 2 * qbytes);  // D-, D+ rows
-  if (e == hipSuccess && nphase == 2) e = hipMalloc(&h->jlist, sizeof(long long) * (size_t)ncells);
+  if (e == hipSuccess && nphase == 2) e = device_alloc(&h->dpath, 2 * qbytes);  // D-, D+ rows
+  if (e == hipSuccess && nphase == 2) e = device_alloc(&h->jlist, sizeof(long long) * (size_t)ncells);
   // the small words in one allocation: CFL ring, time ring, jump-face counts,
   // status, then the team's messages, each on a line of its own
   const size_t words = 4 * 16 + (h->shape.block ? res_words_of(h->res_g, h->nc) : 0);
-  if (e == hipSuccess) e = hipMalloc(&h->slots, sizeof(unsigned long long) * words);
+  if (e == hipSuccess) e = device_alloc(&h->slots, sizeof(unsigned long long) * words);
   if (e == hipSuccess) {
     h->tring = (double*)(h->slots + 16);
     if (nphase == 2) h->jcnt = h->slots + 32;
@@ -1152,7 +1152,7 @@ int hes_solver_run(hes_solver* h, long long max_steps, double t_end, int use_gra
       if (h->dt_hist) HIP_TRY(hipFree(h->dt_hist));
       h->dt_hist = nullptr;
       h->dt_cap = 0;
-      HIP_TRY(hipMalloc(&h->dt_hist, sizeof(double) * (size_t)(max_steps > 0 ? max_steps : 1)));
+      HIP_TRY(device_alloc(&h->dt_hist, sizeof(double) * (size_t)(max_steps > 0 ? max_steps : 1)));
       h->dt_cap = max_steps;
     }
   }
@@ -1253,8 +1253,8 @@ int hes_copy_bandwidth(long long bytes, int reps, double* gbs) {
   const long long nblocks = (n + 255) / 256;
   if (nblocks > 0x7fffffffLL) return fail(HES_ERR_ARG, "copy size too large");
   double *a = nullptr, *b = nullptr;
-  HIP_TRY(hipMalloc(&a, n * 8));
-  hipError_t e = hipMalloc(&b, n * 8);
+  HIP_TRY(device_alloc(&a, n * 8));
+  hipError_t e = device_alloc(&b, n * 8);
   hipEvent_t e0, e1;
   if (e == hipSuccess) e = hipMemset(a, 0, n * 8);
   if (e == hipSuccess) e = hipEventCreate(&e0);

@@ -116,3 +116,32 @@ def test_no_exception_leaves_a_call(host):
         fake.fake_new_fails(0)
         assert np.array_equal(got, q)
     """)
+
+
+def test_kept_memory_is_given_back_when_it_is_short(host):
+    """Device memory that finished calls left for the next ones does not make a
+    later allocation fail."""
+    host("""
+    q = np.ones((14, 100000), order="F")
+    with Solver(EOS, 100000) as s:
+        s.set_state(q)
+    kept = fake.fake_device_used()
+    assert 0 < kept <= 4 * 96 << 20
+    for make in (lambda: Solver(EOS, 50000), lambda: Batch([EOS], [50000]), lambda: Adjoint(EOS, 50000, 4),
+                 lambda: BatchAdjoint([EOS], [50000], 4)):
+        with make():  # its size
+            need = fake.fake_device_used() - kept
+        fake.fake_device_cap(need + kept // 2)
+        make().close()
+        assert fake.fake_device_used() < kept
+        fake.fake_device_cap(NONE)
+        with Solver(EOS, 100000) as s:
+            s.set_state(q)
+        assert fake.fake_device_used() == kept
+    fake.fake_device_cap(kept + 1000)
+    try:
+        Solver(EOS, 100000)
+        assert False
+    except HesError as e:
+        assert "out of memory" in str(e)
+    """)
