@@ -84,44 +84,57 @@ inline void piece_give(Piece& b, bool keep) {
 // the pieces' faults cost what they save.
 constexpr size_t DOWNLOAD_SHARED_MIN = 6 << 20;
 
+// Cells [first, first + cells) of the rows into `out` by way of a space's memory.
+inline hipError_t download_plain(const double* Q, double* out, int nc, long long first,
+                                 long long cells, long long pitch) {
+  const size_t bytes = sizeof(double) * (size_t)nc * (size_t)cells;
+  Space s;
+  hipError_t e = space_take(&s);
+  if (e != hipSuccess) return e;
+  const bool small = bytes <= Space::HOST;
+  if (!small) e = space_device(s, bytes);
+  double* at = (double*)(small ? s.host : s.device);
+  if (e == hipSuccess) e = gather(Q, at, nc, first, cells, pitch, s.stream);
+  if (e == hipSuccess && !small) e = hipMemcpyAsync(out, at, bytes, hipMemcpyDeviceToHost, s.stream);
+  const hipError_t es = hipStreamSynchronize(s.stream);
+  if (e == hipSuccess) e = es;
+  if (e == hipSuccess && small) std::memcpy(out, at, bytes);
+  space_give(s, e == hipSuccess);
+  return e;
+}
+
 // The n states of rows Q (written by work that has been waited for) into `out`.
 inline hipError_t download_state(const double* Q, double* out, int nc, long long n,
                                  long long pitch) {
   const size_t bytes = sizeof(double) * (size_t)nc * (size_t)n;
+  if (bytes < DOWNLOAD_SHARED_MIN) return download_plain(Q, out, nc, 0, n, pitch);
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  if (bytes < DOWNLOAD_SHARED_MIN) {
-    Space s;
-    e = space_take(&s);
-    if (e != hipSuccess) return e;
-    const bool small = bytes <= Space::HOST;
-    if (!small) e = space_device(s, bytes);
-    double* at = (double*)(small ? s.host : s.device);
-    if (e == hipSuccess) e = gather(Q, at, nc, 0, n, pitch, s.stream);
-    if (e == hipSuccess && !small) e = hipMemcpyAsync(out, at, bytes, hipMemcpyDeviceToHost, s.stream);
-    const hipError_t es = hipStreamSynchronize(s.stream);
-    if (e == hipSuccess) e = es;
-    if (e == hipSuccess && small) std::memcpy(out, at, bytes);
-    space_give(s, e == hipSuccess);
-    return e;
-  }
   // cells of a piece: a share of a small state, a whole piece of a large one
   const size_t piece = std::max<size_t>(std::min(Piece::BYTES, bytes / DOWNLOAD_THREADS), 1 << 20);
   const long long per = (long long)(piece / (sizeof(double) * nc));
   const long long parts = (n + per - 1) / per;
   std::atomic<long long> next{0};
   std::atomic<int> failed{(int)hipSuccess};
-  auto work = [&]() {
+  // page_locked: a thread without a piece leaves its share to the others
+  auto work = [&](bool page_locked) {
     Piece b;
     hipError_t we = hipSetDevice(dev);
-    if (we == hipSuccess) we = piece_take(dev, &b);
+    if (we == hipSuccess && page_locked && piece_take(dev, &b) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
     while (we == hipSuccess && failed.load() == (int)hipSuccess) {
       const long long k = next.fetch_add(1);
       if (k >= parts) break;
       const long long c0 = k * per, cells = std::min(per, n - c0);
+      if (!page_locked) {
+        we = download_plain(Q, out + c0 * nc, nc, c0, cells, pitch);
+        continue;
+      }
       we = gather(Q, (double*)b.p, nc, c0, cells, pitch, b.stream);
-      const hipError_t es = b.stream ? hipStreamSynchronize(b.stream) : hipSuccess;
+      const hipError_t es = hipStreamSynchronize(b.stream);
       if (we == hipSuccess) we = es;
       if (we == hipSuccess)
         std::memcpy(out + c0 * nc, b.p, sizeof(double) * (size_t)nc * (size_t)cells);
@@ -132,12 +145,13 @@ inline hipError_t download_state(const double* Q, double* out, int nc, long long
   std::thread threads[DOWNLOAD_THREADS - 1];
   try {
     for (long long k = 1; k < std::min<long long>(DOWNLOAD_THREADS, parts); ++k)
-      threads[k - 1] = std::thread(work);
+      threads[k - 1] = std::thread(work, true);
   } catch (const std::exception&) {  // fewer threads share the work
   }
-  work();
+  work(true);
   for (std::thread& t : threads)
     if (t.joinable()) t.join();
+  work(false);  // what is left when no thread had a piece
   return (hipError_t)failed.load();
 }
 

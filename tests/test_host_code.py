@@ -118,6 +118,21 @@ def test_no_exception_leaves_a_call(host):
     """)
 
 
+def test_state_comes_back_without_page_locked_pieces(host):
+    """A large state's download takes page-locked memory for every thread: with
+    some of it, or none, the state still comes back."""
+    host("""
+    n = 120000  # 13 MB: several pieces
+    q = np.asfortranarray(np.arange(14.0 * n).reshape(14, n, order="F"))
+    for allowed in (0, 1, 3, 10 ** 6):
+        fake.fake_host_fail_from(1 << 20, allowed)
+        with Solver(EOS, n) as s:
+            s.set_state(q)
+            assert np.array_equal(s.get_state(), q), allowed
+            assert np.array_equal(s.get_state(), q), allowed
+    """)
+
+
 def test_kept_memory_is_given_back_when_it_is_short(host):
     """Device memory that finished calls left for the next ones does not make a
     later allocation fail."""
