@@ -1044,7 +1044,6 @@ int hes_adjoint_create(hes_adjoint** out, long long ncells, const double* materi
   if (e == hipSuccess) e = dalloc(&h->rho_t, P);
   if (e == hipSuccess) e = dalloc(&h->u_t, P);
   if (e == hipSuccess) e = dalloc(&h->status, 4);
-  if (e == hipSuccess && h->res.shape.block) e = dalloc(&h->comm, (size_t)comm_words(h));
   if (e == hipSuccess) e = zero_on(h->stream, h->status, 4 * sizeof(int));
   if (e == hipSuccess) {
     // gin = (b0, c0, rho0, cv, t0): the inputs of the generated routines
@@ -1062,6 +1061,13 @@ int hes_adjoint_create(hes_adjoint** out, long long ncells, const double* materi
     if (e == hipSuccess)
       e = copy_on(h->stream, h->slots, sl.data(), sizeof(double*) * sl.size(),
                   hipMemcpyHostToDevice);
+  }
+  if (e == hipSuccess && h->res.shape.block) {
+    e = dalloc(&h->comm, (size_t)comm_words(h));
+    if (no_room(e)) {  // then a launch per step
+      h->plan = h->res = {{0, 0}, 0, 0};
+      e = hipSuccess;
+    }
   }
   if (e != hipSuccess) {
     g_err = std::string("adjoint allocation failed: ") + hipGetErrorString(e);

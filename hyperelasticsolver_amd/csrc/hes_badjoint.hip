@@ -1156,15 +1156,6 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
   up(&h->gmat, nullptr, 2 * (size_t)nproblems);
   up(&h->status, nullptr, 4);
   up(&h->segs, segs.data(), segs.size());
-  if (pl.tiles) {
-    up(&h->teams, pl.teams.data(), pl.teams.size());
-    up(&h->items, pl.items.data(), pl.items.size());
-    up(&h->comm, nullptr, pl.words);
-    h->plan_tiles = h->res_tiles = pl.tiles;
-    h->res_groups = (int)pl.items.size();
-    h->res_waits = pl.waits;
-    h->res_words = pl.words;
-  }
   if (e == hipSuccess) e = zero_on(h->stream, h->status, 4 * sizeof(int));
   if (e == hipSuccess) {
     std::vector<double*> sl;
@@ -1173,6 +1164,24 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
     sl.push_back(h->fq[1]);
     h->nslots = (int)sl.size();
     up(&h->slots, sl.data(), sl.size());
+  }
+  if (e == hipSuccess && pl.tiles) {
+    up(&h->teams, pl.teams.data(), pl.teams.size());
+    up(&h->items, pl.items.data(), pl.items.size());
+    up(&h->comm, nullptr, pl.words);
+    if (no_room(e)) {  // then a launch per step
+      void** mine[] = {(void**)&h->teams, (void**)&h->items, (void**)&h->comm};
+      for (void** p : mine) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+      }
+      e = hipSuccess;
+    } else {
+      h->plan_tiles = h->res_tiles = pl.tiles;
+      h->res_groups = (int)pl.items.size();
+      h->res_waits = pl.waits;
+      h->res_words = pl.words;
+    }
   }
   if (e != hipSuccess) {
     g_err = std::string("batched adjoint allocation failed: ") + hipGetErrorString(e);

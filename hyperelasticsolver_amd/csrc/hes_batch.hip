@@ -729,6 +729,8 @@ int batch_carry(hes_batch* h) {
 
 // ---- the whole loop in one launch ------------------------------------------------
 
+// Its teams and message buffer (7 KB per workgroup, at the end of a creation);
+// without room for them the batch takes a launch per step.
 hipError_t plan_batch_resident(hes_batch* h) {
   h->plan_tiles = h->res_tiles = 0;
   h->res_wait = res_ticks(RES_WAIT_US);
@@ -739,6 +741,14 @@ hipError_t plan_batch_resident(hes_batch* h) {
   if (e == hipSuccess) e = device_alloc(&h->items, sizeof(BResItem) * pl.items.size());
   if (e == hipSuccess) e = device_alloc(&h->res_out, sizeof(BResOut) * (size_t)h->P);
   if (e == hipSuccess) e = device_alloc(&h->comm, sizeof(unsigned long long) * pl.words);
+  if (no_room(e)) {
+    void** mine[] = {(void**)&h->teams, (void**)&h->items, (void**)&h->res_out, (void**)&h->comm};
+    for (void** p : mine) {
+      if (*p) (void)hipFree(*p);
+      *p = nullptr;
+    }
+    return hipSuccess;
+  }
   if (e == hipSuccess)
     e = hipMemsetAsync(h->comm, 0, sizeof(unsigned long long) * pl.words, h->stream);
   if (e == hipSuccess)

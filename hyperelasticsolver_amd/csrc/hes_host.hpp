@@ -157,6 +157,13 @@ hipError_t device_alloc(T** p, size_t bytes) {
   return hipMalloc((void**)p, bytes);
 }
 
+// After an allocation that can be done without: whether there was no room for it.
+inline bool no_room(hipError_t e) {
+  if (e != hipErrorOutOfMemory) return false;
+  (void)hipGetLastError();
+  return true;
+}
+
 inline void space_free(Space& s) {
   if (s.stream) (void)hipStreamDestroy(s.stream);
   if (s.host) (void)hipHostFree(s.host);

@@ -964,8 +964,15 @@ int hes_solver_create(hes_solver** out, int nphase, int flux, long long ncells,
   if (e == hipSuccess && nphase == 2) e = device_alloc(&h->jlist, sizeof(long long) * (size_t)ncells);
   // the small words in one allocation: CFL ring, time ring, jump-face counts,
   // status, then the team's messages, each on a line of its own
-  const size_t words = 4 * 16 + (h->shape.block ? res_words_of(h->res_g, h->nc) : 0);
-  if (e == hipSuccess) e = device_alloc(&h->slots, sizeof(unsigned long long) * words);
+  size_t words = 4 * 16 + (h->shape.block ? res_words_of(h->res_g, h->nc) : 0);
+  if (e == hipSuccess) {
+    e = device_alloc(&h->slots, sizeof(unsigned long long) * words);
+    if (h->shape.block && no_room(e)) {  // then a launch per step
+      h->plan = h->shape = {0, 0};
+      words = 4 * 16;
+      e = device_alloc(&h->slots, sizeof(unsigned long long) * words);
+    }
+  }
   if (e == hipSuccess) {
     h->tring = (double*)(h->slots + 16);
     if (nphase == 2) h->jcnt = h->slots + 32;

@@ -160,3 +160,23 @@ def test_kept_memory_is_given_back_when_it_is_short(host):
     except HesError as e:
         assert "out of memory" in str(e)
     """)
+
+
+def test_no_room_for_the_messages_of_a_team(host):
+    """The buffers of a one-launch time loop can be done without: a handle that
+    has room for everything else is created and takes a launch per step."""
+    host("""
+    n = 300000
+    for make in (lambda: Solver(EOS, n), lambda: Solver((EOS, EOS), 20000, flux="hll"),
+                 lambda: Batch([EOS] * 40, [5000] * 40), lambda: Adjoint(EOS, n, 4, every=2),
+                 lambda: BatchAdjoint([EOS] * 40, [5000] * 40, 4, every=2)):
+        fake.fake_device_cap(NONE)
+        with make() as h:
+            assert h.team() > 0
+            size = fake.fake_device_used()
+        assert fake.fake_device_used() == 0
+        fake.fake_device_cap(size - 1000)
+        with make() as h:
+            assert h.team() == 0 and h.team(1000) == 0
+        assert fake.fake_device_used() == 0
+    """)
