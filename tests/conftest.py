@@ -25,3 +25,23 @@ def pytest_collection_modifyitems(config, items):
 def ora():
     import oracle_bind
     return oracle_bind.load()
+
+
+@pytest.fixture(params=["one launch", "launch per step"])
+def route(request, monkeypatch):
+    """Both routes of a time loop that fits the chip: the launch that takes all
+    steps, and (for every handle the test makes) a launch per step."""
+    if request.param == "one launch":
+        return
+    from hyperelasticsolver_amd.adjoint import Adjoint, BatchAdjoint
+    from hyperelasticsolver_amd.batched import Batch
+    from hyperelasticsolver_amd.solver import Solver
+
+    def per_step(init):
+        def make(self, *args, **kw):
+            init(self, *args, **kw)
+            assert self.team(-1) == 0
+        return make
+
+    for kind in (Solver, Batch, Adjoint, BatchAdjoint):
+        monkeypatch.setattr(kind, "__init__", per_step(kind.__init__))

@@ -63,6 +63,7 @@ def _build(ora, ncells, nph=1, flux="rusanov", seed=0):
 NCELLS = [3, 61, 62, 63, 64, 124, 125, 200, 517]
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("flux", ["rusanov", "hll"])
 def test_batch_equals_single_problem_runs(ora, flux):
     from hyperelasticsolver_amd.solver import Solver
@@ -84,11 +85,13 @@ def test_batch_equals_single_problem_runs(ora, flux):
         assert np.array_equal(Qb[:, b.offsets[p]:b.offsets[p + 1]], Qs), f"problem {p}"
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("flux,fk", [("rusanov", 0), ("hll", 1)])
 def test_batch_over_two_to_the_21_cells(ora, flux, fk):
     """A whole-batch launch over 2^21 cells or more takes the pinned schedule
     (four waves per SIMD); one-problem launches (mode "loop") take the other.
-    Both must give the same bits, and the oracle the same states to 1e-10."""
+    Both, and one launch for all steps, must give the same bits, and the oracle
+    the same states to 1e-10."""
     from hyperelasticsolver_amd.solver import materials_array
     rng = np.random.default_rng(21)
     ncells = [int(n) for n in rng.integers(40000, 52000, 48)]
@@ -115,6 +118,7 @@ def test_batch_over_two_to_the_21_cells(ora, flux, fk):
         assert so == steps and np.all(err <= TOL), (p, err.max())
 
 
+@pytest.mark.usefixtures("route")
 def test_large_problems_in_a_batch_equal_single_problem_runs(ora):
     """Problems above 65536 cells max their CFL speeds into the slot only when
     the slot holds a smaller one; smaller problems always issue the atomic.
@@ -217,6 +221,7 @@ def test_two_phase_batch_equals_single_problem_runs(ora, flux):
             assert np.array_equal(Qb[:, offs[p]:offs[p + 1]], Qs), f"problem {p}"
 
 
+@pytest.mark.usefixtures("route")
 def test_batch_modes_agree_and_autotune_restores(ora):
     print("[batch] modes + autotune", flush=True)
     ncells = [70, 5, 300, 1000, 62]
@@ -235,10 +240,12 @@ def test_batch_modes_agree_and_autotune_restores(ora):
         assert np.array_equal(s, res[0][1][1])
 
 
+@pytest.mark.usefixtures("route")
 def test_every_launch_shape_gives_the_same_bits(ora):
     """Block size, XCD block order and tiles per wave (each wave stepping
     through its tiles in turn) change only the schedule: every shape gives the
-    bits of the default one, eager and graph-replayed."""
+    bits of the default one, eager and graph-replayed.  (Where a graph run is
+    one launch for all steps, the shapes do not enter it.)"""
     print("[batch] launch shapes", flush=True)
     ncells = [70, 5, 300, 1000, 62, 2500, 63, 64]
     ref = None
@@ -259,6 +266,7 @@ def test_every_launch_shape_gives_the_same_bits(ora):
             assert np.array_equal(out[1][0], ref[1][0]) and np.array_equal(out[1][1], ref[1][1])
 
 
+@pytest.mark.usefixtures("route")
 def test_batch_per_problem_t_end(ora):
     print("[batch] per-problem t_end", flush=True)
     ncells = [100, 200]
@@ -346,6 +354,7 @@ def _pieces(ora, rng, eos, nph, k):
     return ora.prim2cons(nph, mats, P), np.sort(rng.uniform(0.1, 0.9, k - 1))
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("nph,flux,mode", [(1, "rusanov", "graph"), (1, "hll", "eager"),
                                            (1, "rusanov", "loop"), (2, "rusanov", "graph")])
 def test_stopped_problems_keep_their_state_and_resume(ora, nph, flux, mode):

@@ -21,7 +21,7 @@ from scipy.optimize import brentq
 
 from test_gpu_solver import MAT_AL, MAT_CU, _piecewise, _rand_two_phase, _two_phase_eos
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("route")]
 
 
 def _pressures(ora, mats, Q):

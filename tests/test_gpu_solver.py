@@ -78,6 +78,7 @@ def _gpu_run(nph, mats, flux, Q0, steps, use_graph=False, t_end=math.inf):
     return Q, r
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("nph,flux,nx,steps,nstates", [
     (1, "rusanov", 300, 60, 4),
     (1, "hll", 300, 60, 4),
@@ -104,6 +105,7 @@ MAT_ALT = np.array([8.93, 6.22, 9.0e-4, 300.0, 3.16, 1.0, 3.577, 2.088])   # mai
 MAT_ALT2 = np.array([2.7, 6.22, 9.0e-4, 300.0, 3.1, 1.0, 3.577, 2.088])
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("nph,flux", [(1, "rusanov"), (1, "hll"), (1, "lxf"),
                                       (2, "rusanov"), (2, "hll"), (2, "lxf")])
 def test_step_parity_general_exponents(ora, nph, flux):
@@ -130,8 +132,10 @@ def test_step_parity_general_exponents(ora, nph, flux):
     np.testing.assert_allclose(r["dt"], dto, rtol=TOL, atol=0)
 
 
+@pytest.mark.usefixtures("route")
 def test_graph_equals_eager(ora):
-    """The hipGraph replay path gives bit-identical states to eager launches."""
+    """The hipGraph replay path (of a launch per step) gives bit-identical
+    states to eager launches."""
     print("[graph] single-phase hll nx=500 steps=125", flush=True)
     mats, Q0, _, _ = _problem(ora, 1, 500, 5, seed=7)
     Qa, ra = _gpu_run(1, mats, "hll", Q0, 125, use_graph=False)
@@ -141,6 +145,7 @@ def test_graph_equals_eager(ora):
     assert ra["t"] == rb["t"]
 
 
+@pytest.mark.usefixtures("route")
 def test_t_end_stops_like_reference(ora):
     """`while t < T` (main.jl:202): same number of steps and same final time."""
     print("[t_end] single-phase rusanov nx=200 T=0.01", flush=True)
@@ -153,6 +158,7 @@ def test_t_end_stops_like_reference(ora):
         assert np.all(rel_err_per_component(Qg, Qo) <= TOL)
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("nph", [1, 2])
 def test_uniform_state_is_bit_invariant(ora, nph):
     """F(Q) - F(Q) = 0 exactly: a uniform state never changes (a known answer of
@@ -169,6 +175,7 @@ def test_uniform_state_is_bit_invariant(ora, nph):
             assert np.array_equal(Qg, Q0), (k, flux)
 
 
+@pytest.mark.usefixtures("route")
 def test_conservation_telescopes(ora):
     """Mass, momentum and energy change only by the frozen end cells' fluxes:
     with identical end states the totals are conserved to round-off."""
@@ -184,6 +191,7 @@ def test_conservation_telescopes(ora):
         assert np.all(np.abs(tot1 - tot0) <= 1e-13 * scale + 1e-300), (tot1 - tot0) / scale
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("flux", ["rusanov", "hll", "lxf"])
 def test_parity_many_blocks(ora, flux):
     """2^16 cells: ~1000 blocks spread over all XCDs, so the CFL max-reduction
@@ -254,6 +262,7 @@ def test_pinned_rusanov_speeds_are_formed_on_request(ora):
     assert moved.sum() > 100 and np.any(c1[0, moved] != c0[0, moved])
 
 
+@pytest.mark.usefixtures("route")
 def test_step_sound_speeds_against_lapack(ora):
     """The step's sound speed of a cell, sqrt of the acoustic tensor's
     eigenvalue of largest modulus (the shifted characteristic cubic, with
@@ -289,6 +298,7 @@ def test_step_sound_speeds_against_lapack(ora):
     assert err.max() <= 1e-12, (err.max(), int(err.argmax()))
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("name,flux", [("config1_rusanov", "rusanov"), ("config1_hll", "hll")])
 def test_golden_config1_full_run(name, flux):
     """1000-cell Riemann problem run to t_end = 0.06 (701 steps) against the
@@ -305,6 +315,7 @@ def test_golden_config1_full_run(name, flux):
     assert abs(r["t"] - float(g["t"])) <= TOL * float(g["t"])
 
 
+@pytest.mark.usefixtures("route")
 def test_golden_testcase6():
     """HyperelasticityMPh test case 6 (main.jl's own two-phase case) with HLL."""
     import os
@@ -323,6 +334,7 @@ def _two_phase_eos(mats):
     return mk(mats[:8]), mk(mats[8:])
 
 
+@pytest.mark.usefixtures("route")
 def test_relaxation_decays_relative_velocity_exactly(ora):
     """Velocity relaxation (an optional source; parity unpinned, the reference
     has none).  On a uniform state the fluxes cancel exactly, so only the
@@ -357,6 +369,7 @@ def test_relaxation_decays_relative_velocity_exactly(ora):
     assert np.array_equal(Q[:, [0, nx - 1]], Q0[:, [0, nx - 1]])
 
 
+@pytest.mark.usefixtures("route")
 def test_relaxation_off_is_the_plain_step_and_conserves(ora):
     """tau = inf gives the source-free step bit for bit; with a finite tau a
     two-phase Riemann run keeps mixture momentum and total energy telescoping."""
@@ -387,6 +400,7 @@ def test_relaxation_off_is_the_plain_step_and_conserves(ora):
         assert abs(t1 - t0) <= 1e-12 * np.abs(Q0[rows]).sum(), rows
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("flux", ["rusanov", "hll"])
 def test_two_phase_every_face_jumps(ora, flux):
     """A tanh volume-fraction profile (main.jl:110-123) makes every face a
@@ -473,6 +487,7 @@ def _mph_eos_pair():
     return Barton2009(), Barton2009()
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("case", [1, 2, 3])
 def test_reference_uniform_test_cases_stay_bit_identical(case):
     """HyperelasticityMPh test cases 1, 2 and 3 (HyperelasticityMPh.jl:276-311)
@@ -491,6 +506,7 @@ def test_reference_uniform_test_cases_stay_bit_identical(case):
         assert np.array_equal(Qg, Q0), flux
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("case", [4, 5])
 def test_test_cases_4_5_are_half_the_single_phase_run(case):
     """Test cases 4 and 5 hold two identical phases at a = 1/2
@@ -515,6 +531,7 @@ def test_test_cases_4_5_are_half_the_single_phase_run(case):
             assert np.all(err <= 1e-12), (flux, p, err.max())
 
 
+@pytest.mark.usefixtures("route")
 def test_moving_volume_fraction_contact_keeps_the_primitives(ora):
     """Test case 10 (HyperelasticityMPh.jl:389-408): both phases and both sides
     share u, F and S, and only the volume fractions jump (0.4/0.6 | 0.6/0.4).
@@ -547,6 +564,7 @@ def test_moving_volume_fraction_contact_keeps_the_primitives(ora):
         assert Qg[0].sum() - Q0[0].sum() == pytest.approx(want, rel=1e-11)
 
 
+@pytest.mark.usefixtures("route")
 def test_volume_fractions_keep_summing_to_one(ora):
     """a1 + a2 = 1 is kept: both phases' volume-fraction rows see the same face
     speed and the same u_I with opposite jumps."""
@@ -559,6 +577,7 @@ def test_volume_fractions_keep_summing_to_one(ora):
         assert np.abs(Qg[0] + Qg[15] - 1.0).max() <= 1e-13, flux
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("live,use_graph", [(12, False), (59, True)])
 def test_two_phase_run_resumed_after_one_no_op_step(ora, live, use_graph):
     """A run whose last launched step is a no-op (t >= t_end) and a run that
