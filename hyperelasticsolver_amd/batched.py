@@ -4,10 +4,10 @@ Each problem has its own length, materials, CFL number and dx, hence its own
 time step (main.jl:204-214 applied per problem).  The state of all problems is
 packed (ncomp x total cells, problems one after another) and lives on the GPU.
 `run(steps, mode="graph")` runs the whole step loop at once: in one launch
-(one phase, problems that fit the chip) or as one captured hipGraph;
-`mode="eager"` takes one launch per step;
+(one phase, problems that fit the chip, where it is the faster: see `team`) or
+as one captured hipGraph; `mode="eager"` takes one launch per step;
 `mode="loop"` is the one-problem-per-launch baseline; `autotune()` picks the
-launch shape by timing each candidate on the actual problem set.
+shape of a launch per step by timing each candidate on the actual problem set.
 """
 import ctypes
 
@@ -111,8 +111,9 @@ class Batch:
         check(lib().hes_batch_set_t_end(self._h, None if v is None else ptr(v)))
 
     def set_launch(self, block=256, xcd=True, tiles_per_wave=1):
-        """Launch shape: block of 64 or 256 threads, XCD-contiguous block order,
-        and tiles of 62 cells each wave takes in turn."""
+        """Shape of a launch per step: block of 64 or 256 threads, XCD-contiguous
+        block order, and tiles of 62 cells each wave takes in turn.  It does not
+        enter a `graph` run in one launch."""
         check(lib().hes_batch_set_launch(self._h, int(block), 1 if xcd else 0, int(tiles_per_wave)))
 
     def run(self, steps, mode="graph"):
@@ -129,8 +130,9 @@ class Batch:
         return team(lib().hes_batch_team, self._h, wait_us)
 
     def autotune(self, steps=3):
-        """Time every launch shape (block, XCD order, tiles per wave) on the
-        current state, restore the state and keep the fastest."""
+        """Time every shape of a launch per step (block, XCD order, tiles per wave)
+        on the current state, restore the state and keep the fastest.  It does
+        not enter a `graph` run in one launch."""
         b = ctypes.c_int()
         x = ctypes.c_int()
         w = ctypes.c_int()

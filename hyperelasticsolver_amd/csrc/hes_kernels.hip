@@ -782,9 +782,9 @@ constexpr long long RES_STEPS = 1LL << 16;  // steps of one launch at most
 // together around the interfaces, so a wave with 64 cells may work on all its
 // faces in turn while most of the chip has none; one launch per step spreads
 // them evenly.  us per step once the interfaces have spread, that against
-// this: HLL, 1000 cells 189 -> 21, 10007 60 -> 21, 27000 42 -> 31, but 59000
-// 38 -> 52, where it is left out; Rusanov 45 -> 14, 25 -> 14, 22 -> 14 and 26
-// -> 20.
+// this (4 pieces, 400 steps in): HLL, 1000 cells 126 -> 21, 10007 47 -> 21, 27000
+// 35 -> 32, but 59000 39 -> 52, where it is left out; Rusanov 38 -> 13, 23 -> 13,
+// 25 -> 13 and 29 -> 18.
 constexpr ResShape RES_SHAPES2[3] = {{256, 16}, {256, 32}, {256, 64}};  // HLL: the first two
 
 void plan_resident(hes_solver* h) {
@@ -1205,8 +1205,9 @@ int hes_solver_team(hes_solver* h, const long long* wait_us, int* workgroups) {
   return HES_OK;
 }
 
-// Time `reps` launches of the step kernel alone on the solver's stream (HIP
-// events bracket exactly these launches).  The state advances by reps steps.
+// Time `reps` steps on the solver's stream: the launch that takes them all (with
+// the clearing of its message slots, 2 us), or the launches of the step kernels
+// alone, captured beforehand.  The state advances by reps steps.
 int hes_solver_time_steps(hes_solver* h, long long reps, float* elapsed_ms) {
   if (!h || !elapsed_ms) return fail(HES_ERR_ARG, "null argument");
   if (!h->has_state) return fail(HES_ERR_ARG, "no state set");

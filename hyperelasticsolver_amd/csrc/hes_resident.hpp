@@ -3,7 +3,7 @@
 //
 // A step needs the maximum CFL speed of the whole state, so a launch per step
 // (k_step) streams every state through memory and pays a launch and its ramp
-// per step: 5.4 us per step at 1000 cells (Rusanov), 20.4 us at 2^18, of which
+// per step: 5.5 us per step at 1000 cells (Rusanov), 20.1 us at 2^18, of which
 // the arithmetic is 2 and 4.  Here a team of workgroups, all resident at once,
 // holds the problem: one cell per lane in registers for the whole run.
 //
@@ -28,12 +28,15 @@
 // has: the launch then ends without a result and the caller's input is whole
 // (results go to another buffer, and only after the last wait).
 //
-// Measured (two phases: see plan_resident), single phase, us per step, one launch per step against this:
-// 1000 cells 5.4 -> 3.4 (Rusanov) and 6.0 -> 3.7 (HLL), 30011 cells 7.2 -> 3.7
-// and 7.9 -> 3.5, 2^18 cells 20.4 -> 9.4 and 19.5 -> 11.8.  What is left: the
-// chain of dependent FP64 operations of one cell (2 us, a wave alone on its
-// SIMD), the team's maximum (1.3 us for 5 workgroups, 2.1 us for 256), and
-// from two waves per SIMD on the FP64 issue rate (0.95 us per tile and SIMD).
+// Measured (two phases: see plan_resident), single phase, 65 pieces, us per
+// step, one launch per step (replayed from a graph) against this: 1000 cells
+// 5.5 -> 3.6 (Rusanov) and 6.2 -> 3.8 (HLL), 30011 cells 7.7 -> 4.0 and 8.5 ->
+// 3.8, 2^18 cells 20.1 -> 9.4 and 21.6 -> 11.8.  What is left: the chain of
+// dependent FP64 operations of one cell (2.2 us Rusanov, 2.9 HLL: one workgroup,
+// which exchanges nothing), the team's exchange (1.1 us more with 2 workgroups,
+// 1.4 with 5, 2.2 with 256; with HLL, whose mid state falls into the wait, 0.8 to
+// 0.9), and from two waves per SIMD on the FP64 issue rate (0.95 us per tile and
+// SIMD).
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -238,7 +241,7 @@ __device__ __forceinline__ ResOut resident_run1(const ResTeam& a, const MatDev& 
                                                 Hook hook = Hook()) {
   constexpr int NC = 14, W = BLK / 64, NT = W * T;
   constexpr bool HOOK = !std::is_same<Hook, ResNoHook>::value;
-  constexpr bool LATE_FLUX = T == 1 && BLK < 1024;
+  constexpr bool LATE_FLUX = T == 1;
   __shared__ double edge[2][NT][2][NC];  // new first and last updated cell of every tile, by parity
   __shared__ double red[2][W];           // every wave's maximum, by parity
   __shared__ double mine_out[2][RES_HALO][NC], theirs[2][RES_HALO][NC];

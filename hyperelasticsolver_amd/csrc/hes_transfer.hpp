@@ -3,8 +3,8 @@
 //
 // A copy into pageable memory runs at the rate of one host thread that copies
 // out of the runtime's staging memory and takes the page faults of a fresh
-// array (9 GB/s; 52 ms for 2^22 cells of 14 components, whose 400 Rusanov
-// steps take 72).  A large state is therefore cut into pieces, and several
+// array (9 GB/s; 47 to 52 ms for 2^22 cells of 14 components, whose 400 Rusanov
+// steps take 72; 10.5 ms as here, 45 GB/s).  A large state is therefore cut into pieces, and several
 // threads each let a kernel write a piece into page-locked memory of their
 // own, in the host's order, and copy it out.
 #pragma once

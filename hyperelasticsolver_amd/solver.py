@@ -182,7 +182,8 @@ class Solver:
         return team(lib().hes_solver_team, self._h, wait_us)
 
     def time_steps(self, reps):
-        """GPU time (ms) of `reps` back-to-back steps, replayed from one captured graph."""
+        """GPU time (ms) of `reps` back-to-back steps: of the one launch that takes
+        them all, or of their launches, replayed from one captured graph."""
         ms = ctypes.c_float()
         check(lib().hes_solver_time_steps(self._h, int(reps), ctypes.byref(ms)))
         return ms.value

@@ -117,10 +117,12 @@ int hes_solver_set_pressure_relaxation(hes_solver* h, double tau);
  * are the same bits either way. */
 int hes_solver_team(hes_solver* h, const long long* wait_us, int* workgroups);
 
-/* Time `reps` back-to-back steps (the step kernels and nothing else) with HIP
- * events on the solver stream; the state advances by reps steps.  The steps
- * are captured into one graph before the first event (as hes_solver_run
- * replays them), so the timed region holds only the graph's launch. */
+/* Time `reps` back-to-back steps with HIP events on the solver stream; the state
+ * advances by reps steps.  Where the steps of a run are one launch, that launch
+ * is timed, with the clearing of the words its workgroups exchange (about 2 us).
+ * Else the steps are captured into one graph before the first event (as
+ * hes_solver_run replays them), so the timed region holds only the graph's
+ * launch: the step kernels and nothing else. */
 int hes_solver_time_steps(hes_solver* h, long long reps, float* elapsed_ms);
 
 /* Measured HBM bandwidth of a plain device copy of `bytes` bytes (read plus
@@ -129,8 +131,8 @@ int hes_solver_time_steps(hes_solver* h, long long reps, float* elapsed_ms);
 int hes_copy_bandwidth(long long bytes, int reps, double* gbs);
 
 /* ---- Batched solver: many independent 1D problems of uneven length (the
- *      reference runs one problem per process, main.jl:130-152) advanced with
- *      one launch per step.  Problem p has ncells[p] >= 3 cells, its own
+ *      reference runs one problem per process, main.jl:130-152) advanced
+ *      together.  Problem p has ncells[p] >= 3 cells, its own
  *      materials (nphase blocks of 8), CFL number, dx and hence its own dt
  *      (main.jl:204-214 per problem) and frozen end cells.  The packed state
  *      is ncomp x sum(ncells), problems one after another (Julia layout). */
@@ -154,22 +156,24 @@ int hes_batch_get_state(hes_batch* h, double* Q_host);
 int hes_batch_get_times(hes_batch* h, double* t, long long* steps);
 /* Per-problem end time (main.jl:202 `while t < T`), NULL for none. */
 int hes_batch_set_t_end(hes_batch* h, const double* t_end);
-/* Launch shape: block of 64 or 256 threads; xcd != 0 deals consecutive blocks
+/* Launch shape of a launch per step: block of 64 or 256 threads; xcd != 0 deals consecutive blocks
  * to one XCD; tiles_per_wave (1..64) adjacent tiles of 62 cells per wave in
  * turn (a grid of ceil(tiles / tiles_per_wave) waves, each lane taking that
- * many cells). */
+ * many cells).  It does not enter a mode-1 run in one launch. */
 int hes_batch_set_launch(hes_batch* h, int block, int xcd, int tiles_per_wave);
 /* Advance every problem by `steps` steps.  mode 0: one launch per step;
  * 1: the whole step loop at once: one launch in which a team of workgroups
- * holds each problem on the chip (one phase, problems of up to about 60000
- * cells), else captured in one hipGraph and launched once;
+ * holds each problem on the chip (one phase, every problem of up to about
+ * 123000 cells; not for thousands of problems of a few tens of cells, where a
+ * launch per step is faster), else captured in one hipGraph and launched once;
  * 2: one launch per problem per step (the per-problem loop). */
 int hes_batch_run(hes_batch* h, long long steps, int mode, float* elapsed_ms);
 /* As hes_solver_team, for mode 1; *workgroups counts all problems' teams. */
 int hes_batch_team(hes_batch* h, const long long* wait_us, int* workgroups);
 /* Time every launch shape (block 64/256 x XCD order on/off x 1, 2 or 4 tiles
- * per wave) for `steps` steps on the current state (which is restored
- * afterwards) and keep the fastest. */
+ * per wave) of a launch per step (mode 0) for `steps` steps on the current state
+ * (which is restored afterwards) and keep the fastest for mode 0, and for mode 1
+ * where it is not one launch (hes_batch_team tells). */
 int hes_batch_autotune(hes_batch* h, int steps, int* block, int* xcd, int* tiles_per_wave,
                        float* ms_per_step);
 
