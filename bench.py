@@ -164,7 +164,10 @@ def batched_problem(seed=4):
 
 
 def time_batched(steps, loop_steps=5, eager_only=False):
-    """eager_only: the step kernels launched one by one with the default launch
+    """The graph-mode run (one launch for all steps of problems that fit the chip:
+    its states stay on the chip, so it has no fraction of the memory rate)
+    beside the per-problem loop and, in `autotune`, the best launch per step.
+    eager_only: the step kernels launched one by one with the default launch
     shape (no autotuning, no captured graph, no per-problem loop), for kernel
     counters."""
     from hyperelasticsolver_amd.batched import Batch
@@ -183,7 +186,8 @@ def time_batched(steps, loop_steps=5, eager_only=False):
                     "ms_per_step": ms / steps}
         tuned = b.autotune(steps=3)
         b.run(2, mode="graph")                     # warm-up
-        ms_graph = b.run(steps, mode="graph")       # whole loop in one hipGraph launch
+        ms_graph = b.run(steps, mode="graph")       # the whole loop at once
+        team = b.team()
         ms_loop = b.run(loop_steps, mode="loop")    # one launch per problem per step
         Q = b.get_state()
     if not np.all(np.isfinite(Q)):
@@ -192,7 +196,9 @@ def time_batched(steps, loop_steps=5, eager_only=False):
     loop_per_step = ms_loop / loop_steps
     return {"value": total * steps / (ms_graph / 1e3), "unit": "cell-updates/s",
             "problems": len(ncells), "cells": total, "steps": steps, "ms_per_step": per_step,
-            "hbm_frac": BYTES_PER_CELL_1PH * total / (per_step / 1e3) / 1e9 / HBM_PEAK_GBS,
+            "one_launch_workgroups": team,
+            "hbm_frac": None if team else
+            BYTES_PER_CELL_1PH * total / (per_step / 1e3) / 1e9 / HBM_PEAK_GBS,
             "loop_ms_per_step": loop_per_step, "speedup_vs_one_problem_per_launch": loop_per_step / per_step,
             "autotune": tuned}
 
@@ -251,8 +257,8 @@ ADJOINT_MODES = ("graph_sparse", "graph_dense", "eager_sparse", "eager_dense")
 
 def time_adjoint(n=1 << 18, steps=2000, every=50, modes=ADJOINT_MODES):
     """(forward + adjoint) / forward: the plain forward is the solver's step
-    loop on the same problem (its steps replayed from one captured graph, as
-    the adjoint's graph modes replay theirs); the adjoint run is its
+    loop on the same problem (one launch for all its steps, as the adjoint's
+    first pass takes them); the adjoint run is its
     checkpointed forward pass plus the reverse pass (recompute + reverse
     steps).  Reported for each launch mode, with zero-tile skipping (the
     default) and without it (every tile of every reverse step evaluated)."""
@@ -304,8 +310,8 @@ def time_batched_adjoint(nprob=256, lo=1024, hi=8192, steps=2000, every=50, seed
     ln 8192))) cells, (rho0, c0, b0) of each scaled by U(0.8, 1.2), two seeded
     pieces split at x = 1/2, 2000 Rusanov steps, checkpoints every 50, each
     problem's target from a run with its b0 * 1.05 and c0 * 0.97.  The plain
-    forward is the batched solver's step loop on the same problems (one
-    captured graph); the adjoint run is the batched adjoint's checkpointed
+    forward is the batched solver's step loop on the same problems (one launch
+    for all its steps); the adjoint run is the batched adjoint's checkpointed
     forward pass plus its reverse pass (graph modes: each replayed from one
     captured graph; eager modes: kernels launched one by one)."""
     from hyperelasticsolver_amd.EquationsOfState import Barton2009
