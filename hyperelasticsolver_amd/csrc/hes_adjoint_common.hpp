@@ -281,11 +281,10 @@ constexpr int seg_cells(int block) { return block / 64 * TILE + 2; }  // of a wo
 constexpr int seg_own(int block) { return seg_cells(block) - 2 * SEG_STEPS; }  // without the halos
 // Threads of a workgroup: beside the reverse steps the larger one, whose halos
 // cost 11% (reverse pass, ms, 256 / 512 threads: 2^18 cells without skipping
-// 70.8 / 69.3, 30000 cells 5.14 / 4.76, 16 small problems 5.66 / 5.32, 256
-// larger ones 239 / 234, 1000 small ones 18.4 / 18.5); the smaller one where
-// workgroups without a cotangent near them end at once (2^18 cells 26.6 /
-// 27.8) and above the chip's size (500000 cells 7.0 / 7.3); 1024 is no better
-// than 512 and slower for many small problems (20.3).
+// 70.8 / 69.3, 30000 cells 5.14 / 4.76); the smaller one where workgroups
+// without a cotangent near them end at once (2^18 cells 26.6 / 27.8) and above
+// the chip's size (500000 cells 7.0 / 7.3).  A batch takes fewer threads and
+// steps.
 constexpr int SEG_BLOCK = 256, SEG_BLOCK_BESIDE = 512;
 struct SegCtx {
   const double* Q;   // state s (14 rows)
@@ -293,7 +292,7 @@ struct SegCtx {
   const unsigned long long* lmax;  // of state s + k at lmax[k * stride]
   long long* istar;  // of state s + k at istar[k * stride] (find)
   long long stride, pitch, lo, hi, o0, o1;  // the problem's cells, this workgroup's
-  int halo, steps, find;
+  int halo, steps, find;  // halo: at least `steps`, or 0 for a whole problem
   double cfl;
 };
 template <int BLK>

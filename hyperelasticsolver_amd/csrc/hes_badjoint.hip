@@ -253,17 +253,27 @@ __global__ void k_badj_nocell(long long* __restrict__ istar, long long m) {
 }
 
 // States s + 1 .. s + steps of every problem from state s (segment_run), a
-// workgroup per entry of the table.  Reverse pass of 256 problems of 1024 ..
-// 8192 cells, the recompute in a launch per step against this: 249 -> 234 ms
-// (the reverse steps, one wave per SIMD, are what it waits for).  Where every
-// problem is short (two tiles at most) a launch is SEG_STEPS_SHORT steps: long
-// launches of many workgroups keep the reverse steps from the SIMDs, and the
-// short problems' states are a small part of what a step moves (reverse pass
-// over 300 steps, ms, a launch per step / 3 steps / 25: 4000 problems of 20 ..
-// 120 cells 19.1 / 19.0 / 19.8, 16000 of 10 .. 62 46.1 / 46.7 / 47.9, 16000 of
-// 63 .. 124 99.6 / 97.6 / 99.3; longer ones lose: 1000 of 100 .. 900 22.9 /
-// 24.1 / 23.1).
-constexpr int SEG_STEPS_SHORT = 3;
+// workgroup per entry of the table.  The reverse steps run beside this, one
+// wave per SIMD, so a launch has to leave them room: short, of small workgroups
+// whose halos are as wide as its steps are many.  Reverse pass of 300 steps, ms,
+// by threads and steps of a launch, beside one launch of a wave per tile and
+// step:
+//                                          a step  128, 2  256, 3  512, 25
+//   4000 problems of 20 .. 120 cells         18.8    18.8    19.1     20.4
+//   the same and 5 of 5000                   19.7    19.6    20.1     21.5
+//   16000 of 10 .. 62                        45.4    45.4    47.5     47.7
+//   1000 of 100 .. 900                       22.6    22.1    22.7     22.6
+//   400 of 20 .. 120, 40 of 2000              7.3     7.2     7.4      8.0
+//   40 of 4000 .. 9000                       12.8    12.4    12.4     12.9
+//   1000 of 1000 .. 1500                     34.8    33.0    32.8     32.6
+//   256 of 1024 .. 8192                      48.1    46.7    46.0     45.6
+// So 128 threads where a problem has 16 tiles or fewer on average, else 256.
+struct BSegShape {
+  int block, steps;
+};
+inline BSegShape bseg_shape(long long tiles, long long problems) {
+  return tiles <= 16 * problems ? BSegShape{128, 2} : BSegShape{256, 3};
+}
 struct BSeg {
   long long lo, hi, o0, o1;  // the problem's cells, the workgroup's
   int p, halo;
@@ -286,12 +296,6 @@ void k_badj_segment(BAdjSegArgs a) {
   const int p = cload(&g->p);
   c.lmax += p;
   segment_run<BLK>(c, uniform_mat(a.mats + p));
-}
-// Threads of its workgroups: the fewest that hold the longest problem whole.
-int seg_block_of(long long longest) {
-  for (int block = 64; block < SEG_BLOCK_BESIDE; block *= 2)
-    if (longest <= seg_cells(block)) return block;
-  return SEG_BLOCK_BESIDE;
 }
 
 // Argmax cell of the CFL speed of every (state, problem) from the per-tile
@@ -748,7 +752,8 @@ struct hes_badjoint {
   BResItem* items = nullptr;
   unsigned long long* comm = nullptr;
   BSeg* segs = nullptr;  // the recompute's workgroups
-  int nsegs = 0, seg_block = 0, seg_steps = 0;  // threads of each; steps of a launch
+  BSegShape seg_shape = {0, 0};
+  int nsegs = 0;
   BTile* tiles = nullptr;
   int* tfirst = nullptr;
   long long* offs = nullptr;
@@ -936,17 +941,13 @@ hipError_t brecord_backward(hes_badjoint* h) {
   hipStream_t st2 = h->stream2;
   HIP_TRY_E(hipEventRecord(h->ev_fork, st));
   HIP_TRY_E(hipStreamWaitEvent(st2, h->ev_fork, 0));
-  void (*segment)(BAdjSegArgs) = h->seg_block == 64    ? k_badj_segment<64>
-                                 : h->seg_block == 128 ? k_badj_segment<128>
-                                 : h->seg_block == 256 ? k_badj_segment<256>
-                                                       : k_badj_segment<SEG_BLOCK_BESIDE>;
   auto recompute = [&](long long c) -> hipError_t {
     const long long s0 = c * h->every;
     const long long end = std::min(s0 + h->every, h->nsteps);
     const int buf = (int)(c & 1);
     // each recomputed state keeps its sound speeds in row 14 of its slot,
     // as the checkpoints do: the reverse step reads its face speeds there
-    for (long long s = s0; s + 1 < end; s += h->seg_steps) {
+    for (long long s = s0; s + 1 < end; s += h->seg_shape.steps) {
       BAdjSegArgs a;
       std::memset((void*)&a, 0, sizeof(a));
       a.segs = h->segs;
@@ -956,9 +957,10 @@ hipError_t brecord_backward(hes_badjoint* h) {
       a.c.lmax = h->lmax + s * h->P;
       a.c.stride = h->P;
       a.c.pitch = h->pitch;
-      a.c.steps = (int)std::min<long long>(h->seg_steps, end - 1 - s);
+      a.c.steps = (int)std::min<long long>(h->seg_shape.steps, end - 1 - s);
       a.c.cfl = h->cfl;
-      hipLaunchKernelGGL(segment, dim3((unsigned)h->nsegs), dim3((unsigned)h->seg_block), 0, st2, a);
+      hipLaunchKernelGGL(h->seg_shape.block == 128 ? k_badj_segment<128> : k_badj_segment<256>,
+                         dim3((unsigned)h->nsegs), dim3((unsigned)h->seg_shape.block), 0, st2, a);
     }
     const int cnt = (int)(end - s0);
     hipLaunchKernelGGL(k_badj_lam, dim3(blocks_of((long long)cnt * h->P, 64)), dim3(64), 0, st2,
@@ -1102,15 +1104,14 @@ int hes_badjoint_create(hes_badjoint** out, int nproblems, const long long* ncel
     h->dev = dev;
     h->cus = cus;
   }
-  h->seg_block = seg_block_of(*std::max_element(ncells, ncells + nproblems));
-  h->seg_steps = h->seg_block <= 128 ? SEG_STEPS_SHORT : SEG_STEPS;
+  h->seg_shape = bseg_shape(h->ntiles, nproblems);
   std::vector<BSeg> segs;
   for (int p = 0; p < nproblems; ++p) {
     const long long lo = h->offs_h[p], hi = h->offs_h[p + 1];
-    const bool whole = hi - lo <= seg_cells(h->seg_block);
-    const int per = whole ? seg_cells(h->seg_block) : seg_own(h->seg_block);
+    const int cells = seg_cells(h->seg_shape.block);
+    const int halo = hi - lo <= cells ? 0 : h->seg_shape.steps, per = cells - 2 * halo;
     for (long long c = lo; c < hi; c += per)
-      segs.push_back({lo, hi, c, std::min(c + per, hi), p, whole ? 0 : SEG_STEPS});
+      segs.push_back({lo, hi, c, std::min(c + per, hi), p, halo});
   }
   h->nsegs = (int)segs.size();
   const BResPlan pl = bres_plan(h->offs_h, h->cus, NQ, false, true);

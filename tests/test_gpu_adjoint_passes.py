@@ -91,12 +91,13 @@ def test_recomputed_states_change_nothing(n):
 
 
 # few workgroups (a tile per wave), more than the chip holds at once (two), a
-# problem that does not fit and runs step by step; then the last lengths that
-# each size of the recompute's workgroups holds, and waves past a short
-# problem's end (its last cell in a wave's first or last lane)
+# problem that does not fit and runs step by step; then the lengths that a
+# workgroup of the recompute holds (126 cells alone, 122 each; with longer
+# problems 250 and 244), one more, and waves past a problem's end (its last cell
+# in a wave's first or last lane)
 BATCHES = [[3, 62, 250, 251, 498, 499, 896, 897, 1000, 9000], [8000] * 40 + [5, 700], [123393, 300],
-           [3, 62, 63, 64], [3, 65, 125, 126], [64, 127, 187, 188, 189, 250], [63, 125, 126, 497, 498],
-           [510, 511, 512, 513, 899, 946, 947]]
+           [3, 62, 63, 64], [3, 65, 125, 126], [123, 124, 127, 128, 129, 183, 184, 185], [243, 244, 245, 247],
+           [20] * 30 + [365, 366, 367, 2000], [1000, 1001, 1200, 1452, 1453, 251, 250, 249, 5000]]
 
 
 @pytest.mark.parametrize("which", range(len(BATCHES)))
